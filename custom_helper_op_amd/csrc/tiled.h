@@ -1276,13 +1276,20 @@ constexpr int backward_record_words() {
   const int w = NV == 1 ? (rec > list ? rec : list) : rec + list;
   return (w + 3) / 4 * 4;
 }
+// The list of a window move between two depths of a chunk, whose records are in use then.
+template <int VEC, int LPP, bool SIX = false>
+constexpr int backward_list_words() {
+  using WN = Window<VEC, LPP, SIX>;
+  return LPP > 1 && WN::SLOTS * 2 > 4 * WN::C ? WN::SLOTS * 2 : 0;
+}
 template <int VEC, int LPP, int NV, bool SIX = false>
 constexpr int backward_lds_words() {
   using WN = Window<VEC, LPP, SIX>;
   // records (or list), windows, one cell (4 texels x C) staged on its way to memory, and for
   // narrow pixels one claim word per window slot
+  // and, where that cell's place is too small for it, the list of a move inside a chunk
   return backward_record_words<VEC, LPP, NV, SIX>() + NV * WN::SLOTS * WN::STRIDE + 4 * WN::C +
-         (LPP <= kClaimLanes ? WN::SLOTS : 0);
+         (LPP <= kClaimLanes ? WN::SLOTS : 0) + backward_list_words<VEC, LPP, SIX>();
 }
 
 // Minimum over the 64 lanes, in registers: four DPP steps reduce each row of 16 lanes,
@@ -1298,8 +1305,9 @@ __device__ __forceinline__ int wave_min(int v) {
 
 // Moves the window of one view to origin (ny, nx): every texel that falls outside the new
 // window is written out with dense global atomics (C consecutive floats per texel, 64/C
-// texels per instruction) and its slot is cleared.  Uniform control flow.
-template <int VEC, int LPP, bool SIX = false>
+// texels per instruction, UN instructions per round: their LDS reads go out together) and its
+// slot is cleared.  Uniform control flow.
+template <int VEC, int LPP, bool SIX = false, int UN = 4>
 __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, float *data,
                                             int *list, float *gview, int srcW, int lane) {
   using WN = Window<VEC, LPP, SIX>;
@@ -1324,7 +1332,6 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, fl
     if (count > 0) {
       wave_sync();
       constexpr int EPI = 64 / WN::C;  // texels per instruction
-      constexpr int UN = 4;            // instructions per round: their LDS reads go out together
       const int sub_e = lane / WN::C, j = lane - sub_e * WN::C;
       const int2 *pairs = reinterpret_cast<const int2 *>(list);
       for (int e0 = 0; e0 < count; e0 += UN * EPI) {
@@ -1529,9 +1536,9 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
     for (int i = 0; i < VEC; ++i) v[k][i] = 0.f;
 }
 
-// Cells that stick out of the window (samples of consecutive depths jumping far apart, as
-// they do close to the cameras) go to memory directly.  Uniform control flow: `m` has the
-// lane bits of every pixel with such a cell (`mine` for the caller's own lanes).  One pixel
+// Cells that no window position covers (the tile's pixels of one depth further apart than the
+// window is wide, on strongly magnified views) go to memory directly.  Uniform control flow:
+// `m` has the lane bits of every pixel with such a cell (`mine` for the caller's own lanes).  One pixel
 // at a time, its lanes lay the four tap images out in LDS as two rows of two adjacent texels
 // and the whole wave adds each row as a dense run of 2*C consecutive floats.  Added lane by
 // lane from the registers, each 16-byte chunk of a texel would carry one float per
@@ -1626,12 +1633,7 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // A compile-time flag: the loop around the kernel's body costs the wide instantiations
 // registers they do not have (the 32-channel kernel spills with it).
 // WIDE: the kernel as it is without the slimming of lean_backward: three waves per SIMD and, for
-// 32 channels, the 8 x 8 window.  For sweeps whose samples of consecutive hypotheses land many
-// texels apart (wide baselines, hypotheses close to the cameras) the two rows more are worth
-// more than the fourth wave: fewer cells stick out of the window and go to memory on their
-// own, and such launches are bound by those atomics, not by latency (six source views with
-// 15-degree rotations and depths from 0.5: 18.9 ms against 20.6 ms slimmed).  The launcher
-// decides (tiled_launch.inc).
+// 32 channels, the 8 x 8 window.  The launcher decides (tiled_launch.inc).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool DG = true,
           bool PV = (CORR == 1), bool VLOOP = false, bool WIDE = false>
 __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) void backward_kernel(const Args<S> a,
@@ -1659,8 +1661,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   float *s_stage = s_data + NV * WN::SLOTS * WN::STRIDE;
   int *s_tags = reinterpret_cast<int *>(s_stage + 4 * WN::C);  // narrow pixels: claim words
   static_assert(LPP > kClaimLanes || NV == 1, "one set of claim words: one view per workgroup");
+  int *s_own_list = s_tags + (LPP <= kClaimLanes ? WN::SLOTS : 0);
+  // (LPP == 1: the records are in registers)
+  int *s_move_list = LPP == 1                                         ? s_list
+                     : backward_list_words<VEC, LPP, kSix>() > 0 ? s_own_list
+                                                                 : reinterpret_cast<int *>(s_stage);
   // CORR 3 only: reference rows, sample rows
-  float *s_v3 = s_stage + 4 * WN::C + (LPP <= kClaimLanes ? WN::SLOTS : 0);
+  float *s_v3 = reinterpret_cast<float *>(s_own_list + backward_list_words<VEC, LPP, kSix>());
   static_assert(CORR != 3 || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
   const float base = per_voxel_depth ? 0.f : a.base_plane[t.pix];
   float ref[VEC];
@@ -1757,6 +1764,41 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // the pixel's depth gradients: the first view of a group that holds them all stores, the
   // later ones add (same lane, same address); several groups add atomically
   const bool dg_store = g.ngroups == 1 && vi == 0, dg_own = g.ngroups == 1;
+  // Runs of a spread chunk that end now (`fire`: whole pixels; called by all lanes).  The
+  // samples of such a chunk land so far apart (hypotheses close to the cameras, wide baselines,
+  // few planes far apart) that its cells do not fit the window together, but the runs that end
+  // at one depth lie about as close to each other as the tile's pixels do, so the window moves
+  // to them: neighbouring pixels share most of their texels (2 x 4 pixels: about 15 instead of
+  // 32 taps), which then leave as one dense run of atomics each, and the rate of the atomics is
+  // what bounds such a launch (32 channels, six views, depths from 0.5, 15-degree rotations:
+  // 18.5 -> 13.3 ms against every cell of such a chunk adding its four texels to memory by itself;
+  // minimum over two views, twelve planes from 1.7 to 16: 632 -> 395 us).  A cell that is still outside (pixels of one depth further apart
+  // than the window, on strongly magnified views) goes to memory by itself.
+  auto end_spread_runs = [&](int n, bool fire) __attribute__((always_inline)) {
+    // (the lane index as a value the compiler cannot see through: what the window's functions
+    // derive from it would be computed in front of all chunks and held through the depth loop)
+    int lane = t.lane;
+    if constexpr (LPP < 8) asm volatile("" : "+v"(lane));
+    const int cl = lane % LPP;
+    const int key = cell[n].y & 0x7fffffff;
+    bool in = WN::inside(key, oy[n], ox[n]);
+    if (__ballot(fire && !in) != 0ull) {
+      const int fh = key >> 16, fw = key & 0xffff;
+      const int ny = wave_min(fire ? fh : WN::kNone), nx = wave_min(fire ? fw : WN::kNone);
+      const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
+      const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
+      window_move<VEC, LPP, kSix, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
+                                  s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane);
+      in = WN::inside(key, oy[n], ox[n]);
+      const bool out = fire && !in;
+      const unsigned long long m = __ballot(out);
+      if (m != 0ull) {
+        flush_cells_to_memory<VEC, LPP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl);
+        if (out) cur[n] = -1;
+      }
+    }
+    if (fire) cell[n].y = in ? (key | WN::kInside) : key;
+  };
   wave_sync();
   for (int d0 = d_lo; d0 < d_hi; d0 += LPP) {
     // Depth hypothesis and valid-view count of lane (p, j)'s voxel: requested before the
@@ -1786,7 +1828,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     int2 r_cell[NV];
     float r_scl = 0.f;
     float4 r_wts[NV], r_dwt[NV];
-    bool chunk_out[NV];  // some cell of this chunk (or the open one) sticks out of the window
+    bool spread[NV];  // the cells of this chunk and the open ones do not fit the window together
     // Issue the loads of this chunk's cost_grad rows now, unconditionally, so that the
     // reprojection below overlaps their latency.  Through the caches: the workgroups of a
     // tile's views read the same rows (streamed, only about a third of the later reads found
@@ -1893,14 +1935,15 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
         }
         // The scatter window has to cover this chunk's cells and the cell still open from
         // the last chunk.  Usually it already does (one vote); otherwise it is centred on
-        // their bounding box, and whatever still sticks out is marked for the memory path.
+        // their bounding box.  A box larger than the window: the window follows the runs that
+        // end, depth by depth (end_spread_runs).
         const bool valid = hit.off >= 0;
         if (valid) {
           const unsigned fh = (unsigned)hit.key >> 16;
           ring_rows[n] |= (1u << WN::ring_row(fh)) | (1u << WN::ring_row(fh + 1u));
         }
         bool in_new = !valid || WN::inside(hit.key, oy[n], ox[n]);
-        chunk_out[n] = false;
+        spread[n] = false;
         if (__ballot(!(in_new && (cur[n] < 0 || cell[n].y < 0))) != 0ull) {
           int my = WN::kNone, mx = WN::kNone, My = -WN::kNone, Mx = -WN::kNone;
           if (valid) my = My = hit.key >> 16, mx = Mx = hit.key & 0xffff;
@@ -1911,13 +1954,16 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
           const int ny = wave_min(my), nx = wave_min(mx);
           const int hy = -wave_min(-My) + 1, hx = -wave_min(-Mx) + 1;  // last row / column used
           const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);  // slack
-          window_move<VEC, LPP, kSix>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0),
-                                nx - (sx > 0 ? sx / 2 : 0), s_data + n * WN::SLOTS * WN::STRIDE,
-                                s_list, gview[n], srcW, t.lane);
-          in_new = !valid || WN::inside(hit.key, oy[n], ox[n]);
-          const int ck = cell[n].y & 0x7fffffff;
-          cell[n].y = WN::inside(ck, oy[n], ox[n]) ? (ck | WN::kInside) : ck;
-          chunk_out[n] = __ballot((valid && !in_new) || (cur[n] >= 0 && cell[n].y >= 0)) != 0ull;
+          spread[n] = sy < 0 || sx < 0;
+          if (spread[n]) {
+            in_new = false;  // decided when the run ends
+            cell[n].y &= 0x7fffffff;
+          } else {
+            window_move<VEC, LPP, kSix>(oy[n], ox[n], ny - sy / 2, nx - sx / 2,
+                                  s_data + n * WN::SLOTS * WN::STRIDE, s_list, gview[n], srcW, t.lane);
+            in_new = true;
+            cell[n].y |= WN::kInside;
+          }
         }
         const int2 rec = make_int2(WN::kPacked ? (int)WN::pack_slots(hit.key) : 0,
                                    (valid && in_new) ? (hit.key | WN::kInside) : hit.key);
@@ -2000,16 +2046,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
       float dvox = 0.f;  // this lane's share of d(loss)/d(depth of this voxel)
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        if (chunk_out[n]) {  // uniform, and false for the whole chunk in the usual case
-          // runs that end at this depth on a cell outside the window: to memory, now
-          const bool fire_out = scl != 0.f && rec_off[n] >= 0 && rec_off[n] != cur[n] &&
-                                cur[n] >= 0 && cell[n].y >= 0;
-          const unsigned long long m = __ballot(fire_out);
-          if (m != 0ull) {
-            flush_cells_to_memory<VEC, LPP>(m, fire_out, cell[n].y, sg[n], s_stage, gview[n], srcW,
-                                            t.lane, t.cl);
-            if (fire_out) cur[n] = -1;
-          }
+        if (spread[n]) {  // uniform, and false for the whole chunk in the usual case
+          const bool fire = scl != 0.f && rec_off[n] >= 0 && rec_off[n] != cur[n] && cur[n] >= 0;
+          end_spread_runs(n, fire);
         }
       }
       // (one view per workgroup: a tap offset implies a non-zero factor, phase 1 reprojects
@@ -2061,7 +2100,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
           const float4 wt = rec_wt[n], dwt = rec_dwt[n];
           if (off >= 0) {
             if (off != cur[n]) {
-              // (a run whose cell sticks out of the window was closed by the uniform block
+              // (a run whose cell the window could not cover was closed by the uniform block
               // above, which left cur[n] = -1)
               // the run on the previous cell ends.  Start fetching the new cell's taps
               // first, then hand the old cell's image to the window while they arrive.
@@ -2170,12 +2209,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // the runs still open, then everything the windows hold
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
-    const bool out = cur[n] >= 0 && cell[n].y >= 0;
-    const unsigned long long m = __ballot(out);
-    if (m != 0ull)
-      flush_cells_to_memory<VEC, LPP>(m, out, cell[n].y, sg[n], s_stage, gview[n], srcW, t.lane,
-                                      t.cl);
-    if (cur[n] >= 0 && !out)
+    if (__ballot(cur[n] >= 0 && cell[n].y >= 0) != 0ull) end_spread_runs(n, cur[n] >= 0);
+    if (cur[n] >= 0)
       window_add<VEC, LPP, false, kSix>((unsigned)cell[n].x, cell[n].y, sg[n],
                            s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
   }
