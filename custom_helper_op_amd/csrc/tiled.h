@@ -1220,7 +1220,7 @@ struct Window {
   // LDS is 10 KB, so that sixteen workgroups fit a CU; four rows measured 2 % slower than eight
   // at equal occupancy, six sit between.  The ring index of a row is then a remainder, not a
   // mask.
-  static constexpr int ROWS = SIX ? 6 : (2 * TH > 8 ? 2 * TH : 8);
+  static constexpr int ROWS = SIX ? 6 : LPP == 16 ? 4 : (2 * TH > 8 ? 2 * TH : 8);
   static constexpr int COLS = 2 * TW > 8 ? 2 * TW : 8;
   static constexpr int SLOTS = ROWS * COLS;
   static constexpr bool kPow2Rows = (ROWS & (ROWS - 1)) == 0;
@@ -1608,12 +1608,13 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // than three).  Up to 32 bytes of scratch remain in two of those instantiations, outside the
 // depth loop: bf16 group-correlation backward 479 -> 462 us cold, 447 -> 417 us warm.
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false) {
-  return nv == 1 && !wide && ((lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
+  return nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
                      (lpp == 4 && corr <= 1 && reduce == 0) ||
                      (lpp == 2 && corr <= 1 && reduce == 0));
 }
 constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false) {
-  return lean_backward(nv, lpp, corr, reduce, wide) ? 4
+  return lpp == 16 && nv == 1                             ? 3
+         : lean_backward(nv, lpp, corr, reduce, wide) ? 4
          : nv == 1 && lpp <= 8                       ? 3
          : nv <= 2                                   ? 2
                                                      : 1;
