@@ -249,11 +249,9 @@ __device__ __forceinline__ void fold_groups(const float *ch, int sub, float *out
 #pragma unroll
     for (int c = 0; c < VEC / 4; ++c)
       out[c] = (ch[4 * c] + ch[4 * c + 1]) + (ch[4 * c + 2] + ch[4 * c + 3]);
-  } else {  // sub == 8 == VEC
-    float s = 0.f;
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) s += ch[c];
-    out[0] = s;
+  } else {  // sub == 8: two lanes of four channels, both left with the sum
+    static_assert(VEC == 4, "a group of eight is two lanes");
+    out[0] = dpp_add<0xB1>((ch[0] + ch[1]) + (ch[2] + ch[3]));  // quad_perm 1,0,3,2
   }
 }
 
@@ -267,22 +265,15 @@ __device__ __forceinline__ void store_groups(S *p, const float *v, int sub) {
     store_vec<S, VEC / 2, whole_lines(C / 2, B)>(p, v);
   } else if (sub == 4) {
     store_vec<S, VEC / 4, whole_lines(C / 4, B)>(p, v);
-  } else {
-    if constexpr (VEC >= 8) store_vec<S, VEC / 8, whole_lines(C / 8, B)>(p, v);
+  } else if (threadIdx.x & 1) {  // sub == 8: the group's second lane
+    store_vec<S, 1, whole_lines(C / 8, B)>(p, v);
   }
 }
 
-template <typename S, int VEC, bool STREAM>
-__device__ __forceinline__ void load_groups(const S *p, float *v, int sub) {
-  if (sub == 1) {
-    load_vec<S, VEC, STREAM>(p, v);
-  } else if (sub == 2) {
-    load_vec<S, VEC / 2, STREAM>(p, v);
-  } else if (sub == 4) {
-    load_vec<S, VEC / 4, STREAM>(p, v);
-  } else {
-    if constexpr (VEC >= 8) load_vec<S, VEC / 8, STREAM>(p, v);
-  }
+// Offset of lane `cl`'s first group in a row of group values (a group of eight: lanes 2g, 2g + 1).
+template <int VEC>
+__device__ __forceinline__ int group_offset(int cl, int sub) {
+  return sub == 8 ? cl >> 1 : cl * (VEC / sub);
 }
 
 // ---- shared front end of both kernels ---------------------------------------------------
@@ -471,6 +462,35 @@ __device__ __forceinline__ void better_pair(float &best, int &code) {
   best = take ? ob : best;
   code = take ? oc : code;
 }
+// A group of eight channels held by two lanes: the odd lane continues the even lane's sum over
+// its own four, in channel order (the result of the odd lane is the group's).
+__device__ __forceinline__ float continue_group(float sum, const float (&val)[4], int cl) {
+  const float head = dpp_move<0xA0>(sum);  // quad_perm 0,0,2,2
+  return (cl & 1) ? (((head + val[0]) + val[1]) + val[2]) + val[3] : sum;
+}
+// The maximum reduce of one accepted view: where a correlation group of this lane is larger than
+// the largest so far (strictly: the earliest view keeps a tie), it and its view are kept.  A
+// group's products are summed in channel order.  One branch on the group width per sample (the
+// width is a run-time value; picking the terms of every group by comparisons instead took, with
+// the wave per SIMD of forward_min_waves, 157 against 140 us on an f16 sweep of 32 channels in
+// eight groups, four views, 237 x 315 x 24).
+__device__ __forceinline__ void keep_larger_groups(float (&best)[4], int (&arg)[4], const float (&val)[4],
+                                                   int sub, int cl, int view) {
+  auto keep = [&](int i, float corr) __attribute__((always_inline)) {
+    if (best[i] < corr) best[i] = corr, arg[i] = view;
+  };
+  if (sub >= 4) {
+    float corr = ((val[0] + val[1]) + val[2]) + val[3];
+    if (sub == 8) corr = continue_group(corr, val, cl);
+    keep(0, corr);
+  } else if (sub == 2) {
+    keep(0, val[0] + val[1]);
+    keep(1, val[2] + val[3]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) keep(c, val[c]);
+  }
+}
 constexpr int kNoPair = 0x7fffffff;  // pair code: source group * 16 + reference group
 
 // The best (source group, reference group) pair of one accepted sample of one pixel, found
@@ -610,7 +630,10 @@ constexpr int forward_squares_words(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 
 // gathers of wide-baseline views (stress workload forward 5.17 -> 4.45 ms).  Three and four
 // views at four lanes per pixel: 102 -> 87 registers without scratch, five waves instead of
 // four (f16 cascade workload forward 122 -> 113 us cold); the other widths would spill.
+// MIN / MAX of four views: 129-131 registers left alone, 8 bytes of scratch at 128 and a fourth wave
+// (six views would spill 60 bytes and more: left alone).
 constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce) {
+  if (reduce != 0 && corr <= 1 && nv == 4 && lpp >= 2) return 4;
   if (corr > 1 || reduce != 0) return 1;
   return nv >= 5 ? 4 : (nv >= 3 && lpp == 4) ? 5 : 1;
 }
@@ -680,7 +703,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
   // pair; MEAN averages the views' maxima, MIN keeps the largest with (view, reference group,
   // source group) as its mask (cost_volume_kernels_gpu_v3.cu.cc:52-146, :148-262)
   const int OC = CORR == 1 ? a.groups : (CORR == 2 || CORR == 3) ? 1 : C;
-  const int gv = VEC / g.sub;  // output values per lane
+  const int goff = group_offset<VEC>(t.cl, g.sub);  // first of this lane's group values in a row
   // the cost rows of the per-channel ops (and the sample rows of the warp-only op) stream past
   // the caches where they cover whole lines
   constexpr bool kNtRows = whole_lines(VEC * LPP, (int)sizeof(S));
@@ -880,16 +903,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
               for (int c = 0; c < VEC; ++c)
                 if (acc[jj][c] > val[c]) acc[jj][c] = val[c], arg[jj][c] = n;
             } else {
-#pragma unroll
-              for (int gi = 0; gi < VEC; ++gi) {
-                if (gi * g.sub < VEC) {
-                  float corr = 0.f;
-#pragma unroll
-                  for (int c = 0; c < VEC; ++c)
-                    if (c >= gi * g.sub && c < (gi + 1) * g.sub) corr += val[c];
-                  if (acc[jj][gi] < corr) acc[jj][gi] = corr, arg[jj][gi] = n;
-                }
-              }
+              keep_larger_groups(acc[jj], arg[jj], val, g.sub, t.cl, n);
             }
           } else {
 #pragma unroll
@@ -927,10 +941,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
             store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc[jj]);
             store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * VEC, arg[jj]);
           } else {
-            store_groups<S, VEC, LPP>(out + t.cl * gv, acc[jj], g.sub);
-            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * gv, arg[jj]);
-            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + t.cl * gv, arg[jj]);
-            else store_ints<VEC / 4, whole_lines(VEC * LPP / 4, 4)>(mout + t.cl * gv, arg[jj]);
+            store_groups<S, VEC, LPP>(out + goff, acc[jj], g.sub);
+            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg[jj]);
+            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg[jj]);
+            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg[jj]);
           }
         } else {
           if (kcnt[jj] > 1) {
@@ -951,7 +965,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
 #pragma unroll
               for (int c = 0; c < VEC; ++c) grp[c] = dflt;
             }
-            store_groups<S, VEC, LPP>(out + t.cl * gv, grp, g.sub);
+            store_groups<S, VEC, LPP>(out + goff, grp, g.sub);
           }
         }
       }
@@ -1077,17 +1091,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
               for (int c = 0; c < VEC; ++c)
                 if (acc[c] > val[c]) acc[c] = val[c], arg[c] = n;
             } else {
-              // groups of sub consecutive channels, summed in channel order from zero
-#pragma unroll
-              for (int gi = 0; gi < VEC; ++gi) {
-                if (gi * g.sub < VEC) {
-                  float corr = 0.f;
-#pragma unroll
-                  for (int c = 0; c < VEC; ++c)
-                    if (c >= gi * g.sub && c < (gi + 1) * g.sub) corr += val[c];
-                  if (acc[gi] < corr) acc[gi] = corr, arg[gi] = n;
-                }
-              }
+              keep_larger_groups(acc, arg, val, g.sub, t.cl, n);
             }
             ++k;
             continue;
@@ -1140,10 +1144,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
             store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc);
             store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * VEC, arg);
           } else {
-            store_groups<S, VEC, LPP>(out + t.cl * gv, acc, g.sub);
-            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * gv, arg);
-            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + t.cl * gv, arg);
-            else store_ints<VEC / 4, whole_lines(VEC * LPP / 4, 4)>(mout + t.cl * gv, arg);
+            store_groups<S, VEC, LPP>(out + goff, acc, g.sub);
+            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg);
+            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg);
+            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg);
           }
         }
         continue;
@@ -1181,7 +1185,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
 #pragma unroll
             for (int c = 0; c < VEC; ++c) grp[c] = dflt;
           }
-          store_groups<S, VEC, LPP>(out + t.cl * gv, grp, g.sub);
+          store_groups<S, VEC, LPP>(out + goff, grp, g.sub);
         }
       }
     }
@@ -1220,6 +1224,11 @@ struct Window {
   // LDS is 10 KB, so that sixteen workgroups fit a CU; four rows measured 2 % slower than eight
   // at equal occupancy, six sit between.  The ring index of a row is then a remainder, not a
   // mask.
+  // Sixteen lanes per pixel (64 channels, 2 x 2 pixels): a slot is 256 bytes, and with eight rows
+  // the window alone held a CU to seven workgroups (20.5 KB each).  Four rows (12.5 KB) let
+  // thirteen in; together with the slimming of lean_backward the gradients run three waves
+  // per SIMD instead of two (group correlation, four views, 254 x 319 x 16, training pass 2.68
+  // -> 1.61 ms; warped features, four views, 73 x 96 x 161: 1218 -> 1045 us).
   static constexpr int ROWS = SIX ? 6 : LPP == 16 ? 4 : (2 * TH > 8 ? 2 * TH : 8);
   static constexpr int COLS = 2 * TW > 8 ? 2 * TW : 8;
   static constexpr int SLOTS = ROWS * COLS;
@@ -1607,6 +1616,8 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // with them the kernels spilled 44-68 bytes around the depth loop and four waves were slower
 // than three).  Up to 32 bytes of scratch remain in two of those instantiations, outside the
 // depth loop: bf16 group-correlation backward 479 -> 462 us cold, 447 -> 417 us warm.
+// Sixteen lanes per pixel (64 channels): slimmed, all of them, to three waves (164-222 registers
+// left alone, 132-164 slimmed; LDS holds them to 13 workgroups per CU, see Window::ROWS).
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false) {
   return nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
                      (lpp == 4 && corr <= 1 && reduce == 0) ||
@@ -1699,7 +1710,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // 3: CostVolumeV3, one upstream gradient per voxel that flows through the best group pair
   constexpr bool kVoxelGrad = CORR == 2 || CORR == 3;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
-  const int gv = VEC / g.sub;
+  const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
+  const int goff = CORR == 1 ? group_offset<VEC>(t.cl, g.sub) : t.cl * VEC;
   const int d_lo = t.d_lo, d_hi = t.d_hi;
   // upstream-gradient rows fetched ahead; the MIN reduce stages the mask rows beside them
   constexpr int PFMAX = (REDUCE || kLean) ? 4 : 8;
@@ -1758,10 +1770,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   }
   const S *cg_lane =
       CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + t.cl * VEC
-                : a.cost_grad + t.pix * D * OC + (kVoxelGrad ? 0 : t.cl * (CORR ? gv : VEC));
+                : a.cost_grad + t.pix * D * OC + (kVoxelGrad ? 0 : goff);
   const int32_t *cnt_src = CORR == 4 ? a.mask_in + t.pix * D * N + t.view0
                                      : a.mask_in + t.pix * D * mask_w;
-  const int32_t *mask_lane = cnt_src + t.cl * (CORR ? gv : VEC);  // this lane's part of a mask row
+  const int32_t *mask_lane = cnt_src + goff;  // this lane's part of a mask row
   // the pixel's depth gradients: the first view of a group that holds them all stores, the
   // later ones add (same lane, same address); several groups add atomically
   const bool dg_store = g.ngroups == 1 && vi == 0, dg_own = g.ngroups == 1;
@@ -1855,8 +1867,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
         };
         if (g.sub == 1) group_rows(std::integral_constant<int, VEC>());
         else if (g.sub == 2) group_rows(std::integral_constant<int, VEC / 2>());
-        else if (g.sub == 4) group_rows(std::integral_constant<int, VEC / 4>());
-        else if constexpr (VEC >= 8) group_rows(std::integral_constant<int, VEC / 8>());
+        else group_rows(std::integral_constant<int, 1>());
       }
 #pragma unroll
       for (int jj = 0; jj < PF; ++jj) {
