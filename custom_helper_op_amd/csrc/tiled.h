@@ -1315,10 +1315,11 @@ __device__ __forceinline__ int wave_min(int v) {
 // Moves the window of one view to origin (ny, nx): every texel that falls outside the new
 // window is written out with dense global atomics (C consecutive floats per texel, 64/C
 // texels per instruction, UN instructions per round: their LDS reads go out together) and its
-// slot is cleared.  Uniform control flow.
+// slot is cleared.  Uniform control flow.  `cm`: channels of a texel in memory (a slot may be
+// padded; padding stays zero and is never written out).
 template <int VEC, int LPP, bool SIX = false, int UN = 4>
 __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, float *data,
-                                            int *list, float *gview, int srcW, int lane) {
+                                            int *list, float *gview, int srcW, int lane, int cm) {
   using WN = Window<VEC, LPP, SIX>;
   if (oy != WN::kNone) {
     wave_sync();  // the adds of the chunk before are complete and visible
@@ -1358,7 +1359,7 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, fl
         for (int u = 0; u < UN; ++u) {
           if (v[u] != 0.f) {
             data[le[u].x * WN::STRIDE + j] = 0.f;
-            atomic_add(gview + (int64_t)le[u].y * WN::C + j, v[u]);
+            atomic_add(gview + (int64_t)le[u].y * cm + j, v[u]);
           }
         }
       }
@@ -1386,7 +1387,7 @@ __device__ __forceinline__ unsigned wave_or(unsigned v) {
 // arithmetic).  All LDS reads of a row are issued together, then its atomics.
 template <int VEC, int LPP, bool SIX = false>
 __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *data, float *gview,
-                                                 int srcW, int lane, unsigned rows) {
+                                                 int srcW, int lane, unsigned rows, int cm) {
   using WN = Window<VEC, LPP, SIX>;
   if (oy == WN::kNone) return;
   wave_sync();  // the last adds are complete and visible
@@ -1411,7 +1412,7 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
         const int sl = e / C, ch = e - sl * C;
         const int ry = sl / WN::COLS, rx = sl - ry * WN::COLS;
         const int y = WN::image_row(ry, oy), x = ox + ((rx - ox) & (WN::COLS - 1));
-        if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * C + ch), v[u]);
+        if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
       }
     }
     return;
@@ -1429,7 +1430,7 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
       const int rx = e / C, ch = e - rx * C;
       const int x = ox + ((rx - ox) & (WN::COLS - 1));
       // (a slot that was never added to holds zero: texels outside the image never are)
-      if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * C + ch), v[u]);
+      if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
     }
   }
 }
@@ -1555,7 +1556,8 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
 template <int VEC, int LPP>
 __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool mine, int key,
                                                       float (&v)[4][VEC], float *stage,
-                                                      float *gview, int srcW, int lane, int cl) {
+                                                      float *gview, int srcW, int lane, int cl,
+                                                      int cm) {
   constexpr int C = VEC * LPP;
   typedef float vecf __attribute__((ext_vector_type(VEC)));
   while (m) {
@@ -1574,15 +1576,16 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
     }
     wave_sync();
     const int fh = k2 >> 16, fw = k2 & 0xffff;
-    float *row0 = gview + (int64_t)(fh * srcW + fw) * C;
-    float *row1 = row0 + (int64_t)srcW * C;
+    float *row0 = gview + (int64_t)(fh * srcW + fw) * cm;
+    float *row1 = row0 + (int64_t)srcW * cm;
 #pragma unroll
     for (int f0 = 0; f0 < 2 * C; f0 += 64) {
       const int f = f0 + lane;
       if (f < 2 * C) {
         const float a0 = stage[f], a1 = stage[2 * C + f];
-        if (a0 != 0.f) atomic_add(row0 + f, a0);
-        if (a1 != 0.f) atomic_add(row1 + f, a1);
+        const int e = f / C * cm + f % C;
+        if (a0 != 0.f) atomic_add(row0 + e, a0);
+        if (a1 != 0.f) atomic_add(row1 + e, a1);
       }
     }
     wave_sync();
@@ -1646,8 +1649,15 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // registers they do not have (the 32-channel kernel spills with it).
 // WIDE: the kernel as it is without the slimming of lean_backward: three waves per SIMD and, for
 // 32 channels, the 8 x 8 window.  The launcher decides (tiled_launch.inc).
+// PAD: fewer channels than the pixel's lanes hold (20, 24, 28 on eight lanes).  The lanes past the
+// last channel compute what the last lane computes and contribute nothing: their gradients are
+// selected to zero (not multiplied: infinities), their window slots stay zero.  A quarter of the
+// arithmetic is idle at 24 channels, but eight pixels share a wave and a scatter window where the
+// lane-per-channel kernels have two pixels and none (training
+// passes of 24 channels: minimum over five views, 63 x 85 x 37, 219 -> 110 us; warped features, 212 x
+// 213 x 86, 627 -> 344 us).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool DG = true,
-          bool PV = (CORR == 1), bool VLOOP = false, bool WIDE = false>
+          bool PV = (CORR == 1), bool VLOOP = false, bool WIDE = false, bool PAD = false>
 __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) void backward_kernel(const Args<S> a,
                                                                           const Geometry g) {
   constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, WIDE);
@@ -1682,9 +1692,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   float *s_v3 = reinterpret_cast<float *>(s_own_list + backward_list_words<VEC, LPP, kSix>());
   static_assert(CORR != 3 || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
   const float base = per_voxel_depth ? 0.f : a.base_plane[t.pix];
+  static_assert(!PAD || CORR != 3, "CostVolumeV3: whole pixels");
+  const int cm = PAD ? C : WN::C;
+  const bool ch_ok = !PAD || t.cl * VEC < C;
+  const int clc = PAD ? min(t.cl, C / VEC - 1) : t.cl;  // the lane whose channels this lane reads
   float ref[VEC];
   if constexpr (CORR != 4) {
-    load_vec<S, VEC, false>(a.ref + t.pix * C + t.cl * VEC, ref);
+    load_vec<S, VEC, false>(a.ref + t.pix * C + clc * VEC, ref);
     if constexpr (CORR == 3) {
 #pragma unroll
       for (int c = 0; c < VEC; ++c) s_v3[t.p * (VEC * LPP) + t.cl * VEC + c] = ref[c];
@@ -1697,7 +1711,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   const int64_t view_elems = (int64_t)srcH * srcW * C;
   float *src_grad_img = kWide ? a.src_grad_acc : reinterpret_cast<float *>(a.src_grad);
   const int row_step = srcW * C;
-  const unsigned lane_ch = (unsigned)(t.cl * VEC);
+  const unsigned lane_ch = (unsigned)(clc * VEC);
   float racc[VEC];
 #pragma unroll
   for (int c = 0; c < VEC; ++c) racc[c] = 0.f;
@@ -1711,7 +1725,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   constexpr bool kVoxelGrad = CORR == 2 || CORR == 3;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
   const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
-  const int goff = CORR == 1 ? group_offset<VEC>(t.cl, g.sub) : t.cl * VEC;
+  const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : clc * VEC;
   const int d_lo = t.d_lo, d_hi = t.d_hi;
   // upstream-gradient rows fetched ahead; the MIN reduce stages the mask rows beside them
   constexpr int PFMAX = (REDUCE || kLean) ? 4 : 8;
@@ -1769,7 +1783,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
       for (int c = 0; c < VEC; ++c) sg[n][k][c] = 0.f;
   }
   const S *cg_lane =
-      CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + t.cl * VEC
+      CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + clc * VEC
                 : a.cost_grad + t.pix * D * OC + (kVoxelGrad ? 0 : goff);
   const int32_t *cnt_src = CORR == 4 ? a.mask_in + t.pix * D * N + t.view0
                                      : a.mask_in + t.pix * D * mask_w;
@@ -1801,12 +1815,12 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
       const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
       const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
       window_move<VEC, LPP, kSix, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
-                                  s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane);
+                                  s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane, cm);
       in = WN::inside(key, oy[n], ox[n]);
       const bool out = fire && !in;
       const unsigned long long m = __ballot(out);
       if (m != 0ull) {
-        flush_cells_to_memory<VEC, LPP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl);
+        flush_cells_to_memory<VEC, LPP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl, cm);
         if (out) cur[n] = -1;
       }
     }
@@ -1972,7 +1986,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
             cell[n].y &= 0x7fffffff;
           } else {
             window_move<VEC, LPP, kSix>(oy[n], ox[n], ny - sy / 2, nx - sx / 2,
-                                  s_data + n * WN::SLOTS * WN::STRIDE, s_list, gview[n], srcW, t.lane);
+                                  s_data + n * WN::SLOTS * WN::STRIDE, s_list, gview[n], srcW, t.lane, cm);
             in_new = true;
             cell[n].y |= WN::kInside;
           }
@@ -2166,6 +2180,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
                 racc[c] = __builtin_fmaf(cg[c], smp, racc[c]);
                 gsrc = cg[c] * ref[c];
               }
+              if constexpr (PAD) gsrc = ch_ok ? gsrc : 0.f;
               sg[n][0][c] = __builtin_fmaf(gsrc, wt.x, sg[n][0][c]);
               sg[n][1][c] = __builtin_fmaf(gsrc, wt.y, sg[n][1][c]);
               sg[n][2][c] = __builtin_fmaf(gsrc, wt.z, sg[n][2][c]);
@@ -2181,6 +2196,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
           }
         }
       }
+      if constexpr (PAD && DG) dvox = ch_ok ? dvox : 0.f;
       if constexpr (!DG) {
         // no depth gradient wanted
       } else if (per_voxel_depth) {
@@ -2230,7 +2246,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
 #pragma unroll
   for (int n = 0; n < NV; ++n)
     window_flush_all<VEC, LPP, kSix>(oy[n], ox[n], s_data + n * WN::SLOTS * WN::STRIDE, gview[n], srcW,
-                               t.lane, wave_or(ring_rows[n]));
+                               t.lane, wave_or(ring_rows[n]), cm);
   wave_sync();  // the next view clears the window
   }  // views of the group
 
@@ -2243,8 +2259,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   } else if (single) {
     // (16-bit storage too: the finished sums go straight to the output, the fp32 image of
     // ref_grad is neither written nor narrowed afterwards)
-    if (t.pix_ok) store_vec<S, VEC, false>(a.ref_grad + t.pix * C + t.cl * VEC, racc);
-  } else if (t.pix_ok) {
+    if (t.pix_ok && ch_ok) store_vec<S, VEC, false>(a.ref_grad + t.pix * C + t.cl * VEC, racc);
+  } else if (t.pix_ok && ch_ok) {
 #pragma unroll
     for (int c = 0; c < VEC; ++c) atomic_add(rg + t.pix * C + t.cl * VEC + c, racc[c]);
   }
