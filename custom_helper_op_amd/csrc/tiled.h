@@ -1806,7 +1806,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     // derive from it would be computed in front of all chunks and held through the depth loop)
     int lane = t.lane;
     if constexpr (LPP < 8) asm volatile("" : "+v"(lane));
-    const int cl = lane % LPP;
+    const int cl = LPP < 8 ? lane % LPP : t.cl;
     const int key = cell[n].y & 0x7fffffff;
     bool in = WN::inside(key, oy[n], ox[n]);
     if (__ballot(fire && !in) != 0ull) {
