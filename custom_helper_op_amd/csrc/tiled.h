@@ -623,9 +623,8 @@ constexpr int forward_squares_words(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 
 // the squared difference / per-group maximum of the correlation with the winning view as
 // mask (-1: none).  The winner must be the reference's, so that reduce uses the literal
 // operand order with every operation rounded separately instead of the fused chains.
-// Minimum waves per SIMD the register allocator has to leave room for (mean of the squared
-// difference or of the group correlation only: the MIN / MAX reduces keep winner indices per
-// depth and channel and would spill).  Five and six views: left alone the compiler takes ~140
+// Minimum waves per SIMD the register allocator has to leave room for (the mean, and the minimum /
+// maximum of four views; elsewhere the winner indices per depth and channel would spill).  Five and six views: left alone the compiler takes ~140
 // registers (three waves); held to 128 it needs no scratch, and the fourth wave hides the tap
 // gathers of wide-baseline views (stress workload forward 5.17 -> 4.45 ms).  Three and four
 // views at four lanes per pixel: 102 -> 87 registers without scratch, five waves instead of
