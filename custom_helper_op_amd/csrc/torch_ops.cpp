@@ -11,6 +11,7 @@
 // (custom_helper_op/cc/kernels/cost_volume_kernels.cc:91-106, :220-243;
 // cost_volume_kernels_v2.cc:93-110; cost_volume_kernels_v3.cc:94-115, :231-255;
 // cost_aggregate_kernels.cc:85-106, :196-226; feature_aggregate_kernels.cc:69-92, :176-210).
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -34,7 +35,6 @@ enum Op { V1 = 0, V2 = 1, AGGREGATE = 2, V3 = 3, FEATURE = 4 };
 
 PyObject *g_invalid_argument = nullptr;  // ops.InvalidArgumentError
 PyObject *g_chop_error = nullptr;        // _lib.ChopError
-PyObject *g_out_of_memory = nullptr;     // torch.OutOfMemoryError
 
 struct InvalidArgument : std::runtime_error {
   using std::runtime_error::runtime_error;
@@ -492,12 +492,10 @@ PyObject *guarded(F &&body) {
       PyErr_SetObject(g_chop_error, args);
       Py_DECREF(args);
     }
-  } catch (const c10::OutOfMemoryError &e) {
-    PyErr_SetString(g_out_of_memory, e.what_without_backtrace());
-  } catch (const c10::Error &e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-  } catch (const std::exception &e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {
+    // torch's own, and what Python code called from here raised: a saved-tensor hook may end the
+    // call with an exception of its own, as checkpointing does where it has recomputed enough
+    torch::translate_exception_to_python(std::current_exception());
   }
   return nullptr;
 }
@@ -606,11 +604,11 @@ PyObject *py_combine_projection(PyObject *, PyObject *const *a, Py_ssize_t n) {
   });
 }
 
-// errors(InvalidArgumentError, ChopError, OutOfMemoryError): the exception classes to raise
+// errors(InvalidArgumentError, ChopError): the exception classes to raise
 PyObject *py_errors(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  if (!count_is(n, 3, "errors")) return nullptr;
-  Py_INCREF(a[0]), Py_INCREF(a[1]), Py_INCREF(a[2]);
-  g_invalid_argument = a[0], g_chop_error = a[1], g_out_of_memory = a[2];
+  if (!count_is(n, 2, "errors")) return nullptr;
+  Py_INCREF(a[0]), Py_INCREF(a[1]);
+  g_invalid_argument = a[0], g_chop_error = a[1];
   Py_RETURN_NONE;
 }
 

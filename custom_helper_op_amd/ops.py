@@ -38,7 +38,7 @@ def _native():
     if _native_module is None:
         _lib.load()
         from . import _chop_torch
-        _chop_torch.errors(InvalidArgumentError, _lib.ChopError, torch.cuda.OutOfMemoryError)
+        _chop_torch.errors(InvalidArgumentError, _lib.ChopError)
         _native_module = _chop_torch
     return _native_module
 

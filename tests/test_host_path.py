@@ -1,0 +1,93 @@
+"""What the native host path keeps of torch's machinery: saved-tensor hooks and checkpointing, the
+types of errors, tracing, forward-mode and functional derivatives -- for every differentiable
+function, on the GPU and, with the C ABI taken from the oracle (host_path.py), on the CPU."""
+import numpy as np
+import pytest
+import torch
+import torch.utils.checkpoint
+
+import custom_helper_op_amd as chop
+import host_path
+from custom_helper_op_amd import _lib, ops
+from custom_helper_op_amd.configs import reference_test_case
+
+FORMS = ("cost_volume", "cost_volume_v2", "cost_volume_v3", "cost_aggregate", "feature_aggregate",
+         "cost_volume_v2_filled", "cost_aggregate_filled")
+
+
+@pytest.fixture(scope="module")
+def cpu_module(tmp_path_factory):
+    return host_path.build_module(tmp_path_factory.mktemp("host_path"))
+
+
+@pytest.fixture(params=["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def device(request, monkeypatch):
+    if request.param == "cpu":
+        module = request.getfixturevalue("cpu_module")[0]
+        module.errors(ops.InvalidArgumentError, _lib.ChopError)
+        monkeypatch.setattr(ops, "_native_module", module)
+    return request.param
+
+
+def _inputs(form, device, grad=True, seed=2):
+    """Positional tensors of a differentiable function, and the function on them."""
+    t = reference_test_case(3, 1, 2, 6, 7, 8, 5, np.float32, seed=seed)
+    t = {k: torch.from_numpy(v).to(device) for k, v in t.items()}
+    t["depth_grid"] = t["base_plane"] + t["offsets"][:, None, None, :]
+    t["default"] = torch.full((), 0.25, device=device)
+    v2 = "_v2" in form
+    keys = [] if form == "feature_aggregate" else ["ref"]
+    keys += ["src"] + (["depth_grid"] if v2 else ["base_plane", "offsets"]) + ["Rs", "Ts"]
+    wanted = {"ref", "src", "depth_grid", "base_plane", "default"} if grad else ()
+    keys += ["default"] if form.endswith("filled") else []
+    ins = [t[k].requires_grad_(k in wanted) for k in keys]
+    kw = {"groups": 2} if v2 or form == "cost_volume_v3" else {}
+    return ins, lambda *a: getattr(chop, form)(*a, **kw)
+
+
+def _gradients(ins, cost, seed=5):
+    up = torch.randn(cost.shape, generator=torch.Generator().manual_seed(seed)).to(cost)
+    return torch.autograd.grad(cost, [x for x in ins if x.requires_grad], up)
+
+
+def _close(got, want):
+    # float32 sums of one order against another: the order of the GPU's atomics is free
+    for g, w in zip(got, want):
+        torch.testing.assert_close(g, w, rtol=1e-5, atol=1e-5 * float(w.abs().max()))
+
+
+class Mine(Exception):
+    pass
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_checkpoint_of_the_bare_operator(form, device):
+    """Its recomputation ends with an exception out of the pack hook, inside the operator's call."""
+    ins, fn = _inputs(form, device)
+    want = _gradients(ins, fn(*ins)[0])
+    cost, mask = torch.utils.checkpoint.checkpoint(fn, *ins, use_reentrant=False)
+    _close(_gradients(ins, cost), want)
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_hooks_see_the_saved_tensors_and_may_raise(form, device):
+    ins, fn = _inputs(form, device)
+    want, packed = _gradients(ins, fn(*ins)[0]), []
+
+    def pack(x):
+        packed.append(x)
+        return x.detach().cpu()
+
+    def raises(x):
+        raise Mine(form)
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda x: x.to(device)):
+        cost, mask = fn(*ins)
+    assert len(packed) == len(ins) + 1
+    _close(_gradients(ins, cost), want)
+    with torch.autograd.graph.saved_tensors_hooks(raises, lambda x: x), pytest.raises(Mine, match=form):
+        fn(*ins)
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: x, raises):
+        cost, mask = fn(*ins)
+    with pytest.raises(Mine, match=form):
+        _gradients(ins, cost)
