@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -35,6 +36,7 @@ enum Op { V1 = 0, V2 = 1, AGGREGATE = 2, V3 = 3, FEATURE = 4 };
 
 PyObject *g_invalid_argument = nullptr;  // ops.InvalidArgumentError
 PyObject *g_chop_error = nullptr;        // _lib.ChopError
+PyObject *g_recorded = nullptr;          // ops._recorded
 
 struct InvalidArgument : std::runtime_error {
   using std::runtime_error::runtime_error;
@@ -532,6 +534,10 @@ PyObject *py_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!count_is(n, kCallArgs + 2, "forward")) return nullptr;
   return guarded([&] {
     const bool differentiable = truth(a[kCallArgs + 1]);
+    // A trace can hold an autograd function of Python; of a call from here it would only hold the
+    // allocations.
+    if (differentiable && torch::jit::tracer::isTracing())
+      return PyObject_Vectorcall(g_recorded, a, kCallArgs + 1, nullptr);
     Call given = call_args(a, differentiable);
     given.default_cost = tensor_arg(a[kCallArgs]);
     Call c = given;
@@ -570,6 +576,22 @@ PyObject *py_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   });
 }
 
+// default_gradient(reduce, cost_grad, cost_mask, default) -> the gradient of the filled forms' scalar
+PyObject *py_default_gradient(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (!count_is(n, 4, "default_gradient")) return nullptr;
+  return guarded([&] {
+    const int reduce = reduce_arg(a[0]);
+    const Tensor g = tensor_arg(a[1]), mask = tensor_arg(a[2]), like = tensor_arg(a[3]);
+    Tensor out;
+    {
+      const WithoutLock unlocked;
+      const c10::AutoGradMode no_grad(false);
+      out = default_gradient(reduce, g.contiguous(), mask, like);
+    }
+    return wrap(out);
+  });
+}
+
 // combine_projection(ref_cam [B,2,4,4], src_cam [B,N,2,4,4], scale [3]) -> (Rs, Ts)
 PyObject *py_combine_projection(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!count_is(n, 3, "combine_projection")) return nullptr;
@@ -604,11 +626,12 @@ PyObject *py_combine_projection(PyObject *, PyObject *const *a, Py_ssize_t n) {
   });
 }
 
-// errors(InvalidArgumentError, ChopError): the exception classes to raise
-PyObject *py_errors(PyObject *, PyObject *const *a, Py_ssize_t n) {
-  if (!count_is(n, 2, "errors")) return nullptr;
-  Py_INCREF(a[0]), Py_INCREF(a[1]);
-  g_invalid_argument = a[0], g_chop_error = a[1];
+// python_side(InvalidArgumentError, ChopError, recorded): the exception classes to raise and what
+// forward() hands a call to that is being recorded
+PyObject *py_python_side(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  if (!count_is(n, 3, "python_side")) return nullptr;
+  Py_INCREF(a[0]), Py_INCREF(a[1]), Py_INCREF(a[2]);
+  g_invalid_argument = a[0], g_chop_error = a[1], g_recorded = a[2];
   Py_RETURN_NONE;
 }
 
@@ -616,7 +639,8 @@ PyMethodDef g_methods[] = {
     {"forward", (PyCFunction)(void (*)(void))py_forward, METH_FASTCALL, nullptr},
     {"backward", (PyCFunction)(void (*)(void))py_backward, METH_FASTCALL, nullptr},
     {"combine_projection", (PyCFunction)(void (*)(void))py_combine_projection, METH_FASTCALL, nullptr},
-    {"errors", (PyCFunction)(void (*)(void))py_errors, METH_FASTCALL, nullptr},
+    {"default_gradient", (PyCFunction)(void (*)(void))py_default_gradient, METH_FASTCALL, nullptr},
+    {"python_side", (PyCFunction)(void (*)(void))py_python_side, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_chop_torch", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -38,9 +38,13 @@ def _native():
     if _native_module is None:
         _lib.load()
         from . import _chop_torch
-        _chop_torch.errors(InvalidArgumentError, _lib.ChopError)
+        _connect(_chop_torch)
         _native_module = _chop_torch
     return _native_module
+
+
+def _connect(module):
+    module.python_side(InvalidArgumentError, _lib.ChopError, _recorded)
 
 
 def _reduce_code(reduce_method):
@@ -232,6 +236,46 @@ def cost_aggregate_filled(ref_image, src_images, base_plane, offsets, Rs, Ts, de
     custom_layers.py:51-57)."""
     return _native().forward(_AGGREGATE, ref_image, src_images, base_plane, offsets, Rs, Ts,
                              reduce_method, 1, half_centor, False, default_cost, True)
+
+
+class _Operator(torch.autograd.Function):
+    """An operator and its registered gradient as a function of Python's autograd, for the modes of
+    torch that record or refuse such a function and cannot see a native node."""
+
+    @staticmethod
+    def forward(ctx, op, ref_image, src_images, depth, offsets, Rs, Ts, reduce_method, groups,
+                half_centor, grid, default_cost):
+        cost, mask = _native().forward(op, ref_image, src_images, depth, offsets, Rs, Ts,
+                                       reduce_method, groups, half_centor, grid, default_cost, False)
+        ctx.save_for_backward(ref_image, src_images, depth, offsets, Rs, Ts, default_cost, mask)
+        ctx.attrs = (op, reduce_method, groups, half_centor, grid)
+        ctx.mark_non_differentiable(mask)
+        return cost, mask
+
+    @staticmethod
+    def backward(ctx, grad_out, _grad_mask):
+        *inputs, default_cost, mask = ctx.saved_tensors
+        op, *attrs = ctx.attrs
+        grads = _native().backward(op, *inputs, *attrs, grad_out, mask, ctx.needs_input_grad[3])
+        default_grad = (_native().default_gradient(attrs[0], grad_out, mask, default_cost)
+                        if ctx.needs_input_grad[11] else None)
+        return (None, *grads, *[None] * 7, default_grad)
+
+
+def _recorded(op, ref_image, src_images, depth, offsets, Rs, Ts, reduce_method, groups, half_centor,
+              grid, default_cost):
+    """What a differentiable function does while a trace is recorded; depth inputs and cameras
+    are taken from where the caller has them, as in ``csrc/torch_ops.cpp``."""
+    device = (src_images if op == _FEATURE else ref_image).device
+
+    def there(x):
+        return x if x is None else (x if torch.is_tensor(x) else torch.as_tensor(x)).to(device)
+
+    offsets, Rs, Ts = there(offsets), there(Rs), there(Ts)
+    if op == _V2:
+        depth = there(depth)
+    return _Operator.apply(op, ref_image, src_images, depth, offsets, Rs, Ts, reduce_method, groups,
+                           half_centor, grid, default_cost)
 
 
 class _DefaultFill(torch.autograd.Function):

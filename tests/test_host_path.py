@@ -8,7 +8,7 @@ import torch.utils.checkpoint
 
 import custom_helper_op_amd as chop
 import host_path
-from custom_helper_op_amd import _lib, ops
+from custom_helper_op_amd import ops
 from custom_helper_op_amd.configs import reference_test_case
 
 FORMS = ("cost_volume", "cost_volume_v2", "cost_volume_v3", "cost_aggregate", "feature_aggregate",
@@ -24,7 +24,7 @@ def cpu_module(tmp_path_factory):
 def device(request, monkeypatch):
     if request.param == "cpu":
         module = request.getfixturevalue("cpu_module")[0]
-        module.errors(ops.InvalidArgumentError, _lib.ChopError)
+        ops._connect(module)
         monkeypatch.setattr(ops, "_native_module", module)
     return request.param
 
@@ -91,3 +91,16 @@ def test_hooks_see_the_saved_tensors_and_may_raise(form, device):
         cost, mask = fn(*ins)
     with pytest.raises(Mine, match=form):
         _gradients(ins, cost)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("grad", [False, True])
+def test_trace_holds_the_operator(form, grad, device):
+    ins, fn = _inputs(form, device, grad)
+    traced = torch.jit.trace(lambda *a: fn(*a), tuple(ins))
+    other, _ = _inputs(form, device, grad, seed=3)
+    cost, mask = traced(*other)
+    want_cost, want_mask = fn(*other)
+    assert torch.equal(cost, want_cost) and torch.equal(mask, want_mask)
+    if grad:
+        _close(_gradients(other, cost), _gradients(other, want_cost))
