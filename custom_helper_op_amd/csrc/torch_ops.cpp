@@ -529,6 +529,13 @@ Call call_args(PyObject *const *a, bool move_small) {
   return c;
 }
 
+// Whether an input carries a tangent of forward-mode differentiation.
+bool has_tangent(const Call &c) {
+  for (const Tensor *t : {&c.ref, &c.src, &c.depth, &c.offsets, &c.Rs, &c.Ts, &c.default_cost})
+    if (t->defined() && t->_fw_grad(0).defined()) return true;
+  return false;
+}
+
 // forward(<call>, default | None, differentiable) -> (cost, mask)
 PyObject *py_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!count_is(n, kCallArgs + 2, "forward")) return nullptr;
@@ -540,6 +547,9 @@ PyObject *py_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
       return PyObject_Vectorcall(g_recorded, a, kCallArgs + 1, nullptr);
     Call given = call_args(a, differentiable);
     given.default_cost = tensor_arg(a[kCallArgs]);
+    // The operators have no forward derivative: Python's autograd function refuses a tangent, which
+    // would be lost on the way through here.
+    if (differentiable && has_tangent(given)) return PyObject_Vectorcall(g_recorded, a, kCallArgs + 1, nullptr);
     Call c = given;
     Tensor cost, mask;
     {
@@ -627,7 +637,7 @@ PyObject *py_combine_projection(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // python_side(InvalidArgumentError, ChopError, recorded): the exception classes to raise and what
-// forward() hands a call to that is being recorded
+// forward() hands a call to in the modes that only an autograd function of Python takes part in
 PyObject *py_python_side(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!count_is(n, 3, "python_side")) return nullptr;
   Py_INCREF(a[0]), Py_INCREF(a[1]), Py_INCREF(a[2]);

@@ -4,6 +4,7 @@ function, on the GPU and, with the C ABI taken from the oracle (host_path.py), o
 import numpy as np
 import pytest
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.utils.checkpoint
 
 import custom_helper_op_amd as chop
@@ -104,3 +105,16 @@ def test_trace_holds_the_operator(form, grad, device):
     assert torch.equal(cost, want_cost) and torch.equal(mask, want_mask)
     if grad:
         _close(_gradients(other, cost), _gradients(other, want_cost))
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("grad", [False, True])
+def test_forward_mode_is_refused(form, grad, device):
+    """There is no forward derivative: an input with a tangent must not give a result without one."""
+    ins, fn = _inputs(form, device, grad)
+    with forward_ad.dual_level():
+        for i in range(len(ins)):
+            dual = [forward_ad.make_dual(x, torch.ones_like(x)) if k == i else x for k, x in enumerate(ins)]
+            with pytest.raises(NotImplementedError, match="forward mode"):
+                fn(*dual)
+        assert fn(*ins)[0].requires_grad == grad
