@@ -20,6 +20,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <mutex>
@@ -529,6 +530,11 @@ Call call_args(PyObject *const *a, bool move_small) {
   return c;
 }
 
+// Whether a transform of torch.func (grad, vmap, jvp, ...) is active on this thread.
+bool in_functional_transform() {
+  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+
 // Whether an input carries a tangent of forward-mode differentiation.
 bool has_tangent(const Call &c) {
   for (const Tensor *t : {&c.ref, &c.src, &c.depth, &c.offsets, &c.Rs, &c.Ts, &c.default_cost})
@@ -542,8 +548,8 @@ PyObject *py_forward(PyObject *, PyObject *const *a, Py_ssize_t n) {
   return guarded([&] {
     const bool differentiable = truth(a[kCallArgs + 1]);
     // A trace can hold an autograd function of Python; of a call from here it would only hold the
-    // allocations.
-    if (differentiable && torch::jit::tracer::isTracing())
+    // allocations.  Under the transforms of torch.func such a function says what it lacks.
+    if (differentiable && (torch::jit::tracer::isTracing() || in_functional_transform()))
       return PyObject_Vectorcall(g_recorded, a, kCallArgs + 1, nullptr);
     Call given = call_args(a, differentiable);
     given.default_cost = tensor_arg(a[kCallArgs]);

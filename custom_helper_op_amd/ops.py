@@ -264,9 +264,9 @@ class _Operator(torch.autograd.Function):
 
 def _recorded(op, ref_image, src_images, depth, offsets, Rs, Ts, reduce_method, groups, half_centor,
               grid, default_cost):
-    """What a differentiable function does while a trace is recorded or where an input carries a
-    forward-mode tangent; depth inputs and cameras are taken from where the caller has them, as in
-    ``csrc/torch_ops.cpp``."""
+    """What a differentiable function does while a trace is recorded, under the transforms of
+    ``torch.func`` and where an input carries a forward-mode tangent; depth inputs and cameras are
+    taken from where the caller has them, as in ``csrc/torch_ops.cpp``."""
     device = (src_images if op == _FEATURE else ref_image).device
 
     def there(x):

@@ -118,3 +118,15 @@ def test_forward_mode_is_refused(form, grad, device):
             with pytest.raises(NotImplementedError, match="forward mode"):
                 fn(*dual)
         assert fn(*ins)[0].requires_grad == grad
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_functional_transforms_are_refused(form, device):
+    ins, fn = _inputs(form, device, grad=False)
+    first, rest = ins[0], ins[1:]
+    for call in (lambda: torch.func.grad(lambda x: fn(x, *rest)[0].sum())(first),
+                 lambda: torch.func.vmap(lambda x: fn(x, *rest)[0])(first[None]),
+                 lambda: torch.func.vmap(lambda z: fn(*ins)[0] + z)(torch.zeros(3, device=device)),
+                 lambda: torch.func.jvp(lambda x: fn(x, *rest)[0], (first,), (first,))):
+        with pytest.raises(RuntimeError, match="functorch transforms"):
+            call()
