@@ -338,6 +338,36 @@ Tensor default_gradient(int reduce, const Tensor &g, const Tensor &mask, const T
   return out.scalar_type() == like.scalar_type() ? out : out.to(like.scalar_type());
 }
 
+// The exception in flight as the interpreter's error; its lock is held.
+void set_error() {
+  try {
+    throw;
+  } catch (const PythonError &) {
+  } catch (const InvalidArgument &e) {
+    PyErr_SetString(g_invalid_argument, e.what());
+  } catch (const LibraryError &e) {
+    PyObject *args = Py_BuildValue("(is)", e.code, e.what());
+    if (args != nullptr) {
+      PyErr_SetObject(g_chop_error, args);
+      Py_DECREF(args);
+    }
+  } catch (...) {
+    // torch's own, and what Python code called from here raised: a saved-tensor hook may end the
+    // call with an exception of its own, as checkpointing does where it has recomputed enough
+    torch::translate_exception_to_python(std::current_exception());
+  }
+}
+
+// The exception in flight as one of Python, for threads that do not hold the lock.
+python_error as_python_error() {
+  const PyGILState_STATE lock = PyGILState_Ensure();
+  set_error();
+  python_error e;
+  e.persist();
+  PyGILState_Release(lock);
+  return e;
+}
+
 // ---- autograd -------------------------------------------------------------------------------
 // The gradient registered for an operator (custom_helper_ops.py:41-61, :74-94, :107-131,
 // :141-161, :174-195): the Grad op is fed the forward's mask; offsets, Rs and Ts receive no
@@ -355,6 +385,17 @@ struct OpBackward : public torch::autograd::Node {
     for (auto *v : {&ref, &src, &depth, &offsets, &Rs, &Ts, &default_cost, &mask}) v->reset_data();
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+    // The engine knows the types of torch's exceptions and of those that come from Python; any other
+    // it raises as a bare RuntimeError.
+    try {
+      return gradients(std::move(grads));
+    } catch (const InvalidArgument &) {
+      throw as_python_error();
+    } catch (const LibraryError &) {
+      throw as_python_error();
+    }
+  }
+  torch::autograd::variable_list gradients(torch::autograd::variable_list &&grads) {
     const std::lock_guard<std::mutex> lock(mutex_);
     const c10::AutoGradMode no_grad(false);
     Call c;
@@ -485,20 +526,8 @@ template <typename F>
 PyObject *guarded(F &&body) {
   try {
     return body();
-  } catch (const PythonError &) {
-    return nullptr;
-  } catch (const InvalidArgument &e) {
-    PyErr_SetString(g_invalid_argument, e.what());
-  } catch (const LibraryError &e) {
-    PyObject *args = Py_BuildValue("(is)", e.code, e.what());
-    if (args != nullptr) {
-      PyErr_SetObject(g_chop_error, args);
-      Py_DECREF(args);
-    }
   } catch (...) {
-    // torch's own, and what Python code called from here raised: a saved-tensor hook may end the
-    // call with an exception of its own, as checkpointing does where it has recomputed enough
-    torch::translate_exception_to_python(std::current_exception());
+    set_error();
   }
   return nullptr;
 }

@@ -1,6 +1,8 @@
 """What the native host path keeps of torch's machinery: saved-tensor hooks and checkpointing, the
 types of errors, tracing, forward-mode and functional derivatives -- for every differentiable
 function, on the GPU and, with the C ABI taken from the oracle (host_path.py), on the CPU."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,7 @@ import torch.utils.checkpoint
 
 import custom_helper_op_amd as chop
 import host_path
-from custom_helper_op_amd import ops
+from custom_helper_op_amd import _lib, ops
 from custom_helper_op_amd.configs import reference_test_case
 
 FORMS = ("cost_volume", "cost_volume_v2", "cost_volume_v3", "cost_aggregate", "feature_aggregate",
@@ -130,3 +132,31 @@ def test_functional_transforms_are_refused(form, device):
                  lambda: torch.func.jvp(lambda x: fn(x, *rest)[0], (first,), (first,))):
         with pytest.raises(RuntimeError, match="functorch transforms"):
             call()
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_errors_of_the_backward_pass_keep_their_types(form, device):
+    ins, fn = _inputs(form, device)
+    ndim = max(x.dim() for x in ins)
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: x, lambda x: x[:, :1] if x.dim() == ndim else x):
+        cost, mask = fn(*ins)
+    with pytest.raises(chop.InvalidArgumentError, match="must compate"):
+        _gradients(ins, cost)
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_status_of_the_library_reaches_the_caller(form, cpu_module, monkeypatch):
+    module, so = cpu_module
+    ops._connect(module)
+    monkeypatch.setattr(ops, "_native_module", module)
+    status = ctypes.c_int.in_dll(ctypes.CDLL(so), "chop_test_status")
+    ins, fn = _inputs(form, "cpu")
+    cost, mask = fn(*ins)
+    try:
+        status.value = 5
+        for call in (lambda: fn(*ins), lambda: _gradients(ins, cost)):
+            with pytest.raises(_lib.ChopError, match="as the test asked") as caught:
+                call()
+            assert caught.value.code == 5
+    finally:
+        status.value = 0
