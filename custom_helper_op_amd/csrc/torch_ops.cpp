@@ -92,8 +92,9 @@ Tensor prepared(const Tensor &t, at::ScalarType dtype, at::Device device, const 
 
 inline bool shaped(const Tensor &t, at::IntArrayRef want) { return t.sizes() == want; }
 
-// Types, devices and shapes of a call's inputs; makes them contiguous and fills in the sizes.
-void check_inputs(Call &c) {
+// Types, devices and shapes of a call's inputs and, for a gradient, of what flows back and of the
+// mask; makes them contiguous and fills in the sizes.
+void check_inputs(Call &c, Tensor *cost_grad = nullptr, Tensor *mask = nullptr) {
   const Tensor &lead = c.op == FEATURE ? c.src : c.ref;
   const at::ScalarType dt = lead.scalar_type();
   const at::Device dev = lead.device();
@@ -115,8 +116,13 @@ void check_inputs(Call &c) {
     c.Rs = prepared(c.Rs, real, dev, "Rs");
     c.Ts = prepared(c.Ts, real, dev, "Ts");
   };
-  depth_inputs();
+  if (c.op != V1) depth_inputs();
   cameras();
+  if (cost_grad != nullptr) {
+    *cost_grad = prepared(*cost_grad, dt, dev, c.op == FEATURE ? "mapped_feature_grad" : "cost_grad");
+    *mask = prepared(*mask, at::kInt, dev, c.op == FEATURE ? "mapped_mask" : "cost_mask");
+  }
+  if (c.op == V1) depth_inputs();
   if (c.op == FEATURE) {
     require(c.src.dim() == 5, "src_images must have rank 5");
     c.B = c.src.size(0), c.N = c.src.size(1), c.srcH = c.src.size(2), c.srcW = c.src.size(3);
@@ -254,8 +260,8 @@ void forward(const Call &c, Tensor &cost, Tensor &mask) {
 }
 
 // Gradient: `depth_grad` stays undefined when it is not wanted (V3 and FeatureAggregate always
-// compute it).  The inputs have been checked; the upstream gradient and the mask are checked here.
-void backward(const Call &c, Tensor cost_grad, Tensor mask, bool want_depth, Tensor &ref_grad, Tensor &src_grad,
+// compute it).  Everything has been checked but the shapes of the upstream gradient and the mask.
+void backward(const Call &c, const Tensor &cost_grad, const Tensor &mask, bool want_depth, Tensor &ref_grad, Tensor &src_grad,
               Tensor &depth_grad) {
   const Tensor &lead = c.op == FEATURE ? c.src : c.ref;
   const at::ScalarType dt = lead.scalar_type();
@@ -325,6 +331,7 @@ void backward(const Call &c, Tensor cost_grad, Tensor mask, bool want_depth, Ten
 // Gradient of the layers' scalar default: the upstream gradient summed over the voxels that
 // received it (16-bit storage is read as stored and summed in float).
 Tensor default_gradient(int reduce, const Tensor &g, const Tensor &mask, const Tensor &like) {
+  require(like.numel() == 1, "default_cost must be a scalar");
   const c10::DeviceGuard guard(g.device());
   const at::ScalarType dt = g.scalar_type();
   const int64_t n_mask = mask.numel(), inner = n_mask ? g.numel() / n_mask : 1;
@@ -402,10 +409,10 @@ struct OpBackward : public torch::autograd::Node {
     c.op = op, c.reduce = reduce, c.half = half, c.groups = groups, c.grid = grid;
     c.ref = ref.unpack(), c.src = src.unpack(), c.depth = depth.unpack(), c.offsets = offsets.unpack();
     c.Rs = Rs.unpack(), c.Ts = Ts.unpack(), c.default_cost = default_cost.unpack();
-    const Tensor m = mask.unpack();
+    Tensor m = mask.unpack();
     Tensor g = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
-    g = g.contiguous();
-    check_inputs(c);
+    // all of them again: a saved-tensor hook may have given back something else
+    check_inputs(c, &g, &m);
     torch::autograd::variable_list out(7);
     backward(c, g, m, task_should_compute_output(2), out[0], out[1], out[2]);
     if (c.default_cost.defined() && task_should_compute_output(6))
@@ -611,10 +618,7 @@ PyObject *py_backward(PyObject *, PyObject *const *a, Py_ssize_t n) {
     {
       const WithoutLock unlocked;
       const c10::AutoGradMode no_grad(false);
-      const Tensor &lead = c.op == FEATURE ? c.src : c.ref;
-      check_inputs(c);
-      cg = prepared(cg, lead.scalar_type(), lead.device(), c.op == FEATURE ? "mapped_feature_grad" : "cost_grad");
-      mask = prepared(mask, at::kInt, lead.device(), c.op == FEATURE ? "mapped_mask" : "cost_mask");
+      check_inputs(c, &cg, &mask);
       backward(c, cg, mask, want_depth, rg, sg, dg);
     }
     return wrap_tuple({&rg, &sg, &dg});
@@ -626,12 +630,13 @@ PyObject *py_default_gradient(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!count_is(n, 4, "default_gradient")) return nullptr;
   return guarded([&] {
     const int reduce = reduce_arg(a[0]);
-    const Tensor g = tensor_arg(a[1]), mask = tensor_arg(a[2]), like = tensor_arg(a[3]);
+    const Tensor g = tensor_arg(a[1]).contiguous(), like = tensor_arg(a[3]);
+    const Tensor mask = prepared(tensor_arg(a[2]), at::kInt, g.device(), "cost_mask");
     Tensor out;
     {
       const WithoutLock unlocked;
       const c10::AutoGradMode no_grad(false);
-      out = default_gradient(reduce, g.contiguous(), mask, like);
+      out = default_gradient(reduce, g, mask, like);
     }
     return wrap(out);
   });

@@ -160,3 +160,42 @@ def test_status_of_the_library_reaches_the_caller(form, cpu_module, monkeypatch)
             assert caught.value.code == 5
     finally:
         status.value = 0
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_what_hooks_give_back_is_checked(form, device):
+    """Tensors of another type than the upstream gradient's, or another mask, never reach a kernel."""
+    ins, fn = _inputs(form, device)
+    for change, match in ((lambda x: x.double() if x.is_floating_point() else x, "grad must have dtype torch.float64"),
+                          (lambda x: x if x.is_floating_point() else x.long(), "mask must have dtype torch.int32"),
+                          (lambda x: x[:0] if x.is_floating_point() and x.dim() else x, "must compate"),
+                          (lambda x: x if x.dim() else x.new_empty(0), "default_cost must be a scalar")):
+        if "default" in match and not form.endswith("filled"):
+            continue
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: x, change):
+            cost, mask = fn(*ins)
+        with pytest.raises(chop.InvalidArgumentError, match=match):
+            _gradients(ins, cost)
+
+
+def test_order_of_the_checks(device):
+    """Types before shapes, and among the types the order in which the operators take them."""
+    ins, fn = _inputs("cost_volume", device, grad=False)
+    cost, mask = fn(*ins)
+    ref, src, plane, offsets, Rs, Ts = ins
+    grid = plane + offsets[:, None, None, :]
+    for match, call in (
+            ("Rs must have", lambda: chop.cost_volume(ref, src, plane.double(), offsets, Rs.double(), Ts)),
+            ("cost_grad must have", lambda: chop.cost_volume_grad(ref, src, plane.double(), offsets, Rs, Ts,
+                                                                  cost.double(), mask)),
+            ("cost_grad must have", lambda: chop.cost_volume_grad(ref[0], src, plane, offsets, Rs, Ts,
+                                                                  cost.double(), mask)),
+            ("cost_mask must have", lambda: chop.cost_volume_grad(ref[0], src, plane, offsets, Rs, Ts, cost,
+                                                                  mask.long())),
+            ("base_plane must have", lambda: chop.cost_aggregate(ref, src, plane.double(), offsets, Rs.double(), Ts)),
+            ("depth_grid must have", lambda: chop.cost_volume_v2(ref, src, grid.double(), Rs.double(), Ts, groups=2)),
+            ("cost_grad must have", lambda: chop.cost_volume_grad_v2(ref[0], src, grid, Rs, Ts, cost.double(), mask,
+                                                                     groups=2)),
+            ("ref image must", lambda: chop.cost_volume_grad(ref[0], src, plane, offsets, Rs, Ts, cost, mask[0]))):
+        with pytest.raises(chop.InvalidArgumentError, match=match):
+            call()
