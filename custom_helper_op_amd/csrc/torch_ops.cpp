@@ -510,6 +510,16 @@ bool truth(PyObject *o) {
   return v != 0;
 }
 
+// half_centor: what int() takes, so that None or a word are refused
+bool half_arg(PyObject *o) {
+  if (PyBool_Check(o)) return o == Py_True;
+  PyObject *number = PyNumber_Long(o);
+  if (number == nullptr) throw PythonError();
+  const int v = PyObject_IsTrue(number);
+  Py_DECREF(number);
+  return v != 0;
+}
+
 PyObject *wrap(const Tensor &t) {
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
@@ -561,7 +571,7 @@ Call call_args(PyObject *const *a, bool move_small) {
   c.Rs = tensor_arg(a[5], small);
   c.Ts = tensor_arg(a[6], small);
   c.groups = groups_arg(a[8]);
-  c.half = truth(a[9]);
+  c.half = half_arg(a[9]);
   c.grid = truth(a[10]);
   return c;
 }

@@ -45,7 +45,7 @@ def _inputs(form, device, grad=True, seed=2):
     keys += ["default"] if form.endswith("filled") else []
     ins = [t[k].requires_grad_(k in wanted) for k in keys]
     kw = {"groups": 2} if v2 or form == "cost_volume_v3" else {}
-    return ins, lambda *a: getattr(chop, form)(*a, **kw)
+    return ins, lambda *a, **more: getattr(chop, form)(*a, **kw, **more)
 
 
 def _gradients(ins, cost, seed=5):
@@ -199,3 +199,14 @@ def test_order_of_the_checks(device):
             ("ref image must", lambda: chop.cost_volume_grad(ref[0], src, plane, offsets, Rs, Ts, cost, mask[0]))):
         with pytest.raises(chop.InvalidArgumentError, match=match):
             call()
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_half_centor_is_a_number(form, device):
+    ins, fn = _inputs(form, device, grad=False)
+    for bad, error in ((None, TypeError), ("no", ValueError), ([], TypeError)):
+        with pytest.raises(error):
+            fn(*ins, half_centor=bad)
+    for yes, no in ((1, 0), (np.True_, np.False_)):
+        assert torch.equal(fn(*ins, half_centor=yes)[0], fn(*ins, half_centor=True)[0])
+        assert torch.equal(fn(*ins, half_centor=no)[0], fn(*ins, half_centor=False)[0])
