@@ -2310,11 +2310,21 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
   g.seg = ((per_seg + LPP - 1) / LPP) * LPP;
   // Segments are whole chunks.  Rounded up they can be twice what was asked for (135 hypotheses of
   // 64 channels: eight segments of 17 become five of 32); a launch with fewer than two waves per
-  // SIMD rounds down instead: its time is that of its longest wave (best pair of 64 channels, six
-  // views, 16 x 21 x 135, forward 183 -> 99 us; group correlation bf16, 21 x 26 x 117, 25.4 -> 15.5 us;
-  // the gradients gain or lose a microsecond or two: 24.1 -> 21.0, 16.4 -> 18.9 us).
-  if (g.nseg > 1 && per_seg > LPP && tiles * ngroups * ((D + g.seg - 1) / g.seg) < 2048)
-    g.seg = per_seg / LPP * LPP;
+  // SIMD rounds down instead: its time is that of its longest wave (forward: best pair of 64
+  // channels, six views, 16 x 21 x 135, 183 -> 99 us; group correlation bf16, 21 x 26 x 117, 25.4 ->
+  // 15.5 us; gradients up to 1.6x: group correlation of 32 channels, 37 x 49 x 28, 27 -> 17 us).
+  // A gradient (vper > 0) pays for every segment, so it rounds up where that costs more than the
+  // longest wave: where the segments and views that add to one pixel's gradient become many (six
+  // views, 105 hypotheses of 32 channels: 13 us rounded up, 18 down), and where the waves no longer
+  // all run side by side -- two or three per SIMD, one where a wave has 16 pixels and more and most
+  // segments would be a single chunk (one view of 16 channels, 36 x 46 x 55: 14 and 17 us).
+  // Measured on 140 launches either side of these lines.
+  if (g.nseg > 1 && per_seg > LPP && tiles * ngroups * ((D + g.seg - 1) / g.seg) < 2048) {
+    const int down = per_seg / LPP * LPP;
+    const int64_t n = (D + down - 1) / down;
+    const int64_t most = LPP >= 16 ? 3072 : LPP >= 8 ? 2400 : n <= 5 ? 2048 : 1024;
+    if (vper == 0 || (ngroups * n <= 35 && tiles * ngroups * n <= most)) g.seg = down;
+  }
   g.nseg = (int)((D + g.seg - 1) / g.seg);
   g.total_units = tiles * g.nseg * g.ngroups;
   g.units_per_seg = (unsigned)(tiles * g.ngroups);
