@@ -1722,6 +1722,20 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // (feature_aggregate_kernels_gpu.cu.cc:219-326)
   // 3: CostVolumeV3, one upstream gradient per voxel that flows through the best group pair
   constexpr bool kVoxelGrad = CORR == 2 || CORR == 3;
+  // One winning view per voxel (or group): a view's runs are few and end far apart in depth.  An open
+  // run from a cell left long ago need not make a chunk spread (kEndLeft), and where few runs end at
+  // a depth moving the window to them costs more than adding them to memory (kFewRuns, in pixels of
+  // the wave; end_spread_runs).  Four views, 136 x 176, 24 planes from 0.9: best pair of 32 channels
+  // 276 -> 186 us (189 with every run outside the window added to memory), dense planes 378 -> 341 us;
+  // CostAggregate of 16 and 8 channels 144 -> 112 and 108 -> 71 us.  The lines: an eighth of the
+  // pixels, but four for the best pair, whose gradient is bound by instructions and leaves the
+  // atomics room (64 channels: none 407, two 313, four 273 us).  The gradients of CostAggregate with
+  // 32 channels and more keep the runs left behind: they have no registers for the check (two
+  // views, dense: 181 us without, 187 with it).  Where a mean or every channel's own winner keeps
+  // all runs short, most pixels of a tile end together and the window pays.
+  constexpr bool kWinners = REDUCE == 1 && (kVoxelGrad || CORR == 1);
+  constexpr bool kEndLeft = kWinners && (CORR != 2 || LPP < 8);
+  constexpr int kFewRuns = !kWinners ? 0 : CORR == 3 ? 4 : PPW / 8;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
   const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
   const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : clc * VEC;
@@ -1808,14 +1822,17 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     const int cl = LPP < 8 ? lane % LPP : t.cl;
     const int key = cell[n].y & 0x7fffffff;
     bool in = WN::inside(key, oy[n], ox[n]);
-    if (__ballot(fire && !in) != 0ull) {
-      const int fh = key >> 16, fw = key & 0xffff;
-      const int ny = wave_min(fire ? fh : WN::kNone), nx = wave_min(fire ? fw : WN::kNone);
-      const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
-      const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
-      window_move<VEC, LPP, kSix, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
-                                  s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane, cm);
-      in = WN::inside(key, oy[n], ox[n]);
+    const unsigned long long outside = __ballot(fire && !in);
+    if (outside != 0ull) {
+      if (kFewRuns == 0 || __popcll(outside) > kFewRuns * LPP) {
+        const int fh = key >> 16, fw = key & 0xffff;
+        const int ny = wave_min(fire ? fh : WN::kNone), nx = wave_min(fire ? fw : WN::kNone);
+        const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
+        const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
+        window_move<VEC, LPP, kSix, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
+                                    s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane, cm);
+        in = WN::inside(key, oy[n], ox[n]);
+      }
       const bool out = fire && !in;
       const unsigned long long m = __ballot(out);
       if (m != 0ull) {
@@ -1976,10 +1993,27 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
             const int cy = (cell[n].y >> 16) & 0x7fff, cx = cell[n].y & 0xffff;
             my = min(my, cy), mx = min(mx, cx), My = max(My, cy), Mx = max(Mx, cx);
           }
-          const int ny = wave_min(my), nx = wave_min(mx);
-          const int hy = -wave_min(-My) + 1, hx = -wave_min(-Mx) + 1;  // last row / column used
-          const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);  // slack
+          int ny = wave_min(my), nx = wave_min(mx);
+          int hy = -wave_min(-My) + 1, hx = -wave_min(-Mx) + 1;  // last row / column used
+          int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);  // slack
           spread[n] = sy < 0 || sx < 0;
+          if constexpr (kEndLeft) {
+            if (spread[n] && __ballot(valid) != 0ull) {
+              // without the open runs: where the chunk's cells fit, the runs it leaves behind end
+              const int fh = hit.key >> 16, fw = hit.key & 0xffff;
+              ny = wave_min(valid ? fh : WN::kNone), nx = wave_min(valid ? fw : WN::kNone);
+              hy = -wave_min(valid ? -fh : WN::kNone) + 1, hx = -wave_min(valid ? -fw : WN::kNone) + 1;
+              sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
+              spread[n] = sy < 0 || sx < 0;
+              const int key = cell[n].y & 0x7fffffff;
+              const bool left = !spread[n] && cur[n] >= 0 && !WN::inside(key, ny - sy / 2, nx - sx / 2);
+              const unsigned long long m = __ballot(left);
+              if (m != 0ull) {
+                flush_cells_to_memory<VEC, LPP>(m, left, key, sg[n], s_stage, gview[n], srcW, t.lane, t.cl, cm);
+                if (left) cur[n] = -1;
+              }
+            }
+          }
           if (spread[n]) {
             in_new = false;  // decided when the run ends
             cell[n].y &= 0x7fffffff;

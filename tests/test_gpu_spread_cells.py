@@ -85,3 +85,26 @@ def test_spread_cells_views_take_turns(oracle):
     assert _lib.load().chop_last_views_per_workgroup() == 2
     for g, w in zip(got, oracle.cost_volume_bwd(*args, cg, mask)):
         assert_backward_close(host(g), w)
+
+
+@pytest.mark.parametrize("C", [4, 8, 16, 32, 64])
+def test_runs_of_seldom_winners(oracle, C):
+    """One winner per voxel or group among six views: a view wins now and then, so its runs stay
+    open while the sweep moves on and few of them end at a depth.  Dense planes (the runs left
+    behind alone do not fit the window), planes far apart, and both in one sweep."""
+    for near, far, rot, shift, D in ((2.0, 12.0, 4.0, 0.2, 47), SWEEPS["apart"] + (13,), SWEEPS["mixed"] + (33,)):
+        print("\n[case] C%d planes %g to %g" % (C, near, far), flush=True)
+        rng, args = _tensors(C + D, 1, 6, 29, 43, C, D, near, far, rot, shift)
+        a2 = (args[0], args[1], args[2] + args[3][:, None, None, :], args[4], args[5])
+        for name, a, groups in (("cost_aggregate", args, ()), ("cost_volume_v2", a2, (C // 4,)),
+                                ("cost_volume_v3", args, (C // 4,))):
+            if name == "cost_volume_v3" and C < 8:
+                continue
+            cost, mask = getattr(oracle, name + "_fwd")(*a, "MIN", *groups)
+            cg = rng.standard_normal(cost.shape).astype(np.float32)
+            grad = {"cost_aggregate": chop.cost_aggregate_grad, "cost_volume_v2": chop.cost_volume_grad_v2,
+                    "cost_volume_v3": chop.cost_volume_grad_v3}[name]
+            got = grad(*[dev(x) for x in a], dev(cg), dev(mask), "MIN", *groups)
+            assert _lib.load().chop_last_kernel_family() == 2
+            for g, w in zip(got, getattr(oracle, name + "_bwd")(*a, cg, mask, "MIN", *groups)):
+                assert_backward_close(host(g), w)
