@@ -1730,7 +1730,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // CostAggregate of 16 and 8 channels 144 -> 112 and 108 -> 71 us.  The lines: an eighth of the
   // pixels, but four for the best pair, whose gradient is bound by instructions and leaves the
   // atomics room (64 channels: none 407, two 313, four 273 us).  The gradients of CostAggregate with
-  // 32 channels and more keep the runs left behind: they have no registers for the check (two
+  // 32 channels and more keep the runs left behind open: the check costs them more than it saves (two
   // views, dense: 181 us without, 187 with it).  Where a mean or every channel's own winner keeps
   // all runs short, most pixels of a tile end together and the window pays.
   constexpr bool kWinners = REDUCE == 1 && (kVoxelGrad || CORR == 1);
@@ -1812,8 +1812,12 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // 32 taps), which then leave as one dense run of atomics each, and the rate of the atomics is
   // what bounds such a launch (32 channels, six views, depths from 0.5, 15-degree rotations:
   // 18.5 -> 13.3 ms against every cell of such a chunk adding its four texels to memory by itself;
-  // minimum over two views, twelve planes from 1.7 to 16: 632 -> 395 us).  A cell that is still outside (pixels of one depth further apart
-  // than the window, on strongly magnified views) goes to memory by itself.
+  // minimum over two views, 260 x 372, twelve planes from 1.7 to 16: 632 -> 351 us).  A cell that is
+  // still outside (pixels of one depth further apart than the window, on strongly magnified views)
+  // goes to memory by itself, and so do a few runs of seldom winners (kFewRuns).  CostVolumeV3's
+  // gradient of a mean spends its time on the pair search: 24 far-apart planes of 32 channels 0-3 %
+  // slower than with every cell added to memory, of 16 channels 1.2-1.5x faster; dense planes 0.8 %
+  // slower (188.4 -> 189.9 us) for the block in its loop.
   auto end_spread_runs = [&](int n, bool fire) __attribute__((always_inline)) {
     // (the lane index as a value the compiler cannot see through: what the window's functions
     // derive from it would be computed in front of all chunks and held through the depth loop)

@@ -5,9 +5,14 @@
 // torch.autograd.Function each way) a tiny forward cost 22 us of host time against 8 us on the
 // GPU and a small training pass 77 us against 33 us.  Here a call parses its arguments once with
 // the interpreter's fast calling convention, releases the interpreter lock, and the backward
-// pass runs without taking it at all.
+// pass takes it for nothing of its own (saved-tensor hooks and errors do).
 //
-// The checks and their order are those of CostVolumeOp::Compute and its siblings
+// A node hung on the result does not take part in everything that an autograd function of Python
+// does: while torch.jit records a trace, under the transforms of torch.func and where an input
+// carries a forward-mode tangent the call goes through one (ops._Operator), which is recorded, or
+// refused with torch's own message.
+//
+// The checks and their order (types, then shapes) are those of CostVolumeOp::Compute and its siblings
 // (custom_helper_op/cc/kernels/cost_volume_kernels.cc:91-106, :220-243;
 // cost_volume_kernels_v2.cc:93-110; cost_volume_kernels_v3.cc:94-115, :231-255;
 // cost_aggregate_kernels.cc:85-106, :196-226; feature_aggregate_kernels.cc:69-92, :176-210).

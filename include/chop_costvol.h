@@ -428,7 +428,7 @@ int chop_last_kernel_family(void);
 int chop_last_views_per_workgroup(void);
 /* No counterpart in the reference.  The tiled gradient kernels for 32 channels exist twice:
  * slimmed to four wavefronts per SIMD with a scatter window of 6 x 8 texels, and at three
- * wavefronts with 8 x 8.  The first is 3-13 % faster (most where wide baselines and
+ * wavefronts with 8 x 8.  The first takes 3-17 % less time (most where wide baselines and
  * hypotheses close to the cameras spread the samples).  Left alone the library
  * picks the second for five or more source views; rows = 6 or 8 fixes the
  * choice for subsequent calls from this thread, 0 returns it to the library.  Returns the
