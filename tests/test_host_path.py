@@ -210,3 +210,28 @@ def test_half_centor_is_a_number(form, device):
     for yes, no in ((1, 0), (np.True_, np.False_)):
         assert torch.equal(fn(*ins, half_centor=yes)[0], fn(*ins, half_centor=True)[0])
         assert torch.equal(fn(*ins, half_centor=no)[0], fn(*ins, half_centor=False)[0])
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_strided_inputs_subsets_and_a_second_pass(form, device):
+    plain, fn = _inputs(form, device)
+    wanted = [i for i, x in enumerate(plain) if x.requires_grad]
+    want = dict(zip(wanted, _gradients(plain, fn(*plain)[0])))
+    for subset in [[i] for i in wanted] + [wanted]:
+        ins = [x.detach() if x.dim() < 3 else x.detach().transpose(1, 2).contiguous().transpose(1, 2) for x in plain]
+        for i in subset:
+            ins[i].requires_grad_(True)
+        cost, mask = fn(*ins)
+        assert cost.requires_grad and not mask.requires_grad
+        up = torch.randn(cost.shape, generator=torch.Generator().manual_seed(5)).to(cost)
+        for retain in (True, False):
+            _close(torch.autograd.grad(cost, [ins[i] for i in subset], up, retain_graph=retain), [want[i] for i in subset])
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(cost, [ins[i] for i in subset], up)
+    with torch.no_grad():
+        assert not fn(*plain)[0].requires_grad
+    cost, mask = fn(*plain)
+    with torch.no_grad():
+        plain[wanted[0]].add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        _gradients(plain, cost)
