@@ -1,6 +1,6 @@
 // Strip kernels: the wave-per-pixel-strip decomposition for every shape the tiled kernels do
-// not take -- float64 (the element type of the reference's own tests), channel counts that
-// are not 4 x a power of two (the reference tests use 3, 5 and 9), any number of views -- for
+// not take -- channel counts that are not 4 x a power of two (the reference tests use 3, 5 and 9),
+// any number of views, pointers that are not 16-byte aligned -- for
 // CostVolume, CostVolumeV2, CostAggregate (both reduces) and FeatureAggregate, all four storage
 // types, up to 64 channels; and for the gradient of CostVolumeV3 in float and double with any
 // group width (the lanes of a pixel find the view's best group pair again through LDS, then
@@ -55,20 +55,6 @@ __device__ __forceinline__ void strip_sync() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// 1 / x to within an ulp or two, for the backward's factors (a full IEEE division costs about
-// ten instructions in float and fifty in double; the gradients are compared at 1e-4).
-__device__ __forceinline__ float quick_recip(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double quick_recip(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-}
-
-// a * b + c in one rounding: the backward's arithmetic (gradients are compared at 1e-4; with
-// contraction off for the whole library a plain a * b + c is two instructions)
-__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double mad(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 // Sum over the 2^shift consecutive lanes of a pixel, left in every one of them.
 template <typename R>

@@ -97,6 +97,17 @@ __device__ __forceinline__ uint32_t narrow_word<bf16_t>(const float *in) {
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+// Two and four values of the arithmetic type as they lie in LDS.
+template <typename R>
+struct alignas(2 * sizeof(R)) Two {
+  R x, y;
+};
+template <typename R>
+struct alignas(16) Four {
+  R x, y, z, w;
+};
 
 template <int BYTES>
 struct Raw;
@@ -117,10 +128,23 @@ struct Raw<2> {
   using type = uint16_t;
 };
 
-// Loads CNT elements of S (CNT*sizeof(S) in {2,4,8,16} bytes, naturally aligned) as floats.
-// STREAM marks data that is touched once (cost rows, upstream gradients): non-temporal.
-template <typename S, int CNT, bool STREAM>
-__device__ __forceinline__ void load_vec(const S *p, float *out) {
+// Loads CNT elements of S (CNT*sizeof(S) in {2,4,8,16,32} bytes, 16-byte aligned from there on) in
+// the arithmetic type.  STREAM marks data that is touched once (cost rows, upstream gradients):
+// non-temporal.  GAP (double only): elements from one pair to the next, see lane_gap.
+template <typename S, int CNT, bool STREAM, int GAP = 2>
+__device__ __forceinline__ void load_vec(const S *p, typename Storage<S>::Real *out) {
+  if constexpr (sizeof(S) == 8) {
+    if constexpr (CNT == 1) {
+      out[0] = STREAM ? __builtin_nontemporal_load(p) : *p;
+    } else {
+#pragma unroll
+      for (int k = 0; k < CNT / 2; ++k) {
+        const f64x2 *q = reinterpret_cast<const f64x2 *>(p + k * GAP);
+        const f64x2 v = STREAM ? __builtin_nontemporal_load(q) : *q;
+        out[2 * k] = v[0], out[2 * k + 1] = v[1];
+      }
+    }
+  } else {
   constexpr int BYTES = CNT * (int)sizeof(S);
   using RawT = typename Raw<BYTES>::type;
   constexpr int PER_WORD = 4 / (int)sizeof(S);
@@ -136,6 +160,7 @@ __device__ __forceinline__ void load_vec(const S *p, float *out) {
 #pragma unroll
     for (int k = 0; k < BYTES / 4; ++k) widen_word<S>(v[k], out + k * PER_WORD);
   }
+  }
 }
 
 // Output rows bypass the caches (non-temporal, STREAM) only where one store of a pixel's lanes covers
@@ -144,8 +169,22 @@ __device__ __forceinline__ void load_vec(const S *p, float *out) {
 // depths, which other store instructions write: streamed, each piece reaches memory on its own
 // as a partial line, while L2 puts the pieces of a cached line together first (the
 // valid-view counts of the MVSNet-stage forward: 134 -> 123 us).
-template <typename S, int CNT, bool STREAM>
-__device__ __forceinline__ void store_vec(S *p, const float *in) {
+template <typename S, int CNT, bool STREAM, int GAP = 2>
+__device__ __forceinline__ void store_vec(S *p, const typename Storage<S>::Real *in) {
+  if constexpr (sizeof(S) == 8) {
+    if constexpr (CNT == 1) {
+      if (STREAM) __builtin_nontemporal_store(in[0], p);
+      else *p = in[0];
+    } else {
+#pragma unroll
+      for (int k = 0; k < CNT / 2; ++k) {
+        f64x2 *q = reinterpret_cast<f64x2 *>(p + k * GAP);
+        const f64x2 v = {in[2 * k], in[2 * k + 1]};
+        if (STREAM) __builtin_nontemporal_store(v, q);
+        else *q = v;
+      }
+    }
+  } else {
   constexpr int BYTES = CNT * (int)sizeof(S);
   using RawT = typename Raw<BYTES>::type;
   constexpr int PER_WORD = 4 / (int)sizeof(S);
@@ -164,16 +203,25 @@ __device__ __forceinline__ void store_vec(S *p, const float *in) {
     __builtin_nontemporal_store(v, q);
   else
     *q = v;
+  }
 }
 
 // The same load without the conversion: CNT elements as they lie in memory, in 32-bit words
 // (a single 16-bit element in the low half of one word).  A wave that widens 16-bit values
 // right after the load waits for memory at that point; keeping the words and widening them
 // where they are used lets the wait fall behind whatever work sits in between.
+// (doubles are kept as doubles)
+template <typename S>
+using RawWord = typename std::conditional<sizeof(S) == 8, double, uint32_t>::type;
 template <typename S, int CNT>
-constexpr int raw_words() { return (CNT * (int)sizeof(S) + 3) / 4; }
-template <typename S, int CNT, bool STREAM>
-__device__ __forceinline__ void load_raw(const S *p, uint32_t *out) {
+constexpr int raw_words() { return (CNT * (int)sizeof(S) + 3) / (int)sizeof(RawWord<S>); }
+__device__ __forceinline__ float raw_to_real(uint32_t w) { return __uint_as_float(w); }
+__device__ __forceinline__ double raw_to_real(double w) { return w; }
+template <typename S, int CNT, bool STREAM, int GAP = 2>
+__device__ __forceinline__ void load_raw(const S *p, RawWord<S> *out) {
+  if constexpr (sizeof(S) == 8) {
+    load_vec<S, CNT, STREAM, GAP>(p, out);
+  } else {
   constexpr int BYTES = CNT * (int)sizeof(S);
   using RawT = typename Raw<BYTES>::type;
   const RawT *q = reinterpret_cast<const RawT *>(p);
@@ -184,9 +232,14 @@ __device__ __forceinline__ void load_raw(const S *p, uint32_t *out) {
 #pragma unroll
     for (int k = 0; k < BYTES / 4; ++k) out[k] = v[k];
   }
+  }
 }
 template <typename S, int CNT>
-__device__ __forceinline__ void widen_raw(const uint32_t *in, float *out) {
+__device__ __forceinline__ void widen_raw(const RawWord<S> *in, typename Storage<S>::Real *out) {
+  if constexpr (sizeof(S) == 8) {
+#pragma unroll
+    for (int k = 0; k < CNT; ++k) out[k] = in[k];
+  } else {
   constexpr int BYTES = CNT * (int)sizeof(S);
   constexpr int PER_WORD = 4 / (int)sizeof(S);
   if constexpr (BYTES == 2) {
@@ -197,11 +250,45 @@ __device__ __forceinline__ void widen_raw(const uint32_t *in, float *out) {
 #pragma unroll
     for (int k = 0; k < BYTES / 4; ++k) widen_word<S>(in[k], out + k * PER_WORD);
   }
+  }
 }
 
 // (the choice is made at compile time from the row's width: a run-time test in front of every
 // row store cost the MVSNet-stage forward 20 us)
 constexpr bool whole_lines(int elements, int elem_bytes) { return elements * elem_bytes >= 128; }
+
+// Which channels a lane owns.  Four consecutive ones, 16 bytes in float.  In double four would be 32
+// bytes, which one access cannot move: each of two accesses of a pixel's lanes would touch every
+// other 16 bytes of the row, and a streamed row would leave as half lines.  So in double a lane
+// owns two pairs, one in each half of the row (channels 2 cl and half + 2 cl), and every access
+// of a pixel is one contiguous run.  Not where a lane's channels have to be neighbours (correlation
+// groups) and not with idle lanes (their pairs would lie in the other half).
+constexpr int lane_gap(int lpp, int corr, int elem_bytes, bool pad) {
+  return elem_bytes == 8 && corr != 1 && !pad ? 2 * lpp : 2;
+}
+// first channel of lane `cl`; channel c (0..3) is that + c / 2 * gap + c % 2
+__device__ __forceinline__ int lane_first(int cl, int gap) { return gap == 2 ? cl * 4 : cl * 2; }
+
+// This lane's four channels of an LDS row of channels (at `p`: the first).
+template <int GAP, typename R>
+__device__ __forceinline__ void slot_read(const R *p, R (&v)[4]) {
+  if constexpr (sizeof(R) == 4) {
+    const Four<R> w = *reinterpret_cast<const Four<R> *>(p);
+    v[0] = w.x, v[1] = w.y, v[2] = w.z, v[3] = w.w;
+  } else {
+    const Two<R> lo = *reinterpret_cast<const Two<R> *>(p), hi = *reinterpret_cast<const Two<R> *>(p + GAP);
+    v[0] = lo.x, v[1] = lo.y, v[2] = hi.x, v[3] = hi.y;
+  }
+}
+template <int GAP, typename R>
+__device__ __forceinline__ void slot_write(R *p, const R (&v)[4]) {
+  if constexpr (sizeof(R) == 4) {
+    *reinterpret_cast<Four<R> *>(p) = Four<R>{v[0], v[1], v[2], v[3]};
+  } else {
+    *reinterpret_cast<Two<R> *>(p) = Two<R>{v[0], v[1]};
+    *reinterpret_cast<Two<R> *>(p + GAP) = Two<R>{v[2], v[3]};
+  }
+}
 
 // Orders this wave's LDS traffic: the lanes of a wavefront execute in lockstep and the
 // LDS returns a wave's operations in issue order, so only the compiler has to be kept
@@ -222,12 +309,21 @@ __device__ __forceinline__ void wave_sync() {
 // lane of the group.  Cross-lane moves in registers: quad permutes, then the half-row and
 // row mirrors (a mirror pairs lane i with lane WIDTH-1-i; the quad steps finish the sum).
 template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-  const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false);
-  return v + __int_as_float(moved);
+__device__ __forceinline__ int dpp_move(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
 }
-template <int WIDTH>
-__device__ __forceinline__ float group_sum(float v) {
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __int_as_float(dpp_move<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  return __hiloint2double(dpp_move<CTRL>(__double2hiint(v)), dpp_move<CTRL>(__double2loint(v)));
+}
+template <int CTRL, typename R>
+__device__ __forceinline__ R dpp_add(R v) { return v + dpp_move<CTRL>(v); }
+template <int WIDTH, typename R>
+__device__ __forceinline__ R group_sum(R v) {
   static_assert(WIDTH == 1 || WIDTH == 2 || WIDTH == 4 || WIDTH == 8 || WIDTH == 16, "group width");
   if constexpr (WIDTH >= 16) v = dpp_add<0x140>(v);  // row_mirror
   if constexpr (WIDTH >= 8) v = dpp_add<0x141>(v);   // row_half_mirror
@@ -237,8 +333,8 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 // Sums the per-channel values of each correlation group: out[g] for g < VEC/sub.
-template <int VEC>
-__device__ __forceinline__ void fold_groups(const float *ch, int sub, float *out) {
+template <int VEC, typename R>
+__device__ __forceinline__ void fold_groups(const R *ch, int sub, R *out) {
   if (sub == 1) {
 #pragma unroll
     for (int c = 0; c < VEC; ++c) out[c] = ch[c];
@@ -256,7 +352,7 @@ __device__ __forceinline__ void fold_groups(const float *ch, int sub, float *out
 }
 
 template <typename S, int VEC, int LPP>
-__device__ __forceinline__ void store_groups(S *p, const float *v, int sub) {
+__device__ __forceinline__ void store_groups(S *p, const typename Storage<S>::Real *v, int sub) {
   // p already points at this lane's first group; a pixel's row holds VEC * LPP / sub values
   constexpr int C = VEC * LPP, B = (int)sizeof(S);
   if (sub == 1) {
@@ -277,10 +373,10 @@ __device__ __forceinline__ int group_offset(int cl, int sub) {
 }
 
 // ---- shared front end of both kernels ---------------------------------------------------
-template <int NV>
+template <int NV, typename R>
 struct Cameras {
-  float zc[NV], wc[NV], hc[NV];  // rows of R applied to (ref_w, ref_h, 1)
-  float t0[NV], t1[NV], t2[NV];
+  R zc[NV], wc[NV], hc[NV];  // rows of R applied to (ref_w, ref_h, 1)
+  R t0[NV], t1[NV], t2[NV];
 };
 
 template <int LPP>
@@ -361,14 +457,16 @@ __device__ __forceinline__ bool locate_tile(const Args<S> &a, const Geometry &g,
 }
 
 template <typename S, int NV>
-__device__ __forceinline__ void load_cameras(const Args<S> &a, int b, int view0, float ref_w,
-                                             float ref_h, Cameras<NV> &c) {
+__device__ __forceinline__ void load_cameras(const Args<S> &a, int b, int view0,
+                                             typename Storage<S>::Real ref_w,
+                                             typename Storage<S>::Real ref_h,
+                                             Cameras<NV, typename Storage<S>::Real> &c) {
   const int N = (int)a.N;
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
     const int nn = view0 + n < N ? view0 + n : 0;
-    const float *Rm = a.Rs + ((int64_t)b * N + nn) * 9;
-    const float *t = a.Ts + ((int64_t)b * N + nn) * 3;
+    const auto *Rm = a.Rs + ((int64_t)b * N + nn) * 9;
+    const auto *t = a.Ts + ((int64_t)b * N + nn) * 3;
     // same association as the per-voxel expression: (R6*w + R7*h) + R8
     c.zc[n] = Rm[6] * ref_w + Rm[7] * ref_h + Rm[8];
     c.wc[n] = Rm[0] * ref_w + Rm[1] * ref_h + Rm[2];
@@ -378,45 +476,47 @@ __device__ __forceinline__ void load_cameras(const Args<S> &a, int b, int view0,
 }
 
 // One reprojection with hoisted row products; bit-identical to warp.h's project().
+template <typename R>
 struct Hit {
   int off;     // element offset of tap (fh,fw) inside the view's image, or -1
   int key;     // (fh << 16) | fw
-  float k00, k01, k11, k10;
-  float dh, dw;
-  float z, w3d, h3d;
+  R k00, k01, k11, k10;
+  R dh, dw;
+  R z, w3d, h3d;
 };
 
-template <int NV>
-__device__ __forceinline__ void reproject(const Cameras<NV> &c, int n, float depth, float half,
-                                          float src_h_max, float src_w_max, int srcW, int C,
-                                          Hit &r) {
+template <int NV, typename R>
+__device__ __forceinline__ void reproject(const Cameras<NV, R> &c, int n, R depth, R half,
+                                          R src_h_max, R src_w_max, int srcW, int C,
+                                          Hit<R> &r) {
   r.off = -1;
   r.key = 0;
-  r.k00 = r.k01 = r.k11 = r.k10 = 0.f;
+  r.k00 = r.k01 = r.k11 = r.k10 = R(0);
   r.z = c.zc[n] * depth + c.t2[n];
-  if (r.z <= 0.f) return;
+  if (r.z <= R(0)) return;
   r.w3d = c.wc[n] * depth + c.t0[n];
-  float sw = r.w3d / r.z;
+  R sw = r.w3d / r.z;
   r.h3d = c.hc[n] * depth + c.t1[n];
-  float sh = r.h3d / r.z;
+  R sh = r.h3d / r.z;
   sw = sw - half;
   sh = sh - half;
-  if (sh > 0.f && sw > 0.f && sh < src_h_max && sw < src_w_max) {
+  if (sh > R(0) && sw > R(0) && sh < src_h_max && sw < src_w_max) {
     const int fh = static_cast<int>(sh), fw = static_cast<int>(sw);
-    r.dh = sh - static_cast<float>(fh);
-    r.dw = sw - static_cast<float>(fw);
+    r.dh = sh - static_cast<R>(fh);
+    r.dw = sw - static_cast<R>(fw);
     r.k11 = r.dh * r.dw;
-    r.k10 = r.dh * (1.f - r.dw);
-    r.k00 = (1.f - r.dh) * (1.f - r.dw);
-    r.k01 = (1.f - r.dh) * r.dw;
+    r.k10 = r.dh * (R(1) - r.dw);
+    r.k00 = (R(1) - r.dh) * (R(1) - r.dw);
+    r.k01 = (R(1) - r.dh) * r.dw;
     r.off = (fh * srcW + fw) * C;
     r.key = (fh << 16) | fw;
   }
 }
 
 template <typename S>
-__device__ __forceinline__ float voxel_depth(const Args<S> &a, int64_t pix, int b, int d,
-                                             float base) {
+__device__ __forceinline__ typename Storage<S>::Real voxel_depth(const Args<S> &a, int64_t pix, int b,
+                                                                 int d,
+                                                                 typename Storage<S>::Real base) {
   return a.depth_grid ? a.depth_grid[pix * a.D + d] : base + a.offsets[(int64_t)b * a.D + d];
 }
 
@@ -443,15 +543,46 @@ __device__ __forceinline__ void store_ints(int32_t *p, const int *v) {
   }
 }
 
-// ---- CostVolumeV3: the largest correlation of any source group with any reference group ------
-// A value of another lane of the same pixel, in registers.
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+// A row of winners per channel, four of this lane's.
+template <int VEC, int LPP, int GAP>
+__device__ __forceinline__ void store_winners(int32_t *p, const int *v) {
+  if constexpr (GAP == 2) {
+    store_ints<VEC, whole_lines(VEC * LPP, 4)>(p, v);
+  } else {
+    store_ints<2, false>(p, v);
+    store_ints<2, false>(p + GAP, v + 2);
+  }
 }
-template <int CTRL>
-__device__ __forceinline__ int dpp_move(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+
+// ---- CostVolumeV3: the largest correlation of any source group with any reference group ------
+// The mean over k accepted views.  In its literal form the division rounds like the reference's:
+// halving and quartering are exact, so only other counts pay for one.
+template <bool LIT, typename R>
+__device__ __forceinline__ void mean_of(R (&acc)[4], int k) {
+  if constexpr (LIT) {
+    if (k == 2 || k == 4) {
+      const R part = k == 2 ? R(0.5) : R(0.25);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] *= part;
+    } else if (k > 2) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] /= static_cast<R>(k);
+    }
+  } else if (k > 1) {
+    const R inv = quick_recip(static_cast<R>(k));
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] *= inv;
+  }
+}
+// The group values of a lane: its channels' sums folded, or (literal form, add_groups) already so.
+template <bool LIT, typename R>
+__device__ __forceinline__ void fold_or_keep(const R (&acc)[4], int sub, R (&out)[4]) {
+  if constexpr (LIT) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) out[c] = acc[c];
+  } else {
+    fold_groups<4>(acc, sub, out);
+  }
 }
 // One butterfly step of "largest value, earliest pair on a tie" (both partners end equal).
 template <int CTRL>
@@ -464,8 +595,9 @@ __device__ __forceinline__ void better_pair(float &best, int &code) {
 }
 // A group of eight channels held by two lanes: the odd lane continues the even lane's sum over
 // its own four, in channel order (the result of the odd lane is the group's).
-__device__ __forceinline__ float continue_group(float sum, const float (&val)[4], int cl) {
-  const float head = dpp_move<0xA0>(sum);  // quad_perm 0,0,2,2
+template <typename R>
+__device__ __forceinline__ R continue_group(R sum, const R (&val)[4], int cl) {
+  const R head = dpp_move<0xA0>(sum);  // quad_perm 0,0,2,2
   return (cl & 1) ? (((head + val[0]) + val[1]) + val[2]) + val[3] : sum;
 }
 // The maximum reduce of one accepted view: where a correlation group of this lane is larger than
@@ -474,13 +606,14 @@ __device__ __forceinline__ float continue_group(float sum, const float (&val)[4]
 // width is a run-time value; picking the terms of every group by comparisons instead took, with
 // the wave per SIMD of forward_min_waves, 157 against 140 us on an f16 sweep of 32 channels in
 // eight groups, four views, 237 x 315 x 24).
-__device__ __forceinline__ void keep_larger_groups(float (&best)[4], int (&arg)[4], const float (&val)[4],
+template <typename R>
+__device__ __forceinline__ void keep_larger_groups(R (&best)[4], int (&arg)[4], const R (&val)[4],
                                                    int sub, int cl, int view) {
-  auto keep = [&](int i, float corr) __attribute__((always_inline)) {
+  auto keep = [&](int i, R corr) __attribute__((always_inline)) {
     if (best[i] < corr) best[i] = corr, arg[i] = view;
   };
   if (sub >= 4) {
-    float corr = ((val[0] + val[1]) + val[2]) + val[3];
+    R corr = ((val[0] + val[1]) + val[2]) + val[3];
     if (sub == 8) corr = continue_group(corr, val, cl);
     keep(0, corr);
   } else if (sub == 2) {
@@ -489,6 +622,22 @@ __device__ __forceinline__ void keep_larger_groups(float (&best)[4], int (&arg)[
   } else {
 #pragma unroll
     for (int c = 0; c < 4; ++c) keep(c, val[c]);
+  }
+}
+// The mean's literal form: one view's products, added up group by group in channel order, join the
+// sums of the views before it.
+template <typename R>
+__device__ __forceinline__ void add_groups(R (&acc)[4], const R (&val)[4], int sub, int cl) {
+  if (sub >= 4) {
+    R corr = ((val[0] + val[1]) + val[2]) + val[3];
+    if (sub == 8) corr = continue_group(corr, val, cl);
+    acc[0] += corr;
+  } else if (sub == 2) {
+    acc[0] += val[0] + val[1];
+    acc[1] += val[2] + val[3];
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] += val[c];
   }
 }
 constexpr int kNoPair = 0x7fffffff;  // pair code: source group * 16 + reference group
@@ -541,7 +690,7 @@ __device__ __forceinline__ void v3_best_pair(const float (&smp)[VEC], const floa
 // reference group, :494-512).  `rows` = two LDS arrays of 64*VEC floats: the pixel rows of
 // the reference image (written once by the caller) and of this sample.
 template <int VEC, int LPP, int SUB, int REDUCE>
-__device__ __forceinline__ void v3_pair_gradients(const float4 wt, const float (&tap)[4][VEC],
+__device__ __forceinline__ void v3_pair_gradients(const Four<float> wt, const float (&tap)[4][VEC],
                                                   float cg, int pair, float *rows, int p, int cl,
                                                   float (&racc)[VEC], float (&gsrc)[VEC]) {
   constexpr int C = VEC * LPP, LPG = SUB / 4;
@@ -610,14 +759,15 @@ __device__ __forceinline__ void keep_alive(const Touched &w) {
   asm volatile("" ::"v"(w.a), "v"(w.b));  // no instruction: the two registers count as read here
 }
 
-template <int NV>
-constexpr int forward_lds_words(int lpp) {
-  return lpp > 1 ? NV * 64 * 5 : 0;
+template <int NV, typename R = float>
+constexpr int forward_lds_bytes(int lpp) {
+  return lpp > 1 ? NV * 64 * (4 * (int)sizeof(R) + 4) : 0;
 }
-// The minimum of the summed squared difference also stages one chunk of squares per view:
-// a row of C (+4 padding, so that the eight readers of a pixel hit different banks) floats
-// per (pixel, depth).
-constexpr int forward_squares_words(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 4) : 0; }
+// The sums of squares that have to be added up in channel order (the minimum, and the mean in its
+// literal form) also stage one chunk of squares per view: a row of C (+4 padding, so that the
+// eight readers of a pixel hit different banks) values per (pixel, depth).
+template <typename R = float>
+constexpr int forward_squares_bytes(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 4) * (int)sizeof(R) : 0; }
 
 // REDUCE: 0 mean over the accepted views (mask = their number), 1 per-channel minimum of
 // the squared difference / per-group maximum of the correlation with the winning view as
@@ -631,20 +781,36 @@ constexpr int forward_squares_words(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 
 // four (f16 cascade workload forward 122 -> 113 us cold); the other widths would spill.
 // MIN / MAX of four views: 129-131 registers left alone, 8 bytes of scratch at 128 and a fourth wave
 // (six views would spill 60 bytes and more: left alone).
-constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce) {
+// (float arithmetic; in double the registers are left to the compiler)
+constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce, bool wide_real) {
+  if (wide_real) return 1;
   if (reduce != 0 && corr <= 1 && nv == 4 && lpp >= 2) return 4;
   if (corr > 1 || reduce != 0) return 1;
   return nv >= 5 ? 4 : (nv >= 3 && lpp == 4) ? 5 : 1;
 }
 
-template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0>
+// LIT: the mean in the reference's operand order too, every operation rounded by itself, so that the
+// result is the plain evaluation's to the bit.  Double is always evaluated that way: the rows are
+// twice as long and the stores bound the launch as before (two views, 32 channels, 128 x 160 x 192:
+// 1.04 GB in 243 us, 4.3 TB/s; 430 us with a lane per channel, which reads every record and offset
+// once for two pixels instead of eight).
+template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool LIT = (sizeof(S) == 8)>
 // At most five waves per SIMD: with six (the two-view instantiation needs only 80 VGPRs)
 // the waves of a CU evict each other's taps from L1 and the kernel is 6 % slower.  The lower
 // bound: see forward_min_waves.
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))) void forward_kernel(
+__attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, sizeof(S) == 8), 5))) void forward_kernel(
     const Args<S> a, const Geometry g) {
+  using R = typename Storage<S>::Real;
+  using R4 = Four<R>;
   constexpr int PPW = 64 / LPP;
+  // bytes of a float4's worth of records per float of lane offset (p4, q4 below)
+  constexpr unsigned kR4 = sizeof(R);
+  constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), false);
+  // Three views and more in double: the views take turns with one set of taps (four sets of four
+  // channels are 128 registers), also in the ops that keep a set per view in float.
+  constexpr bool kOneSet = sizeof(R) == 8 && NV >= 3;
+  constexpr int NT = kOneSet ? 1 : NV;
   extern __shared__ __align__(16) unsigned char smem[];
   Tile<LPP> t;
   // (one or two views only: the instantiations for more views are held to a register budget
@@ -656,43 +822,45 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
     return;
   }
   const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
-  const float half = a.half;
+  const R half = a.half;
+  const int ch0 = lane_first(t.cl, GAP);
   // LDS records: wts[NV][LPP][PPW] then off[NV][LPP][PPW], addressed as (lane-dependent
   // byte offset) + (compile-time constant) so that the constant lands in the instruction's
   // offset field instead of costing a register per unrolled depth
-  constexpr int kWts = 0, kOff = NV * 64 * 16;
+  constexpr int kWts = 0, kOff = NV * 64 * (int)sizeof(R4), kRec = kOff + NV * 64 * 4;
   const unsigned p4 = (unsigned)t.p * 4u;                 // reader: pixel p
   const unsigned q4 = (unsigned)(t.cl * PPW + t.p) * 4u;  // writer: lane (p, j)
 
-  Cameras<NV> cam;
-  load_cameras<S, NV>(a, t.b, t.view0, static_cast<float>(t.w) + half,
-                      static_cast<float>(t.h) + half, cam);
-  const float base = a.depth_grid ? 0.f : a.base_plane[t.pix];
-  float ref[VEC];
+  // (one set: the views' row products, twelve registers each, are computed where a chunk needs them)
+  const R ref_w = static_cast<R>(t.w) + half, ref_h = static_cast<R>(t.h) + half;
+  Cameras<NT, R> cam;
+  if constexpr (!kOneSet) load_cameras<S, NT>(a, t.b, t.view0, ref_w, ref_h, cam);
+  const R base = a.depth_grid ? R(0) : a.base_plane[t.pix];
+  R ref[VEC];
   if constexpr (CORR != 4) {
-    load_vec<S, VEC, false>(a.ref + t.pix * C + t.cl * VEC, ref);
+    load_vec<S, VEC, false, GAP>(a.ref + t.pix * C + ch0, ref);
     if constexpr (CORR == 3) {
       // CostVolumeV3: every lane of a pixel reads all of the pixel's reference groups
       static_assert(CORR != 3 || (LPP > 1 && VEC == 4), "CostVolumeV3: wide pixels");
-      float *s_ref = reinterpret_cast<float *>(smem + NV * 64 * 20);  // behind the records
+      float *s_ref = reinterpret_cast<float *>(smem + kRec);  // behind the records
 #pragma unroll
       for (int c = 0; c < VEC; ++c) s_ref[t.p * (VEC * LPP) + t.cl * VEC + c] = ref[c];
       wave_sync();
     }
   } else {
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) ref[c] = 0.f;  // the warp-only op has no reference image
+    for (int c = 0; c < VEC; ++c) ref[c] = R(0);  // the warp-only op has no reference image
   }
   const S *view[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n)
-    view[n] = a.src + ((int64_t)t.b * N + (n < N ? n : 0)) * srcH * srcW * C + t.cl * VEC;
+    view[n] = a.src + ((int64_t)t.b * N + (n < N ? n : 0)) * srcH * srcW * C + ch0;
   const int row_step = srcW * C;
 
-  float tap[NV][4][VEC];
-  int cur[NV];
+  R tap[NT][4][VEC];
+  int cur[NT];
 #pragma unroll
-  for (int n = 0; n < NV; ++n) cur[n] = -1;
+  for (int n = 0; n < NT; ++n) cur[n] = -1;
 
   // CORR: 0 squared difference per channel, 1 group correlation, 2 squared difference
   // summed over all channels (one value per voxel), 4 the samples themselves, one row per
@@ -706,134 +874,185 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
   // the cost rows of the per-channel ops (and the sample rows of the warp-only op) stream past
   // the caches where they cover whole lines
   constexpr bool kNtRows = whole_lines(VEC * LPP, (int)sizeof(S));
+  // one value per voxel that is added up in channel order
+  constexpr bool kRowSums = CORR == 2 && (REDUCE == 1 || LIT);
   const int d_lo = t.d_lo, d_hi = t.d_hi;
   // the cost-map layers' default fill folded into the store: where no view was accepted the
   // scalar is written instead of the cost (custom_layers.py:52-57, :78-83)
   const bool fill = a.default_cost != nullptr;
-  const float dflt = fill ? *a.default_cost : 0.f;
+  const R dflt = fill ? *a.default_cost : R(0);
   // this pixel's output rows (the 64-bit product once per wave, not once per depth)
   S *const out_pix = a.cost + t.pix * D * OC;
   int32_t *const mask_pix = a.mask + t.pix * D * OC;
   for (int d0 = d_lo; d0 < d_hi; d0 += LPP) {
     // ---- phase 1: reprojection by lane (p, j = cl) --------------------------------------
     int r_off[NV];
-    float4 r_wts[NV];
+    R4 r_wts[NV];
     unsigned vmask = 0u;  // views accepted for lane (p, j)'s own voxel
     {
       const int d = d0 + t.cl;
       const bool d_ok = d < d_hi;
-      const float depth = d_ok ? voxel_depth(a, t.pix, t.b, d, base) : 1.f;
+      const R depth = d_ok ? voxel_depth(a, t.pix, t.b, d, base) : R(1);
       int cnt = 0;
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        Hit hit;
+        Hit<R> hit;
         hit.off = -1;
-        hit.k00 = hit.k01 = hit.k11 = hit.k10 = 0.f;
-        if (n < N && d_ok) reproject<NV>(cam, n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
+        hit.k00 = hit.k01 = hit.k11 = hit.k10 = R(0);
+        if constexpr (kOneSet) load_cameras<S, 1>(a, t.b, n, ref_w, ref_h, cam);
+        if (n < N && d_ok)
+          reproject<NT, R>(cam, kOneSet ? 0 : n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
         cnt += hit.off >= 0;
-        if constexpr (CORR == 2 && REDUCE == 1) vmask |= (hit.off >= 0 ? 1u : 0u) << n;
+        if constexpr (kRowSums) vmask |= (hit.off >= 0 ? 1u : 0u) << n;
         if constexpr (CORR == 4) {
           if (n < N && d_ok && t.pix_ok)
             a.mask[(t.pix * D + d) * N + n] = hit.off >= 0 ? 1 : 0;
         }
         if constexpr (LPP > 1) {
           lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = hit.off;
-          lds_at<float4>(smem, q4 * 4u, kWts + (n * LPP * PPW) * 16) =
-              make_float4(hit.k00, hit.k01, hit.k11, hit.k10);
+          lds_at<R4>(smem, q4 * kR4, kWts + (n * LPP * PPW) * (int)sizeof(R4)) =
+              R4{hit.k00, hit.k01, hit.k11, hit.k10};
         } else {
           r_off[n] = hit.off;
-          r_wts[n] = make_float4(hit.k00, hit.k01, hit.k11, hit.k10);
+          r_wts[n] = R4{hit.k00, hit.k01, hit.k11, hit.k10};
         }
       }
       if constexpr (REDUCE == 0 && CORR != 4)
         if (d_ok && t.pix_ok) a.mask[t.pix * D + d] = cnt;
     }
     if constexpr (LPP > 1) wave_sync();
-    if constexpr (CORR == 2 && REDUCE == 1) {
+    if constexpr (kRowSums) {
       // Minimum over the views of the squared difference summed over ALL channels
       // (cost_aggregate_kernels_gpu.cu.cc:128-229).  The mask names the winning view, so the
       // sum has to be the reference's: channel 0 first, every product and sum rounded
       // separately.  View by view, the channel lanes leave the chunk's squares in LDS and the
-      // lane that owns voxel (p, d0 + cl) adds its row up in channel order.
-      constexpr int kSq = NV * 64 * 20;             // behind the records
-      constexpr int ROWB = (VEC * LPP + 4) * 4;     // bytes per (pixel, depth) row
-      float best = 3.402823466e+38f;                // numeric_limits<T>::max(), :170
+      // lane that owns voxel (p, d0 + cl) adds its row up in channel order.  The mean in its
+      // literal form is one such sum through all accepted views (:33-125).
+      constexpr int kSq = kRec;                           // behind the records
+      constexpr int ROWB = (VEC * LPP + 4) * (int)sizeof(R);  // bytes per (pixel, depth) row
+      R best = REDUCE == 1 ? Limits<R>::max() : R(0);     // numeric_limits<T>::max(), :170
       int win = -1;
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        float own = 0.f;  // LPP == 1: this lane holds the whole pixel
+        constexpr int kMany = kOneSet ? 0 : 1;
+        R(&tp)[4][VEC] = tap[n * kMany];
+        int &cur1 = cur[n * kMany];
+        if constexpr (kOneSet) cur1 = -1;
+        R own[VEC];  // LPP == 1: this lane holds the whole pixel
 #pragma unroll
         for (int jj = 0; jj < LPP; ++jj) {
           if (d0 + jj >= d_hi) {
             if constexpr (LPP >= 16) continue; else break;
           }
           int off;
-          float4 wt;
+          R4 wt;
           if constexpr (LPP > 1) {
             off = lds_at<int>(smem, p4, kOff + ((n * LPP + jj) * PPW) * 4);
-            wt = lds_at<float4>(smem, p4 * 4u, kWts + ((n * LPP + jj) * PPW) * 16);
+            wt = lds_at<R4>(smem, p4 * kR4, kWts + ((n * LPP + jj) * PPW) * (int)sizeof(R4));
           } else {
             off = r_off[n];
             wt = r_wts[n];
           }
-          float sq[VEC];
+          R sq[VEC];
 #pragma unroll
-          for (int c = 0; c < VEC; ++c) sq[c] = 0.f;
+          for (int c = 0; c < VEC; ++c) sq[c] = R(0);
           if (off >= 0) {
-            if (off != cur[n]) {
-              cur[n] = off;
+            if (off != cur1) {
+              cur1 = off;
               const S *q = view[n] + off;
-              load_vec<S, VEC, false>(q, tap[n][0]);
-              load_vec<S, VEC, false>(q + C, tap[n][1]);
-              load_vec<S, VEC, false>(q + row_step + C, tap[n][2]);
-              load_vec<S, VEC, false>(q + row_step, tap[n][3]);
+              load_vec<S, VEC, false, GAP>(q, tp[0]);
+              load_vec<S, VEC, false, GAP>(q + C, tp[1]);
+              load_vec<S, VEC, false, GAP>(q + row_step + C, tp[2]);
+              load_vec<S, VEC, false, GAP>(q + row_step, tp[3]);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const float smp = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
-                                wt.w * tap[n][3][c];
-              const float diff = smp - ref[c];
+              const R smp = wt.x * tp[0][c] + wt.y * tp[1][c] + wt.z * tp[2][c] + wt.w * tp[3][c];
+              const R diff = smp - ref[c];
               sq[c] = diff * diff;
             }
           }
           if constexpr (LPP > 1) {
-            lds_at<float4>(smem, (unsigned)(t.p * LPP * ROWB + t.cl * VEC * 4), kSq + jj * ROWB) =
-                make_float4(sq[0], sq[1], sq[2], sq[3]);
+            const unsigned own_at = (unsigned)(t.p * LPP * ROWB + ch0 * (int)sizeof(R));
+            slot_write<GAP>(&lds_at<R>(smem, own_at, kSq + jj * ROWB), sq);
           } else {
-            own = 0.f;
 #pragma unroll
-            for (int c = 0; c < VEC; ++c) own += sq[c];
+            for (int c = 0; c < VEC; ++c) own[c] = sq[c];
           }
         }
-        if constexpr (LPP > 1) {
-          wave_sync();
-          if ((vmask >> n) & 1u) {
-            float tot = 0.f;
+        if constexpr (LPP > 1) wave_sync();
+        if ((vmask >> n) & 1u) {
+          R tot = REDUCE == 1 ? R(0) : best;
+          if constexpr (LPP > 1) {
 #pragma unroll
             for (int k = 0; k < LPP; ++k) {
-              const float4 v = lds_at<float4>(
-                  smem, (unsigned)((t.p * LPP + t.cl) * ROWB), kSq + k * VEC * 4);
+              const R4 v = lds_at<R4>(smem, (unsigned)((t.p * LPP + t.cl) * ROWB),
+                                      kSq + k * VEC * (int)sizeof(R));
               tot += v.x;
               tot += v.y;
               tot += v.z;
               tot += v.w;
             }
-            if (best > tot) best = tot, win = n;  // strict: the earliest view keeps a tie (:217)
+          } else {
+#pragma unroll
+            for (int c = 0; c < VEC; ++c) tot += own[c];
           }
-          wave_sync();
-        } else {
-          if (((vmask >> n) & 1u) && best > own) best = own, win = n;
+          if constexpr (REDUCE == 0) best = tot;
+          else if (best > tot) best = tot, win = n;  // strict: the earliest view keeps a tie (:217)
         }
+        if constexpr (LPP > 1) wave_sync();
       }
       const int d = d0 + t.cl;
       if (d < d_hi && t.pix_ok) {
-        const float out = win >= 0 ? best / static_cast<float>(C) : dflt;  // :222-227
-        reinterpret_cast<float *>(a.cost)[t.pix * D + d] = out;
-        a.mask[t.pix * D + d] = win;
+        R out = dflt;
+        if constexpr (REDUCE == 1) {
+          if (win >= 0) out = best / static_cast<R>(C);  // :222-227
+          a.mask[t.pix * D + d] = win;
+        } else {
+          if (vmask != 0u) out = best / static_cast<R>(__popc(vmask) * C);  // :118-123
+        }
+        reinterpret_cast<R *>(a.cost)[t.pix * D + d] = out;
       }
       continue;
     }
-    if constexpr ((CORR == 0 || CORR == 1) && (NV >= 5 || (NV >= 3 && LPP == 4))) {
+    if constexpr (CORR == 4 && kOneSet) {
+      // the samples alone, view by view (a row per voxel and view: nothing is summed)
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        int cur1 = -1;
+#pragma unroll
+        for (int jj = 0; jj < LPP; ++jj) {
+          if (d0 + jj >= d_hi || n >= N) continue;
+          const int off = LPP > 1 ? lds_at<int>(smem, p4, kOff + ((n * LPP + jj) * PPW) * 4) : r_off[n];
+          R smp[VEC];
+#pragma unroll
+          for (int c = 0; c < VEC; ++c) smp[c] = R(0);
+          if (off >= 0) {
+            R4 wt;
+            if constexpr (LPP > 1)
+              wt = lds_at<R4>(smem, p4 * kR4, kWts + ((n * LPP + jj) * PPW) * (int)sizeof(R4));
+            else
+              wt = r_wts[n];
+            if (off != cur1) {
+              cur1 = off;
+              const S *q = view[n] + off;
+              load_vec<S, VEC, false, GAP>(q, tap[0][0]);
+              load_vec<S, VEC, false, GAP>(q + C, tap[0][1]);
+              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[0][2]);
+              load_vec<S, VEC, false, GAP>(q + row_step, tap[0][3]);
+            }
+#pragma unroll
+            for (int c = 0; c < VEC; ++c)
+              smp[c] = wt.x * tap[0][0][c] + wt.y * tap[0][1][c] + wt.z * tap[0][2][c] + wt.w * tap[0][3][c];
+          }
+          if (t.pix_ok)
+            store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d0 + jj) * N + n) * C + ch0, smp);
+        }
+      }
+      if constexpr (LPP > 1) wave_sync();
+      continue;
+    }
+    if constexpr ((CORR == 0 || CORR == 1) && (NV >= 5 || (NV >= 3 && LPP == 4) || kOneSet)) {
       // ---- phase 2, one view at a time (many views) ---------------------------------------
       // With every view's four taps live at once the kernel needs ~25 registers per view
       // (171 for six views: two waves per SIMD).  Here a block of up to eight depths keeps
@@ -843,10 +1062,12 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
       // depth-by-depth loop.  (Measurements decide where this form is used: for three or four
       // views the depth-by-depth loop needs fewer registers at 32+ channels, and with one or
       // two lanes per pixel its taps, which survive from chunk to chunk, matter more.)
-      constexpr int DB = LPP < 8 ? LPP : 8;
+      // (double: blocks of four depths, whose accumulators take the registers of eight in float)
+      constexpr int kMostDB = sizeof(R) == 8 ? 4 : 8;
+      constexpr int DB = LPP < kMostDB ? LPP : kMostDB;
 #pragma unroll
       for (int j0 = 0; j0 < LPP; j0 += DB) {
-      float acc[DB][VEC];
+      R acc[DB][VEC];
       int arg[REDUCE == 1 ? DB : 1][VEC];
       int kcnt[DB];
 #pragma unroll
@@ -854,14 +1075,14 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
         kcnt[jj] = 0;
 #pragma unroll
         for (int c = 0; c < VEC; ++c) {
-          acc[jj][c] = REDUCE == 0 ? 0.f : CORR == 0 ? 3.402823466e+38f : 1.175494351e-38f;
+          acc[jj][c] = REDUCE == 0 ? R(0) : CORR == 0 ? Limits<R>::max() : Limits<R>::min_positive();
           if constexpr (REDUCE == 1) arg[jj][c] = -1;
         }
       }
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         int cur1 = -1;
-        float tp[4][VEC];
+        R tp[4][VEC];
 #pragma unroll
         for (int jj = 0; jj < DB; ++jj) {
           if (d0 + j0 + jj >= d_hi) continue;
@@ -871,33 +1092,38 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
           else
             off = r_off[n];
           if (off < 0) continue;
-          float4 wt;
+          R4 wt;
           if constexpr (LPP > 1)
-            wt = lds_at<float4>(smem, p4 * 4u, kWts + ((n * LPP + j0 + jj) * PPW) * 16);
+            wt = lds_at<R4>(smem, p4 * kR4, kWts + ((n * LPP + j0 + jj) * PPW) * (int)sizeof(R4));
           else
             wt = r_wts[n];
           if (off != cur1) {
             cur1 = off;
             const S *q = view[n] + off;
-            load_vec<S, VEC, false>(q, tp[0]);
-            load_vec<S, VEC, false>(q + C, tp[1]);
-            load_vec<S, VEC, false>(q + row_step + C, tp[2]);
-            load_vec<S, VEC, false>(q + row_step, tp[3]);
+            load_vec<S, VEC, false, GAP>(q, tp[0]);
+            load_vec<S, VEC, false, GAP>(q + C, tp[1]);
+            load_vec<S, VEC, false, GAP>(q + row_step + C, tp[2]);
+            load_vec<S, VEC, false, GAP>(q + row_step, tp[3]);
           }
           ++kcnt[jj];
-          if constexpr (REDUCE == 1) {
-            float val[VEC];
+          if constexpr (REDUCE == 1 || LIT) {
+            R val[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const float smp = wt.x * tp[0][c] + wt.y * tp[1][c] + wt.z * tp[2][c] + wt.w * tp[3][c];
+              const R smp = wt.x * tp[0][c] + wt.y * tp[1][c] + wt.z * tp[2][c] + wt.w * tp[3][c];
               if (CORR == 0) {
-                const float diff = smp - ref[c];
+                const R diff = smp - ref[c];
                 val[c] = diff * diff;
               } else {
                 val[c] = smp * ref[c];
               }
             }
-            if (CORR == 0) {
+            if (REDUCE == 0 && CORR == 0) {
+#pragma unroll
+              for (int c = 0; c < VEC; ++c) acc[jj][c] += val[c];
+            } else if (REDUCE == 0) {
+              add_groups(acc[jj], val, g.sub, t.cl);
+            } else if (CORR == 0) {
 #pragma unroll
               for (int c = 0; c < VEC; ++c)
                 if (acc[jj][c] > val[c]) acc[jj][c] = val[c], arg[jj][c] = n;
@@ -908,17 +1134,17 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
               if (CORR != 1) {
-                float diff = __builtin_fmaf(wt.x, tp[0][c], -ref[c]);
-                diff = __builtin_fmaf(wt.y, tp[1][c], diff);
-                diff = __builtin_fmaf(wt.z, tp[2][c], diff);
-                diff = __builtin_fmaf(wt.w, tp[3][c], diff);
-                acc[jj][c] = __builtin_fmaf(diff, diff, acc[jj][c]);
+                R diff = mad(wt.x, tp[0][c], -ref[c]);
+                diff = mad(wt.y, tp[1][c], diff);
+                diff = mad(wt.z, tp[2][c], diff);
+                diff = mad(wt.w, tp[3][c], diff);
+                acc[jj][c] = mad(diff, diff, acc[jj][c]);
               } else {
-                float smp = wt.x * tp[0][c];
-                smp = __builtin_fmaf(wt.y, tp[1][c], smp);
-                smp = __builtin_fmaf(wt.z, tp[2][c], smp);
-                smp = __builtin_fmaf(wt.w, tp[3][c], smp);
-                acc[jj][c] = __builtin_fmaf(smp, ref[c], acc[jj][c]);
+                R smp = wt.x * tp[0][c];
+                smp = mad(wt.y, tp[1][c], smp);
+                smp = mad(wt.z, tp[2][c], smp);
+                smp = mad(wt.w, tp[3][c], smp);
+                acc[jj][c] = mad(smp, ref[c], acc[jj][c]);
               }
             }
           }
@@ -937,8 +1163,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
               if (arg[jj][c] < 0) acc[jj][c] = dflt;
           }
           if (CORR == 0) {
-            store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc[jj]);
-            store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * VEC, arg[jj]);
+            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc[jj]);
+            store_winners<VEC, LPP, GAP>(mout + ch0, arg[jj]);
           } else {
             store_groups<S, VEC, LPP>(out + goff, acc[jj], g.sub);
             if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg[jj]);
@@ -946,20 +1172,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
             else if (g.sub == 4 || (t.cl & 1)) store_ints<1, whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg[jj]);
           }
         } else {
-          if (kcnt[jj] > 1) {
-            const float inv = __builtin_amdgcn_rcpf(static_cast<float>(kcnt[jj]));
-#pragma unroll
-            for (int c = 0; c < VEC; ++c) acc[jj][c] *= inv;
-          }
+          mean_of<LIT>(acc[jj], kcnt[jj]);
           if (CORR == 0) {
             if (fill && kcnt[jj] == 0) {
 #pragma unroll
               for (int c = 0; c < VEC; ++c) acc[jj][c] = dflt;
             }
-            store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc[jj]);
+            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc[jj]);
           } else {
-            float grp[VEC];
-            fold_groups<VEC>(acc[jj], g.sub, grp);
+            R grp[VEC];
+            fold_or_keep<LIT>(acc[jj], g.sub, grp);
             if (fill && kcnt[jj] == 0) {
 #pragma unroll
               for (int c = 0; c < VEC; ++c) grp[c] = dflt;
@@ -972,7 +1194,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
       if constexpr (LPP > 1) wave_sync();
       continue;
     }
-    float agg_out = 0.f;
+    R agg_out = R(0);
     int v3_out[3] = {-1, -1, -1};
     // ---- phase 2: channel arithmetic by lane (p, channel slice) ---------------------------
 #pragma unroll
@@ -983,25 +1205,25 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
         // from unrolling it and sends its register arrays to scratch memory)
         if constexpr (LPP >= 16) continue; else break;
       }
-      float acc[VEC];
+      R acc[VEC];
       int arg[VEC];  // REDUCE == 1: winning view per channel (or per group)
 #pragma unroll
       for (int c = 0; c < VEC; ++c) {
         // numeric_limits::max() / ::min() seeds, cost_volume_kernels_gpu.cu.cc:174-177 and
         // cost_volume_kernels_gpu_v2.cu.cc:179
-        acc[c] = REDUCE == 0 ? 0.f : CORR == 0 ? 3.402823466e+38f : 1.175494351e-38f;
+        acc[c] = REDUCE == 0 ? R(0) : CORR == 0 ? Limits<R>::max() : Limits<R>::min_positive();
         arg[c] = -1;
       }
       int k = 0;
       float v3_acc = REDUCE == 0 ? 0.f : 1.175494351e-38f;  // :76, :193
       int v3_view = -1, v3_code = 0;
 #pragma unroll
-      for (int n = 0; n < NV; ++n) {
+      for (int n = 0; n < NT; ++n) {
         int off;
-        float4 wt;
+        R4 wt;
         if constexpr (LPP > 1) {
           off = lds_at<int>(smem, p4, kOff + ((n * LPP + jj) * PPW) * 4);
-          wt = lds_at<float4>(smem, p4 * 4u, kWts + ((n * LPP + jj) * PPW) * 16);
+          wt = lds_at<R4>(smem, p4 * kR4, kWts + ((n * LPP + jj) * PPW) * (int)sizeof(R4));
         } else {
           off = r_off[n];
           wt = r_wts[n];
@@ -1011,10 +1233,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
             if (off != cur[n]) {
               cur[n] = off;
               const S *q = view[n] + off;
-              load_vec<S, VEC, false>(q, tap[n][0]);
-              load_vec<S, VEC, false>(q + C, tap[n][1]);
-              load_vec<S, VEC, false>(q + row_step + C, tap[n][2]);
-              load_vec<S, VEC, false>(q + row_step, tap[n][3]);
+              load_vec<S, VEC, false, GAP>(q, tap[n][0]);
+              load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
+              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
+              load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
             }
             float smp[VEC];
 #pragma unroll
@@ -1022,7 +1244,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
               smp[c] = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
                        wt.w * tap[n][3][c];
             const float *ref_row =
-                reinterpret_cast<const float *>(smem + NV * 64 * 20) + t.p * (VEC * LPP);
+                reinterpret_cast<const float *>(smem + kRec) + t.p * (VEC * LPP);
             float best;
             int code;
             if (g.sub == 8)
@@ -1042,17 +1264,17 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
         if constexpr (CORR == 4) {
           // the sample in the reference's operand order (bit-identical to the plain
           // evaluation), zeros for a view that is not accepted
-          float smp[VEC];
+          R smp[VEC];
 #pragma unroll
-          for (int c = 0; c < VEC; ++c) smp[c] = 0.f;
+          for (int c = 0; c < VEC; ++c) smp[c] = R(0);
           if (off >= 0) {
             if (off != cur[n]) {
               cur[n] = off;
               const S *q = view[n] + off;
-              load_vec<S, VEC, false>(q, tap[n][0]);
-              load_vec<S, VEC, false>(q + C, tap[n][1]);
-              load_vec<S, VEC, false>(q + row_step + C, tap[n][2]);
-              load_vec<S, VEC, false>(q + row_step, tap[n][3]);
+              load_vec<S, VEC, false, GAP>(q, tap[n][0]);
+              load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
+              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
+              load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
@@ -1060,32 +1282,37 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
                        wt.w * tap[n][3][c];
           }
           if (n < N && t.pix_ok)
-            store_vec<S, VEC, kNtRows>(a.cost + ((t.pix * D + d) * N + n) * C + t.cl * VEC, smp);
+            store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d) * N + n) * C + ch0, smp);
           continue;
         }
         if (off >= 0) {
           if (off != cur[n]) {
             cur[n] = off;
             const S *q = view[n] + off;
-            load_vec<S, VEC, false>(q, tap[n][0]);
-            load_vec<S, VEC, false>(q + C, tap[n][1]);
-            load_vec<S, VEC, false>(q + row_step + C, tap[n][2]);
-            load_vec<S, VEC, false>(q + row_step, tap[n][3]);
+            load_vec<S, VEC, false, GAP>(q, tap[n][0]);
+            load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
+            load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
+            load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
           }
-          if constexpr (REDUCE == 1) {
-            float val[VEC];
+          if constexpr (REDUCE == 1 || LIT) {
+            R val[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const float smp = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
-                                wt.w * tap[n][3][c];
-              if (CORR == 0) {
-                const float diff = smp - ref[c];
+              const R smp = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
+                            wt.w * tap[n][3][c];
+              if (CORR != 1) {
+                const R diff = smp - ref[c];
                 val[c] = diff * diff;
               } else {
                 val[c] = smp * ref[c];
               }
             }
-            if (CORR == 0) {
+            if (REDUCE == 0 && CORR != 1) {
+#pragma unroll
+              for (int c = 0; c < VEC; ++c) acc[c] += val[c];
+            } else if (REDUCE == 0) {
+              add_groups(acc, val, g.sub, t.cl);
+            } else if (CORR == 0) {
 #pragma unroll
               for (int c = 0; c < VEC; ++c)
                 if (acc[c] > val[c]) acc[c] = val[c], arg[c] = n;
@@ -1099,17 +1326,17 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
           for (int c = 0; c < VEC; ++c) {
             if (CORR != 1) {
               // sample - ref as one chain of fused multiply-adds
-              float diff = __builtin_fmaf(wt.x, tap[n][0][c], -ref[c]);
-              diff = __builtin_fmaf(wt.y, tap[n][1][c], diff);
-              diff = __builtin_fmaf(wt.z, tap[n][2][c], diff);
-              diff = __builtin_fmaf(wt.w, tap[n][3][c], diff);
-              acc[c] = __builtin_fmaf(diff, diff, acc[c]);
+              R diff = mad(wt.x, tap[n][0][c], -ref[c]);
+              diff = mad(wt.y, tap[n][1][c], diff);
+              diff = mad(wt.z, tap[n][2][c], diff);
+              diff = mad(wt.w, tap[n][3][c], diff);
+              acc[c] = mad(diff, diff, acc[c]);
             } else {
-              float smp = wt.x * tap[n][0][c];
-              smp = __builtin_fmaf(wt.y, tap[n][1][c], smp);
-              smp = __builtin_fmaf(wt.z, tap[n][2][c], smp);
-              smp = __builtin_fmaf(wt.w, tap[n][3][c], smp);
-              acc[c] = __builtin_fmaf(smp, ref[c], acc[c]);
+              R smp = wt.x * tap[n][0][c];
+              smp = mad(wt.y, tap[n][1][c], smp);
+              smp = mad(wt.z, tap[n][2][c], smp);
+              smp = mad(wt.w, tap[n][3][c], smp);
+              acc[c] = mad(smp, ref[c], acc[c]);
             }
           }
           ++k;
@@ -1140,8 +1367,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
           S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
           int32_t *mout = mask_pix + d * OC;
           if (CORR == 0) {
-            store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc);
-            store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + t.cl * VEC, arg);
+            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc);
+            store_winners<VEC, LPP, GAP>(mout + ch0, arg);
           } else {
             store_groups<S, VEC, LPP>(out + goff, acc, g.sub);
             if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg);
@@ -1155,20 +1382,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
         // one value per voxel: the pixel's lanes add up their channels; the lane whose
         // slice index equals the depth's place in the chunk keeps the result, so that the
         // chunk is stored as LPP consecutive floats per pixel
-        float tot = group_sum<LPP>((acc[0] + acc[1]) + (acc[2] + acc[3]));
-        tot = k > 0 ? tot / static_cast<float>(k * C) : dflt;
+        R tot = group_sum<LPP>((acc[0] + acc[1]) + (acc[2] + acc[3]));
+        tot = k > 0 ? tot / static_cast<R>(k * C) : dflt;
         if constexpr (LPP > 1) {
           if (t.cl == jj) agg_out = tot;
         } else {
-          if (t.pix_ok) reinterpret_cast<float *>(a.cost)[t.pix * D + d] = tot;
+          if (t.pix_ok) reinterpret_cast<R *>(a.cost)[t.pix * D + d] = tot;
         }
         continue;
       }
-      if (k > 1) {
-        const float inv = __builtin_amdgcn_rcpf(static_cast<float>(k));
-#pragma unroll
-        for (int c = 0; c < VEC; ++c) acc[c] *= inv;
-      }
+      mean_of<LIT>(acc, k);
       if (t.pix_ok) {
         S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
         if (CORR == 0) {
@@ -1176,10 +1399,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
 #pragma unroll
             for (int c = 0; c < VEC; ++c) acc[c] = dflt;
           }
-          store_vec<S, VEC, kNtRows>(out + t.cl * VEC, acc);
+          store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc);
         } else {
-          float grp[VEC];
-          fold_groups<VEC>(acc, g.sub, grp);
+          R grp[VEC];
+          fold_or_keep<LIT>(acc, g.sub, grp);
           if (fill && k == 0) {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) grp[c] = dflt;
@@ -1190,7 +1413,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
     }
     if constexpr ((CORR == 2 || CORR == 3) && LPP > 1) {
       if (t.pix_ok && d0 + t.cl < d_hi)
-        reinterpret_cast<float *>(a.cost)[t.pix * D + d0 + t.cl] = agg_out;
+        reinterpret_cast<R *>(a.cost)[t.pix * D + d0 + t.cl] = agg_out;
     }
     if constexpr (CORR == 3 && REDUCE == 1) {
       if (t.pix_ok && d0 + t.cl < d_hi) {
@@ -1211,14 +1434,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE), 5))
 // holds exactly the texels [oy, oy+ROWS) x [ox, ox+COLS).  Because the slot of a texel
 // depends only on its coordinates, the four slots of a cell are computed once, by the lane
 // that reprojects the voxel, and travel with the record.
-template <int VEC, int LPP, bool SIX = false>
+// The forms of the window: left to the tile's shape, or fixed by the kernel that owns it.
+enum { kPlainWindow = 0, kSixRows = 6, kFourRows = 4 };
+template <int VEC, int LPP, int FORM = kPlainWindow>
 struct Window {
   static constexpr int PPW = 64 / LPP;
   // twice the tile's height by twice its width, at least eight each way: room for the
   // samples' drift in either direction (8 x 8 against 4 x 16 for the 2 x 4 pixels of 32
   // channels: 357 -> 338 us on the MVSNet-stage workload)
   static constexpr int TH = tile_rows(PPW), TW = PPW / TH;
-  // SIX (eight lanes per pixel, 32 channels, 2 x 4 pixels, kernels held to four waves per
+  // kSixRows (eight lanes per pixel, 32 channels, 2 x 4 pixels, kernels held to four waves per
   // SIMD: see backward_waves): six rows instead of eight.  With a 6 KB window the workgroup's
   // LDS is 10 KB, so that sixteen workgroups fit a CU; four rows measured 2 % slower than eight
   // at equal occupancy, six sit between.  The ring index of a row is then a remainder, not a
@@ -1228,7 +1453,10 @@ struct Window {
   // thirteen in; together with the slimming of lean_backward the gradients run three waves
   // per SIMD instead of two (group correlation, four views, 254 x 319 x 16, training pass 2.68
   // -> 1.61 ms; warped features, four views, 73 x 96 x 161: 1218 -> 1045 us).
-  static constexpr int ROWS = SIX ? 6 : LPP == 16 ? 4 : (2 * TH > 8 ? 2 * TH : 8);
+  // Double doubles a slot: kFourRows for eight lanes per pixel.
+  static constexpr int ROWS = FORM == kSixRows                 ? 6
+                              : FORM == kFourRows || LPP == 16 ? 4
+                                                               : (2 * TH > 8 ? 2 * TH : 8);
   static constexpr int COLS = 2 * TW > 8 ? 2 * TW : 8;
   static constexpr int SLOTS = ROWS * COLS;
   static constexpr bool kPow2Rows = (ROWS & (ROWS - 1)) == 0;
@@ -1270,34 +1498,39 @@ struct Window {
 // (see window_add), which needs one claim word per window slot.
 constexpr int kClaimLanes = 8;
 
-// LDS words of the backward kernel: the records of one chunk
-//   float4 wts, dwt [NV*64] | int off [NV*64] | int2 cell {slots, key|inside} [NV*64] |
-//   float scale [64] | float dst [64]
+// LDS bytes of the backward kernel: the records of one chunk
+//   Four wts, dwt [NV*64] | int2 cell {slots, key|inside} [NV*64] | int off [NV*64] |
+//   R scale [64] | R dst [64] (per-voxel depth gradients and CostVolumeV3)
+// The slim form (double, slim_double) keeps one Four {dh, dw, d sh / d depth, d sw / d depth} for both
+// sets of weights, which the lanes expand where a depth starts (ten operations): 64 bytes less
+// per voxel.
 // then the list of texels leaving a window, then the windows.  With one view per workgroup
 // the list shares the record space: a window only moves before the chunk's records are
 // written.
-template <int VEC, int LPP, int NV, bool SIX = false>
-constexpr int backward_record_words() {
-  using WN = Window<VEC, LPP, SIX>;
-  const int rec = LPP > 1 ? NV * 64 * 11 + 128 : 0;
-  const int list = WN::SLOTS * 2;
-  const int w = NV == 1 ? (rec > list ? rec : list) : rec + list;
-  return (w + 3) / 4 * 4;
+template <typename R, int VEC, int LPP, int NV, int FORM = kPlainWindow, bool SLIM = false, bool DST = true>
+constexpr int backward_record_bytes() {
+  using WN = Window<VEC, LPP, FORM>;
+  const int fours = SLIM ? 1 : 2;
+  const int rec = LPP > 1 ? NV * 64 * (fours * 4 * (int)sizeof(R) + 12) + (DST ? 2 : 1) * 64 * (int)sizeof(R) : 0;
+  const int list = WN::SLOTS * 8;
+  const int b = NV == 1 ? (rec > list ? rec : list) : rec + list;
+  return (b + 31) / 32 * 32;
 }
 // The list of a window move between two depths of a chunk, whose records are in use then.
-template <int VEC, int LPP, bool SIX = false>
-constexpr int backward_list_words() {
-  using WN = Window<VEC, LPP, SIX>;
-  return LPP > 1 && WN::SLOTS * 2 > 4 * WN::C ? WN::SLOTS * 2 : 0;
+template <typename R, int VEC, int LPP, int FORM = kPlainWindow>
+constexpr int backward_list_bytes() {
+  using WN = Window<VEC, LPP, FORM>;
+  return LPP > 1 && WN::SLOTS * 8 > 4 * WN::C * (int)sizeof(R) ? WN::SLOTS * 8 : 0;
 }
-template <int VEC, int LPP, int NV, bool SIX = false>
-constexpr int backward_lds_words() {
-  using WN = Window<VEC, LPP, SIX>;
+template <typename R, int VEC, int LPP, int NV, int FORM = kPlainWindow, bool SLIM = false, bool DST = true>
+constexpr int backward_lds_bytes() {
+  using WN = Window<VEC, LPP, FORM>;
   // records (or list), windows, one cell (4 texels x C) staged on its way to memory, and for
   // narrow pixels one claim word per window slot
   // and, where that cell's place is too small for it, the list of a move inside a chunk
-  return backward_record_words<VEC, LPP, NV, SIX>() + NV * WN::SLOTS * WN::STRIDE + 4 * WN::C +
-         (LPP <= kClaimLanes ? WN::SLOTS : 0) + backward_list_words<VEC, LPP, SIX>();
+  return backward_record_bytes<R, VEC, LPP, NV, FORM, SLIM, DST>() +
+         (NV * WN::SLOTS * WN::STRIDE + 4 * WN::C) * (int)sizeof(R) +
+         (LPP <= kClaimLanes ? WN::SLOTS * 4 : 0) + backward_list_bytes<R, VEC, LPP, FORM>();
 }
 
 // Minimum over the 64 lanes, in registers: four DPP steps reduce each row of 16 lanes,
@@ -1316,10 +1549,10 @@ __device__ __forceinline__ int wave_min(int v) {
 // texels per instruction, UN instructions per round: their LDS reads go out together) and its
 // slot is cleared.  Uniform control flow.  `cm`: channels of a texel in memory (a slot may be
 // padded; padding stays zero and is never written out).
-template <int VEC, int LPP, bool SIX = false, int UN = 4>
-__device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, float *data,
-                                            int *list, float *gview, int srcW, int lane, int cm) {
-  using WN = Window<VEC, LPP, SIX>;
+template <int VEC, int LPP, int FORM = kPlainWindow, int UN = 4, typename R>
+__device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R *data,
+                                            int *list, R *gview, int srcW, int lane, int cm) {
+  using WN = Window<VEC, LPP, FORM>;
   if (oy != WN::kNone) {
     wave_sync();  // the adds of the chunk before are complete and visible
     int count = 0;
@@ -1345,7 +1578,7 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, fl
       const int2 *pairs = reinterpret_cast<const int2 *>(list);
       for (int e0 = 0; e0 < count; e0 += UN * EPI) {
         int2 le[UN];
-        float v[UN];
+        R v[UN];
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
           const int e = e0 + u * EPI + sub_e;
@@ -1353,11 +1586,11 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, fl
           if (e >= count) le[u].x = -1;
         }
 #pragma unroll
-        for (int u = 0; u < UN; ++u) v[u] = le[u].x >= 0 ? data[le[u].x * WN::STRIDE + j] : 0.f;
+        for (int u = 0; u < UN; ++u) v[u] = le[u].x >= 0 ? data[le[u].x * WN::STRIDE + j] : R(0);
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
-          if (v[u] != 0.f) {
-            data[le[u].x * WN::STRIDE + j] = 0.f;
+          if (v[u] != R(0)) {
+            data[le[u].x * WN::STRIDE + j] = R(0);
             atomic_add(gview + (int64_t)le[u].y * cm + j, v[u]);
           }
         }
@@ -1384,10 +1617,10 @@ __device__ __forceinline__ unsigned wave_or(unsigned v) {
 // set when a cell used ring row r; a short sweep over few hypotheses touches three or four
 // of the eight, and the untouched ones need neither their LDS reads nor their address
 // arithmetic).  All LDS reads of a row are issued together, then its atomics.
-template <int VEC, int LPP, bool SIX = false>
-__device__ __forceinline__ void window_flush_all(int oy, int ox, const float *data, float *gview,
+template <int VEC, int LPP, int FORM = kPlainWindow, typename R>
+__device__ __forceinline__ void window_flush_all(int oy, int ox, const R *data, R *gview,
                                                  int srcW, int lane, unsigned rows, int cm) {
-  using WN = Window<VEC, LPP, SIX>;
+  using WN = Window<VEC, LPP, FORM>;
   if (oy == WN::kNone) return;
   wave_sync();  // the last adds are complete and visible
   constexpr int C = WN::C;
@@ -1398,11 +1631,12 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
     // instructions whose LDS reads go out together, so that the wave waits for the LDS once
     // per batch instead of once per row (315 against 325 us on the MVSNet-stage workload)
     constexpr int NI = WN::SLOTS * C / 64;
-    constexpr int BATCH = NI < 32 ? NI : 32;
+    constexpr int MOST = sizeof(R) == 4 ? 32 : NI % 16 == 0 ? 16 : 8;
+    constexpr int BATCH = NI < MOST ? NI : MOST;
     static_assert(NI % BATCH == 0, "whole batches");
 #pragma unroll 1
     for (int i0 = 0; i0 < NI; i0 += BATCH) {
-      float v[BATCH];
+      R v[BATCH];
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) v[u] = data[(i0 + u) * 64 + lane];
 #pragma unroll
@@ -1411,7 +1645,7 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
         const int sl = e / C, ch = e - sl * C;
         const int ry = sl / WN::COLS, rx = sl - ry * WN::COLS;
         const int y = WN::image_row(ry, oy), x = ox + ((rx - ox) & (WN::COLS - 1));
-        if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
+        if (v[u] != R(0)) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
       }
     }
     return;
@@ -1420,7 +1654,7 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
   for (int ry = 0; ry < WN::ROWS; ++ry) {
     if (!((rows >> ry) & 1u)) continue;  // uniform
     const int y = WN::image_row(ry, oy);
-    float v[PER_ROW];
+    R v[PER_ROW];
 #pragma unroll
     for (int u = 0; u < PER_ROW; ++u) v[u] = data[(ry * PER_ROW + u) * 64 + lane];
 #pragma unroll
@@ -1429,7 +1663,7 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
       const int rx = e / C, ch = e - rx * C;
       const int x = ox + ((rx - ox) & (WN::COLS - 1));
       // (a slot that was never added to holds zero: texels outside the image never are)
-      if (v[u] != 0.f) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
+      if (v[u] != R(0)) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
     }
   }
 }
@@ -1448,11 +1682,10 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const float *da
 // from 429 to 400 us; against LDS atomics it halved the time of the 8-channel workloads.
 // 16 lanes per pixel (four pixels per wave): the pixels that fire in the same instruction
 // take turns, one pixel per round with its four taps in flight together.
-template <int VEC, int LPP, bool LEAN = false, bool SIX = false>
-__device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4][VEC],
-                                           float *data, int *tags, int lane, int cl) {
-  using WN = Window<VEC, LPP, SIX>;
-  typedef float vecf __attribute__((ext_vector_type(VEC)));
+template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP = 2, typename R>
+__device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VEC],
+                                           R *data, int *tags, int lane, int cl) {
+  using WN = Window<VEC, LPP, FORM>;
   if (key < 0) {
     // the whole cell lies inside the window (the usual case)
     if constexpr (!WN::kPacked) slots = 0;
@@ -1466,22 +1699,21 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
       const int rx0 = fw & (WN::COLS - 1), rx1 = (fw + 1) & (WN::COLS - 1);
       slot[0] = ry0 + rx0, slot[1] = ry0 + rx1, slot[2] = ry1 + rx1, slot[3] = ry1 + rx0;
     }
-    float *base = data + cl * VEC;
+    R *base = data + lane_first(cl, GAP);
     if constexpr (LPP > kClaimLanes) {
       unsigned long long firing = __ballot(true);
       while (firing) {
         const int lead = __ffsll((long long)firing) - 1;
         firing &= ~(((1ull << LPP) - 1ull) << lead);  // retire this pixel's lanes
         if (lane - cl == lead) {
-          vecf old[4];
+          R old[4][VEC];
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            old[k] = *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE);
+          for (int k = 0; k < 4; ++k) slot_read<GAP>(base + slot[k] * WN::STRIDE, old[k]);
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) old[k][i] += v[k][i];
-            *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE) = old[k];
+            slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
         if (firing) wave_sync();
@@ -1496,21 +1728,21 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
         if constexpr (LEAN) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            vecf old = *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE);
+            R old[VEC];
+            slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) old[i] += v[k][i];
-            *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE) = old;
+            slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
           }
         } else {
-          vecf old[4];
+          R old[4][VEC];
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            old[k] = *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE);
+          for (int k = 0; k < 4; ++k) slot_read<GAP>(base + slot[k] * WN::STRIDE, old[k]);
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) old[k][i] += v[k][i];
-            *reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE) = old[k];
+            slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
         pending = false;
@@ -1522,11 +1754,11 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
         if (go) {
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            vecf *d = reinterpret_cast<vecf *>(base + slot[k] * WN::STRIDE);
-            vecf old = *d;
+            R old[VEC];
+            slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
             for (int i = 0; i < VEC; ++i) old[i] += v[k][i];
-            *d = old;
+            slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
             // (the next tap may be the texel another pixel has just updated: the LDS keeps a
             // wave's operations in order, the compiler is held to it here)
             wave_sync();
@@ -1542,7 +1774,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
 #pragma unroll
   for (int k = 0; k < 4; ++k)
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) v[k][i] = 0.f;
+    for (int i = 0; i < VEC; ++i) v[k][i] = R(0);
 }
 
 // Cells that no window position covers (the tile's pixels of one depth further apart than the
@@ -1552,13 +1784,11 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, float (&v)[4
 // and the whole wave adds each row as a dense run of 2*C consecutive floats.  Added lane by
 // lane from the registers, each 16-byte chunk of a texel would carry one float per
 // instruction, and the atomics cost per chunk, not per float.
-template <int VEC, int LPP>
+template <int VEC, int LPP, int GAP, typename R>
 __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool mine, int key,
-                                                      float (&v)[4][VEC], float *stage,
-                                                      float *gview, int srcW, int lane, int cl,
+                                                      R (&v)[4][VEC], R *stage, R *gview, int srcW, int lane, int cl,
                                                       int cm) {
   constexpr int C = VEC * LPP;
-  typedef float vecf __attribute__((ext_vector_type(VEC)));
   while (m) {
     const int lead = __ffsll((long long)m) - 1;
     m &= ~(((1ull << LPP) - 1ull) << lead);
@@ -1566,25 +1796,21 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
     if (lane - cl == lead) {
       // taps 00, 01 (row fh), then 10, 11 (row fh + 1); v is ordered 00, 01, 11, 10
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        vecf w;
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) w[i] = v[k][i];
-        *reinterpret_cast<vecf *>(stage + (k == 2 ? 3 : k == 3 ? 2 : k) * C + cl * VEC) = w;
-      }
+      for (int k = 0; k < 4; ++k)
+        slot_write<GAP>(stage + (k == 2 ? 3 : k == 3 ? 2 : k) * C + lane_first(cl, GAP), v[k]);
     }
     wave_sync();
     const int fh = k2 >> 16, fw = k2 & 0xffff;
-    float *row0 = gview + (int64_t)(fh * srcW + fw) * cm;
-    float *row1 = row0 + (int64_t)srcW * cm;
+    R *row0 = gview + (int64_t)(fh * srcW + fw) * cm;
+    R *row1 = row0 + (int64_t)srcW * cm;
 #pragma unroll
     for (int f0 = 0; f0 < 2 * C; f0 += 64) {
       const int f = f0 + lane;
       if (f < 2 * C) {
-        const float a0 = stage[f], a1 = stage[2 * C + f];
+        const R a0 = stage[f], a1 = stage[2 * C + f];
         const int e = f / C * cm + f % C;
-        if (a0 != 0.f) atomic_add(row0 + e, a0);
-        if (a1 != 0.f) atomic_add(row1 + e, a1);
+        if (a0 != R(0)) atomic_add(row0 + e, a0);
+        if (a1 != R(0)) atomic_add(row1 + e, a1);
       }
     }
     wave_sync();
@@ -1593,7 +1819,7 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) v[k][i] = 0.f;
+      for (int i = 0; i < VEC; ++i) v[k][i] = R(0);
   }
 }
 
@@ -1620,13 +1846,25 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // depth loop: bf16 group-correlation backward 479 -> 462 us cold, 447 -> 417 us warm.
 // Sixteen lanes per pixel (64 channels): slimmed, all of them, to three waves (164-222 registers
 // left alone, 132-164 slimmed; LDS holds them to 13 workgroups per CU, see Window::ROWS).
-constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false) {
-  return nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
+// Double: the slimmed code at two waves per SIMD (taps, tap sums and rows of four channels are 100
+// registers before anything else, 182-206 in all), whole records and the six-row window, which fit two waves'
+// share of the LDS.  Held to 168 registers for a third wave, with the slim records (slim_double), the cameras'
+// row products computed again for every chunk and a window of four rows, the gradients that stream
+// upstream rows spill 76-130 bytes around the depth loop, and a reload from scratch waits for the
+// rows requested before it: 32 channels, two views, 128 x 160 x 192: 745 us against 532 (lane per
+// channel: 940), minimum over three views x 64 751 against 372 (673).  CostAggregate has no rows and
+// does not spill: three views, 149 x 220 x 116, 524 against 584 us (1460); 64 channels, where LDS holds
+// either form to seven workgroups, 364 against 275 us (630); one lane per pixel has no records in LDS.
+constexpr bool slim_double(int lpp, int corr) { return corr == 2 && lpp > 1 && lpp <= 8; }
+constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false,
+                             bool wide_real = false) {
+  return wide_real ? true : nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
                      (lpp == 4 && corr <= 1 && reduce == 0) ||
                      (lpp == 2 && corr <= 1 && reduce == 0));
 }
-constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false) {
-  return lpp == 16 && nv == 1                             ? 3
+constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false,
+                             bool wide_real = false) {
+  return wide_real ? (slim_double(lpp, corr) ? 3 : 2) : lpp == 16 && nv == 1                             ? 3
          : lean_backward(nv, lpp, corr, reduce, wide) ? 4
          : nv == 1 && lpp <= 8                       ? 3
          : nv <= 2                                   ? 2
@@ -1657,47 +1895,57 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // 213 x 86, 627 -> 344 us).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool DG = true,
           bool PV = (CORR == 1), bool VLOOP = false, bool WIDE = false, bool PAD = false>
-__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) void backward_kernel(const Args<S> a,
-                                                                          const Geometry g) {
-  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, WIDE);
-  constexpr bool kSix = kLean && LPP == 8;
-  using WN = Window<VEC, LPP, kSix>;
+__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE, sizeof(S) == 8)) void backward_kernel(
+    const Args<S> a, const Geometry g) {
+  using R = typename Storage<S>::Real;
+  using R4 = Four<R>;
+  constexpr bool kDouble = sizeof(S) == 8;
+  constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
+  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, WIDE, kDouble);
+  constexpr bool kSlim = kDouble && slim_double(LPP, CORR);
+  constexpr int kForm = !(kLean && LPP == 8) ? kPlainWindow : kSlim ? kFourRows : kSixRows;
+  using WN = Window<VEC, LPP, kForm>;
   constexpr int PPW = 64 / LPP;
   constexpr bool kWide = sizeof(S) == 2;  // gradients accumulate in fp32 images
   extern __shared__ __align__(16) unsigned char smem[];
   Tile<LPP> t;
   if (!locate_tile<S, LPP>(a, g, t)) return;
   const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
-  const float half = a.half;
+  const R half = a.half;
   constexpr bool per_voxel_depth = PV;
+  constexpr bool kDstWords = !kSlim || PV;
   // byte offsets of the record arrays; a record is addressed as (lane-dependent byte offset)
   // + (compile-time constant), so that the constant lands in the instruction's offset field
-  constexpr int kWts = 0, kDwt = kWts + NV * 64 * 16, kCell = kDwt + NV * 64 * 16,
-                kOff = kCell + NV * 64 * 8, kScl = kOff + NV * 64 * 4, kDst = kScl + 64 * 4;
+  constexpr int kB = (int)sizeof(R), kB4 = (int)sizeof(R4);
+  constexpr int kWts = 0, kDwt = kWts + (kSlim ? 0 : NV * 64 * kB4), kCell = kDwt + NV * 64 * kB4,
+                kOff = kCell + NV * 64 * 8, kScl = kOff + NV * 64 * 4, kDst = kScl + 64 * kB;
   const unsigned p4 = (unsigned)t.p * 4u;                      // reader: pixel p
   const unsigned q4 = (unsigned)(t.cl * PPW + t.p) * 4u;       // writer: lane (p, j)
+  const unsigned p1 = p4 * (unsigned)(kB / 4), q1 = q4 * (unsigned)(kB / 4);  // one R per voxel
+  const unsigned pw = p4 * (unsigned)kB, qw = q4 * (unsigned)kB;               // four
   int *s_list = NV == 1 ? reinterpret_cast<int *>(smem)
-                        : reinterpret_cast<int *>(smem) + (LPP > 1 ? NV * 64 * 11 + 128 : 0);
-  float *s_data = reinterpret_cast<float *>(smem) + backward_record_words<VEC, LPP, NV, kSix>();
-  float *s_stage = s_data + NV * WN::SLOTS * WN::STRIDE;
+                        : reinterpret_cast<int *>(smem + (LPP > 1 ? kDst + 64 * kB : 0));
+  R *s_data = reinterpret_cast<R *>(smem + backward_record_bytes<R, VEC, LPP, NV, kForm, kSlim, kDstWords>());
+  R *s_stage = s_data + NV * WN::SLOTS * WN::STRIDE;
   int *s_tags = reinterpret_cast<int *>(s_stage + 4 * WN::C);  // narrow pixels: claim words
   static_assert(LPP > kClaimLanes || NV == 1, "one set of claim words: one view per workgroup");
   int *s_own_list = s_tags + (LPP <= kClaimLanes ? WN::SLOTS : 0);
   // (LPP == 1: the records are in registers)
   int *s_move_list = LPP == 1                                         ? s_list
-                     : backward_list_words<VEC, LPP, kSix>() > 0 ? s_own_list
+                     : backward_list_bytes<R, VEC, LPP, kForm>() > 0 ? s_own_list
                                                                  : reinterpret_cast<int *>(s_stage);
   // CORR 3 only: reference rows, sample rows
-  float *s_v3 = reinterpret_cast<float *>(s_own_list + backward_list_words<VEC, LPP, kSix>());
+  float *s_v3 = reinterpret_cast<float *>(s_own_list + backward_list_bytes<R, VEC, LPP, kForm>() / 4);
   static_assert(CORR != 3 || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
-  const float base = per_voxel_depth ? 0.f : a.base_plane[t.pix];
+  const R base = per_voxel_depth ? R(0) : a.base_plane[t.pix];
   static_assert(!PAD || CORR != 3, "CostVolumeV3: whole pixels");
   const int cm = PAD ? C : WN::C;
   const bool ch_ok = !PAD || t.cl * VEC < C;
   const int clc = PAD ? min(t.cl, C / VEC - 1) : t.cl;  // the lane whose channels this lane reads
-  float ref[VEC];
+  const int ch0 = lane_first(clc, GAP);
+  R ref[VEC];
   if constexpr (CORR != 4) {
-    load_vec<S, VEC, false>(a.ref + t.pix * C + clc * VEC, ref);
+    load_vec<S, VEC, false, GAP>(a.ref + t.pix * C + ch0, ref);
     if constexpr (CORR == 3) {
 #pragma unroll
       for (int c = 0; c < VEC; ++c) s_v3[t.p * (VEC * LPP) + t.cl * VEC + c] = ref[c];
@@ -1705,16 +1953,18 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   } else {
     static_assert(CORR != 4 || NV == 1, "the warp-only gradient runs one view per workgroup");
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) ref[c] = 0.f;
+    for (int c = 0; c < VEC; ++c) ref[c] = R(0);
   }
   const int64_t view_elems = (int64_t)srcH * srcW * C;
-  float *src_grad_img = kWide ? a.src_grad_acc : reinterpret_cast<float *>(a.src_grad);
+  R *src_grad_img;
+  if constexpr (kWide) src_grad_img = a.src_grad_acc;
+  else src_grad_img = a.src_grad;
   const int row_step = srcW * C;
-  const unsigned lane_ch = (unsigned)(clc * VEC);
-  float racc[VEC];
+  const unsigned lane_ch = (unsigned)ch0;
+  R racc[VEC];
 #pragma unroll
-  for (int c = 0; c < VEC; ++c) racc[c] = 0.f;
-  float dacc = 0.f;  // base-plane gradient partial of this lane
+  for (int c = 0; c < VEC; ++c) racc[c] = R(0);
+  R dacc = R(0);  // base-plane gradient partial of this lane
 
   // CORR: 0 squared difference per channel, 1 group correlation, 2 squared difference
   // summed over all channels (one upstream gradient per voxel), 4 the warp alone: one
@@ -1738,7 +1988,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   constexpr int kFewRuns = !kWinners ? 0 : CORR == 3 ? 4 : PPW / 8;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
   const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
-  const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : clc * VEC;
+  const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : ch0;
   const int d_lo = t.d_lo, d_hi = t.d_hi;
   // upstream-gradient rows fetched ahead; the MIN reduce stages the mask rows beside them
   constexpr int PFMAX = (REDUCE || kLean) ? 4 : 8;
@@ -1750,7 +2000,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   // element steps from one depth to the next in the upstream gradient and in the mask
   const int cg_step = CORR == 4 ? N * C : OC;
   const int cnt_step = CORR == 4 ? N : mask_w;
-  const float *dv_src = per_voxel_depth ? a.depth_grid + t.pix * D : a.offsets + (int64_t)t.b * D;
+  const R *dv_src = per_voxel_depth ? a.depth_grid + t.pix * D : a.offsets + (int64_t)t.b * D;
   // The views of this workgroup's group take turns (NV at a time; NV = 1 in every launch):
   // each gets the scatter window to itself and leaves it empty.  What belongs to the pixel
   // (reference gradient, depth gradients, the upstream rows in the caches) is shared, so a
@@ -1767,12 +2017,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     asm volatile("" : "+v"(t.lane), "+v"(t.cl), "+v"(t.p), "+v"(t.pix), "+v"(t.h), "+v"(t.w));
   }
   for (int k = t.lane * 4; k < NV * WN::SLOTS * WN::STRIDE; k += 256)
-    *reinterpret_cast<float4 *>(s_data + k) = make_float4(0.f, 0.f, 0.f, 0.f);
-  Cameras<NV> cam;
-  load_cameras<S, NV>(a, t.b, t.view0, static_cast<float>(t.w) + half,
-                      static_cast<float>(t.h) + half, cam);
+    *reinterpret_cast<R4 *>(s_data + k) = R4{R(0), R(0), R(0), R(0)};
+  Cameras<NV, R> cam;
+  if constexpr (!kSlim)
+    load_cameras<S, NV>(a, t.b, t.view0, static_cast<R>(t.w) + half, static_cast<R>(t.h) + half, cam);
+  int cam_w = t.w, cam_h = t.h;
   const S *view[NV];
-  float *gview[NV];  // gradient image of the view, no lane offset
+  R *gview[NV];  // gradient image of the view, no lane offset
   int oy[NV], ox[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
@@ -1781,7 +2032,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     gview[n] = src_grad_img + vo;
     oy[n] = ox[n] = WN::kNone;
   }
-  float tap[NV][4][VEC], sg[NV][4][VEC];
+  R tap[NV][4][VEC], sg[NV][4][VEC];
   int cur[NV];     // tap offset of the open run, -1: none
   int2 cell[NV];   // its slots and key (bit 31: inside the window)
   unsigned ring_rows[NV];  // ring rows of the window this lane's accepted cells mapped to
@@ -1793,10 +2044,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int c = 0; c < VEC; ++c) sg[n][k][c] = 0.f;
+      for (int c = 0; c < VEC; ++c) sg[n][k][c] = R(0);
   }
   const S *cg_lane =
-      CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + clc * VEC
+      CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + ch0
                 : a.cost_grad + t.pix * D * OC + (kVoxelGrad ? 0 : goff);
   const int32_t *cnt_src = CORR == 4 ? a.mask_in + t.pix * D * N + t.view0
                                      : a.mask_in + t.pix * D * mask_w;
@@ -1833,14 +2084,14 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
         const int ny = wave_min(fire ? fh : WN::kNone), nx = wave_min(fire ? fw : WN::kNone);
         const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
         const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
-        window_move<VEC, LPP, kSix, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
+        window_move<VEC, LPP, kForm, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
                                     s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane, cm);
         in = WN::inside(key, oy[n], ox[n]);
       }
       const bool out = fire && !in;
       const unsigned long long m = __ballot(out);
       if (m != 0ull) {
-        flush_cells_to_memory<VEC, LPP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl, cm);
+        flush_cells_to_memory<VEC, LPP, GAP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl, cm);
         if (out) cur[n] = -1;
       }
     }
@@ -1851,14 +2102,14 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     // Depth hypothesis and valid-view count of lane (p, j)'s voxel: requested before the
     // chunk's upstream-gradient rows, because loads return in order and the reprojection
     // should wait for these two words only.
-    float dv = 1.f, cg_vox = 0.f;
+    R dv = R(1), cg_vox = R(0);
     int cnt = REDUCE ? -1 : 0;  // "nothing to do" for a lane without a voxel
     int v3_pair = kNoPair;
     if (d0 + t.cl < d_hi) {
       dv = dv_src[d0 + t.cl];
       if (t.pix_ok) cnt = cnt_src[(int64_t)(d0 + t.cl) * cnt_step];
       if constexpr (kVoxelGrad)  // the voxel's one upstream gradient rides with its record
-        cg_vox = reinterpret_cast<const float *>(cg_lane)[d0 + t.cl];
+        cg_vox = reinterpret_cast<const R *>(cg_lane)[d0 + t.cl];
       if constexpr (CORR == 3 && REDUCE == 1) {
         if (t.pix_ok) {
           const int64_t m3 = (int64_t)(d0 + t.cl) * 3;
@@ -1873,8 +2124,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     }
     int r_off[NV];
     int2 r_cell[NV];
-    float r_scl = 0.f;
-    float4 r_wts[NV], r_dwt[NV];
+    R r_scl = R(0);
+    R4 r_wts[NV], r_dwt[NV];
     bool spread[NV];  // the cells of this chunk and the open ones do not fit the window together
     // Issue the loads of this chunk's cost_grad rows now, unconditionally, so that the
     // reprojection below overlaps their latency.  Through the caches: the workgroups of a
@@ -1885,7 +2136,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     // kernel's output, which a load that allocates has to push out first.
     // (whole rows are kept as loaded and widened to float where a depth uses them; group
     // rows, whose width is a run-time value, are widened here and kept as float bits)
-    uint32_t cgw[kVoxelGrad ? 1 : PF][(CORR == 0 || CORR == 4) ? raw_words<S, VEC>() : VEC];
+    RawWord<S> cgw[kVoxelGrad ? 1 : PF][(CORR == 0 || CORR == 4) ? raw_words<S, VEC>() : VEC];
     int mrow[kMaskRows ? PF : 1][VEC];
     auto load_rows = [&](int first) {
       if constexpr (CORR == 1) {
@@ -1896,7 +2147,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
 #pragma unroll
           for (int jj = 0; jj < PF; ++jj) {
             const int d = min(first + jj, d_hi - 1);
-            load_vec<S, CNT, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<float *>(cgw[jj]));
+            load_vec<S, CNT, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<R *>(cgw[jj]));
           }
         };
         if (g.sub == 1) group_rows(std::integral_constant<int, VEC>());
@@ -1910,13 +2161,16 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
         // (each view of FeatureAggregate has rows of its own: streamed where they cover whole
         // lines)
         if constexpr (CORR == 0)
-          load_raw<S, VEC, false>(src_cg, cgw[jj]);
+          load_raw<S, VEC, false, GAP>(src_cg, cgw[jj]);
         if constexpr (CORR == 4)
-          load_raw<S, VEC, whole_lines(VEC * LPP, (int)sizeof(S))>(src_cg, cgw[jj]);
+          load_raw<S, VEC, whole_lines(VEC * LPP, (int)sizeof(S)), GAP>(src_cg, cgw[jj]);
         if constexpr (kMaskRows) {
           const int32_t *m = mask_lane + (int64_t)d * OC;
           const int cntv = CORR == 0 ? VEC : gv;
-          if (cntv == 4) {
+          if (GAP != 2) {
+            const int2 lo = *reinterpret_cast<const int2 *>(m), hi = *reinterpret_cast<const int2 *>(m + GAP);
+            mrow[jj][0] = lo.x, mrow[jj][1] = lo.y, mrow[jj][2] = hi.x, mrow[jj][3] = hi.y;
+          } else if (cntv == 4) {
             typedef int i32x4 __attribute__((ext_vector_type(4)));
             const i32x4 *q = reinterpret_cast<const i32x4 *>(m);
             const i32x4 v = *q;
@@ -1934,49 +2188,60 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
     };
     if constexpr (!kVoxelGrad) load_rows(d0);
     {
-      const float depth = d0 + t.cl < d_hi ? (per_voxel_depth ? dv : base + dv) : 1.f;
+      const R depth = d0 + t.cl < d_hi ? (per_voxel_depth ? dv : base + dv) : R(1);
       // factor the reduce applies to the upstream gradient: squared difference 2/k,
       // correlation 1/k, summed squared difference 2*cost_grad/(k*C) (the whole per-voxel
       // factor); zero marks a voxel that contributes nothing
-      float scl = 0.f;
+      // (a division in double is fifty instructions: there the reciprocal serves)
+      if constexpr (kSlim) {
+        // (computed again for every chunk: as values of the whole walk they would be 24 registers; the
+        // compiler would make them that if it could see through the pixel's coordinates)
+        asm volatile("" : "+v"(cam_w), "+v"(cam_h));
+        load_cameras<S, NV>(a, t.b, t.view0, static_cast<R>(cam_w) + half, static_cast<R>(cam_h) + half, cam);
+      }
+      R scl = R(0);
       if constexpr (REDUCE == 0) {
         if (cnt > 0) {
-          if constexpr (CORR == 2)
-            scl = 2.f * (cg_vox / static_cast<float>(cnt * C));
+          if constexpr (CORR == 2 && kDouble)
+            scl = R(2) * cg_vox * quick_recip(static_cast<R>(cnt * C));
+          else if constexpr (CORR == 2)
+            scl = R(2) * (cg_vox / static_cast<R>(cnt * C));
           else if constexpr (CORR == 3)
-            scl = cg_vox / static_cast<float>(cnt);  // cost_volume_kernels_gpu_v3.cu.cc:426
+            scl = cg_vox / static_cast<R>(cnt);  // cost_volume_kernels_gpu_v3.cu.cc:426
           else
-            scl = (CORR == 0 ? 2.f : 1.f) * __builtin_amdgcn_rcpf(static_cast<float>(cnt));
+            scl = (CORR == 0 ? R(2) : R(1)) * quick_recip(static_cast<R>(cnt));
         }
       } else {
         // no division by the view count; `cnt` holds the first mask entry of the voxel (or,
         // for the summed squared difference, its winning view)
         if constexpr (CORR == 2) {
-          if (cnt == t.view0) scl = 2.f * (cg_vox / static_cast<float>(C));
+          if (cnt == t.view0) scl = R(2) * (cg_vox / static_cast<R>(C));
         } else if constexpr (CORR == 3) {
           if (cnt == t.view0) scl = cg_vox;  // cost_volume_kernels_gpu_v3.cu.cc:621-622
         } else {
-          if (cnt >= 0) scl = CORR == 0 ? 2.f : 1.f;
+          if (cnt >= 0) scl = CORR == 0 ? R(2) : R(1);
         }
       }
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        Hit hit;
+        Hit<R> hit;
         hit.off = -1;
         hit.key = 0;
-        hit.k00 = hit.k01 = hit.k11 = hit.k10 = 0.f;
-        float4 dw4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t.view0 + n < N && scl != 0.f) {
-          reproject<NV>(cam, n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
+        hit.k00 = hit.k01 = hit.k11 = hit.k10 = R(0);
+        hit.dh = hit.dw = R(0);
+        R4 dw4 = R4{R(0), R(0), R(0), R(0)};
+        if (t.view0 + n < N && scl != R(0)) {
+          reproject<NV, R>(cam, n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
           if (DG && hit.off >= 0) {
             // d(sample)/d(depth) = sum over taps of dwt * tap, from
             //   d/d(src_h) = t1*dw + (t10 - t00),  d/d(src_w) = t1*dh + (t01 - t00),
             //   t1 = t11 - t10 - t01 + t00, chained through the perspective divide.
-            const float inv = __builtin_amdgcn_rcpf(hit.z * hit.z);
-            const float ah = (cam.hc[n] * hit.z - cam.zc[n] * hit.h3d) * inv;
-            const float aw = (cam.wc[n] * hit.z - cam.zc[n] * hit.w3d) * inv;
-            const float cp = ah * hit.dw + aw * hit.dh;
-            dw4 = make_float4(cp - ah - aw, aw - cp, cp, ah - cp);  // taps 00, 01, 11, 10
+            const R inv = quick_recip(hit.z * hit.z);
+            const R ah = (cam.hc[n] * hit.z - cam.zc[n] * hit.h3d) * inv;
+            const R aw = (cam.wc[n] * hit.z - cam.zc[n] * hit.w3d) * inv;
+            const R cp = ah * hit.dw + aw * hit.dh;
+            dw4 = R4{cp - ah - aw, aw - cp, cp, ah - cp};
+            if constexpr (kSlim) dw4 = R4{R(0), R(0), ah, aw};  // taps 00, 01, 11, 10
           }
         }
         // The scatter window has to cover this chunk's cells and the cell still open from
@@ -2013,7 +2278,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
               const bool left = !spread[n] && cur[n] >= 0 && !WN::inside(key, ny - sy / 2, nx - sx / 2);
               const unsigned long long m = __ballot(left);
               if (m != 0ull) {
-                flush_cells_to_memory<VEC, LPP>(m, left, key, sg[n], s_stage, gview[n], srcW, t.lane, t.cl, cm);
+                flush_cells_to_memory<VEC, LPP, GAP>(m, left, key, sg[n], s_stage, gview[n], srcW, t.lane, t.cl, cm);
                 if (left) cur[n] = -1;
               }
             }
@@ -2022,7 +2287,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
             in_new = false;  // decided when the run ends
             cell[n].y &= 0x7fffffff;
           } else {
-            window_move<VEC, LPP, kSix>(oy[n], ox[n], ny - sy / 2, nx - sx / 2,
+            window_move<VEC, LPP, kForm>(oy[n], ox[n], ny - sy / 2, nx - sx / 2,
                                   s_data + n * WN::SLOTS * WN::STRIDE, s_list, gview[n], srcW, t.lane, cm);
             in_new = true;
             cell[n].y |= WN::kInside;
@@ -2033,39 +2298,42 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
         if constexpr (LPP > 1) {
           lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = hit.off;
           lds_at<int2>(smem, q4 * 2u, kCell + (n * LPP * PPW) * 8) = rec;
-          lds_at<float4>(smem, q4 * 4u, kWts + (n * LPP * PPW) * 16) =
-              make_float4(hit.k00, hit.k01, hit.k11, hit.k10);
-          if constexpr (DG) lds_at<float4>(smem, q4 * 4u, kDwt + (n * LPP * PPW) * 16) = dw4;
+          if constexpr (kSlim) {
+            lds_at<R4>(smem, qw, kWts + (n * LPP * PPW) * kB4) = R4{hit.dh, hit.dw, dw4.z, dw4.w};
+          } else {
+            lds_at<R4>(smem, qw, kWts + (n * LPP * PPW) * kB4) = R4{hit.k00, hit.k01, hit.k11, hit.k10};
+            if constexpr (DG) lds_at<R4>(smem, qw, kDwt + (n * LPP * PPW) * kB4) = dw4;
+          }
         } else {
           r_off[n] = hit.off;
           r_cell[n] = rec;
-          r_wts[n] = make_float4(hit.k00, hit.k01, hit.k11, hit.k10);
+          r_wts[n] = R4{hit.k00, hit.k01, hit.k11, hit.k10};
           r_dwt[n] = dw4;
         }
       }
       if constexpr (LPP > 1) {
-        lds_at<float>(smem, q4, kScl) = scl;
+        lds_at<R>(smem, q1, kScl) = scl;
         if constexpr (CORR == 3)
           lds_at<int>(smem, q4, kDst) = v3_pair;  // (this op has no per-voxel depth gradient)
-        else
-          lds_at<float>(smem, q4, kDst) = 0.f;
+        else if constexpr (kDstWords)
+          lds_at<R>(smem, q1, kDst) = R(0);
       } else {
         r_scl = scl;
       }
     }
     if constexpr (LPP > 1) wave_sync();
     int rb_off[2][NV];
-    float4 rb_wt[2][NV], rb_dwt[2][NV];
-    float rb_scl[2];
+    R4 rb_wt[2][NV], rb_dwt[2][NV];
+    R rb_scl[2];
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
       if constexpr (LPP > 1) {
         rb_off[0][n] = lds_at<int>(smem, p4, kOff + (n * LPP * PPW) * 4);
-        rb_wt[0][n] = lds_at<float4>(smem, p4 * 4u, kWts + (n * LPP * PPW) * 16);
-        if constexpr (DG)
-          rb_dwt[0][n] = lds_at<float4>(smem, p4 * 4u, kDwt + (n * LPP * PPW) * 16);
+        rb_wt[0][n] = lds_at<R4>(smem, pw, kWts + (n * LPP * PPW) * kB4);
+        if constexpr (DG && !kSlim)
+          rb_dwt[0][n] = lds_at<R4>(smem, pw, kDwt + (n * LPP * PPW) * kB4);
         else
-          rb_dwt[0][n] = make_float4(0.f, 0.f, 0.f, 0.f);
+          rb_dwt[0][n] = R4{R(0), R(0), R(0), R(0)};
       } else {
         rb_off[0][n] = r_off[n];
         rb_wt[0][n] = r_wts[n];
@@ -2073,7 +2341,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
       }
     }
     if constexpr (LPP > 1)
-      rb_scl[0] = lds_at<float>(smem, p4, kScl);
+      rb_scl[0] = lds_at<R>(smem, p1, kScl);
     else
       rb_scl[0] = r_scl;
 #pragma unroll
@@ -2094,38 +2362,38 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
 #pragma unroll
           for (int n = 0; n < NV; ++n) {
             rb_off[nb][n] = lds_at<int>(smem, p4, kOff + ((n * LPP + jj + kAhead) * PPW) * 4);
-            rb_wt[nb][n] = lds_at<float4>(smem, p4 * 4u, kWts + ((n * LPP + jj + kAhead) * PPW) * 16);
-            if constexpr (DG)
-              rb_dwt[nb][n] = lds_at<float4>(smem, p4 * 4u, kDwt + ((n * LPP + jj + kAhead) * PPW) * 16);
+            rb_wt[nb][n] = lds_at<R4>(smem, pw, kWts + ((n * LPP + jj + kAhead) * PPW) * kB4);
+            if constexpr (DG && !kSlim)
+              rb_dwt[nb][n] = lds_at<R4>(smem, pw, kDwt + ((n * LPP + jj + kAhead) * PPW) * kB4);
             else
-              rb_dwt[nb][n] = make_float4(0.f, 0.f, 0.f, 0.f);
+              rb_dwt[nb][n] = R4{R(0), R(0), R(0), R(0)};
           }
-          rb_scl[nb] = lds_at<float>(smem, p4, kScl + ((jj + kAhead) * PPW) * 4);
+          rb_scl[nb] = lds_at<R>(smem, p1, kScl + ((jj + kAhead) * PPW) * kB);
         }
       }
       const int *rec_off = rb_off[cb];
-      const float4 *rec_wt = rb_wt[cb], *rec_dwt = rb_dwt[cb];
-      const float scl = rb_scl[cb];
-      float dvox = 0.f;  // this lane's share of d(loss)/d(depth of this voxel)
+      const R4 *rec_wt = rb_wt[cb], *rec_dwt = rb_dwt[cb];
+      const R scl = rb_scl[cb];
+      R dvox = R(0);  // this lane's share of d(loss)/d(depth of this voxel)
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         if (spread[n]) {  // uniform, and false for the whole chunk in the usual case
-          const bool fire = scl != 0.f && rec_off[n] >= 0 && rec_off[n] != cur[n] && cur[n] >= 0;
+          const bool fire = scl != R(0) && rec_off[n] >= 0 && rec_off[n] != cur[n] && cur[n] >= 0;
           end_spread_runs(n, fire);
         }
       }
       // (one view per workgroup: a tap offset implies a non-zero factor, phase 1 reprojects
       // only voxels that have one; one test instead of two per depth)
-      if (NV == 1 ? rec_off[0] >= 0 : scl != 0.f) {
-        float cg[VEC];
+      if (NV == 1 ? rec_off[0] >= 0 : scl != R(0)) {
+        R cg[VEC];
         {
-          float raw[VEC];
+          R raw[VEC];
           if constexpr (!kVoxelGrad) {
             if (CORR == 0 || CORR == 4)
               widen_raw<S, VEC>(cgw[jj % PF], raw);
             else
 #pragma unroll
-              for (int c = 0; c < VEC; ++c) raw[c] = __uint_as_float(cgw[jj % PF][c]);
+              for (int c = 0; c < VEC; ++c) raw[c] = raw_to_real(cgw[jj % PF][c]);
           }
           if constexpr (kVoxelGrad) {
 #pragma unroll
@@ -2153,14 +2421,20 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
                               : g.sub == 2              ? mr[c / 2]
                               : g.sub == 4              ? mr[c / 4]
                                                         : mr[0];
-              if (win != t.view0) cg[c] = 0.f;
+              if (win != t.view0) cg[c] = R(0);
             }
           }
         }
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
           const int off = rec_off[n];
-          const float4 wt = rec_wt[n], dwt = rec_dwt[n];
+          R4 wt = rec_wt[n], dwt = rec_dwt[n];
+          if constexpr (kSlim) {
+            const R dh = wt.x, dw = wt.y, ah = wt.z, aw = wt.w, k11 = dh * dw, k01 = dw - k11;
+            wt = R4{(R(1) - dh) - k01, k01, k11, dh - k11};
+            const R cp = mad(ah, dw, aw * dh), bp = aw - cp;
+            dwt = R4{-ah - bp, bp, cp, ah - cp};
+          }
           if (off >= 0) {
             if (off != cur[n]) {
               // (a run whose cell the window could not cover was closed by the uniform block
@@ -2172,12 +2446,12 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
               const unsigned e1 = e0 + (unsigned)row_step * (unsigned)sizeof(S);
               const char *vb = reinterpret_cast<const char *>(view[n]);
               const unsigned cb = (unsigned)C * (unsigned)sizeof(S);
-              load_vec<S, VEC, false>(reinterpret_cast<const S *>(vb + e0), tap[n][0]);
-              load_vec<S, VEC, false>(reinterpret_cast<const S *>(vb + (e0 + cb)), tap[n][1]);
-              load_vec<S, VEC, false>(reinterpret_cast<const S *>(vb + (e1 + cb)), tap[n][2]);
-              load_vec<S, VEC, false>(reinterpret_cast<const S *>(vb + e1), tap[n][3]);
+              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + e0), tap[n][0]);
+              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + (e0 + cb)), tap[n][1]);
+              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + (e1 + cb)), tap[n][2]);
+              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + e1), tap[n][3]);
               if (cur[n] >= 0)
-                window_add<VEC, LPP, kLean, kSix>((unsigned)cell[n].x, cell[n].y, sg[n],
+                window_add<VEC, LPP, kLean, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n],
                                             s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
               cur[n] = off;
               if constexpr (LPP > 1)
@@ -2185,7 +2459,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
               else
                 cell[n] = r_cell[n];
             }
-            float gs3[VEC];
+            R gs3[VEC];
             if constexpr (CORR == 3) {
               const int pair = REDUCE ? lds_at<int>(smem, p4, kDst + (jj * PPW) * 4) : 0;
               if (g.sub == 8)
@@ -2197,49 +2471,49 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              float gsrc;  // d(loss)/d(sample of this channel)
+              R gsrc;  // d(loss)/d(sample of this channel)
               if constexpr (CORR == 3) {
                 gsrc = gs3[c];
               } else if constexpr (CORR == 4) {
                 gsrc = cg[c];
               } else if (CORR != 1) {
-                float diff = __builtin_fmaf(wt.x, tap[n][0][c], -ref[c]);
-                diff = __builtin_fmaf(wt.y, tap[n][1][c], diff);
-                diff = __builtin_fmaf(wt.z, tap[n][2][c], diff);
-                diff = __builtin_fmaf(wt.w, tap[n][3][c], diff);
+                R diff = mad(wt.x, tap[n][0][c], -ref[c]);
+                diff = mad(wt.y, tap[n][1][c], diff);
+                diff = mad(wt.z, tap[n][2][c], diff);
+                diff = mad(wt.w, tap[n][3][c], diff);
                 gsrc = diff * cg[c];
                 racc[c] -= gsrc;
               } else {
-                float smp = wt.x * tap[n][0][c];
-                smp = __builtin_fmaf(wt.y, tap[n][1][c], smp);
-                smp = __builtin_fmaf(wt.z, tap[n][2][c], smp);
-                smp = __builtin_fmaf(wt.w, tap[n][3][c], smp);
-                racc[c] = __builtin_fmaf(cg[c], smp, racc[c]);
+                R smp = wt.x * tap[n][0][c];
+                smp = mad(wt.y, tap[n][1][c], smp);
+                smp = mad(wt.z, tap[n][2][c], smp);
+                smp = mad(wt.w, tap[n][3][c], smp);
+                racc[c] = mad(cg[c], smp, racc[c]);
                 gsrc = cg[c] * ref[c];
               }
-              if constexpr (PAD) gsrc = ch_ok ? gsrc : 0.f;
-              sg[n][0][c] = __builtin_fmaf(gsrc, wt.x, sg[n][0][c]);
-              sg[n][1][c] = __builtin_fmaf(gsrc, wt.y, sg[n][1][c]);
-              sg[n][2][c] = __builtin_fmaf(gsrc, wt.z, sg[n][2][c]);
-              sg[n][3][c] = __builtin_fmaf(gsrc, wt.w, sg[n][3][c]);
+              if constexpr (PAD) gsrc = ch_ok ? gsrc : R(0);
+              sg[n][0][c] = mad(gsrc, wt.x, sg[n][0][c]);
+              sg[n][1][c] = mad(gsrc, wt.y, sg[n][1][c]);
+              sg[n][2][c] = mad(gsrc, wt.z, sg[n][2][c]);
+              sg[n][3][c] = mad(gsrc, wt.w, sg[n][3][c]);
               if constexpr (DG) {
-                float ds = dwt.x * tap[n][0][c];
-                ds = __builtin_fmaf(dwt.y, tap[n][1][c], ds);
-                ds = __builtin_fmaf(dwt.z, tap[n][2][c], ds);
-                ds = __builtin_fmaf(dwt.w, tap[n][3][c], ds);
-                dvox = __builtin_fmaf(gsrc, ds, dvox);
+                R ds = dwt.x * tap[n][0][c];
+                ds = mad(dwt.y, tap[n][1][c], ds);
+                ds = mad(dwt.z, tap[n][2][c], ds);
+                ds = mad(dwt.w, tap[n][3][c], ds);
+                dvox = mad(gsrc, ds, dvox);
               }
             }
           }
         }
       }
-      if constexpr (PAD && DG) dvox = ch_ok ? dvox : 0.f;
+      if constexpr (PAD && DG) dvox = ch_ok ? dvox : R(0);
       if constexpr (!DG) {
         // no depth gradient wanted
       } else if (per_voxel_depth) {
         if constexpr (LPP > 1) {
-          const float tot = group_sum<LPP>(dvox);
-          if (t.cl == 0) lds_at<float>(smem, p4, kDst + (jj * PPW) * 4) = tot;
+          const R tot = group_sum<LPP>(dvox);
+          if (t.cl == 0) lds_at<R>(smem, p1, kDst + (jj * PPW) * kB) = tot;
         } else {
           if (t.pix_ok) {
             if (dg_store)
@@ -2259,7 +2533,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
       if (DG && per_voxel_depth) {
         const int d = d0 + t.cl;
         if (d < d_hi && t.pix_ok) {
-          const float tot = lds_at<float>(smem, q4, kDst);
+          const R tot = lds_at<R>(smem, q1, kDst);
           if (dg_store)
             a.depth_grad[t.pix * D + d] = tot;
           else if (dg_own)
@@ -2276,33 +2550,35 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE)) vo
   for (int n = 0; n < NV; ++n) {
     if (__ballot(cur[n] >= 0 && cell[n].y >= 0) != 0ull) end_spread_runs(n, cur[n] >= 0);
     if (cur[n] >= 0)
-      window_add<VEC, LPP, false, kSix>((unsigned)cell[n].x, cell[n].y, sg[n],
+      window_add<VEC, LPP, false, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n],
                            s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
   }
   wave_sync();
 #pragma unroll
   for (int n = 0; n < NV; ++n)
-    window_flush_all<VEC, LPP, kSix>(oy[n], ox[n], s_data + n * WN::SLOTS * WN::STRIDE, gview[n], srcW,
+    window_flush_all<VEC, LPP, kForm>(oy[n], ox[n], s_data + n * WN::SLOTS * WN::STRIDE, gview[n], srcW,
                                t.lane, wave_or(ring_rows[n]), cm);
   wave_sync();  // the next view clears the window
   }  // views of the group
 
   // pixel-owned gradients: one store when this workgroup saw every depth, otherwise one
   // atomic add per depth segment into the zero-filled outputs
-  float *rg = kWide ? a.ref_grad_acc : reinterpret_cast<float *>(a.ref_grad);
+  R *rg;
+  if constexpr (kWide) rg = a.ref_grad_acc;
+  else rg = a.ref_grad;
   const bool single = g.nseg * g.ngroups == 1;
   if constexpr (CORR == 4) {
     // no reference image, no gradient for it
   } else if (single) {
     // (16-bit storage too: the finished sums go straight to the output, the fp32 image of
     // ref_grad is neither written nor narrowed afterwards)
-    if (t.pix_ok && ch_ok) store_vec<S, VEC, false>(a.ref_grad + t.pix * C + t.cl * VEC, racc);
+    if (t.pix_ok && ch_ok) store_vec<S, VEC, false, GAP>(a.ref_grad + t.pix * C + ch0, racc);
   } else if (t.pix_ok && ch_ok) {
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) atomic_add(rg + t.pix * C + t.cl * VEC + c, racc[c]);
+    for (int c = 0; c < VEC; ++c) atomic_add(rg + t.pix * C + ch0 + c / 2 * GAP + c % 2, racc[c]);
   }
   if (DG && !per_voxel_depth) {
-    const float tot = group_sum<LPP>(dacc);
+    const R tot = group_sum<LPP>(dacc);
     if (t.cl == 0 && t.pix_ok) {
       if (single)
         a.depth_grad[t.pix] = tot;

@@ -132,6 +132,21 @@ __device__ __forceinline__ R depth_chain(const Sample<R> &s, R h_grad, R w_grad)
          (s.z * s.z);
 }
 
+// ---- arithmetic that is not part of the rounding contract ----------------------------------
+// 1 / x to within an ulp or two, for the gradients' factors (a full IEEE division costs about
+// ten instructions in float and fifty in double; the gradients are compared at 1e-4).
+__device__ __forceinline__ float quick_recip(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double quick_recip(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+
+// a * b + c in one rounding: the backward's arithmetic (gradients are compared at 1e-4; with
+// contraction off for the whole library a plain a * b + c is two instructions)
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double mad(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // ---- atomics ------------------------------------------------------------------------------
 // Hardware floating-point add at the L2 (global_atomic_add_f32 / _f64); the destination
 // is ordinary coarse-grained device memory owned by the caller.

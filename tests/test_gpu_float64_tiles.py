@@ -1,0 +1,71 @@
+"""Float64 on the tile-shaped kernels: pixels of 4 to 64 channels, some lanes idle (20, 24, 28), one to
+seven views (seven: the forward pass keeps a lane per channel), depth ranges that end inside a chunk.
+
+An unforced call takes them, the strip family forced takes a lane per channel.  Forward both are the
+plain evaluation: equal to each other and to the oracle to the bit.  Gradients: the sums come in
+another order, each of up to a few hundred terms, so 1e-10 of the gradient's rms (the oracle's own
+bar in float64) holds with three digits to spare.
+"""
+import numpy as np
+import pytest
+import torch
+
+import custom_helper_op_amd as chop
+from custom_helper_op_amd import _lib
+from custom_helper_op_amd.configs import reference_test_case
+from gpu_util import assert_backward_close, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _announce(request):
+    print("\n[case] %s" % request.node.nodeid, flush=True)
+    yield
+    _lib.load().chop_set_kernel_family(0)
+
+
+def _both(run):
+    out = []
+    for family in (0, 2):
+        _lib.load().chop_set_kernel_family(family)
+        out.append([host(x) for x in run()])
+        assert _lib.load().chop_last_kernel_family() == 3
+    return out
+
+
+@pytest.mark.parametrize("C", [4, 8, 16, 20, 24, 28, 32, 64])
+@pytest.mark.parametrize("N,H,W,D", [(1, 13, 17, 5), (2, 7, 9, 35), (4, 12, 10, 16), (7, 6, 11, 9)])
+@pytest.mark.parametrize("op,reduce,groups", [("v1", "MEAN", 1), ("v1", "MIN", 1), ("v2", "MEAN", 4),
+                                              ("v2", "MIN", 2), ("aggregate", "MEAN", 1),
+                                              ("aggregate", "MIN", 1), ("feature", "MEAN", 1)])
+def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
+    t = reference_test_case(3, 2, N, H, W, C, D, np.float64, seed=C + N)
+    t["Ts"] = (t["Ts"] + np.linspace(-0.5, 0.5, N)[None, :, None]).astype(np.float64)
+    args = tuple(t[k] for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts"))
+    extra = (reduce,)
+    if op == "v1":
+        fwd, bwd = chop.cost_volume_raw, chop.cost_volume_grad
+        want_fwd, want_bwd = oracle.cost_volume_fwd, oracle.cost_volume_bwd
+    elif op == "aggregate":
+        fwd, bwd = chop.cost_aggregate_raw, chop.cost_aggregate_grad
+        want_fwd, want_bwd = oracle.cost_aggregate_fwd, oracle.cost_aggregate_bwd
+    elif op == "feature":
+        args, extra = args[1:], ()
+        fwd, bwd = chop.feature_aggregate_raw, chop.feature_aggregate_grad
+        want_fwd, want_bwd = oracle.feature_aggregate_fwd, oracle.feature_aggregate_bwd
+    else:
+        grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
+        args, extra = (t["ref"], t["src"], grid, t["Rs"], t["Ts"]), (reduce, groups)
+        fwd, bwd = chop.cost_volume_v2_raw, chop.cost_volume_grad_v2
+        want_fwd, want_bwd = oracle.cost_volume_v2_fwd, oracle.cost_volume_v2_bwd
+    ins = [dev(x) for x in args]
+    want = want_fwd(*args, *extra)
+    for got in _both(lambda: fwd(*ins, *extra)):
+        for g, w in zip(got, want):
+            assert np.array_equal(g, w)
+    cg = np.random.default_rng(5).standard_normal(want[0].shape)
+    grads = want_bwd(*args, cg, want[1], *extra)
+    for got in _both(lambda: bwd(*ins, dev(cg), dev(want[1]), *extra)):
+        for g, w in zip(got, grads):
+            assert_backward_close(g, w, 1e-10)
