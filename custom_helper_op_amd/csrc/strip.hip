@@ -42,7 +42,7 @@ constexpr int kDB = 8;  // depths per chunk (16 measured slower everywhere: regi
 
 struct StripGeom {
   int lpp_shift;        // log2(LPP)
-  int nseg, seg;        // depth segments, depths per segment (a multiple of kDB)
+  int nseg, seg;        // depth segments, depths per segment (a multiple of kDB, or fewer)
   int vg;               // views reprojected together: min(N, max(1, LPP / kDB))
   int carry;            // backward: open runs survive the end of a chunk (in LDS)
   int cache;            // backward: a texel cache in LDS between the runs and memory
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(64, W4 ? 4 : 1) void strip_backward_kernel(const Ar
 
 
 template <typename S>
-StripGeom strip_geometry(const Args<S> &a) {
+StripGeom strip_geometry(const Args<S> &a, bool backward) {
   StripGeom g;
   g.lpp_shift = 0;
   while ((1 << g.lpp_shift) < a.C) ++g.lpp_shift;
@@ -738,6 +738,20 @@ StripGeom strip_geometry(const Args<S> &a) {
   while (nseg < 16 && g.tiles * nseg < 256 * 80 && a.D / (nseg * 2) >= 2 * kDB) nseg *= 2;
   const int per = (int)((a.D + nseg - 1) / nseg);
   g.seg = (per + kDB - 1) / kDB * kDB;
+  // A launch below two waves per SIMD lasts as long as its longest wave: segments of less than a
+  // chunk then (3 channels, two views, 12 x 16 x 9, double, 12 tiles: forward 11.3 -> 5.8 us, gradient
+  // 17.2 -> 9.5 us; bf16 group correlation, four views, 16 x 17 x 28: 50 -> 9 and 76 -> 16 us; at one
+  // wave per SIMD instead: 24 channels, three views, 38 x 43 x 25 15 against 11 us).  Every segment of a
+  // gradient adds to its pixels' sums: two depths at least and 48 segments at most (two views, 15 x 21 x
+  // 94: 41 us in five segments, 17 in 47, 30 in 94; three views, 18 x 19 x 186: 40, 21 in 47, 36 in 93).
+  if (g.tiles * ((a.D + g.seg - 1) / g.seg) < 2048) {
+    int64_t len = (g.tiles * a.D + 2047) / 2048;
+    if (backward) {
+      if (len < 2) len = 2;
+      if (len < (a.D + 47) / 48) len = (a.D + 47) / 48;
+    }
+    if (len < g.seg) g.seg = (int)(len <= kDB ? len : len / kDB * kDB);
+  }
   g.nseg = (int)((a.D + g.seg - 1) / g.seg);
   // carried runs: N * 64 lanes * (4 sums + tap offset + cell); given up beyond 16 KiB, or
   // where records and runs together would pass the launch limit (one channel in float64:
@@ -780,7 +794,8 @@ bool strip_supported(const Args<S> &a) {
   const bool grid = a.depth_grid != nullptr;
   if (a.corr == GROUP_CORRELATION ? !grid : grid && !(a.corr == SQUARED_DIFFERENCE && sizeof(S) == 2))
     return false;
-  const StripGeom g = strip_geometry(a);
+  // (the gradient never has more segments)
+  const StripGeom g = strip_geometry(a, false);
   return g.tiles * g.nseg < (int64_t)1 << 31;
 }
 
@@ -796,7 +811,7 @@ bool strip_pair_backward_supported(const Args<S> &a) {
     if (a.groups < 1 || a.C % a.groups != 0) return false;
     if (a.srcH < 2 || a.srcW < 2) return false;
     if (a.srcH * a.srcW * a.C >= (int64_t)1 << 31) return false;
-    const StripGeom g = strip_geometry(a);
+    const StripGeom g = strip_geometry(a, true);
     if (a.groups > 16) return false;  // very many groups: the search of groups^2 pairs dominates
     return g.tiles * g.nseg < (int64_t)1 << 31;
   }
@@ -805,7 +820,7 @@ bool strip_pair_backward_supported(const Args<S> &a) {
 template <typename S>
 hipError_t launch_strip_forward(const Args<S> &a, hipStream_t stream) {
   using R = typename Storage<S>::Real;
-  const StripGeom g = strip_geometry(a);
+  const StripGeom g = strip_geometry(a, false);
   // CostAggregate adds one row of 64 values per depth of a chunk
   const size_t smem = strip_lds_bytes<R>(4, (64 >> g.lpp_shift) * g.vg * kDB) +
                       (a.corr == SUM_SQUARED_DIFFERENCE ? (size_t)kDB * 64 * sizeof(R) : 0);
@@ -834,7 +849,7 @@ hipError_t launch_strip_forward(const Args<S> &a, hipStream_t stream) {
 template <typename S>
 hipError_t launch_strip_backward(const Args<S> &a, hipStream_t stream) {
   using R = typename Storage<S>::Real;
-  const StripGeom g = strip_geometry(a);
+  const StripGeom g = strip_geometry(a, true);
   const int64_t n_ref = a.pixels() * a.C;
   const int64_t n_src = a.B * a.N * a.srcH * a.srcW * a.C;
   hipError_t err;

@@ -2620,6 +2620,15 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
   g.vper = vper;
   // twenty waves per SIMD over the launch: the tail of a launch with fewer is measurable
   g.nseg = choose_segments(tiles * ngroups, D, LPP, 256 * 4 * 20);
+  // A forward launch below two waves per SIMD lasts as long as its longest wave, and a segment costs
+  // it nothing but the set-up: segments down to one chunk (32 channels in 8 groups, five views, 32 x 32 x 5:
+  // 12.6 -> 9.9 us; samples of 8 channels, four views, 22 x 26 x 17: 10.7 -> 7.5 us; double, 8
+  // channels, four views, 182 x 245 x 12: 47 -> 38 us; at four waves per SIMD a correlation of 32
+  // double channels, six views, 120 x 131 x 23, is slower: 191 -> 202 us).
+  if (vper == 0 && tiles * g.nseg < 2048) {
+    const int64_t chunks = (D + LPP - 1) / LPP, want = (2048 + tiles - 1) / tiles;
+    g.nseg = (int)(want < chunks ? want : chunks);
+  }
   const int per_seg = (int)((D + g.nseg - 1) / g.nseg);
   g.seg = ((per_seg + LPP - 1) / LPP) * LPP;
   // Segments are whole chunks.  Rounded up they can be twice what was asked for (135 hypotheses of
