@@ -42,7 +42,10 @@ namespace tiled {
 // change (MVSNet-stage workload, 8 pixels: 0.49 of them for 2 x 4 against 0.61 for 1 x 8;
 // f16 cascade workload, 16 pixels: 0.49-0.68 per view for 4 x 4 against 0.57-0.75 for 2 x 8),
 // and its footprint in the source image has fewer texels per pixel.
-constexpr int tile_rows(int ppw) { return ppw >= 64 ? 8 : ppw >= 16 ? 4 : ppw >= 2 ? 2 : 1; }
+// `tall`: eight pixels as 4 x 2.
+constexpr int tile_rows(int ppw, bool tall = false) {
+  return ppw >= 64 ? 8 : ppw >= 16 || tall ? 4 : ppw >= 2 ? 2 : 1;
+}
 
 struct Geometry {
   int hw;                  // H*W
@@ -389,7 +392,7 @@ struct Tile {
   int64_t pix;
 };
 
-template <typename S, int LPP>
+template <typename S, int LPP, bool TALL = false>
 __device__ __forceinline__ bool locate_tile(const Args<S> &a, const Geometry &g, Tile<LPP> &t) {
   constexpr int PPW = 64 / LPP;
   t.lane = threadIdx.x;
@@ -442,7 +445,7 @@ __device__ __forceinline__ bool locate_tile(const Args<S> &a, const Geometry &g,
     // at more nearly the same depths than those of a long row, so fewer wave iterations carry
     // a cell change (0.49 against 0.62 of them on the MVSNet-stage workload).  Tiles that
     // stick out of the image have their outside pixels switched off.
-    constexpr int TH = tile_rows(PPW), TW = PPW / TH;
+    constexpr int TH = tile_rows(PPW, TALL), TW = PPW / TH;
     const int ty = t_in / g.tiles_x, tx = t_in - ty * g.tiles_x;
     const int py = t.p / TW;
     const int y = ty * TH + py, x = tx * TW + (t.p - py * TW);
@@ -1435,7 +1438,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 // depends only on its coordinates, the four slots of a cell are computed once, by the lane
 // that reprojects the voxel, and travel with the record.
 // The forms of the window: left to the tile's shape, or fixed by the kernel that owns it.
-enum { kPlainWindow = 0, kSixRows = 6, kFourRows = 4 };
+enum { kNotEight = 0, kEightWide = 1, kEightTall = 2 };  // backward_kernel's EIGHT
+enum { kPlainWindow = 0, kSixRows = 6, kFourRows = 4, kSixColumns = 8 };
 template <int VEC, int LPP, int FORM = kPlainWindow>
 struct Window {
   static constexpr int PPW = 64 / LPP;
@@ -1457,22 +1461,42 @@ struct Window {
   static constexpr int ROWS = FORM == kSixRows                 ? 6
                               : FORM == kFourRows || LPP == 16 ? 4
                                                                : (2 * TH > 8 ? 2 * TH : 8);
-  static constexpr int COLS = 2 * TW > 8 ? 2 * TW : 8;
+  // kSixColumns: the same turned by ninety degrees, for a tile of 4 x 2 pixels.
+  static constexpr int COLS = FORM == kSixColumns ? 6 : (2 * TW > 8 ? 2 * TW : 8);
   static constexpr int SLOTS = ROWS * COLS;
-  static constexpr bool kPow2Rows = (ROWS & (ROWS - 1)) == 0;
-  // ring row of image row `fh` (not negative)
-  static __device__ __forceinline__ int ring_row(unsigned fh) {
-    return kPow2Rows ? (int)(fh & (unsigned)(ROWS - 1)) : (int)(fh % (unsigned)ROWS);
-  }
-  // image row of ring row `ry` for a window whose first row is `oy` (any sign)
-  static __device__ __forceinline__ int image_row(int ry, int oy) {
-    if constexpr (kPow2Rows) {
-      return oy + ((ry - oy) & (ROWS - 1));
+  // place of image row / column `i` (not negative) in a ring of LEN
+  template <int LEN>
+  static __device__ __forceinline__ int ring(unsigned i) {
+    if constexpr ((LEN & (LEN - 1)) == 0) {
+      return (int)(i & (unsigned)(LEN - 1));
     } else {
-      int m = (ry - oy) % ROWS;
-      return oy + (m < 0 ? m + ROWS : m);
+      // (i / 6 for every i up to 32769; a general division by a constant takes the high half of a
+      // product, four times the issue time of a 24-bit one)
+      static_assert(LEN == 6, "the reciprocal below");
+      return (int)(i - (__umul24(i, 10923u) >> 16) * 6u);
     }
   }
+  // the place after `r`
+  template <int LEN>
+  static __device__ __forceinline__ int ring_next(int r) {
+    if constexpr ((LEN & (LEN - 1)) == 0) return (r + 1) & (LEN - 1);
+    else return r == LEN - 1 ? 0 : r + 1;
+  }
+  static __device__ __forceinline__ int ring_row(unsigned fh) { return ring<ROWS>(fh); }
+  static __device__ __forceinline__ int ring_col(unsigned fw) { return ring<COLS>(fw); }
+  // image row / column at place `r` of a ring whose window starts at `o` (any sign)
+  template <int LEN>
+  static __device__ __forceinline__ int unring(int r, int o) {
+    if constexpr ((LEN & (LEN - 1)) == 0) {
+      return o + ((r - o) & (LEN - 1));
+    } else {
+      const int first = o >= 0 ? o % LEN : (LEN - 1) - (-1 - o) % LEN;  // (o is uniform)
+      const int m = r - first;
+      return o + (m < 0 ? m + LEN : m);
+    }
+  }
+  static __device__ __forceinline__ int image_row(int ry, int oy) { return unring<ROWS>(ry, oy); }
+  static __device__ __forceinline__ int image_col(int rx, int ox) { return unring<COLS>(rx, ox); }
   static constexpr int C = VEC * LPP;
   static constexpr int STRIDE = C;      // one slot = C consecutive words: 16-byte lane accesses
   static constexpr int kNone = 0x3fffffff;
@@ -1482,8 +1506,8 @@ struct Window {
   // slots of the taps 00, 01, 11, 10 of cell `key`, one byte each
   static __device__ __forceinline__ unsigned pack_slots(int key) {
     const int fh = (key >> 16) & 0x7fff, fw = key & 0xffff;
-    const int ry0 = ring_row((unsigned)fh) * COLS, ry1 = ring_row((unsigned)fh + 1u) * COLS;
-    const int rx0 = fw & (COLS - 1), rx1 = (fw + 1) & (COLS - 1);
+    const int r0 = ring_row((unsigned)fh), ry0 = r0 * COLS, ry1 = ring_next<ROWS>(r0) * COLS;
+    const int rx0 = ring_col((unsigned)fw), rx1 = ring_next<COLS>(rx0);
     return (unsigned)(ry0 + rx0) | ((unsigned)(ry0 + rx1) << 8) | ((unsigned)(ry1 + rx1) << 16) |
            ((unsigned)(ry1 + rx0) << 24);
   }
@@ -1544,6 +1568,13 @@ __device__ __forceinline__ int wave_min(int v) {
              min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
+// Adds to element `e` of a view's image, whose 2^29 elements at most (make_plan) are addressed as the
+// view's uniform base plus 32 bits of bytes.
+template <typename R>
+__device__ __forceinline__ void atomic_at(R *image, unsigned e, R v) {
+  atomic_add(reinterpret_cast<R *>(reinterpret_cast<char *>(image) + e * (unsigned)sizeof(R)), v);
+}
+
 // Moves the window of one view to origin (ny, nx): every texel that falls outside the new
 // window is written out with dense global atomics (C consecutive floats per texel, 64/C
 // texels per instruction, UN instructions per round: their LDS reads go out together) and its
@@ -1559,7 +1590,7 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R 
     for (int sb = 0; sb < WN::SLOTS; sb += 64) {
       const int s = sb + lane;  // (a window of 48 slots: the last lanes have none)
       const int ry = s / WN::COLS, rx = s % WN::COLS;
-      const int y = WN::image_row(ry, oy), x = ox + ((rx - ox) & (WN::COLS - 1));
+      const int y = WN::image_row(ry, oy), x = WN::image_col(rx, ox);
       const bool leaving = s < WN::SLOTS && !((unsigned)(y - ny) < (unsigned)WN::ROWS &&
                                               (unsigned)(x - nx) < (unsigned)WN::COLS);
       const unsigned long long m = __ballot(leaving);
@@ -1591,7 +1622,7 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R 
         for (int u = 0; u < UN; ++u) {
           if (v[u] != R(0)) {
             data[le[u].x * WN::STRIDE + j] = R(0);
-            atomic_add(gview + (int64_t)le[u].y * cm + j, v[u]);
+            atomic_at(gview, (unsigned)le[u].y * (unsigned)cm + (unsigned)j, v[u]);
           }
         }
       }
@@ -1644,8 +1675,8 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const R *data, 
         const int e = (i0 + u) * 64 + lane;  // float index inside the window
         const int sl = e / C, ch = e - sl * C;
         const int ry = sl / WN::COLS, rx = sl - ry * WN::COLS;
-        const int y = WN::image_row(ry, oy), x = ox + ((rx - ox) & (WN::COLS - 1));
-        if (v[u] != R(0)) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
+        const int y = WN::image_row(ry, oy), x = WN::image_col(rx, ox);
+        if (v[u] != R(0)) atomic_at(gview, (unsigned)(y * srcW + x) * (unsigned)cm + (unsigned)ch, v[u]);
       }
     }
     return;
@@ -1661,9 +1692,9 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const R *data, 
     for (int u = 0; u < PER_ROW; ++u) {
       const int e = u * 64 + lane;  // float index inside the row
       const int rx = e / C, ch = e - rx * C;
-      const int x = ox + ((rx - ox) & (WN::COLS - 1));
+      const int x = WN::image_col(rx, ox);
       // (a slot that was never added to holds zero: texels outside the image never are)
-      if (v[u] != R(0)) atomic_add(gview + ((int64_t)(y * srcW + x) * cm + ch), v[u]);
+      if (v[u] != R(0)) atomic_at(gview, (unsigned)(y * srcW + x) * (unsigned)cm + (unsigned)ch, v[u]);
     }
   }
 }
@@ -1696,7 +1727,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
     } else {
       const int fh = (key >> 16) & 0x7fff, fw = key & 0xffff;
       const int ry0 = WN::ring_row((unsigned)fh) * WN::COLS, ry1 = WN::ring_row((unsigned)fh + 1u) * WN::COLS;
-      const int rx0 = fw & (WN::COLS - 1), rx1 = (fw + 1) & (WN::COLS - 1);
+      const int rx0 = WN::ring_col((unsigned)fw), rx1 = WN::ring_col((unsigned)fw + 1u);
       slot[0] = ry0 + rx0, slot[1] = ry0 + rx1, slot[2] = ry1 + rx1, slot[3] = ry1 + rx0;
     }
     R *base = data + lane_first(cl, GAP);
@@ -1884,8 +1915,9 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // VLOOP: the workgroup's view group holds several views, which take turns (g.vper of them).
 // A compile-time flag: the loop around the kernel's body costs the wide instantiations
 // registers they do not have (the 32-channel kernel spills with it).
-// WIDE: the kernel as it is without the slimming of lean_backward: three waves per SIMD and, for
-// 32 channels, the 8 x 8 window.  The launcher decides (tiled_launch.inc).
+// EIGHT: 32 channels with a window of eight rows, for many views.  kEightWide: 8 x 8 texels and the kernel
+// without the slimming of lean_backward, three waves per SIMD; kEightTall: 8 x 6 over tiles of 4 x 2
+// pixels, the slimmed form turned by ninety degrees.  The launcher decides (tiled_launch.inc).
 // PAD: fewer channels than the pixel's lanes hold (20, 24, 28 on eight lanes).  The lanes past the
 // last channel compute what the last lane computes and contribute nothing: their gradients are
 // selected to zero (not multiplied: infinities), their window slots stay zero.  A quarter of the
@@ -1894,22 +1926,22 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // passes of 24 channels: minimum over five views, 63 x 85 x 37, 219 -> 110 us; warped features, 212 x
 // 213 x 86, 627 -> 344 us).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool DG = true,
-          bool PV = (CORR == 1), bool VLOOP = false, bool WIDE = false, bool PAD = false>
-__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE, sizeof(S) == 8)) void backward_kernel(
+          bool PV = (CORR == 1), bool VLOOP = false, int EIGHT = kNotEight, bool PAD = false>
+__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, sizeof(S) == 8)) void backward_kernel(
     const Args<S> a, const Geometry g) {
   using R = typename Storage<S>::Real;
   using R4 = Four<R>;
   constexpr bool kDouble = sizeof(S) == 8;
   constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
-  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, WIDE, kDouble);
+  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, kDouble);
   constexpr bool kSlim = kDouble && slim_double(LPP, CORR);
-  constexpr int kForm = !(kLean && LPP == 8) ? kPlainWindow : kSlim ? kFourRows : kSixRows;
+  constexpr int kForm = !(kLean && LPP == 8) ? kPlainWindow : kSlim ? kFourRows : EIGHT == kEightTall ? kSixColumns : kSixRows;
   using WN = Window<VEC, LPP, kForm>;
   constexpr int PPW = 64 / LPP;
   constexpr bool kWide = sizeof(S) == 2;  // gradients accumulate in fp32 images
   extern __shared__ __align__(16) unsigned char smem[];
   Tile<LPP> t;
-  if (!locate_tile<S, LPP>(a, g, t)) return;
+  if (!locate_tile<S, LPP, EIGHT == kEightTall>(a, g, t)) return;
   const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
   const R half = a.half;
   constexpr bool per_voxel_depth = PV;
@@ -2250,8 +2282,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, WIDE, siz
         // end, depth by depth (end_spread_runs).
         const bool valid = hit.off >= 0;
         if (valid) {
-          const unsigned fh = (unsigned)hit.key >> 16;
-          ring_rows[n] |= (1u << WN::ring_row(fh)) | (1u << WN::ring_row(fh + 1u));
+          const int r0 = WN::ring_row((unsigned)hit.key >> 16);
+          ring_rows[n] |= (1u << r0) | (1u << WN::template ring_next<WN::ROWS>(r0));
         }
         bool in_new = !valid || WN::inside(hit.key, oy[n], ox[n]);
         spread[n] = false;
@@ -2603,7 +2635,7 @@ inline int choose_segments(int64_t tiles, int64_t D, int lpp, int64_t target_uni
 
 template <int LPP>
 inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int sub, int ngroups = 1,
-                              int vper = 0) {
+                              int vper = 0, bool tall = false) {
   constexpr int PPW = 64 / LPP;
   Geometry g;
   g.hw = (int)(H * W);
@@ -2611,7 +2643,7 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
     g.tiles_x = (int)W;
     g.tiles_per_image = g.hw;
   } else {
-    constexpr int TH = tile_rows(PPW), TW = PPW / TH;
+    const int TH = tile_rows(PPW, tall), TW = PPW / TH;
     g.tiles_x = (int)((W + TW - 1) / TW);
     g.tiles_per_image = g.tiles_x * (int)((H + TH - 1) / TH);
   }

@@ -428,10 +428,9 @@ int chop_last_kernel_family(void);
  * image, all views of a pixel tile in one workgroup); 0 if the last backward call did not run
  * the tiled kernels.  For the tests. */
 int chop_last_views_per_workgroup(void);
-/* No counterpart in the reference.  The tiled gradient kernels for 32 channels exist twice:
- * slimmed to four wavefronts per SIMD with a scatter window of 6 x 8 texels, and at three
- * wavefronts with 8 x 8.  The first takes 3-17 % less time (most where wide baselines and
- * hypotheses close to the cameras spread the samples).  Left alone the library
+/* No counterpart in the reference.  The tiled gradient kernels for 32 channels exist with
+ * a scatter window of six rows of texels (6 x 8, four wavefronts per SIMD) and of eight (8 x 8 at three
+ * wavefronts, or in long sweeps over large images 8 x 6 at four).  Left alone the library
  * picks the second for five or more source views; rows = 6 or 8 fixes the
  * choice for subsequent calls from this thread, 0 returns it to the library.  Returns the
  * previous value.  Results agree within the gradient tolerance either way. */
