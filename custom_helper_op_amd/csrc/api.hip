@@ -68,8 +68,11 @@ int check_dims(const Dims &d, int reduce, int groups, bool correlation) {
 // What chop_last_kernel_family() reports for the tile-shaped kernels: 2, in float64 3 -- its
 // tile-shaped and its lane-per-channel kernels give the same bits forward (the plain evaluation's) and
 // stand behind one code.
+// Likewise forward for channel counts that leave lanes idle (20, 24, 28).
 template <typename S>
-constexpr int tiled_family() { return sizeof(S) == 8 ? 3 : 2; }
+int tiled_family(const Args<S> &a, bool forward) {
+  return sizeof(S) == 8 || (forward && (a.C & (a.C - 1)) != 0) ? 3 : 2;
+}
 
 int launch_status(hipError_t err, const char *what) {
   if (err == hipSuccess) return CHOP_OK;
@@ -110,7 +113,7 @@ int forward(void *stream, int reduce, int half_centor, const Dims &d, int groups
   a.default_cost = default_cost;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_kernel_family == 0 && tiled_forward_supported(a)) {
-    g_last_family = tiled_family<S>();
+    g_last_family = tiled_family(a, true);
     return launch_status(launch_tiled_forward(a, s), "tiled forward launch");
   }
   if (g_kernel_family != 1 && strip_supported(a)) {
@@ -180,7 +183,7 @@ int backward(void *stream, int reduce, int half_centor, const Dims &d, int group
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_kernel_family == 0 && work && tiled_backward_supported(a)) {
-    g_last_family = tiled_family<S>();
+    g_last_family = tiled_family(a, false);
     return launch_status(launch_tiled_backward(a, s), "tiled backward launch");
   }
   if (g_kernel_family != 1 && work && strip_supported(a)) {
@@ -294,7 +297,7 @@ int feature_call(void *stream, int half_centor, const Dims &d, const S *src, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_kernel_family == 0 && work) {
     if (backward ? tiled_backward_supported(a) : tiled_forward_supported(a)) {
-      g_last_family = tiled_family<S>();
+      g_last_family = tiled_family(a, !backward);
       return backward ? launch_status(launch_tiled_backward(a, s), "tiled FeatureAggregate backward launch")
                       : launch_status(launch_tiled_forward(a, s), "tiled FeatureAggregate forward launch");
     }

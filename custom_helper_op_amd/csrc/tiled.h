@@ -354,18 +354,18 @@ __device__ __forceinline__ void fold_groups(const R *ch, int sub, R *out) {
   }
 }
 
-template <typename S, int VEC, int LPP>
+template <typename S, int VEC, int LPP, bool PAD>
 __device__ __forceinline__ void store_groups(S *p, const typename Storage<S>::Real *v, int sub) {
   // p already points at this lane's first group; a pixel's row holds VEC * LPP / sub values
   constexpr int C = VEC * LPP, B = (int)sizeof(S);
   if (sub == 1) {
-    store_vec<S, VEC, whole_lines(C, B)>(p, v);
+    store_vec<S, VEC, !PAD && whole_lines(C, B)>(p, v);
   } else if (sub == 2) {
-    store_vec<S, VEC / 2, whole_lines(C / 2, B)>(p, v);
+    store_vec<S, VEC / 2, !PAD && whole_lines(C / 2, B)>(p, v);
   } else if (sub == 4) {
-    store_vec<S, VEC / 4, whole_lines(C / 4, B)>(p, v);
+    store_vec<S, VEC / 4, !PAD && whole_lines(C / 4, B)>(p, v);
   } else if (threadIdx.x & 1) {  // sub == 8: the group's second lane
-    store_vec<S, 1, whole_lines(C / 8, B)>(p, v);
+    store_vec<S, 1, !PAD && whole_lines(C / 8, B)>(p, v);
   }
 }
 
@@ -547,10 +547,10 @@ __device__ __forceinline__ void store_ints(int32_t *p, const int *v) {
 }
 
 // A row of winners per channel, four of this lane's.
-template <int VEC, int LPP, int GAP>
+template <int VEC, int LPP, int GAP, bool PAD>
 __device__ __forceinline__ void store_winners(int32_t *p, const int *v) {
   if constexpr (GAP == 2) {
-    store_ints<VEC, whole_lines(VEC * LPP, 4)>(p, v);
+    store_ints<VEC, !PAD && whole_lines(VEC * LPP, 4)>(p, v);
   } else {
     store_ints<2, false>(p, v);
     store_ints<2, false>(p + GAP, v + 2);
@@ -797,7 +797,14 @@ constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce, bool wide
 // twice as long and the stores bound the launch as before (two views, 32 channels, 128 x 160 x 192:
 // 1.04 GB in 243 us, 4.3 TB/s; 430 us with a lane per channel, which reads every record and offset
 // once for two pixels instead of eight).
-template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool LIT = (sizeof(S) == 8)>
+// PAD: fewer channels than the pixel's lanes hold (20, 24, 28 on eight lanes), as in the gradient kernel
+// below: the lanes past the last channel repeat the last lane's work and store nothing.  Literal, so
+// that the results are those of the lane-per-channel kernels, where two pixels share a wave instead of
+// eight (24 channels: mean over two views, 89 x 106 x 192, four images 433 -> 255 us; aggregate, six
+// views, 130 x 153 x 56, 362 -> 182 us; f16 groups, five views, 111 x 152 x 25, 155 -> 73 us; minimum
+// over five views, 63 x 85 x 37, 47 -> 36 us).
+template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool PAD = false,
+          bool LIT = (sizeof(S) == 8 || PAD)>
 // At most five waves per SIMD: with six (the two-view instantiation needs only 80 VGPRs)
 // the waves of a CU evict each other's taps from L1 and the kernel is 6 % slower.  The lower
 // bound: see forward_min_waves.
@@ -809,7 +816,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   constexpr int PPW = 64 / LPP;
   // bytes of a float4's worth of records per float of lane offset (p4, q4 below)
   constexpr unsigned kR4 = sizeof(R);
-  constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), false);
+  constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
+  static_assert(!PAD || CORR != 3, "CostVolumeV3: whole pixels");
   // Three views and more in double: the views take turns with one set of taps (four sets of four
   // channels are 128 registers), also in the ops that keep a set per view in float.
   constexpr bool kOneSet = sizeof(R) == 8 && NV >= 3;
@@ -826,7 +834,9 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   }
   const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
   const R half = a.half;
-  const int ch0 = lane_first(t.cl, GAP);
+  const bool ch_ok = !PAD || t.cl * VEC < C;
+  const int clc = PAD ? min(t.cl, C / VEC - 1) : t.cl;  // the lane whose channels this lane holds
+  const int ch0 = lane_first(clc, GAP);
   // LDS records: wts[NV][LPP][PPW] then off[NV][LPP][PPW], addressed as (lane-dependent
   // byte offset) + (compile-time constant) so that the constant lands in the instruction's
   // offset field instead of costing a register per unrolled depth
@@ -873,10 +883,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   // pair; MEAN averages the views' maxima, MIN keeps the largest with (view, reference group,
   // source group) as its mask (cost_volume_kernels_gpu_v3.cu.cc:52-146, :148-262)
   const int OC = CORR == 1 ? a.groups : (CORR == 2 || CORR == 3) ? 1 : C;
-  const int goff = group_offset<VEC>(t.cl, g.sub);  // first of this lane's group values in a row
+  const int goff = group_offset<VEC>(clc, g.sub);  // first of this lane's group values in a row
   // the cost rows of the per-channel ops (and the sample rows of the warp-only op) stream past
   // the caches where they cover whole lines
-  constexpr bool kNtRows = whole_lines(VEC * LPP, (int)sizeof(S));
+  constexpr bool kNtRows = !PAD && whole_lines(VEC * LPP, (int)sizeof(S));
   // one value per voxel that is added up in channel order
   constexpr bool kRowSums = CORR == 2 && (REDUCE == 1 || LIT);
   const int d_lo = t.d_lo, d_hi = t.d_hi;
@@ -989,6 +999,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           if constexpr (LPP > 1) {
 #pragma unroll
             for (int k = 0; k < LPP; ++k) {
+              if (PAD && k * VEC >= C) continue;  // (uniform)
               const R4 v = lds_at<R4>(smem, (unsigned)((t.p * LPP + t.cl) * ROWB),
                                       kSq + k * VEC * (int)sizeof(R));
               tot += v.x;
@@ -1048,7 +1059,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             for (int c = 0; c < VEC; ++c)
               smp[c] = wt.x * tap[0][0][c] + wt.y * tap[0][1][c] + wt.z * tap[0][2][c] + wt.w * tap[0][3][c];
           }
-          if (t.pix_ok)
+          if (t.pix_ok && ch_ok)
             store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d0 + jj) * N + n) * C + ch0, smp);
         }
       }
@@ -1156,7 +1167,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
       for (int jj = 0; jj < DB; ++jj) {
         const int d = d0 + j0 + jj;
-        if (d >= d_hi || !t.pix_ok) continue;
+        if (d >= d_hi || !t.pix_ok || !ch_ok) continue;
         S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
         if constexpr (REDUCE == 1) {
           int32_t *mout = mask_pix + d * OC;
@@ -1167,12 +1178,12 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           }
           if (CORR == 0) {
             store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc[jj]);
-            store_winners<VEC, LPP, GAP>(mout + ch0, arg[jj]);
+            store_winners<VEC, LPP, GAP, PAD>(mout + ch0, arg[jj]);
           } else {
-            store_groups<S, VEC, LPP>(out + goff, acc[jj], g.sub);
-            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg[jj]);
-            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg[jj]);
-            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg[jj]);
+            store_groups<S, VEC, LPP, PAD>(out + goff, acc[jj], g.sub);
+            if (g.sub == 1) store_ints<VEC, !PAD && whole_lines(VEC * LPP, 4)>(mout + goff, arg[jj]);
+            else if (g.sub == 2) store_ints<VEC / 2, !PAD && whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg[jj]);
+            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, !PAD && whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg[jj]);
           }
         } else {
           mean_of<LIT>(acc[jj], kcnt[jj]);
@@ -1189,7 +1200,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
               for (int c = 0; c < VEC; ++c) grp[c] = dflt;
             }
-            store_groups<S, VEC, LPP>(out + goff, grp, g.sub);
+            store_groups<S, VEC, LPP, PAD>(out + goff, grp, g.sub);
           }
         }
       }
@@ -1284,7 +1295,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               smp[c] = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
                        wt.w * tap[n][3][c];
           }
-          if (n < N && t.pix_ok)
+          if (n < N && t.pix_ok && ch_ok)
             store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d) * N + n) * C + ch0, smp);
           continue;
         }
@@ -1366,17 +1377,17 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           for (int c = 0; c < VEC; ++c)
             if (arg[c] < 0) acc[c] = dflt;
         }
-        if (t.pix_ok) {
+        if (t.pix_ok && ch_ok) {
           S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
           int32_t *mout = mask_pix + d * OC;
           if (CORR == 0) {
             store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc);
-            store_winners<VEC, LPP, GAP>(mout + ch0, arg);
+            store_winners<VEC, LPP, GAP, PAD>(mout + ch0, arg);
           } else {
-            store_groups<S, VEC, LPP>(out + goff, acc, g.sub);
-            if (g.sub == 1) store_ints<VEC, whole_lines(VEC * LPP, 4)>(mout + goff, arg);
-            else if (g.sub == 2) store_ints<VEC / 2, whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg);
-            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg);
+            store_groups<S, VEC, LPP, PAD>(out + goff, acc, g.sub);
+            if (g.sub == 1) store_ints<VEC, !PAD && whole_lines(VEC * LPP, 4)>(mout + goff, arg);
+            else if (g.sub == 2) store_ints<VEC / 2, !PAD && whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg);
+            else if (g.sub == 4 || (t.cl & 1)) store_ints<1, !PAD && whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg);
           }
         }
         continue;
@@ -1395,7 +1406,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         continue;
       }
       mean_of<LIT>(acc, k);
-      if (t.pix_ok) {
+      if (t.pix_ok && ch_ok) {
         S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
         if (CORR == 0) {
           if (fill && k == 0) {
@@ -1410,7 +1421,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
             for (int c = 0; c < VEC; ++c) grp[c] = dflt;
           }
-          store_groups<S, VEC, LPP>(out + goff, grp, g.sub);
+          store_groups<S, VEC, LPP, PAD>(out + goff, grp, g.sub);
         }
       }
     }

@@ -419,9 +419,9 @@ int chop_cost_volume_sample_coords_f64(void *stream, int half_centor, int64_t B,
  * by the tests to cover all three. */
 int chop_set_kernel_family(int family);
 /* Which family served the last forward/backward call of this thread: 0 none yet,
- * 1 general kernels, 2 tiled kernels, 3 strip kernels.  In double 3 stands for the tiled kernels
- * as well, which an unforced call takes where the shape qualifies (the forward results of the two
- * are the same to the bit). */
+ * 1 general kernels, 2 tiled kernels, 3 strip kernels.  In double, and forward for 20, 24 and 28
+ * channels, 3 stands for the tiled kernels as well, which an unforced call takes where the shape
+ * qualifies (the forward results of the two are the same to the bit). */
 int chop_last_kernel_family(void);
 /* How many source views one workgroup of the last tiled backward call of this thread went
  * through in turn (1: every view had workgroups of its own; N: narrow pixels on a large
