@@ -237,12 +237,10 @@ int v3_call(void *stream, int reduce, int half_centor, const Dims &d, int groups
   a.ref_grad = ref_grad, a.src_grad = src_grad, a.depth_grad = base_plane_grad;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (g_kernel_family == 0 && work) {
-    if constexpr (std::is_same<S, float>::value) {
-      if (backward ? tiled_backward_supported(a) : tiled_forward_supported(a)) {
-        g_last_family = 2;
-        return backward ? launch_status(launch_tiled_backward(a, s), "tiled CostVolumeV3 backward launch")
-                        : launch_status(launch_tiled_forward(a, s), "tiled CostVolumeV3 forward launch");
-      }
+    if (backward ? tiled_backward_supported(a) : tiled_forward_supported(a)) {
+      g_last_family = tiled_family(a, !backward);
+      return backward ? launch_status(launch_tiled_backward(a, s), "tiled CostVolumeV3 backward launch")
+                      : launch_status(launch_tiled_forward(a, s), "tiled CostVolumeV3 forward launch");
     }
   }
   if (g_kernel_family != 1 && work && backward && strip_pair_backward_supported(a)) {

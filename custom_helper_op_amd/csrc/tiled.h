@@ -267,7 +267,7 @@ constexpr bool whole_lines(int elements, int elem_bytes) { return elements * ele
 // of a pixel is one contiguous run.  Not where a lane's channels have to be neighbours (correlation
 // groups) and not with idle lanes (their pairs would lie in the other half).
 constexpr int lane_gap(int lpp, int corr, int elem_bytes, bool pad) {
-  return elem_bytes == 8 && corr != 1 && !pad ? 2 * lpp : 2;
+  return elem_bytes == 8 && corr != 1 && corr != 3 && corr != 5 && !pad ? 2 * lpp : 2;
 }
 // first channel of lane `cl`; channel c (0..3) is that + c / 2 * gap + c % 2
 __device__ __forceinline__ int lane_first(int cl, int gap) { return gap == 2 ? cl * 4 : cl * 2; }
@@ -588,9 +588,9 @@ __device__ __forceinline__ void fold_or_keep(const R (&acc)[4], int sub, R (&out
   }
 }
 // One butterfly step of "largest value, earliest pair on a tie" (both partners end equal).
-template <int CTRL>
-__device__ __forceinline__ void better_pair(float &best, int &code) {
-  const float ob = dpp_move<CTRL>(best);
+template <int CTRL, typename R>
+__device__ __forceinline__ void better_pair(R &best, int &code) {
+  const R ob = dpp_move<CTRL>(best);
   const int oc = dpp_move<CTRL>(code);
   const bool take = ob > best || (ob == best && oc < code);
   best = take ? ob : best;
@@ -643,7 +643,30 @@ __device__ __forceinline__ void add_groups(R (&acc)[4], const R (&val)[4], int s
     for (int c = 0; c < 4; ++c) acc[c] += val[c];
   }
 }
-constexpr int kNoPair = 0x7fffffff;  // pair code: source group * 16 + reference group
+constexpr int kNoPair = 0x7fffffff;
+constexpr int kPairRow = 64;  // pair code: source group * kPairRow + reference group
+// Largest value and smallest integer over the lanes of a pixel, left in every one of them (a NaN
+// gives way to a number: one instruction each, the lane move is part of it).
+__device__ __forceinline__ float larger(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ double larger(double a, double b) { return __builtin_fmax(a, b); }
+template <int LPP, typename R>
+__device__ __forceinline__ R group_max(R v) {
+  if constexpr (LPP >= 2) v = larger(v, dpp_move<0xB1>(v));
+  if constexpr (LPP >= 4) v = larger(v, dpp_move<0x4E>(v));
+  if constexpr (LPP >= 8) v = larger(v, dpp_move<0x141>(v));
+  if constexpr (LPP >= 16) v = larger(v, dpp_move<0x140>(v));
+  return v;
+}
+template <int LPP>
+__device__ __forceinline__ int group_min(int v) {
+  if constexpr (LPP >= 2) v = min(v, dpp_move<0xB1>(v));
+  if constexpr (LPP >= 4) v = min(v, dpp_move<0x4E>(v));
+  if constexpr (LPP >= 8) v = min(v, dpp_move<0x141>(v));
+  if constexpr (LPP >= 16) v = min(v, dpp_move<0x140>(v));
+  return v;
+}
+// (CORR 3: groups of four and eight channels; CORR 5: of one and two)
+constexpr bool best_pair_op(int corr) { return corr == 3 || corr == 5; }
 
 // The best (source group, reference group) pair of one accepted sample of one pixel, found
 // by the pixel's LPP lanes exactly as the reference's loop finds it
@@ -654,36 +677,112 @@ constexpr int kNoPair = 0x7fffffff;  // pair code: source group * 16 + reference
 // strict "<" from the smallest positive float, so the earliest pair keeps a tie.
 // `ref_row`: the pixel's reference channels in LDS.  Every lane of the pixel returns the same
 // best value (the seed when no pair exceeds it) and pair code (kNoPair then).
-template <int VEC, int LPP, int SUB>
-__device__ __forceinline__ void v3_best_pair(const float (&smp)[VEC], const float *ref_row, int cl,
-                                             float &best, int &code) {
-  static_assert(VEC == 4 && (SUB == 4 || SUB == 8), "a group is one lane or two");
-  constexpr int C = VEC * LPP, G = C / SUB, LPG = SUB / 4;
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  const int group = cl / LPG, koff = (cl % LPG) * 4;
-  best = __FLT_MIN__;
+// Every pair is one thread's own loop in the general kernel, which these widths and double ran before
+// (groups of one, two views, 41 x 54 x 9, two images of 32 channels: forward 360 -> 11 us, gradient 380
+// -> 32 us; double, groups of two, three views, 213 x 309 x 33: 2330 -> 1045 and 3700 -> 1570 us).  One
+// class loses: the minimum's gradient of narrow groups over a large image and two views (383 x 534 x
+// 27: 1090 -> 1250 us, with a forward pass of 6100 -> 300 us), where few channels receive anything.
+// Groups of two channels: a lane's four are two source groups.  Groups of one (every channel with every
+// channel): the largest product of a source value is with the pixel's largest reference value, or with
+// its smallest where the source value is negative, because rounding keeps the order; so `ends` (the
+// two, ref_ends) replace the search, and the pair is then the first source channel and the first
+// reference channel whose product is that value.
+template <typename R, int VEC, int LPP, int SUB, bool CODE>
+__device__ __forceinline__ void v3_best_pair(const R (&smp)[VEC], const R *ref_row, const Two<R> &ends, int cl,
+                                             R &best, int &code) {
+  static_assert(VEC == 4 && (SUB == 1 || SUB == 2 || SUB == 4 || SUB == 8), "a group: part of a lane, one lane or two");
+  constexpr int C = VEC * LPP, G = C / SUB, LPG = SUB <= 4 ? 1 : SUB / 4;
+  const int group = SUB >= 4 ? cl / LPG : cl * (4 / SUB), koff = (cl % LPG) * 4;
+  best = Limits<R>::min_positive();
   code = kNoPair;
+  if constexpr (SUB == 1) {
+    R top[VEC];
 #pragma unroll
-  for (int gi = 0; gi < G; ++gi) {
-    const f4 r = *reinterpret_cast<const f4 *>(ref_row + gi * SUB + koff);
-    const float p0 = smp[0] * r[0], p1 = smp[1] * r[1], p2 = smp[2] * r[2], p3 = smp[3] * r[3];
-    float dot = ((p0 + p1) + p2) + p3;  // (0 + p0 differs from p0 in the sign of zero only)
-    if constexpr (LPG == 2) {
-      const float head = dpp_move<0xA0>(dot);  // quad_perm 0,0,2,2: the even lane's four terms
-      dot = (((head + p0) + p1) + p2) + p3;    // complete in the odd lane
+    for (int c = 0; c < VEC; ++c) {
+      top[c] = smp[c] * (smp[c] > R(0) ? ends.y : ends.x);
+      best = larger(best, top[c]);
     }
-    if (best < dot) {
-      best = dot;
-      code = group * 16 + gi;
+    best = group_max<LPP>(best);
+    if constexpr (!CODE) return;
+    int gs = kNoPair;
+#pragma unroll
+    for (int c = VEC - 1; c >= 0; --c)
+      if (top[c] == best) gs = group + c;
+    gs = group_min<LPP>(gs);
+    if (gs != kNoPair) {  // (the seed itself may equal a product: such a pair does not exceed it)
+      const int cs = gs & 3;
+      const R own = cs == 0 ? smp[0] : cs == 1 ? smp[1] : cs == 2 ? smp[2] : smp[3];
+      const R s = __shfl(own, gs >> 2, LPP);
+      const Four<R> r = *reinterpret_cast<const Four<R> *>(ref_row + cl * 4);
+      int gi = kNoPair;
+      if (s * r.w == best) gi = group + 3;
+      if (s * r.z == best) gi = group + 2;
+      if (s * r.y == best) gi = group + 1;
+      if (s * r.x == best) gi = group;
+      gi = group_min<LPP>(gi);
+      if (Limits<R>::min_positive() < best) code = gs * kPairRow + gi;
+    }
+    return;
+  } else if constexpr (SUB == 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll 4
+      for (int g2 = 0; g2 < G; g2 += 2) {
+        const Four<R> r = *reinterpret_cast<const Four<R> *>(ref_row + g2 * 2);
+        const R d0 = smp[2 * u] * r.x + smp[2 * u + 1] * r.y, d1 = smp[2 * u] * r.z + smp[2 * u + 1] * r.w;
+        if constexpr (CODE) {
+          if (best < d0) best = d0, code = (group + u) * kPairRow + g2;
+          if (best < d1) best = d1, code = (group + u) * kPairRow + g2 + 1;
+        } else {
+          best = larger(best, larger(d0, d1));
+        }
+      }
+    }
+    if constexpr (CODE) {
+      if constexpr (LPP >= 2) better_pair<0xB1>(best, code);    // quad_perm 1,0,3,2
+      if constexpr (LPP >= 4) better_pair<0x4E>(best, code);    // quad_perm 2,3,0,1
+      if constexpr (LPP >= 8) better_pair<0x141>(best, code);   // row_half_mirror
+      if constexpr (LPP >= 16) better_pair<0x140>(best, code);  // row_mirror
+    } else {
+      best = group_max<LPP>(best);
+    }
+  } else {
+    // The largest value first (one instruction per pair, the lanes' tournament included), then the
+    // first pair that has it: keeping value and pair together takes three and a longer tournament
+    // (32 channels in four groups, two views, 120 x 152 x 64: forward, which needs no pair, 78 -> 60 us,
+    // gradient 199 -> 189 us).
+    R dot[G];
+#pragma unroll
+    for (int gi = 0; gi < G; ++gi) {
+      const Four<R> r = *reinterpret_cast<const Four<R> *>(ref_row + gi * SUB + koff);
+      const R p0 = smp[0] * r.x, p1 = smp[1] * r.y, p2 = smp[2] * r.z, p3 = smp[3] * r.w;
+      dot[gi] = ((p0 + p1) + p2) + p3;  // (0 + p0 differs from p0 in the sign of zero only)
+      if constexpr (LPG == 2) {
+        const R head = dpp_move<0xA0>(dot[gi]);  // quad_perm 0,0,2,2: the even lane's four terms
+        dot[gi] = (((head + p0) + p1) + p2) + p3;    // complete in the odd lane
+      }
+    }
+    const bool mine = LPG == 1 || (cl & 1) != 0;
+    R top = dot[0];
+#pragma unroll
+    for (int gi = 1; gi < G; ++gi) top = larger(top, dot[gi]);
+    best = group_max<LPP>(larger(best, mine ? top : best));
+    if constexpr (CODE) {
+#pragma unroll
+      for (int gi = G - 1; gi >= 0; --gi)
+        if (dot[gi] == best) code = group * kPairRow + gi;
+      code = group_min<LPP>(mine ? code : kNoPair);
+      if (!(Limits<R>::min_positive() < best)) code = kNoPair;  // no pair exceeds the seed
     }
   }
-  if constexpr (LPG == 2) {
-    if ((cl & 1) == 0) best = __FLT_MIN__, code = kNoPair;
-  }
-  if constexpr (LPP >= 2) better_pair<0xB1>(best, code);    // quad_perm 1,0,3,2
-  if constexpr (LPP >= 4) better_pair<0x4E>(best, code);    // quad_perm 2,3,0,1
-  if constexpr (LPP >= 8) better_pair<0x141>(best, code);   // row_half_mirror
-  if constexpr (LPP >= 16) better_pair<0x140>(best, code);  // row_mirror
+}
+
+// Smallest and largest reference value of a pixel, NaN apart.
+template <int LPP, typename R>
+__device__ __forceinline__ Two<R> ref_ends(const R (&ref)[4]) {
+  const R hi = larger(larger(ref[0], ref[1]), larger(ref[2], ref[3]));
+  const R lo = -larger(larger(-ref[0], -ref[1]), larger(-ref[2], -ref[3]));
+  return Two<R>{-group_max<LPP>(-lo), group_max<LPP>(hi)};
 }
 
 // The gradient of one accepted sample flows through one pair: the view's best pair, found
@@ -692,38 +791,48 @@ __device__ __forceinline__ void v3_best_pair(const float (&smp)[VEC], const floa
 // group); racc += the reference gradient of this lane's channels (zero outside the winning
 // reference group, :494-512).  `rows` = two LDS arrays of 64*VEC floats: the pixel rows of
 // the reference image (written once by the caller) and of this sample.
-template <int VEC, int LPP, int SUB, int REDUCE>
-__device__ __forceinline__ void v3_pair_gradients(const Four<float> wt, const float (&tap)[4][VEC],
-                                                  float cg, int pair, float *rows, int p, int cl,
-                                                  float (&racc)[VEC], float (&gsrc)[VEC]) {
-  constexpr int C = VEC * LPP, LPG = SUB / 4;
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  float *ref_row = rows + p * C, *smp_row = rows + 64 * VEC + p * C;
-  const int group = cl / LPG, koff = (cl % LPG) * 4;
-  float smp[VEC];
+template <typename R, int VEC, int LPP, int SUB, int REDUCE>
+__device__ __forceinline__ void v3_pair_gradients(const Four<R> wt, const R (&tap)[4][VEC], const Two<R> &ends,
+                                                  R cg, int pair, R *rows, int p, int cl,
+                                                  R (&racc)[VEC], R (&gsrc)[VEC]) {
+  constexpr int C = VEC * LPP, LPG = SUB <= 4 ? 1 : SUB / 4;
+  R *ref_row = rows + p * C, *smp_row = rows + 64 * VEC + p * C;
+  const int group = SUB >= 4 ? cl / LPG : cl * (4 / SUB), koff = (cl % LPG) * 4;
+  R smp[VEC];
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     smp[c] = wt.x * tap[0][c] + wt.y * tap[1][c] + wt.z * tap[2][c] + wt.w * tap[3][c];
-  *reinterpret_cast<f4 *>(smp_row + cl * 4) = f4{smp[0], smp[1], smp[2], smp[3]};
+  *reinterpret_cast<Four<R> *>(smp_row + cl * 4) = Four<R>{smp[0], smp[1], smp[2], smp[3]};
   int code = pair;
   if constexpr (REDUCE == 0) {
-    float best;
-    v3_best_pair<VEC, LPP, SUB>(smp, ref_row, cl, best, code);
+    R best;
+    v3_best_pair<R, VEC, LPP, SUB, true>(smp, ref_row, ends, cl, best, code);
   }
   const bool any = code != kNoPair;
-  const int gi_w = code & 15, gs_w = code >> 4;
+  const int gi_w = any ? code % kPairRow : 0, gs_w = any ? code / kPairRow : 0;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) gsrc[c] = 0.f;
-  if (any && group == gs_w) {
-    const f4 r = *reinterpret_cast<const f4 *>(ref_row + gi_w * SUB + koff);
+  for (int c = 0; c < 4; ++c) gsrc[c] = R(0);
+  if constexpr (SUB >= 4) {
+    if (any && group == gs_w) {
+      const Four<R> r = *reinterpret_cast<const Four<R> *>(ref_row + gi_w * SUB + koff);
+      gsrc[0] = cg * r.x, gsrc[1] = cg * r.y, gsrc[2] = cg * r.z, gsrc[3] = cg * r.w;
+    }
+  } else {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) gsrc[c] = cg * r[c];
+    for (int c = 0; c < 4; ++c)
+      if (any && group + c / SUB == gs_w) gsrc[c] = cg * ref_row[gi_w * SUB + c % SUB];
   }
   wave_sync();  // the sample row is complete
-  if (any && group == gi_w) {
-    const f4 m = *reinterpret_cast<const f4 *>(smp_row + gs_w * SUB + koff);
+  if constexpr (SUB >= 4) {
+    if (any && group == gi_w) {
+      const Four<R> m = *reinterpret_cast<const Four<R> *>(smp_row + gs_w * SUB + koff);
+      racc[0] = mad(cg, m.x, racc[0]), racc[1] = mad(cg, m.y, racc[1]);
+      racc[2] = mad(cg, m.z, racc[2]), racc[3] = mad(cg, m.w, racc[3]);
+    }
+  } else {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) racc[c] = __builtin_fmaf(cg, m[c], racc[c]);
+    for (int c = 0; c < 4; ++c)
+      if (any && group + c / SUB == gi_w) racc[c] = mad(cg, smp_row[gs_w * SUB + c % SUB], racc[c]);
   }
 }
 
@@ -817,10 +926,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   // bytes of a float4's worth of records per float of lane offset (p4, q4 below)
   constexpr unsigned kR4 = sizeof(R);
   constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
-  static_assert(!PAD || CORR != 3, "CostVolumeV3: whole pixels");
+  static_assert(!PAD || !best_pair_op(CORR), "CostVolumeV3: whole pixels");
   // Three views and more in double: the views take turns with one set of taps (four sets of four
   // channels are 128 registers), also in the ops that keep a set per view in float.
-  constexpr bool kOneSet = sizeof(R) == 8 && NV >= 3;
+  constexpr bool kOneSet = sizeof(R) == 8 && NV >= 3 && !best_pair_op(CORR);
   constexpr int NT = kOneSet ? 1 : NV;
   extern __shared__ __align__(16) unsigned char smem[];
   Tile<LPP> t;
@@ -852,10 +961,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   R ref[VEC];
   if constexpr (CORR != 4) {
     load_vec<S, VEC, false, GAP>(a.ref + t.pix * C + ch0, ref);
-    if constexpr (CORR == 3) {
+    if constexpr (best_pair_op(CORR)) {
       // CostVolumeV3: every lane of a pixel reads all of the pixel's reference groups
-      static_assert(CORR != 3 || (LPP > 1 && VEC == 4), "CostVolumeV3: wide pixels");
-      float *s_ref = reinterpret_cast<float *>(smem + kRec);  // behind the records
+      static_assert(!best_pair_op(CORR) || (LPP > 1 && VEC == 4), "CostVolumeV3: wide pixels");
+      R *s_ref = reinterpret_cast<R *>(smem + kRec);  // behind the records
 #pragma unroll
       for (int c = 0; c < VEC; ++c) s_ref[t.p * (VEC * LPP) + t.cl * VEC + c] = ref[c];
       wave_sync();
@@ -864,6 +973,9 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
     for (int c = 0; c < VEC; ++c) ref[c] = R(0);  // the warp-only op has no reference image
   }
+  constexpr int kWideSub = CORR == 5 ? 2 : 8;  // CostVolumeV3: the wider of the kernel's two group widths
+  Two<R> ends{};
+  if constexpr (CORR == 5) ends = ref_ends<LPP>(ref);
   const S *view[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n)
@@ -882,7 +994,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   // 3: CostVolumeV3, per view the largest correlation of any (source group, reference group)
   // pair; MEAN averages the views' maxima, MIN keeps the largest with (view, reference group,
   // source group) as its mask (cost_volume_kernels_gpu_v3.cu.cc:52-146, :148-262)
-  const int OC = CORR == 1 ? a.groups : (CORR == 2 || CORR == 3) ? 1 : C;
+  const int OC = CORR == 1 ? a.groups : (CORR == 2 || best_pair_op(CORR)) ? 1 : C;
   const int goff = group_offset<VEC>(clc, g.sub);  // first of this lane's group values in a row
   // the cost rows of the per-channel ops (and the sample rows of the warp-only op) stream past
   // the caches where they cover whole lines
@@ -1229,7 +1341,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         arg[c] = -1;
       }
       int k = 0;
-      float v3_acc = REDUCE == 0 ? 0.f : 1.175494351e-38f;  // :76, :193
+      R v3_acc = REDUCE == 0 ? R(0) : Limits<R>::min_positive();  // :76, :193
       int v3_view = -1, v3_code = 0;
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
@@ -1242,7 +1354,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           off = r_off[n];
           wt = r_wts[n];
         }
-        if constexpr (CORR == 3) {
+        if constexpr (best_pair_op(CORR)) {
           if (off >= 0) {
             if (off != cur[n]) {
               cur[n] = off;
@@ -1252,19 +1364,18 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
               load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
             }
-            float smp[VEC];
+            R smp[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
               smp[c] = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
                        wt.w * tap[n][3][c];
-            const float *ref_row =
-                reinterpret_cast<const float *>(smem + kRec) + t.p * (VEC * LPP);
-            float best;
+            const R *ref_row = reinterpret_cast<const R *>(smem + kRec) + t.p * (VEC * LPP);
+            R best;
             int code;
-            if (g.sub == 8)
-              v3_best_pair<VEC, LPP, 8>(smp, ref_row, t.cl, best, code);
+            if (g.sub == kWideSub)
+              v3_best_pair<R, VEC, LPP, kWideSub, REDUCE == 1>(smp, ref_row, ends, t.cl, best, code);
             else
-              v3_best_pair<VEC, LPP, 4>(smp, ref_row, t.cl, best, code);
+              v3_best_pair<R, VEC, LPP, kWideSub / 2, REDUCE == 1>(smp, ref_row, ends, t.cl, best, code);
             if constexpr (REDUCE == 0) {
               v3_acc += best;  // the seed when no pair exceeds it (:113-131)
             } else if (v3_acc < best) {
@@ -1357,16 +1468,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         }
       }
       if constexpr (CORR == 4) continue;  // every view's row is already stored
-      if constexpr (CORR == 3) {
+      if constexpr (best_pair_op(CORR)) {
         // the lane whose slice index equals the depth's place in the chunk keeps the voxel
         if (t.cl == jj) {
           if constexpr (REDUCE == 0) {
-            agg_out = k > 0 ? v3_acc / static_cast<float>(k) : 0.f;  // :136-141
+            agg_out = k > 0 ? v3_acc / static_cast<R>(k) : R(0);  // :136-141
           } else {
-            agg_out = v3_view >= 0 ? v3_acc : 0.f;  // :253-257
+            agg_out = v3_view >= 0 ? v3_acc : R(0);  // :253-257
             v3_out[0] = v3_view;
-            v3_out[1] = v3_view >= 0 ? (v3_code & 15) : -1;
-            v3_out[2] = v3_view >= 0 ? (v3_code >> 4) : -1;
+            v3_out[1] = v3_view >= 0 ? v3_code % kPairRow : -1;
+            v3_out[2] = v3_view >= 0 ? v3_code / kPairRow : -1;
           }
         }
         continue;
@@ -1425,11 +1536,11 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         }
       }
     }
-    if constexpr ((CORR == 2 || CORR == 3) && LPP > 1) {
+    if constexpr ((CORR == 2 || best_pair_op(CORR)) && LPP > 1) {
       if (t.pix_ok && d0 + t.cl < d_hi)
         reinterpret_cast<R *>(a.cost)[t.pix * D + d0 + t.cl] = agg_out;
     }
-    if constexpr (CORR == 3 && REDUCE == 1) {
+    if constexpr (best_pair_op(CORR) && REDUCE == 1) {
       if (t.pix_ok && d0 + t.cl < d_hi) {
         int32_t *m = a.mask + (t.pix * D + d0 + t.cl) * 3;
         m[0] = v3_out[0], m[1] = v3_out[1], m[2] = v3_out[2];
@@ -1978,10 +2089,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                      : backward_list_bytes<R, VEC, LPP, kForm>() > 0 ? s_own_list
                                                                  : reinterpret_cast<int *>(s_stage);
   // CORR 3 only: reference rows, sample rows
-  float *s_v3 = reinterpret_cast<float *>(s_own_list + backward_list_bytes<R, VEC, LPP, kForm>() / 4);
-  static_assert(CORR != 3 || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
+  R *s_v3 = reinterpret_cast<R *>(s_own_list + backward_list_bytes<R, VEC, LPP, kForm>() / 4);
+  static_assert(!best_pair_op(CORR) || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
   const R base = per_voxel_depth ? R(0) : a.base_plane[t.pix];
-  static_assert(!PAD || CORR != 3, "CostVolumeV3: whole pixels");
+  static_assert(!PAD || !best_pair_op(CORR), "CostVolumeV3: whole pixels");
   const int cm = PAD ? C : WN::C;
   const bool ch_ok = !PAD || t.cl * VEC < C;
   const int clc = PAD ? min(t.cl, C / VEC - 1) : t.cl;  // the lane whose channels this lane reads
@@ -1989,7 +2100,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   R ref[VEC];
   if constexpr (CORR != 4) {
     load_vec<S, VEC, false, GAP>(a.ref + t.pix * C + ch0, ref);
-    if constexpr (CORR == 3) {
+    if constexpr (best_pair_op(CORR)) {
 #pragma unroll
       for (int c = 0; c < VEC; ++c) s_v3[t.p * (VEC * LPP) + t.cl * VEC + c] = ref[c];
     }
@@ -1998,6 +2109,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
     for (int c = 0; c < VEC; ++c) ref[c] = R(0);
   }
+  constexpr int kWideSub = CORR == 5 ? 2 : 8;  // CostVolumeV3: the wider of the kernel's two group widths
+  Two<R> ends{};
+  if constexpr (CORR == 5 && REDUCE == 0) ends = ref_ends<LPP>(ref);
   const int64_t view_elems = (int64_t)srcH * srcW * C;
   R *src_grad_img;
   if constexpr (kWide) src_grad_img = a.src_grad_acc;
@@ -2014,7 +2128,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   // upstream-gradient row and one 0/1 mask entry per (voxel, view)
   // (feature_aggregate_kernels_gpu.cu.cc:219-326)
   // 3: CostVolumeV3, one upstream gradient per voxel that flows through the best group pair
-  constexpr bool kVoxelGrad = CORR == 2 || CORR == 3;
+  constexpr bool kVoxelGrad = CORR == 2 || best_pair_op(CORR);
   // One winning view per voxel (or group): a view's runs are few and end far apart in depth.  An open
   // run from a cell left long ago need not make a chunk spread (kEndLeft), and where few runs end at
   // a depth moving the window to them costs more than adding them to memory (kFewRuns, in pixels of
@@ -2028,7 +2142,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   // all runs short, most pixels of a tile end together and the window pays.
   constexpr bool kWinners = REDUCE == 1 && (kVoxelGrad || CORR == 1);
   constexpr bool kEndLeft = kWinners && (CORR != 2 || LPP < 8);
-  constexpr int kFewRuns = !kWinners ? 0 : CORR == 3 ? 4 : PPW / 8;
+  constexpr int kFewRuns = !kWinners ? 0 : best_pair_op(CORR) ? 4 : PPW / 8;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
   const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
   const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : ch0;
@@ -2039,7 +2153,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   constexpr bool kMaskRows = REDUCE == 1 && !kVoxelGrad;
   // mask entries per voxel: the MIN reduce of CostVolumeV3 records (view, reference group,
   // source group)
-  const int mask_w = kMaskRows ? OC : (CORR == 3 && REDUCE == 1) ? 3 : 1;
+  const int mask_w = kMaskRows ? OC : (best_pair_op(CORR) && REDUCE == 1) ? 3 : 1;
   // element steps from one depth to the next in the upstream gradient and in the mask
   const int cg_step = CORR == 4 ? N * C : OC;
   const int cnt_step = CORR == 4 ? N : mask_w;
@@ -2153,13 +2267,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       if (t.pix_ok) cnt = cnt_src[(int64_t)(d0 + t.cl) * cnt_step];
       if constexpr (kVoxelGrad)  // the voxel's one upstream gradient rides with its record
         cg_vox = reinterpret_cast<const R *>(cg_lane)[d0 + t.cl];
-      if constexpr (CORR == 3 && REDUCE == 1) {
+      if constexpr (best_pair_op(CORR) && REDUCE == 1) {
         if (t.pix_ok) {
           const int64_t m3 = (int64_t)(d0 + t.cl) * 3;
           const int gi = cnt_src[m3 + 1], gs = cnt_src[m3 + 2];
           // a recorded group outside the image's groups: the voxel is skipped
           if ((unsigned)gi < (unsigned)a.groups && (unsigned)gs < (unsigned)a.groups)
-            v3_pair = gs * 16 + gi;
+            v3_pair = gs * kPairRow + gi;
           else
             cnt = -1;
         }
@@ -2249,7 +2363,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             scl = R(2) * cg_vox * quick_recip(static_cast<R>(cnt * C));
           else if constexpr (CORR == 2)
             scl = R(2) * (cg_vox / static_cast<R>(cnt * C));
-          else if constexpr (CORR == 3)
+          else if constexpr (best_pair_op(CORR))
             scl = cg_vox / static_cast<R>(cnt);  // cost_volume_kernels_gpu_v3.cu.cc:426
           else
             scl = (CORR == 0 ? R(2) : R(1)) * quick_recip(static_cast<R>(cnt));
@@ -2259,7 +2373,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
         // for the summed squared difference, its winning view)
         if constexpr (CORR == 2) {
           if (cnt == t.view0) scl = R(2) * (cg_vox / static_cast<R>(C));
-        } else if constexpr (CORR == 3) {
+        } else if constexpr (best_pair_op(CORR)) {
           if (cnt == t.view0) scl = cg_vox;  // cost_volume_kernels_gpu_v3.cu.cc:621-622
         } else {
           if (cnt >= 0) scl = CORR == 0 ? R(2) : R(1);
@@ -2356,7 +2470,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       }
       if constexpr (LPP > 1) {
         lds_at<R>(smem, q1, kScl) = scl;
-        if constexpr (CORR == 3)
+        if constexpr (best_pair_op(CORR))
           lds_at<int>(smem, q4, kDst) = v3_pair;  // (this op has no per-voxel depth gradient)
         else if constexpr (kDstWords)
           lds_at<R>(smem, q1, kDst) = R(0);
@@ -2503,19 +2617,19 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                 cell[n] = r_cell[n];
             }
             R gs3[VEC];
-            if constexpr (CORR == 3) {
+            if constexpr (best_pair_op(CORR)) {
               const int pair = REDUCE ? lds_at<int>(smem, p4, kDst + (jj * PPW) * 4) : 0;
-              if (g.sub == 8)
-                v3_pair_gradients<VEC, LPP, 8, REDUCE>(wt, tap[n], scl, pair, s_v3, t.p, t.cl, racc,
-                                                       gs3);
+              if (g.sub == kWideSub)
+                v3_pair_gradients<R, VEC, LPP, kWideSub, REDUCE>(wt, tap[n], ends, scl, pair, s_v3, t.p,
+                                                                 t.cl, racc, gs3);
               else
-                v3_pair_gradients<VEC, LPP, 4, REDUCE>(wt, tap[n], scl, pair, s_v3, t.p, t.cl, racc,
-                                                       gs3);
+                v3_pair_gradients<R, VEC, LPP, kWideSub / 2, REDUCE>(wt, tap[n], ends, scl, pair, s_v3, t.p,
+                                                                     t.cl, racc, gs3);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
               R gsrc;  // d(loss)/d(sample of this channel)
-              if constexpr (CORR == 3) {
+              if constexpr (best_pair_op(CORR)) {
                 gsrc = gs3[c];
               } else if constexpr (CORR == 4) {
                 gsrc = cg[c];
