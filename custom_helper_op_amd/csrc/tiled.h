@@ -877,9 +877,19 @@ constexpr int forward_lds_bytes(int lpp) {
 }
 // The sums of squares that have to be added up in channel order (the minimum, and the mean in its
 // literal form) also stage one chunk of squares per view: a row of C (+4 padding, so that the
-// eight readers of a pixel hit different banks) values per (pixel, depth).
-template <typename R = float>
-constexpr int forward_squares_bytes(int lpp) { return lpp > 1 ? 64 * (4 * lpp + 4) * (int)sizeof(R) : 0; }
+// readers of a pixel hit different banks) values per (pixel, depth).  From eight lanes on half the
+// chunk's depths at a time: whole chunks are 9 KB (32 channels), in double 18 KB, which with the
+// records held a CU to twelve workgroups and to five (minimum over three views, 135 x 181 x 48, 83 ->
+// 67 us with the segments of choose_segments; double, mean over three views, 149 x 220 x 116, 607 ->
+// 480 us).  Not with five and six views in float, whose registers hold the kernel to three waves
+// anyway (five views, 108 x 126 x 77: 147 us, 157 in halves).
+constexpr int squares_depths(int lpp, int nv, bool wide_real) {
+  return lpp >= 8 && (wide_real || nv <= 4) ? lpp / 2 : lpp;
+}
+template <int NV, typename R = float>
+constexpr int forward_squares_bytes(int lpp) {
+  return lpp > 1 ? 64 / lpp * squares_depths(lpp, NV, sizeof(R) == 8) * (4 * lpp + 4) * (int)sizeof(R) : 0;
+}
 
 // REDUCE: 0 mean over the accepted views (mask = their number), 1 per-channel minimum of
 // the squared difference / per-group maximum of the correlation with the winning view as
@@ -1064,8 +1074,11 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         int &cur1 = cur[n * kMany];
         if constexpr (kOneSet) cur1 = -1;
         R own[VEC];  // LPP == 1: this lane holds the whole pixel
+        constexpr int HALF = squares_depths(LPP, NV, sizeof(R) == 8);  // depths staged together
 #pragma unroll
-        for (int jj = 0; jj < LPP; ++jj) {
+        for (int j0 = 0; j0 < LPP; j0 += HALF) {
+#pragma unroll
+        for (int jj = j0; jj < j0 + HALF; ++jj) {
           if (d0 + jj >= d_hi) {
             if constexpr (LPP >= 16) continue; else break;
           }
@@ -1098,21 +1111,21 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             }
           }
           if constexpr (LPP > 1) {
-            const unsigned own_at = (unsigned)(t.p * LPP * ROWB + ch0 * (int)sizeof(R));
-            slot_write<GAP>(&lds_at<R>(smem, own_at, kSq + jj * ROWB), sq);
+            const unsigned own_at = (unsigned)(t.p * HALF * ROWB + ch0 * (int)sizeof(R));
+            slot_write<GAP>(&lds_at<R>(smem, own_at, kSq + (jj - j0) * ROWB), sq);
           } else {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) own[c] = sq[c];
           }
         }
         if constexpr (LPP > 1) wave_sync();
-        if ((vmask >> n) & 1u) {
+        if (((vmask >> n) & 1u) && (HALF == LPP || (unsigned)(t.cl - j0) < (unsigned)HALF)) {
           R tot = REDUCE == 1 ? R(0) : best;
           if constexpr (LPP > 1) {
 #pragma unroll
             for (int k = 0; k < LPP; ++k) {
               if (PAD && k * VEC >= C) continue;  // (uniform)
-              const R4 v = lds_at<R4>(smem, (unsigned)((t.p * LPP + t.cl) * ROWB),
+              const R4 v = lds_at<R4>(smem, (unsigned)((t.p * HALF + (HALF == LPP ? t.cl : t.cl % HALF)) * ROWB),
                                       kSq + k * VEC * (int)sizeof(R));
               tot += v.x;
               tot += v.y;
@@ -1127,6 +1140,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           else if (best > tot) best = tot, win = n;  // strict: the earliest view keeps a tie (:217)
         }
         if constexpr (LPP > 1) wave_sync();
+        }  // half of the chunk
       }
       const int d = d0 + t.cl;
       if (d < d_hi && t.pix_ok) {
@@ -2748,9 +2762,12 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 // ---- host side -------------------------------------------------------------------------------
 // Depth segments: enough workgroups to fill 256 CUs several times over while every segment
 // keeps at least 16 hypotheses for the register-resident taps to pay off.
-inline int choose_segments(int64_t tiles, int64_t D, int lpp, int64_t target_units) {
+inline int choose_segments(int64_t tiles, int64_t D, int lpp, int64_t target_units, bool row_sums) {
   int nseg = 1;
-  const int64_t min_len = lpp > 16 ? lpp : 16;
+  // (sums in channel order: three waves per SIMD and long chunks, so the last round of workgroups is
+  // the one to keep short: five views, 108 x 126 x 77, 147 -> 129 us; for the others shorter segments
+  // load more taps again: f16 groups, four views, 237 x 315 x 24, 147 -> 171 us)
+  const int64_t least = row_sums ? 8 : 16, min_len = lpp > least ? lpp : least;
   while (nseg < 8 && tiles * nseg < target_units && D / (nseg * 2) >= min_len) nseg *= 2;
   // a problem that does not even give every SIMD one wave: shorter segments still
   const int64_t short_len = lpp > 4 ? lpp : 4;
@@ -2760,7 +2777,7 @@ inline int choose_segments(int64_t tiles, int64_t D, int lpp, int64_t target_uni
 
 template <int LPP>
 inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int sub, int ngroups = 1,
-                              int vper = 0, bool tall = false) {
+                              int vper = 0, bool tall = false, bool row_sums = false) {
   constexpr int PPW = 64 / LPP;
   Geometry g;
   g.hw = (int)(H * W);
@@ -2776,7 +2793,7 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
   g.ngroups = ngroups;
   g.vper = vper;
   // twenty waves per SIMD over the launch: the tail of a launch with fewer is measurable
-  g.nseg = choose_segments(tiles * ngroups, D, LPP, 256 * 4 * 20);
+  g.nseg = choose_segments(tiles * ngroups, D, LPP, 256 * 4 * 20, row_sums);
   // A forward launch below two waves per SIMD lasts as long as its longest wave, and a segment costs
   // it nothing but the set-up: segments down to one chunk (32 channels in 8 groups, five views, 32 x 32 x 5:
   // 12.6 -> 9.9 us; samples of 8 channels, four views, 22 x 26 x 17: 10.7 -> 7.5 us; double, 8
