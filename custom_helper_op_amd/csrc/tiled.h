@@ -1835,6 +1835,16 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const R *data, 
   }
 }
 
+// The source gradient of one channel of a lane, summed over an open run: taps 00, 01, 11, 10.
+// Four adjacent registers: an accumulator of the matrix cores (see the depth loop).
+// (matrix accumulators; elsewhere four values of their own)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename R>
+struct LooseSums {
+  R v[4];
+  __device__ __forceinline__ R &operator[](int k) { return v[k]; }
+};
+
 // Adds the four tap images of a finished run into the window (a cell that sticks out of the
 // window never gets here: flush_cells_to_memory takes it).  Called from divergent code by all
 // LPP lanes of every pixel whose run just ended.  Float LDS atomics cost about three cycles
@@ -1849,9 +1859,9 @@ __device__ __forceinline__ void window_flush_all(int oy, int ox, const R *data, 
 // from 429 to 400 us; against LDS atomics it halved the time of the 8-channel workloads.
 // 16 lanes per pixel (four pixels per wave): the pixels that fire in the same instruction
 // take turns, one pixel per round with its four taps in flight together.
-template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP = 2, typename R>
-__device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VEC],
-                                           R *data, int *tags, int lane, int cl) {
+template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP = 2, typename R, typename T>
+__device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC], R *data,
+                                           int *tags, int lane, int cl) {
   using WN = Window<VEC, LPP, FORM>;
   if (key < 0) {
     // the whole cell lies inside the window (the usual case)
@@ -1879,7 +1889,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] += v[k][i];
+            for (int i = 0; i < VEC; ++i) old[k][i] += v[i][k];
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
@@ -1898,7 +1908,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
             R old[VEC];
             slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] += v[k][i];
+            for (int i = 0; i < VEC; ++i) old[i] += v[i][k];
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
           }
         } else {
@@ -1908,7 +1918,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] += v[k][i];
+            for (int i = 0; i < VEC; ++i) old[k][i] += v[i][k];
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
@@ -1924,7 +1934,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
             R old[VEC];
             slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] += v[k][i];
+            for (int i = 0; i < VEC; ++i) old[i] += v[i][k];
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
             // (the next tap may be the texel another pixel has just updated: the LDS keeps a
             // wave's operations in order, the compiler is held to it here)
@@ -1939,9 +1949,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
   }
   // (a cell that sticks out of the window never gets here: flush_cells_to_memory took it)
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) v[k][i] = R(0);
+  for (int i = 0; i < VEC; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
 }
 
 // Cells that no window position covers (the tile's pixels of one depth further apart than the
@@ -1951,9 +1959,9 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, R (&v)[4][VE
 // and the whole wave adds each row as a dense run of 2*C consecutive floats.  Added lane by
 // lane from the registers, each 16-byte chunk of a texel would carry one float per
 // instruction, and the atomics cost per chunk, not per float.
-template <int VEC, int LPP, int GAP, typename R>
+template <int VEC, int LPP, int GAP, typename R, typename T>
 __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool mine, int key,
-                                                      R (&v)[4][VEC], R *stage, R *gview, int srcW, int lane, int cl,
+                                                      T (&v)[VEC], R *stage, R *gview, int srcW, int lane, int cl,
                                                       int cm) {
   constexpr int C = VEC * LPP;
   while (m) {
@@ -1964,7 +1972,10 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
       // taps 00, 01 (row fh), then 10, 11 (row fh + 1); v is ordered 00, 01, 11, 10
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        slot_write<GAP>(stage + (k == 2 ? 3 : k == 3 ? 2 : k) * C + lane_first(cl, GAP), v[k]);
+      {
+        const R w[VEC] = {v[0][k], v[1][k], v[2][k], v[3][k]};
+        slot_write<GAP>(stage + (k == 2 ? 3 : k == 3 ? 2 : k) * C + lane_first(cl, GAP), w);
+      }
     }
     wave_sync();
     const int fh = k2 >> 16, fw = k2 & 0xffff;
@@ -1984,9 +1995,7 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
   }
   if (mine) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) v[k][i] = R(0);
+    for (int i = 0; i < VEC; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
   }
 }
 
@@ -2026,7 +2035,7 @@ constexpr bool slim_double(int lpp, int corr) { return corr == 2 && lpp > 1 && l
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false,
                              bool wide_real = false) {
   return wide_real ? true : nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
-                     (lpp == 4 && corr <= 1 && reduce == 0) ||
+                     (lpp == 4 && ((corr <= 1 && reduce == 0) || corr == 2 || corr == 4)) ||
                      (lpp == 2 && corr <= 1 && reduce == 0));
 }
 constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false,
@@ -2102,6 +2111,18 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   int *s_move_list = LPP == 1                                         ? s_list
                      : backward_list_bytes<R, VEC, LPP, kForm>() > 0 ? s_own_list
                                                                  : reinterpret_cast<int *>(s_stage);
+  // The source gradient of a channel is an outer product, four weights times one gradient per depth: for
+  // the warp alone, with four lanes and more per pixel, the matrix cores add it, a block of four
+  // lanes (channels) at a time and the lanes' channels one after the other: four instructions instead of
+  // sixteen multiply-adds, in the same single rounding.  They write every lane, whatever the execution
+  // mask: a lane without a sample takes part with a gradient of zero.  (Samples of 16 channels, three views, 97 x 129 x 40, two images: 103 -> 98 us at
+  // four waves per SIMD, 94-96 with the matrix cores; 32 channels, five views, 247 x 274 x 72: 1945 ->
+  // 1850 us; its error against 64-bit sums is that of the multiply-adds.)  The other gradients
+  // have no registers left for it: 32 channels, two views, spill 32-52 bytes at four waves and lose
+  // more (252 -> 263-338 us), 16 channels and CostAggregate gain nothing.
+  constexpr bool kMatrix = CORR == 4 && !kDouble && LPP >= 4;
+  using Sums = typename std::conditional<kMatrix, f32x4, LooseSums<R>>::type;
+  const unsigned own_tap = pw + (unsigned)(t.lane & 3) * (unsigned)kB;
   // CORR 3 only: reference rows, sample rows
   R *s_v3 = reinterpret_cast<R *>(s_own_list + backward_list_bytes<R, VEC, LPP, kForm>() / 4);
   static_assert(!best_pair_op(CORR) || (NV == 1 && LPP > 1 && VEC == 4), "CostVolumeV3: one view, wide pixels");
@@ -2203,7 +2224,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     gview[n] = src_grad_img + vo;
     oy[n] = ox[n] = WN::kNone;
   }
-  R tap[NV][4][VEC], sg[NV][4][VEC];
+  R tap[NV][4][VEC];
+  Sums sg[NV][VEC];
   int cur[NV];     // tap offset of the open run, -1: none
   int2 cell[NV];   // its slots and key (bit 31: inside the window)
   unsigned ring_rows[NV];  // ring rows of the window this lane's accepted cells mapped to
@@ -2213,9 +2235,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     ring_rows[n] = 0u;
     cell[n] = make_int2(0, 0);
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int c = 0; c < VEC; ++c) sg[n][k][c] = R(0);
+    for (int c = 0; c < VEC; ++c) sg[n][c] = Sums{R(0), R(0), R(0), R(0)};
   }
   const S *cg_lane =
       CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + ch0
@@ -2495,7 +2515,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     if constexpr (LPP > 1) wave_sync();
     int rb_off[2][NV];
     R4 rb_wt[2][NV], rb_dwt[2][NV];
-    R rb_scl[2];
+    R rb_scl[2], own_w = R(0);
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
       if constexpr (LPP > 1) {
@@ -2511,6 +2531,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
         rb_dwt[0][n] = r_dwt[n];
       }
     }
+    if constexpr (kMatrix) own_w = lds_at<R>(smem, own_tap, kWts);
     if constexpr (LPP > 1)
       rb_scl[0] = lds_at<R>(smem, p1, kScl);
     else
@@ -2545,6 +2566,11 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       const int *rec_off = rb_off[cb];
       const R4 *rec_wt = rb_wt[cb], *rec_dwt = rb_dwt[cb];
       const R scl = rb_scl[cb];
+      if constexpr (kMatrix)
+        if (jj > 0) own_w = lds_at<R>(smem, own_tap, kWts + (jj * PPW) * kB4);
+      R gmat[VEC];  // d(loss)/d(sample) of this lane's channels for the matrix cores
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) gmat[c] = R(0);
       R dvox = R(0);  // this lane's share of d(loss)/d(depth of this voxel)
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
@@ -2569,6 +2595,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
           if constexpr (kVoxelGrad) {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) cg[c] = scl;
+          } else if (CORR == 4) {
+            // (each view of FeatureAggregate has rows of its own: no factor)
+#pragma unroll
+            for (int c = 0; c < VEC; ++c) cg[c] = raw[c];
           } else if (CORR == 0 || g.sub == 1) {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) cg[c] = raw[c] * scl;
@@ -2663,10 +2693,14 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                 gsrc = cg[c] * ref[c];
               }
               if constexpr (PAD) gsrc = ch_ok ? gsrc : R(0);
-              sg[n][0][c] = mad(gsrc, wt.x, sg[n][0][c]);
-              sg[n][1][c] = mad(gsrc, wt.y, sg[n][1][c]);
-              sg[n][2][c] = mad(gsrc, wt.z, sg[n][2][c]);
-              sg[n][3][c] = mad(gsrc, wt.w, sg[n][3][c]);
+              if constexpr (kMatrix) {
+                gmat[c] = gsrc;
+              } else {
+                sg[n][c][0] = mad(gsrc, wt.x, sg[n][c][0]);
+                sg[n][c][1] = mad(gsrc, wt.y, sg[n][c][1]);
+                sg[n][c][2] = mad(gsrc, wt.z, sg[n][c][2]);
+                sg[n][c][3] = mad(gsrc, wt.w, sg[n][c][3]);
+              }
               if constexpr (DG) {
                 R ds = dwt.x * tap[n][0][c];
                 ds = mad(dwt.y, tap[n][1][c], ds);
@@ -2677,6 +2711,11 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             }
           }
         }
+      }
+      if constexpr (kMatrix) {
+#pragma unroll
+        for (int c = 0; c < VEC; ++c)
+          sg[0][c] = __builtin_amdgcn_mfma_f32_4x4x1f32(own_w, gmat[c], sg[0][c], 0, 0, 0);
       }
       if constexpr (PAD && DG) dvox = ch_ok ? dvox : R(0);
       if constexpr (!DG) {
