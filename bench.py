@@ -361,7 +361,7 @@ def main():
     ap.add_argument("--feature", action="store_true",
                     help="time FeatureAggregate on the workload's tensors")
     ap.add_argument("--float64", action="store_true",
-                    help="time a float32 CostVolume workload's tensors as float64 (strip kernels)")
+                    help="time a float32 CostVolume workload's tensors as float64")
     ap.add_argument("--channels", type=int, default=0, metavar="C",
                     help="keep only the first C feature channels of a float32 CostVolume workload")
     ap.add_argument("--kernel-family", choices=["auto", "general", "strip"], default="auto",

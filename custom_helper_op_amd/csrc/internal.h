@@ -105,8 +105,8 @@ hipError_t launch_general_backward(const Args<S> &a, hipStream_t stream);
 
 // Strip kernels: one wavefront per strip of pixels, one lane per channel, depth innermost.
 // CostVolume, CostVolumeV2, CostAggregate and FeatureAggregate with up to 64 channels, any view
-// count, all storage types: what the tiled kernels decline (float64, channel counts other than 4 x 2^k)
-// runs here.
+// count, all storage types: what the tiled kernels decline (channel counts other than 4 x 2^k and 20,
+// 24, 28; unaligned pointers; more than six views forward) runs here.
 template <typename S>
 bool strip_supported(const Args<S> &a);
 // ... and the gradient of CostVolumeV3 (float, double; the forward pass has no strip kernel)
@@ -149,7 +149,7 @@ hipError_t launch_tiled_backward_wide(const Args<S> &a, hipStream_t stream);
 // it per host thread for chop_last_views_per_workgroup).
 void note_views_per_workgroup(int views);
 // The calling thread's choice between the two 32-channel tiled gradient kernels
-// (chop_set_backward_window): 0 the launcher decides, 6 slimmed, 8 wide.
+// (chop_set_backward_window): 0 the launcher decides, 6 or 8 rows.
 int backward_window_mode();
 // ... and which of the two the launcher took (0: a shape that has only one kernel)
 void note_backward_window(int rows);

@@ -1077,6 +1077,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         constexpr int HALF = squares_depths(LPP, NV, sizeof(R) == 8);  // depths staged together
 #pragma unroll
         for (int j0 = 0; j0 < LPP; j0 += HALF) {
+        if (j0 > 0 && d0 + j0 >= d_hi) continue;  // (uniform: nothing in the second half)
 #pragma unroll
         for (int jj = j0; jj < j0 + HALF; ++jj) {
           if (d0 + jj >= d_hi) {
@@ -2014,7 +2015,8 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // rows keep them above 140) and not CostVolumeV3 (its two extra LDS rows per pixel are 2 KB).
 // Four lanes per pixel (16 channels), gradients of a mean: 130 registers left alone, 121 lean
 // (held to 128 without the slimming they spilled three to five); the window of the 4 x 4 pixel
-// tile is 4 KB.  Two lanes per pixel (8 channels): 119-125 lean, and 122-128 where the views of
+// tile is 4 KB.  CostAggregate and FeatureAggregate the same (134 -> 117-120; six views, 497 x 700 x 41:
+// 3.55 -> 3.11 ms).  Two lanes per pixel (8 channels): 119-125 lean, and 122-128 where the views of
 // a tile take turns in the workgroup (VLOOP) -- once the compiler is kept from carrying two
 // dozen lane-only values through the view loop (see the barrier at the head of that loop;
 // with them the kernels spilled 44-68 bytes around the depth loop and four waves were slower
