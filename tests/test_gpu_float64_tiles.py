@@ -69,3 +69,20 @@ def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
     for got in _both(lambda: bwd(*ins, dev(cg), dev(want[1]), *extra)):
         for g, w in zip(got, grads):
             assert_backward_close(g, w, 1e-10)
+
+
+@pytest.mark.parametrize("reduce", ["MEAN", "MIN"])
+@pytest.mark.parametrize("C,H,W,D", [(64, 7, 9, 11), (64, 7, 9, 12), (32, 128, 128, 5), (32, 127, 129, 5),
+                                     (32, 128, 128, 6), (16, 181, 182, 2), (16, 181, 182, 3)])
+def test_gradients_of_few_depths(C, H, W, D, reduce):
+    """Both sides of the line below which the gradients of group correlation keep a lane per channel:
+    3/4 depth per lane of a pixel, and up to 32 channels only where the launch fills the chip.  The
+    oracle would take minutes at these sizes; the two families agree as above."""
+    t = reference_test_case(3, 1, 2, H, W, C, D, np.float64, seed=C + D)
+    grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
+    ins = [dev(x) for x in (t["ref"], t["src"], grid, t["Rs"], t["Ts"])]
+    cost, mask = chop.cost_volume_v2_raw(*ins, reduce, 4)
+    cg = dev(np.random.default_rng(7).standard_normal(tuple(cost.shape)))
+    here, lanes = _both(lambda: chop.cost_volume_grad_v2(*ins, cg, mask, reduce, 4))
+    for g, w in zip(here, lanes):
+        assert_backward_close(g, w, 1e-10)
