@@ -73,7 +73,8 @@ def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
 
 @pytest.mark.parametrize("reduce", ["MEAN", "MIN"])
 @pytest.mark.parametrize("C,H,W,D", [(64, 7, 9, 11), (64, 7, 9, 12), (32, 128, 128, 5), (32, 127, 129, 5),
-                                     (32, 128, 128, 6), (16, 181, 182, 2), (16, 181, 182, 3)])
+                                     (32, 128, 128, 6), (16, 181, 182, 2), (16, 181, 182, 3),
+                                     (64, 181, 182, 12)])
 def test_gradients_of_few_depths(C, H, W, D, reduce):
     """Both sides of the line below which the gradients of group correlation keep a lane per channel:
     3/4 depth per lane of a pixel, and up to 32 channels only where the launch fills the chip.  The
@@ -84,5 +85,30 @@ def test_gradients_of_few_depths(C, H, W, D, reduce):
     cost, mask = chop.cost_volume_v2_raw(*ins, reduce, 4)
     cg = dev(np.random.default_rng(7).standard_normal(tuple(cost.shape)))
     here, lanes = _both(lambda: chop.cost_volume_grad_v2(*ins, cg, mask, reduce, 4))
+    for g, w in zip(here, lanes):
+        assert_backward_close(g, w, 1e-10)
+
+
+@pytest.mark.parametrize("op", ["v1", "v2"])
+@pytest.mark.parametrize("C,N,H,W,D", [(8, 1, 9, 7, 11), (8, 1, 9, 7, 12), (32, 2, 9, 7, 11), (32, 1, 9, 7, 11),
+                                       (32, 4, 9, 7, 12), (32, 5, 9, 7, 12), (64, 2, 9, 7, 12),
+                                       (64, 3, 9, 7, 12), (64, 3, 91, 91, 12), (64, 5, 91, 91, 12)])
+def test_lines_of_small_launches(op, C, N, H, W, D):
+    """Both sides of the lines at which launches of few depths, few tiles or many views keep a lane per
+    channel: forward equal to the bit, gradients as above."""
+    t = reference_test_case(3, 1, N, H, W, C, D, np.float64, seed=C + N)
+    if op == "v1":
+        ins = [dev(t[k]) for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts")]
+        fwd, bwd, extra = chop.cost_volume_raw, chop.cost_volume_grad, ("MEAN",)
+    else:
+        grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
+        ins = [dev(x) for x in (t["ref"], t["src"], grid, t["Rs"], t["Ts"])]
+        fwd, bwd, extra = chop.cost_volume_v2_raw, chop.cost_volume_grad_v2, ("MEAN", 4)
+    here, lanes = _both(lambda: fwd(*ins, *extra))
+    for g, w in zip(here, lanes):
+        assert np.array_equal(g, w)
+    cg = dev(np.random.default_rng(9).standard_normal(here[0].shape))
+    mask = dev(here[1])
+    here, lanes = _both(lambda: bwd(*ins, cg, mask, *extra))
     for g, w in zip(here, lanes):
         assert_backward_close(g, w, 1e-10)
