@@ -92,7 +92,8 @@ def test_gradients_of_few_depths(C, H, W, D, reduce):
 @pytest.mark.parametrize("op", ["v1", "v2"])
 @pytest.mark.parametrize("C,N,H,W,D", [(8, 1, 9, 7, 11), (8, 1, 9, 7, 12), (32, 2, 9, 7, 11), (32, 1, 9, 7, 11),
                                        (32, 4, 9, 7, 12), (32, 5, 9, 7, 12), (64, 2, 9, 7, 12),
-                                       (64, 3, 9, 7, 12), (64, 3, 91, 91, 12), (64, 5, 91, 91, 12)])
+                                       (64, 3, 9, 7, 12), (64, 3, 91, 91, 12), (64, 5, 91, 91, 12),
+                                       (64, 6, 91, 91, 12)])
 def test_lines_of_small_launches(op, C, N, H, W, D):
     """Both sides of the lines at which launches of few depths, few tiles or many views keep a lane per
     channel: forward equal to the bit, gradients as above."""
