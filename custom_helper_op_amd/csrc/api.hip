@@ -9,6 +9,7 @@
 #include <string>
 
 #include "../../include/chop_costvol.h"
+#include "choice.h"
 #include "internal.h"
 
 namespace chop {
@@ -17,6 +18,7 @@ namespace {
 thread_local std::string g_last_error = "";
 thread_local int g_kernel_family = 0;
 thread_local int g_last_family = 0;
+thread_local int g_last_shape = 0;  // the kernels that ran: 1 general, 2 tile-shaped, 3 a lane per channel
 thread_local int g_last_views_per_workgroup = 0;
 thread_local int g_last_backward_window = 0;
 thread_local int g_backward_window = 0;  // 0: the launcher decides, 6, 8 (chop_set_backward_window)
@@ -65,14 +67,28 @@ int check_dims(const Dims &d, int reduce, int groups, bool correlation) {
       return fail(CHOP_ERR_NULL_POINTER, std::string("null pointer: ") + #p);          \
   } while (0)
 
+void note_general() { g_last_family = g_last_shape = 1; }
+void note_strip() { g_last_family = g_last_shape = 3; }
 // What chop_last_kernel_family() reports for the tile-shaped kernels: 2, in float64 3 -- its
 // tile-shaped and its lane-per-channel kernels give the same bits forward (the plain evaluation's) and
 // stand behind one code.
 // Likewise forward for channel counts that leave lanes idle (20, 24, 28).
+// chop_last_kernel_shape() tells them apart.
 template <typename S>
-int tiled_family(const Args<S> &a, bool forward) {
-  return sizeof(S) == 8 || (forward && (a.C & (a.C - 1)) != 0) ? 3 : 2;
+void note_tiled(const Args<S> &a, bool forward) {
+  g_last_family = sizeof(S) == 8 || (forward && (a.C & (a.C - 1)) != 0) ? 3 : 2;
+  g_last_shape = 2;
 }
+// Whether the tile-shaped kernels take a call: any they can serve if they are asked for (family 3), left
+// alone those they are the faster ones for.
+template <typename S>
+bool takes_tiles(const Args<S> &a, bool is_backward) {
+  if (g_kernel_family != 0 && g_kernel_family != 3) return false;
+  if (!(is_backward ? tiled_backward_supported(a) : tiled_forward_supported(a))) return false;
+  return g_kernel_family == 3 || !lanes_are_faster(a, is_backward);
+}
+// A gradient call begins: nothing is known of its kernels (the tiled launcher says more).
+void note_backward_call() { g_last_views_per_workgroup = g_last_backward_window = 0; }
 
 int launch_status(hipError_t err, const char *what) {
   if (err == hipSuccess) return CHOP_OK;
@@ -112,15 +128,15 @@ int forward(void *stream, int reduce, int half_centor, const Dims &d, int groups
   a.depth_grid = depth_grid, a.Rs = Rs, a.Ts = Ts, a.cost = cost, a.mask = mask;
   a.default_cost = default_cost;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (g_kernel_family == 0 && tiled_forward_supported(a)) {
-    g_last_family = tiled_family(a, true);
+  if (takes_tiles(a, false)) {
+    note_tiled(a, true);
     return launch_status(launch_tiled_forward(a, s), "tiled forward launch");
   }
   if (g_kernel_family != 1 && strip_supported(a)) {
-    g_last_family = 3;
+    note_strip();
     return launch_status(launch_strip_forward(a, s), "strip forward launch");
   }
-  g_last_family = 1;
+  note_general();
   return launch_status(launch_general_forward(a, s), "general forward launch");
 }
 
@@ -136,6 +152,7 @@ int backward(void *stream, int reduce, int half_centor, const Dims &d, int group
   if (int rc = check_dims(d, reduce, groups, corr == GROUP_CORRELATION)) return rc;
   const int64_t pixels = d.B * d.H * d.W, voxels = pixels * d.D;
   const int64_t n_ref = pixels * d.C, n_src = d.B * d.N * d.srcH * d.srcW * d.C;
+  note_backward_call();
   const bool per_voxel_depth = needs_depth_grid || depth_grid != nullptr;
   const int64_t n_depth = per_voxel_depth ? voxels : pixels;
   if (n_ref == 0 && n_src == 0 && n_depth == 0) return CHOP_OK;
@@ -182,15 +199,15 @@ int backward(void *stream, int reduce, int half_centor, const Dims &d, int group
     a.ref_grad_acc = a.src_grad_acc + ((n_src + 63) / 64) * 64;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (g_kernel_family == 0 && work && tiled_backward_supported(a)) {
-    g_last_family = tiled_family(a, false);
+  if (work && takes_tiles(a, true)) {
+    note_tiled(a, false);
     return launch_status(launch_tiled_backward(a, s), "tiled backward launch");
   }
   if (g_kernel_family != 1 && work && strip_supported(a)) {
-    g_last_family = 3;
+    note_strip();
     return launch_status(launch_strip_backward(a, s), "strip backward launch");
   }
-  g_last_family = 1;
+  note_general();
   return launch_status(launch_general_backward(a, s), "general backward launch");
 }
 
@@ -208,6 +225,7 @@ int v3_call(void *stream, int reduce, int half_centor, const Dims &d, int groups
   const int64_t n_ref = pixels * d.C, n_src = d.B * d.N * d.srcH * d.srcW * d.C;
   const bool work = voxels > 0 && d.C > 0;
   if (backward) {
+    note_backward_call();
     if (n_ref == 0 && n_src == 0 && pixels == 0) return CHOP_OK;
     REQUIRE_PTR(ref_grad, n_ref);
     REQUIRE_PTR(src_grad, n_src);
@@ -236,18 +254,16 @@ int v3_call(void *stream, int reduce, int half_centor, const Dims &d, int groups
   a.cost = cost, a.mask = mask, a.cost_grad = cost_grad, a.mask_in = mask_in;
   a.ref_grad = ref_grad, a.src_grad = src_grad, a.depth_grad = base_plane_grad;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (g_kernel_family == 0 && work) {
-    if (backward ? tiled_backward_supported(a) : tiled_forward_supported(a)) {
-      g_last_family = tiled_family(a, !backward);
-      return backward ? launch_status(launch_tiled_backward(a, s), "tiled CostVolumeV3 backward launch")
-                      : launch_status(launch_tiled_forward(a, s), "tiled CostVolumeV3 forward launch");
-    }
+  if (work && takes_tiles(a, backward)) {
+    note_tiled(a, !backward);
+    return backward ? launch_status(launch_tiled_backward(a, s), "tiled CostVolumeV3 backward launch")
+                    : launch_status(launch_tiled_forward(a, s), "tiled CostVolumeV3 forward launch");
   }
   if (g_kernel_family != 1 && work && backward && strip_pair_backward_supported(a)) {
-    g_last_family = 3;
+    note_strip();
     return launch_status(launch_strip_backward(a, s), "strip CostVolumeV3 backward launch");
   }
-  g_last_family = 1;
+  note_general();
   if (backward) return launch_status(launch_v3_backward(a, s), "CostVolumeV3 backward launch");
   return launch_status(launch_v3_forward(a, s), "CostVolumeV3 forward launch");
 }
@@ -267,6 +283,7 @@ int feature_call(void *stream, int half_centor, const Dims &d, const S *src, con
   const int64_t n_src = d.B * d.N * d.srcH * d.srcW * d.C;
   const bool work = rows > 0 && d.C > 0;
   if (backward) {
+    note_backward_call();
     if (n_src == 0 && pixels == 0) return CHOP_OK;
     REQUIRE_PTR(src_grad, n_src);
     REQUIRE_PTR(base_plane_grad, pixels);
@@ -293,19 +310,17 @@ int feature_call(void *stream, int half_centor, const Dims &d, const S *src, con
   a.cost = mapped, a.mask = mapped_mask, a.cost_grad = mapped_grad, a.mask_in = mask_in;
   a.src_grad = src_grad, a.depth_grad = base_plane_grad;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (g_kernel_family == 0 && work) {
-    if (backward ? tiled_backward_supported(a) : tiled_forward_supported(a)) {
-      g_last_family = tiled_family(a, !backward);
-      return backward ? launch_status(launch_tiled_backward(a, s), "tiled FeatureAggregate backward launch")
-                      : launch_status(launch_tiled_forward(a, s), "tiled FeatureAggregate forward launch");
-    }
+  if (work && takes_tiles(a, backward)) {
+    note_tiled(a, !backward);
+    return backward ? launch_status(launch_tiled_backward(a, s), "tiled FeatureAggregate backward launch")
+                    : launch_status(launch_tiled_forward(a, s), "tiled FeatureAggregate forward launch");
   }
   if (g_kernel_family != 1 && work && strip_supported(a)) {
-    g_last_family = 3;
+    note_strip();
     return backward ? launch_status(launch_strip_backward(a, s), "strip FeatureAggregate backward launch")
                     : launch_status(launch_strip_forward(a, s), "strip FeatureAggregate forward launch");
   }
-  g_last_family = 1;
+  note_general();
   if (backward) return launch_status(launch_feature_backward(a, s), "FeatureAggregate backward launch");
   return launch_status(launch_feature_forward(a, s), "FeatureAggregate forward launch");
 }
@@ -363,7 +378,7 @@ extern "C" {
 
 int chop_abi_version(void) { return 1; }
 
-int chop_last_views_per_workgroup(void) { return g_last_family == 2 ? g_last_views_per_workgroup : 0; }
+int chop_last_views_per_workgroup(void) { return g_last_views_per_workgroup; }
 
 int chop_init(void) {
   hipError_t err = hipSuccess;
@@ -379,13 +394,17 @@ const char *chop_last_error_string(void) { return g_last_error.c_str(); }
 
 int chop_set_kernel_family(int family) {
   const int prev = g_kernel_family;
-  g_kernel_family = family == 1 || family == 2 ? family : 0;
+  g_kernel_family = family >= 1 && family <= 3 ? family : 0;
   return prev;
 }
 
 int chop_last_kernel_family(void) { return g_last_family; }
 
-int chop_last_backward_window(void) { return g_last_family == 2 ? g_last_backward_window : 0; }
+// For the tests, no part of the ABI: chop_last_kernel_family() with the kernels told apart in every type
+// and direction -- 0 none yet, 1 general, 2 tile-shaped, 3 a lane per channel.
+int chop_last_kernel_shape(void) { return g_last_shape; }
+
+int chop_last_backward_window(void) { return g_last_backward_window; }
 
 int chop_set_backward_window(int rows) {
   const int prev = g_backward_window;

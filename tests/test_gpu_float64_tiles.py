@@ -1,7 +1,8 @@
 """Float64 on the tile-shaped kernels: pixels of 4 to 64 channels, some lanes idle (20, 24, 28), one to
 seven views (seven: the forward pass keeps a lane per channel), depth ranges that end inside a chunk.
 
-An unforced call takes them, the strip family forced takes a lane per channel.  Forward both are the
+Family 3 asks for them wherever they can serve the shape, family 2 for a lane per channel, and the shape
+reported says that they ran (which of the two an unforced call takes: test_kernel_choice.py).  Forward both are the
 plain evaluation: equal to each other and to the oracle to the bit.  Gradients: the sums come in
 another order, each of up to a few hundred terms, so 1e-10 of the gradient's rms (the oracle's own
 bar in float64) holds with three digits to spare.
@@ -25,21 +26,27 @@ def _announce(request):
     _lib.load().chop_set_kernel_family(0)
 
 
-def _both(run):
+def _both(run, tiles=True):
+    """`run` with the tiles asked for and with a lane per channel.  `tiles`: whether the tiles can serve it."""
     out = []
-    for family in (0, 2):
+    for family, shape in ((3, 2 if tiles else 3), (2, 3)):
         _lib.load().chop_set_kernel_family(family)
         out.append([host(x) for x in run()])
         assert _lib.load().chop_last_kernel_family() == 3
+        assert _lib.load().chop_last_kernel_shape() == shape
     return out
 
 
 @pytest.mark.parametrize("C", [4, 8, 16, 20, 24, 28, 32, 64])
 @pytest.mark.parametrize("N,H,W,D", [(1, 13, 17, 5), (2, 7, 9, 35), (4, 12, 10, 16), (7, 6, 11, 9)])
 @pytest.mark.parametrize("op,reduce,groups", [("v1", "MEAN", 1), ("v1", "MIN", 1), ("v2", "MEAN", 4),
-                                              ("v2", "MIN", 2), ("aggregate", "MEAN", 1),
-                                              ("aggregate", "MIN", 1), ("feature", "MEAN", 1)])
+                                              ("v2", "MIN", 2), ("v2", "MEAN", "four"), ("v2", "MIN", "two"),
+                                              ("aggregate", "MEAN", 1), ("aggregate", "MIN", 1),
+                                              ("feature", "MEAN", 1)])
 def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
+    # (groups of a width in words: as many as the channels make of them)
+    groups = {"four": C // 4, "two": C // 2}.get(groups, groups)
+    can = op != "v2" or C // groups in (1, 2, 4) or (C // groups == 8 and C > 4)
     t = reference_test_case(3, 2, N, H, W, C, D, np.float64, seed=C + N)
     t["Ts"] = (t["Ts"] + np.linspace(-0.5, 0.5, N)[None, :, None]).astype(np.float64)
     args = tuple(t[k] for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts"))
@@ -61,12 +68,12 @@ def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
         want_fwd, want_bwd = oracle.cost_volume_v2_fwd, oracle.cost_volume_v2_bwd
     ins = [dev(x) for x in args]
     want = want_fwd(*args, *extra)
-    for got in _both(lambda: fwd(*ins, *extra)):
+    for got in _both(lambda: fwd(*ins, *extra), can and C > 4 and N <= 6):
         for g, w in zip(got, want):
             assert np.array_equal(g, w)
     cg = np.random.default_rng(5).standard_normal(want[0].shape)
     grads = want_bwd(*args, cg, want[1], *extra)
-    for got in _both(lambda: bwd(*ins, dev(cg), dev(want[1]), *extra)):
+    for got in _both(lambda: bwd(*ins, dev(cg), dev(want[1]), *extra), can):
         for g, w in zip(got, grads):
             assert_backward_close(g, w, 1e-10)
 
@@ -76,15 +83,16 @@ def test_tiles_against_lanes(oracle, C, N, H, W, D, op, reduce, groups):
                                      (32, 128, 128, 6), (16, 181, 182, 2), (16, 181, 182, 3),
                                      (64, 181, 182, 12)])
 def test_gradients_of_few_depths(C, H, W, D, reduce):
-    """Both sides of the line below which the gradients of group correlation keep a lane per channel:
-    3/4 depth per lane of a pixel, and up to 32 channels only where the launch fills the chip.  The
-    oracle would take minutes at these sizes; the two families agree as above."""
+    """Sizes on both sides of the line below which the gradients of group correlation keep a lane per
+    channel: 3/4 depth per lane of a pixel, and up to 32 channels only where the launch fills the chip.
+    The oracle would take minutes at these sizes; the two families agree as above."""
     t = reference_test_case(3, 1, 2, H, W, C, D, np.float64, seed=C + D)
     grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
     ins = [dev(x) for x in (t["ref"], t["src"], grid, t["Rs"], t["Ts"])]
-    cost, mask = chop.cost_volume_v2_raw(*ins, reduce, 4)
+    groups = 4 if C < 64 else 8     # (groups of sixteen channels are not on the tiles)
+    cost, mask = chop.cost_volume_v2_raw(*ins, reduce, groups)
     cg = dev(np.random.default_rng(7).standard_normal(tuple(cost.shape)))
-    here, lanes = _both(lambda: chop.cost_volume_grad_v2(*ins, cg, mask, reduce, 4))
+    here, lanes = _both(lambda: chop.cost_volume_grad_v2(*ins, cg, mask, reduce, groups))
     for g, w in zip(here, lanes):
         assert_backward_close(g, w, 1e-10)
 
@@ -95,8 +103,8 @@ def test_gradients_of_few_depths(C, H, W, D, reduce):
                                        (64, 3, 9, 7, 12), (64, 3, 91, 91, 12), (64, 5, 91, 91, 12),
                                        (64, 6, 91, 91, 12)])
 def test_lines_of_small_launches(op, C, N, H, W, D):
-    """Both sides of the lines at which launches of few depths, few tiles or many views keep a lane per
-    channel: forward equal to the bit, gradients as above."""
+    """Sizes around which launches of few depths, few tiles or many views keep a lane per channel: forward
+    equal to the bit, gradients as above."""
     t = reference_test_case(3, 1, N, H, W, C, D, np.float64, seed=C + N)
     if op == "v1":
         ins = [dev(t[k]) for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts")]
@@ -104,7 +112,7 @@ def test_lines_of_small_launches(op, C, N, H, W, D):
     else:
         grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
         ins = [dev(x) for x in (t["ref"], t["src"], grid, t["Rs"], t["Ts"])]
-        fwd, bwd, extra = chop.cost_volume_v2_raw, chop.cost_volume_grad_v2, ("MEAN", 4)
+        fwd, bwd, extra = chop.cost_volume_v2_raw, chop.cost_volume_grad_v2, ("MEAN", 4 if C < 64 else 8)
     here, lanes = _both(lambda: fwd(*ins, *extra))
     for g, w in zip(here, lanes):
         assert np.array_equal(g, w)
@@ -113,3 +121,19 @@ def test_lines_of_small_launches(op, C, N, H, W, D):
     here, lanes = _both(lambda: bwd(*ins, cg, mask, *extra))
     for g, w in zip(here, lanes):
         assert_backward_close(g, w, 1e-10)
+
+
+def test_gradient_reports_its_launch():
+    """After a tile-shaped gradient in double: one view per workgroup, the one window there is; after any
+    other gradient nothing; a forward pass in between changes neither."""
+    lib = _lib.load()
+    t = reference_test_case(3, 1, 2, 9, 7, 32, 9, np.float64, seed=1)
+    ins = [dev(t[k]) for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts")]
+    cost, mask = chop.cost_volume_raw(*ins)
+    for family, views in ((3, 1), (2, 0), (3, 1), (1, 0)):
+        lib.chop_set_kernel_family(family)
+        chop.cost_volume_grad(*ins, cost, mask)
+        lib.chop_set_kernel_family(5 - family if family > 1 else 3)
+        chop.cost_volume_raw(*ins)
+        assert lib.chop_last_views_per_workgroup() == views
+        assert lib.chop_last_backward_window() == 0

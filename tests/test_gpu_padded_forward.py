@@ -41,10 +41,11 @@ def test_idle_lanes(oracle, C, N, H, W, D, reduce):
     for name, call in calls.items():
         for dt in (None, torch.float16, torch.bfloat16) if name[0] == "v" else (None,):
             got = []
-            for family in (0, 2):
+            for family, shape in ((3, 2 if N <= 6 else 3), (2, 3)):
                 _lib.load().chop_set_kernel_family(family)
                 got.append([host(x) for x in call(dt)[:2]])
                 assert _lib.load().chop_last_kernel_family() == 3
+                assert _lib.load().chop_last_kernel_shape() == shape
             for a, b in zip(*got):
                 assert np.array_equal(a, b), (name, dt)
             if dt is None and name in want:

@@ -11,6 +11,16 @@ from custom_helper_op_amd.configs import reference_test_case
 from gpu_util import assert_backward_close, dev, host
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _tiles():
+    """Every call on the tiled kernels, also those for which another is the faster one."""
+    _lib.load().chop_set_kernel_family(3)
+    yield
+    _lib.load().chop_set_kernel_family(0)
+
+
 KEYS = ("ref", "src", "base_plane", "offsets", "Rs", "Ts")
 
 
@@ -48,11 +58,13 @@ def test_narrow_groups(oracle, C, sub, dtype, values):
                 want, want_mask = oracle.cost_volume_v3_fwd(*args, reduce, G)
             cost, mask = chop.cost_volume_v3_raw(*ins, reduce, G)
             assert _lib.load().chop_last_kernel_family() == (2 if dtype == np.float32 else 3)
+            assert _lib.load().chop_last_kernel_shape() == 2
             assert np.array_equal(host(mask), want_mask)
             assert np.array_equal(host(cost), want, equal_nan=True)
             if values == "specials":
                 continue  # (a gradient of infinities is NaN wherever it lands)
             cg = np.random.default_rng(1).standard_normal(want.shape).astype(dtype)
             got = chop.cost_volume_grad_v3(*ins, dev(cg), dev(want_mask), reduce, G)
+            assert _lib.load().chop_last_kernel_shape() == 2
             for g, w in zip(got, oracle.cost_volume_v3_bwd(*args, cg, want_mask, reduce, G)):
                 assert_backward_close(host(g), w, 1e-4 if dtype == np.float32 else 1e-10)

@@ -1,0 +1,80 @@
+"""Which kernels a call is given to.  The choice is made on the host, from sizes, types and pointer
+alignment alone, before anything is launched: without a GPU the launch then fails, and
+`chop_last_kernel_shape` says what it would have run (1 a thread per element, 2 tile-shaped, 3 a lane per
+channel).  Never run where there is a GPU: the pointers are no pointers."""
+import ctypes
+
+import pytest
+import torch
+
+from custom_helper_op_amd import _lib
+
+pytestmark = pytest.mark.skipif(torch.cuda.device_count() > 0, reason="made-up pointers: only without a GPU")
+GENERAL, TILES, LANES = 1, 2, 3
+REDUCE = {"MEAN": 0, "MIN": 1}
+
+
+@pytest.fixture(autouse=True)
+def _unforced():
+    yield
+    _lib.load().chop_set_kernel_family(0)
+
+
+def ran(op, direction, C, N, H, W, D, reduce="MEAN", dtype="f64", groups=0, B=1, family=0, offset=0):
+    """The kernels a call would have run.  `groups`: 0 is groups of four channels."""
+    lib = _lib.load()
+    lib.chop_set_kernel_family(family)
+    p = [ctypes.c_void_p(4096 + offset)] * 12
+    dims = (B, H, W, C, D, N, H, W)
+    g = groups or max(C // 4, 1)
+    name, fwd, bwd = {"v1": ("cost_volume", 8, 11), "v2": ("cost_volume_v2", 7, 10),
+                      "v3": ("cost_volume_v3", 8, 11), "layer": ("cost_aggregate", 8, 11),
+                      "feat": ("feature_aggregate", 7, 9)}[op]
+    head = (None, 1) if op == "feat" else (None, REDUCE[reduce], 1)
+    tail = (g,) if op in ("v2", "v3") else ()
+    if dtype in ("f16", "bf16"):
+        head = (None, {"f16": 1, "bf16": 2}[dtype]) + head[1:]
+        extra = 1 if op == "v1" else 0            # the depth_grid argument
+        status = (getattr(lib, "chop_%s_fwd_16" % name)(*head, *dims, *tail, *p[:fwd + extra])
+                  if direction == "f" else
+                  getattr(lib, "chop_%s_bwd_16" % name)(*head, *dims, *tail, *p[:bwd + extra],
+                                                        ctypes.c_void_p(4096), 1 << 50))
+    else:
+        status = getattr(lib, "chop_%s_%swd_%s" % (name, direction, dtype))(
+            *head, *dims, *tail, *p[:fwd if direction == "f" else bwd])
+    assert status == 5, lib.chop_last_error_string()     # CHOP_ERR_LAUNCH: no device
+    return lib.chop_last_kernel_shape()
+
+
+@pytest.mark.parametrize("op", ["v1", "v2", "v3", "layer", "feat"])
+@pytest.mark.parametrize("direction", ["f", "b"])
+def test_forced_and_unaligned(op, direction):
+    """Every type at a size that the tile-shaped kernels take unasked, the families forced, and pointers off
+    the 16-byte grid, which they decline (CostVolumeV3 has no forward pass with a lane per channel)."""
+    for dtype in ("f32", "f64") + (("f16", "bf16") if op in ("v1", "v2") else ()):
+        call = lambda **kw: ran(op, direction, 16, 3, 128, 160, 64, dtype=dtype, **kw)
+        lanes = GENERAL if op == "v3" and direction == "f" else LANES
+        assert call() == TILES
+        assert call(family=3) == TILES
+        assert call(family=2) == lanes
+        assert call(family=1) == GENERAL
+        assert call(offset={"f32": 4, "f64": 8}.get(dtype, 2)) == lanes
+        assert call(offset={"f32": 4, "f64": 8}.get(dtype, 2), family=3) == lanes
+
+
+def test_families_keep_their_codes():
+    """`chop_last_kernel_family` says 3 for tiles in double and for idle lanes forward; the shape does not."""
+    lib = _lib.load()
+    assert ran("v1", "f", 24, 3, 128, 160, 64, dtype="f32") == TILES and lib.chop_last_kernel_family() == 3
+    assert ran("v1", "b", 24, 3, 128, 160, 64, dtype="f32") == TILES and lib.chop_last_kernel_family() == 2
+    assert ran("v1", "b", 32, 3, 128, 160, 64) == TILES and lib.chop_last_kernel_family() == 3
+    assert ran("v1", "b", 32, 3, 128, 160, 64, family=2) == LANES and lib.chop_last_kernel_family() == 3
+
+
+def test_asked_for():
+    """Family 3: the tiles wherever they can serve the shape, and only there."""
+    for C, N, want in ((4, 2, LANES), (8, 2, TILES), (64, 6, TILES), (64, 7, LANES), (12, 2, LANES), (28, 2, TILES)):
+        assert ran("v1", "f", C, N, 9, 7, 6, family=3) == want
+    assert ran("v1", "b", 4, 1, 9, 7, 6, family=3) == TILES
+    assert ran("v2", "b", 64, 4, 38, 40, 6, "MIN", family=3) == TILES
+    assert ran("v2", "b", 64, 4, 38, 40, 6, "MIN") == LANES
