@@ -1663,7 +1663,7 @@ constexpr int kClaimLanes = 8;
 //   Four wts, dwt [NV*64] | int2 cell {slots, key|inside} [NV*64] | int off [NV*64] |
 //   R scale [64] | R dst [64] (per-voxel depth gradients and CostVolumeV3)
 // The slim form (double, slim_double) keeps one Four {dh, dw, d sh / d depth, d sw / d depth} for both
-// sets of weights, which the lanes expand where a depth starts (ten operations): 64 bytes less
+// sets of weights, which the lanes expand where a depth starts (eleven operations): 64 bytes less
 // per voxel.
 // then the list of texels leaving a window, then the windows.  With one view per workgroup
 // the list shares the record space: a window only moves before the chunk's records are
@@ -2633,8 +2633,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
           const int off = rec_off[n];
           R4 wt = rec_wt[n], dwt = rec_dwt[n];
           if constexpr (kSlim) {
-            const R dh = wt.x, dw = wt.y, ah = wt.z, aw = wt.w, k11 = dh * dw, k01 = dw - k11;
-            wt = R4{(R(1) - dh) - k01, k01, k11, dh - k11};
+            // (each weight the rounded product of its two factors, as reproject() has it: three of them
+            // come cheaper by subtraction, and lose their relative accuracy where they are small)
+            const R dh = wt.x, dw = wt.y, ah = wt.z, aw = wt.w, eh = R(1) - dh, ew = R(1) - dw;
+            wt = R4{eh * ew, eh * dw, dh * dw, dh * ew};
             const R cp = mad(ah, dw, aw * dh), bp = aw - cp;
             dwt = R4{-ah - bp, bp, cp, ah - cp};
           }

@@ -137,3 +137,39 @@ def test_gradient_reports_its_launch():
         chop.cost_volume_raw(*ins)
         assert lib.chop_last_views_per_workgroup() == views
         assert lib.chop_last_backward_window() == 0
+
+
+def _shifted_view(C, H, W, shift, seed):
+    """One view that sees every pixel moved by `shift` texels right and down, at the single depth 1."""
+    rng = np.random.default_rng(seed)
+    ref, src = rng.standard_normal((1, H, W, C)), rng.standard_normal((1, 1, H, W, C))
+    Rs, Ts = np.eye(3)[None, None].copy(), np.array([shift, shift, 0.0])[None, None].copy()
+    return ref, src, np.zeros((1, H, W, 1)), np.ones((1, 1)), Rs, Ts
+
+
+def _gradients(op, args, cg, reduce):
+    name = {"v1": "cost_volume", "aggregate": "cost_aggregate"}[op]
+    ins = [dev(x) for x in args]
+    _, mask = getattr(chop, name + "_raw")(*ins, reduce)
+    _lib.load().chop_set_kernel_family(3)
+    got = getattr(chop, name + "_grad")(*ins, dev(cg), mask, reduce)
+    assert _lib.load().chop_last_kernel_shape() == 2
+    return [host(g) for g in got], host(mask), name
+
+
+@pytest.mark.parametrize("reduce", ["MEAN", "MIN"])
+@pytest.mark.parametrize("op", ["v1", "aggregate"])
+@pytest.mark.parametrize("C", [8, 16, 24, 32, 64])
+def test_small_weights_keep_their_accuracy(oracle, op, C, reduce):
+    """Both fractions 2^-20 short of one: the first texel receives the weight 2^-40 and nothing else.  A
+    weight that is the product of its factors is right to an ulp of itself, one left over by subtraction
+    to an ulp of one, 2^-12 of itself.  The bar: eight roundings of a gradient's chain, where the
+    difference of sample and reference may cancel to a hundredth: 8 x 100 x 2^-53 < 1e-12."""
+    args = _shifted_view(C, 6, 7, 1.0 - 2.0 ** -20, C)
+    cg = np.random.default_rng(1).standard_normal((1, 6, 7, 1) + ((C,) if op == "v1" else ()))
+    got, mask, name = _gradients(op, args, cg, reduce)
+    want = getattr(oracle, name + "_bwd")(*args, cg, mask, reduce)
+    corner, at = got[1][0, 0, 0, 0], want[1][0, 0, 0, 0]
+    near = np.abs(at) > 0.01 * np.abs(at).max()
+    assert near.sum() > C // 2
+    np.testing.assert_allclose(corner[near], at[near], rtol=1e-12)
