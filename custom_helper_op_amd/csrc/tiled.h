@@ -2682,10 +2682,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               } else if constexpr (CORR == 4) {
                 gsrc = cg[c];
               } else if (CORR != 1) {
-                R diff = mad(wt.x, tap[n][0][c], -ref[c]);
+                // (double: the sample first, then the difference: sums of the sample's parts are the
+                // smaller numbers to round, and the lane-per-channel kernels have it so)
+                R diff = kDouble ? wt.x * tap[n][0][c] : mad(wt.x, tap[n][0][c], -ref[c]);
                 diff = mad(wt.y, tap[n][1][c], diff);
                 diff = mad(wt.z, tap[n][2][c], diff);
                 diff = mad(wt.w, tap[n][3][c], diff);
+                if constexpr (kDouble) diff -= ref[c];
                 gsrc = diff * cg[c];
                 racc[c] -= gsrc;
               } else {

@@ -173,3 +173,23 @@ def test_small_weights_keep_their_accuracy(oracle, op, C, reduce):
     near = np.abs(at) > 0.01 * np.abs(at).max()
     assert near.sum() > C // 2
     np.testing.assert_allclose(corner[near], at[near], rtol=1e-12)
+
+
+@pytest.mark.parametrize("reduce", ["MEAN", "MIN"])
+@pytest.mark.parametrize("op", ["v1", "aggregate"])
+@pytest.mark.parametrize("C", [4, 8, 16, 24, 32, 64])
+def test_difference_of_a_finished_sample(oracle, op, C, reduce):
+    """Samples that are small against the reference: four parts of 0.225 x 2^-52 each, whose sum changes the
+    reference of one by an ulp and none of which does alone.  Every operation up to the difference is then exact
+    or rounds as the plain evaluation's, so the reference's gradient is the oracle's to the bit."""
+    args = list(_shifted_view(C, 6, 7, 0.5, C))
+    args[0], args[1] = np.ones_like(args[0]), np.full_like(args[1], 0.9 * 2.0 ** -52)
+    cg = np.ones((1, 6, 7, 1) + ((C,) if op == "v1" else ()))
+    got, mask, name = _gradients(op, args, cg, reduce)
+    want = getattr(oracle, name + "_bwd")(*args, cg, mask, reduce)
+    plain = 2.0 / (C if op == "aggregate" else 1)
+    assert np.any((want[0] != 0) & (want[0] != plain))     # (the ulp is there to be lost)
+    if C in (4, 8, 16, 32, 64) or op == "v1":              # (1 / C is exact)
+        assert np.array_equal(got[0], want[0])
+    else:
+        np.testing.assert_allclose(got[0], want[0], rtol=3e-16)
