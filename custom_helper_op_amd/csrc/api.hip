@@ -19,6 +19,7 @@ thread_local std::string g_last_error = "";
 thread_local int g_kernel_family = 0;
 thread_local int g_last_family = 0;
 thread_local int g_last_shape = 0;  // the kernels that ran: 1 general, 2 tile-shaped, 3 a lane per channel
+thread_local int g_last_segments = 0;
 thread_local int g_last_views_per_workgroup = 0;
 thread_local int g_last_backward_window = 0;
 thread_local int g_backward_window = 0;  // 0: the launcher decides, 6, 8 (chop_set_backward_window)
@@ -367,6 +368,7 @@ void *scratch_if_known() {
 }  // namespace
 
 void note_views_per_workgroup(int views) { g_last_views_per_workgroup = views; }
+void note_segments(int segments, bool by_segment) { g_last_segments = by_segment ? -segments : segments; }
 int backward_window_mode() { return g_backward_window; }
 void note_backward_window(int rows) { g_last_backward_window = rows; }
 
@@ -403,6 +405,10 @@ int chop_last_kernel_family(void) { return g_last_family; }
 // For the tests, no part of the ABI: chop_last_kernel_family() with the kernels told apart in every type
 // and direction -- 0 none yet, 1 general, 2 tile-shaped, 3 a lane per channel.
 int chop_last_kernel_shape(void) { return g_last_shape; }
+
+// Likewise: the depth segments of the last call that the tile-shaped or the lane-per-channel kernels
+// served, negative where all tiles' first segments went before all second ones.
+int chop_last_segments(void) { return g_last_segments; }
 
 int chop_last_backward_window(void) { return g_last_backward_window; }
 

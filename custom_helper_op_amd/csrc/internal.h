@@ -148,6 +148,9 @@ hipError_t launch_tiled_backward_wide(const Args<S> &a, hipStream_t stream);
 // The tiled backward launcher reports how many views a workgroup took in turn (api.hip keeps
 // it per host thread for chop_last_views_per_workgroup).
 void note_views_per_workgroup(int views);
+// ... and every tiled or strip launcher into how many depth segments it cut a call, and whether these
+// run one after the other (for the tests, chop_last_segments).
+void note_segments(int segments, bool by_segment);
 // The calling thread's choice between the two 32-channel tiled gradient kernels
 // (chop_set_backward_window): 0 the launcher decides, 6 or 8 rows.
 int backward_window_mode();

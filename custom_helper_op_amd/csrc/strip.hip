@@ -821,6 +821,7 @@ template <typename S>
 hipError_t launch_strip_forward(const Args<S> &a, hipStream_t stream) {
   using R = typename Storage<S>::Real;
   const StripGeom g = strip_geometry(a, false);
+  note_segments(g.nseg, false);
   // CostAggregate adds one row of 64 values per depth of a chunk
   const size_t smem = strip_lds_bytes<R>(4, (64 >> g.lpp_shift) * g.vg * kDB) +
                       (a.corr == SUM_SQUARED_DIFFERENCE ? (size_t)kDB * 64 * sizeof(R) : 0);
@@ -850,6 +851,7 @@ template <typename S>
 hipError_t launch_strip_backward(const Args<S> &a, hipStream_t stream) {
   using R = typename Storage<S>::Real;
   const StripGeom g = strip_geometry(a, true);
+  note_segments(g.nseg, false);
   const int64_t n_ref = a.pixels() * a.C;
   const int64_t n_src = a.B * a.N * a.srcH * a.srcW * a.C;
   hipError_t err;

@@ -47,6 +47,10 @@ constexpr int tile_rows(int ppw, bool tall = false) {
   return ppw >= 64 ? 8 : ppw >= 16 || tall ? 4 : ppw >= 2 ? 2 : 1;
 }
 
+// A forward launch gives each XCD one band of tiles: the segments of a tile one after the other
+// (kBands), or all first segments of the band, then all second ones (kBandsBySegment).
+constexpr int kBands = -1, kBandsBySegment = -2;
+
 struct Geometry {
   int hw;                  // H*W
   int tiles_per_image;     // ceil(hw / PPW)
@@ -56,8 +60,8 @@ struct Geometry {
   int seg;                 // depths per segment, multiple of LPP
   int64_t total_units;     // B * tiles_per_image * nseg * ngroups
   unsigned units_per_seg;  // B * tiles_per_image * ngroups
-  int64_t units_per_xcd;   // ceil(total_units / 8)
-  int xcd_shift;           // log2 of the units dealt to one XCD at a time; -1: one band per XCD
+  int64_t units_per_xcd;   // kBands: ceil(total_units / 8); kBandsBySegment: ceil(units_per_seg / 8)
+  int xcd_shift;           // log2 of the units dealt to one XCD at a time, or kBands, kBandsBySegment
   int64_t grid;            // workgroups to launch
   int tiles_x;             // tiles per image row (a tile: tile_rows(PPW) rows of pixels)
   int sub;                 // channels per correlation group (1 for squared difference)
@@ -408,7 +412,9 @@ __device__ __forceinline__ bool locate_tile(const Args<S> &a, const Geometry &g,
                             ? x * (unsigned)g.units_per_xcd + r
                             : ((r >> g.xcd_shift) << (g.xcd_shift + 3)) + (x << g.xcd_shift) +
                                   (r & ((1u << g.xcd_shift) - 1u));
-  if (unit >= (unsigned)g.total_units) return false;
+  // (pixels of one and two lanes never come segment by segment, see make_geometry)
+  const bool by_segment = LPP >= 4 && g.xcd_shift == kBandsBySegment;
+  if (!by_segment && unit >= (unsigned)g.total_units) return false;
   // the groups of one (tile, segment) are neighbours in launch order: they stream the same
   // upstream-gradient rows at about the same time, through the same L2
   unsigned tile;
@@ -425,11 +431,14 @@ __device__ __forceinline__ bool locate_tile(const Args<S> &a, const Geometry &g,
     tile = rem / (unsigned)g.ngroups;
     t.view0 = (int)(rem - tile * (unsigned)g.ngroups) * g.vper;
   } else {
-    const unsigned per_tile = (unsigned)(g.nseg * g.ngroups);
-    tile = unit / per_tile;
-    const int rem = (int)(unit - tile * per_tile);
-    segi = rem / g.ngroups;
-    t.view0 = (rem - segi * g.ngroups) * g.vper;
+    // (one view group.  One division for both orders: a unit into tile and segment, or a place in an
+    // XCD's launches into segment and tile of its band)
+    const unsigned num = by_segment ? r : unit, den = by_segment ? (unsigned)g.units_per_xcd : (unsigned)g.nseg;
+    const unsigned quot = num / den, rem = num - quot * den;
+    tile = by_segment ? x * den + rem : quot;
+    segi = (int)(by_segment ? quot : rem);
+    t.view0 = 0;
+    if (by_segment && tile >= g.units_per_seg) return false;
   }
   t.d_lo = segi * g.seg;
   t.d_hi = min((int)a.D, t.d_lo + g.seg);
@@ -2873,11 +2882,25 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
   g.units_per_seg = (unsigned)(tiles * g.ngroups);
   // backward: runs of 32 units (the view groups of a tile are neighbours and mostly share
   // a run, hence an L2)
-  g.xcd_shift = vper > 0 ? 5 : -1;
-  g.units_per_xcd = (g.total_units + 7) / 8;
-  const int64_t round_to = g.xcd_shift >= 0 ? (int64_t)8 << g.xcd_shift : 8;
-  g.grid = g.xcd_shift >= 0 ? (g.total_units + round_to - 1) / round_to * round_to
-                            : g.units_per_xcd * 8;
+  // Forward: one band of tiles per XCD.  Its workgroups go to the CUs in turn, so two segments of a
+  // tile that follow each other in the launch put all first segments on every other CU, all second
+  // ones on the rest; where the last segment is a short one half of the chip then waits for the other
+  // half (minimum of CostAggregate, 32 channels, four views, 135 x 181: 17, 20, 24 and 31 depths in
+  // segments of 16 all took 59 us).  A launch whose last segment is shorter than three quarters of the
+  // others goes segment by segment and ends on the short ones (17 and 20 depths 59 -> 39 us, 24 60 -> 40
+  // us; group correlation, six views, 114 x 117 x 21, 38 -> 34 us).  Segments about as long as each other
+  // stay beside each other: they share the lines of the output in which one ends and the next begins.
+  // So do those of narrow pixels (up to eight channels) at any length: their waves write pieces of a few
+  // bytes (CostAggregate of 8 channels, 326 x 430 x 82, 83 -> 140 us segment by segment), and the second
+  // order costs their kernels two registers (six views of that op lost a wave per SIMD: 27 -> 42 us).
+  const int64_t last = D - (int64_t)(g.nseg - 1) * g.seg;
+  const bool by_segment = vper == 0 && g.nseg > 1 && LPP >= 4 && 4 * last <= 3 * (int64_t)g.seg;
+  g.xcd_shift = vper > 0 ? 5 : by_segment ? kBandsBySegment : kBands;
+  g.units_per_xcd = ((by_segment ? tiles : g.total_units) + 7) / 8;
+  const int64_t round_to = vper > 0 ? (int64_t)8 << g.xcd_shift : 8;
+  g.grid = vper > 0     ? (g.total_units + round_to - 1) / round_to * round_to
+           : by_segment ? g.units_per_xcd * 8 * g.nseg
+                        : g.units_per_xcd * 8;
   g.sub = sub;
   g.src_h_max = g.src_w_max = 0.f;  // set by the launcher from the source image size
   return g;

@@ -78,3 +78,25 @@ def test_asked_for():
     assert ran("v1", "b", 4, 1, 9, 7, 6, family=3) == TILES
     assert ran("v2", "b", 64, 4, 38, 40, 6, "MIN", family=3) == TILES
     assert ran("v2", "b", 64, 4, 38, 40, 6, "MIN") == LANES
+
+
+def segments(*args, **kw):
+    """Depth segments of the call; negative: all tiles' first segments before all second ones."""
+    ran(*args, **kw)
+    return _lib.load().chop_last_segments()
+
+
+def test_uneven_segments_go_one_after_the_other():
+    """Side by side a short last segment leaves every other compute unit idle; segments about as long as each
+    other stay side by side, and so do narrow pixels with one value per voxel."""
+    layer = dict(reduce="MIN", dtype="f32")
+    assert segments("layer", "f", 32, 4, 135, 181, 17, **layer) == -2       # 16 + 1
+    assert segments("layer", "f", 32, 4, 135, 181, 24, **layer) == -2       # 16 + 8
+    assert segments("layer", "f", 32, 4, 135, 181, 31, **layer) == 2        # 16 + 15
+    assert segments("layer", "f", 32, 4, 135, 181, 32, **layer) == 4        # 4 x 8
+    assert segments("v1", "f", 32, 6, 114, 117, 21, dtype="f32") == -2      # 16 + 5
+    assert segments("layer", "f", 8, 1, 326, 430, 82, **layer) == 7         # 6 x 12 + 10, narrow
+    assert segments("layer", "f", 8, 6, 147, 154, 14, B=2, dtype="f32") > 0
+    assert segments("feat", "f", 16, 1, 60, 80, 17, dtype="f32") < 0
+    assert segments("v1", "f", 32, 2, 128, 160, 192, dtype="f32") == 8      # 8 x 24
+    assert segments("v1", "f", 32, 2, 8, 8, 3, dtype="f32") == 1
