@@ -86,6 +86,18 @@ def segments(*args, **kw):
     return _lib.load().chop_last_segments()
 
 
+def test_many_taps_stay_in_one_round():
+    """Five and six views that hold their taps side by side run two waves per SIMD: more than 2048 waves
+    would be a second round."""
+    assert segments("layer", "f", 8, 6, 135, 181, 24, reduce="MIN", dtype="f32") == 2
+    assert segments("layer", "f", 8, 4, 135, 181, 24, reduce="MIN", dtype="f32") == 3
+    assert segments("layer", "f", 8, 6, 135, 181, 24, reduce="MEAN", dtype="f32") == 3     # (three waves)
+    assert segments("feat", "f", 32, 6, 44, 62, 107, dtype="f32") == -5     # 4 x 24 + 11
+    assert segments("feat", "f", 32, 4, 44, 62, 107, dtype="f32") == -7     # 6 x 16 + 11
+    assert segments("feat", "f", 8, 6, 139, 157, 33, dtype="f64") == 3      # 2 x 16 + 1, rounded down
+    assert segments("feat", "f", 32, 6, 8, 12, 33, dtype="f32") == -5       # twelve tiles: single chunks
+
+
 def test_uneven_segments_go_one_after_the_other():
     """Side by side a short last segment leaves every other compute unit idle; segments about as long as each
     other stay side by side, and so do narrow pixels with one value per voxel."""
