@@ -740,17 +740,29 @@ StripGeom strip_geometry(const Args<S> &a, bool backward) {
   g.seg = (per + kDB - 1) / kDB * kDB;
   // A launch below two waves per SIMD lasts as long as its longest wave: segments of less than a
   // chunk then (3 channels, two views, 12 x 16 x 9, double, 12 tiles: forward 11.3 -> 5.8 us, gradient
-  // 17.2 -> 9.5 us; bf16 group correlation, four views, 16 x 17 x 28: 50 -> 9 and 76 -> 16 us; at one
-  // wave per SIMD instead: 24 channels, three views, 38 x 43 x 25 15 against 11 us).  Every segment of a
-  // gradient adds to its pixels' sums: two depths at least and 48 segments at most (two views, 15 x 21 x
-  // 94: 41 us in five segments, 17 in 47, 30 in 94; three views, 18 x 19 x 186: 40, 21 in 47, 36 in 93).
-  if (g.tiles * ((a.D + g.seg - 1) / g.seg) < 2048) {
+  // 17.2 -> 9.5 us; bf16 group correlation, four views, 16 x 17 x 28: 50 -> 9 and 76 -> 16 us; forward at
+  // one wave per SIMD instead: 24 channels, three views, 38 x 43 x 25 15 against 11 us).  Every segment of
+  // a gradient adds to its pixels' sums: two depths at least and 48 segments at most (two views, 15 x 21 x
+  // 94: 41 us in five segments, 17 in 47, 30 in 94; three views, 18 x 19 x 186: 40, 21 in 47, 36 in 93), and
+  // only below one wave per SIMD (bf16, 3 channels, five views, two images of 100 x 128 x 9, 1600 strips: 87
+  // us whole, 112 in two), half a wave where there is next to nothing to cut (double, group correlation of 32
+  // channels, five views, 38 x 40 x 5, 760 strips: 31 whole, 45 in two and three).  CostAggregate in
+  // double adds its rows up chunk by chunk: no less than one (64 channels, 26 x 34 x 3: 16.5 -> 20.3 us).
+  // Segments as even as their number allows: the longest is what the launch lasts (double, 64 channels,
+  // 38 x 40 x 6 in 5 + 1: gradient 15 -> 20 us).
+  const bool whole_chunks = !backward && a.corr == SUM_SQUARED_DIFFERENCE && sizeof(S) == 8 && a.D <= kDB;
+  const int64_t full = !backward ? 2048 : a.D <= 5 ? 512 : 1024;
+  if (g.tiles * ((a.D + g.seg - 1) / g.seg) < full && !whole_chunks) {
     int64_t len = (g.tiles * a.D + 2047) / 2048;
     if (backward) {
       if (len < 2) len = 2;
       if (len < (a.D + 47) / 48) len = (a.D + 47) / 48;
     }
-    if (len < g.seg) g.seg = (int)(len <= kDB ? len : len / kDB * kDB);
+    if (len < g.seg) {
+      g.seg = (int)(len <= kDB ? len : len / kDB * kDB);
+      const int64_t n = (a.D + g.seg - 1) / g.seg;
+      g.seg = (int)((a.D + n - 1) / n);
+    }
   }
   g.nseg = (int)((a.D + g.seg - 1) / g.seg);
   // carried runs: N * 64 lanes * (4 sums + tap offset + cell); given up beyond 16 KiB, or

@@ -86,6 +86,23 @@ def segments(*args, **kw):
     return _lib.load().chop_last_segments()
 
 
+def test_strips_are_cut_where_it_pays():
+    """A lane per channel: launches below two waves per SIMD (gradients: one; half a wave for next to no
+    depths) are cut below a chunk, into segments as even as their number allows."""
+    bf16 = dict(dtype="bf16", family=2)
+    assert segments("v1", "b", 3, 5, 100, 128, 9, B=2, **bf16) == 1         # 1600 strips
+    assert segments("v1", "b", 3, 5, 100, 128, 9, **bf16) == 3              # 800 strips, 3 x 3
+    assert segments("v1", "f", 3, 5, 100, 128, 9, B=2, **bf16) == 2         # 5 + 4
+    assert segments("v1", "b", 64, 3, 38, 40, 6, family=2) == 1             # 1520 strips
+    assert segments("v2", "b", 32, 5, 38, 40, 5, family=2) == 1             # 760 strips, five depths
+    assert segments("v2", "b", 32, 5, 38, 40, 6, family=2) == 2
+    assert segments("layer", "f", 64, 5, 26, 34, 3, family=2) == 1
+    assert segments("layer", "f", 64, 5, 26, 34, 9, family=2) > 1
+    assert segments("v1", "f", 64, 5, 26, 34, 3, family=2) == 2
+    assert segments("v1", "f", 3, 2, 12, 16, 9, family=2) == 9              # twelve strips: depth by depth
+    assert segments("v1", "b", 3, 2, 12, 16, 9, family=2) == 5
+
+
 def test_many_taps_stay_in_one_round():
     """Five and six views that hold their taps side by side run two waves per SIMD: more than 2048 waves
     would be a second round."""
