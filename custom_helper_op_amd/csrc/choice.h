@@ -1,7 +1,8 @@
 // Which calls that the tile-shaped kernels could serve keep a lane per channel because it is the faster
-// one (the strip kernels; CostVolumeV3 with more than 16 groups: a thread per voxel).  Only double has
-// such calls: its tiles need twice the registers and run two waves per SIMD, and its lane-per-channel
-// kernels are held to four.  Times in microseconds, lane per channel against tiles, as "12 : 15".
+// one (the strip kernels; CostVolumeV3 with more than 16 groups: a thread per voxel).  A lane per channel
+// spreads a depth over more lanes and needs fewer registers, so it wins where a launch is bound by the chain
+// of steps in one wave and not by work.  Times in microseconds, lane per channel against tiles, as
+// "12 : 15"; float64 where nothing else is said.
 #pragma once
 
 #include "internal.h"
@@ -9,33 +10,80 @@
 namespace chop {
 
 template <typename S>
-bool lanes_are_faster(const Args<S> &a, bool backward) {
-  if (sizeof(S) != 8) return false;
-  const int64_t lpp = a.C > 16 && a.C < 32 ? 8 : a.C / 4;  // lanes of a pixel
-  const bool few_tiles = a.pixels() * lpp / 64 < 2048;
-  if (backward) {
-    // Gradients of group correlation over a few depths: clearing and writing back a workgroup's window
-    // costs the same for two depths as for a whole chunk, and wide pixels share it between few pixels.
-    // The line: 3/4 depth per lane of a pixel.  64 channels, two views, 200 x 260: 4 depths 246 : 436, 8
-    // depths 415 : 595; three views, 90 x 100: 4 depths 100 : 146, 12 depths 166 : 161.  32 channels,
-    // three views, 138 x 151: 2 depths 140 : 175, 4 depths 190 : 200, 6 depths 227 : 219.  16 channels: 2
-    // depths 77 : 83, 4 depths 108 : 93.  Where the tiles do not fill the chip the launch is bound by
-    // latency and the tiles' shorter chains win up to 32 channels (five views, 60 x 80, 600 tiles: 32
-    // channels, 2 depths 45 : 38), but not at 64 (70 : 89).
-    // The minimum at 64 channels at any depth: each view's workgroups pass over the other views' voxels
-    // with four pixels to a wave.  200 x 260, four views: 12 depths 1001 : 1455, 32 depths 1833 : 2454,
-    // one hypothesis field 1421 : 1622; two views, 32 depths 1109 : 1224, one hypothesis field 886 : 842.
-    if (a.corr == GROUP_CORRELATION &&
-        ((4 * a.D < 3 * lpp && (lpp == 16 || !few_tiles)) || (lpp == 16 && a.reduce != 0)))
-      return true;
-    // One view over a few depths, few tiles: narrow pixels have only the clearing and writing back to do
-    // (38 x 40 x 6, 8 channels: group correlation 10.6 : 13.6, squared differences 8.5 : 11.9; 16 channels
-    // 16.6 : 16.3).
-    return a.N == 1 && lpp <= 2 && a.D < 12 && few_tiles &&
-           (a.corr == GROUP_CORRELATION || a.corr == SQUARED_DIFFERENCE);
+int64_t lanes_of_a_pixel(const Args<S> &a) {
+  return a.C > 16 && a.C < 32 ? 8 : a.C / 4;
+}
+
+// Values, in double or with idle lanes (20, 24 and 28 channels in any type).  A tile's wave takes a chunk of
+// as many depths as a pixel has lanes through every view, one view's taps after the other's: until every
+// SIMD has a wave of its own, a launch takes as long as one wave, and the chain grows with the views.
+//   waves  32 channels, squared differences:  three views, 190 (38 x 40 x 6) 7.8 : 11.1, 570 10.5 : 14.8,
+//          950 14.8 : 14.9, 1050 (50 x 56 x 24) 18.4 : 17.6, 1800 23.7 : 17.5; two views, 190 6.5 : 7.5,
+//          380 7.7 : 8.9, 570 10.2 : 9.8; one view, 120 5.5 : 6.1, 190 5.6 : 5.3, 570 7.7 : 6.8.  24 channels
+//          in float32, three views: 570 9.9 : 12.1, 1200 15.2 : 13.3.
+//   16 channels leave each lane half as many chains: squared differences, three views, 364 8.4 : 9.3, 600
+//   10.3 : 9.8; group correlation 200 8.5 : 9.8, 546 11.5 : 10.5.  8 channels: tiles at any size.
+//   CostAggregate and FeatureAggregate hold less per view (four views, 32 channels: with differences 180
+//   12.5 : 13.2, 380 14.7 : 16.0, 700 16.7 : 16.5; samples alone 380 12.2 : 16.4, 570 18.2 : 17.9).
+// Few depths shorten the tiles' chain, not the lanes' (one view, 38 x 40: 3 depths 5.4 : 4.5; CostAggregate,
+// four views, 64 channels, 20 x 24: 3 depths 13.4 : 9.7).
+template <typename S>
+bool lanes_are_faster_forward(const Args<S> &a) {
+  const bool idle_lanes = a.C > 16 && a.C < 32;
+  if ((sizeof(S) != 8 && !idle_lanes) || a.corr == BEST_GROUP_PAIR) return false;
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64;
+  const int64_t waves = tiles * ((a.D + lpp - 1) / lpp);
+  if (lpp <= 2) {
+    // One view's minimum at 8 channels writes and does next to nothing else.  Where the volume is far beyond
+    // the caches the strips' rows go out faster: group correlation, 200 x 260, 48 depths 65.7 : 76.1, 333 x
+    // 390, 24 depths 79.1 : 104 (200 x 260, 24 depths 42.1 : 36.4); squared differences, 200 x 260, 86 depths
+    // 149 : 182 (100 x 130, 86 depths 58.8 : 57.8).
+    return lpp == 2 && a.N == 1 && a.reduce != 0 &&
+           ((a.corr == GROUP_CORRELATION && waves >= 32768) ||
+            (a.corr == SQUARED_DIFFERENCE && waves >= 65536));
   }
-  // Squared differences of many views, or of 64 channels and three views in launches of few tiles.
-  return a.corr == SQUARED_DIFFERENCE && ((lpp >= 8 && a.N >= 5) || (lpp == 16 && a.N >= 3 && few_tiles));
+  // Two waves of the squared differences' minimum of many views fit a SIMD: a little over 2048 tiles leave a
+  // second round nearly empty, until the depths can be cut to fill it (five views, 32 channels, 2400 tiles:
+  // 12 depths 64.5 : 72.4, 24 depths 101 : 115, 48 depths 189 : 172; 3250 tiles, 12 depths 83.4 : 73.8).
+  if (a.corr == SQUARED_DIFFERENCE && a.reduce != 0 && a.N >= 5 && lpp >= 8 && tiles > 2048 &&
+      tiles <= 2560 && a.D <= 24)
+    return true;
+  const bool one_value = a.corr == SUM_SQUARED_DIFFERENCE, samples = a.corr == WARP_ONLY;
+  int64_t line;
+  if (lpp == 4)
+    line = one_value || a.N == 1 ? 0 : (a.corr == SQUARED_DIFFERENCE ? 512 : 256) / (a.N == 2 ? 2 : 1);
+  else if (one_value)
+    line = a.N == 1 ? 0 : a.N == 2 ? 192 : 384;
+  else
+    line = a.N == 1 ? 192 : a.N == 2 || samples ? 384 : 768;
+  return waves < line && (one_value ? 2 * a.D >= lpp : a.D >= 4 || a.N >= 3);
+}
+
+template <typename S>
+bool lanes_are_faster(const Args<S> &a, bool backward) {
+  if (!backward) return lanes_are_faster_forward(a);
+  if (sizeof(S) != 8) return false;
+  const int64_t lpp = lanes_of_a_pixel(a);
+  const bool few_tiles = a.pixels() * lpp / 64 < 2048;
+  // Gradients of group correlation over a few depths: clearing and writing back a workgroup's window
+  // costs the same for two depths as for a whole chunk, and wide pixels share it between few pixels.
+  // The line: 3/4 depth per lane of a pixel.  64 channels, two views, 200 x 260: 4 depths 246 : 436, 8
+  // depths 415 : 595; three views, 90 x 100: 4 depths 100 : 146, 12 depths 166 : 161.  32 channels,
+  // three views, 138 x 151: 2 depths 140 : 175, 4 depths 190 : 200, 6 depths 227 : 219.  16 channels: 2
+  // depths 77 : 83, 4 depths 108 : 93.  Where the tiles do not fill the chip the launch is bound by
+  // latency and the tiles' shorter chains win up to 32 channels (five views, 60 x 80, 600 tiles: 32
+  // channels, 2 depths 45 : 38), but not at 64 (70 : 89).
+  // The minimum at 64 channels at any depth: each view's workgroups pass over the other views' voxels
+  // with four pixels to a wave.  200 x 260, four views: 12 depths 1001 : 1455, 32 depths 1833 : 2454,
+  // one hypothesis field 1421 : 1622; two views, 32 depths 1109 : 1224, one hypothesis field 886 : 842.
+  if (a.corr == GROUP_CORRELATION &&
+      ((4 * a.D < 3 * lpp && (lpp == 16 || !few_tiles)) || (lpp == 16 && a.reduce != 0)))
+    return true;
+  // One view over a few depths, few tiles: narrow pixels have only the clearing and writing back to do
+  // (38 x 40 x 6, 8 channels: group correlation 10.6 : 13.6, squared differences 8.5 : 11.9; 16 channels
+  // 16.6 : 16.3).
+  return a.N == 1 && lpp <= 2 && a.D < 12 && few_tiles &&
+         (a.corr == GROUP_CORRELATION || a.corr == SQUARED_DIFFERENCE);
 }
 
 }  // namespace chop

@@ -80,6 +80,34 @@ def test_asked_for():
     assert ran("v2", "b", 64, 4, 38, 40, 6, "MIN") == LANES
 
 
+def sides(direction, lanes, tiles):
+    """Calls on either side of a line: `(op, C, N, H, W, D, keywords)`."""
+    for want, calls in ((LANES, lanes), (TILES, tiles)):
+        for op, C, N, H, W, D, *kw in calls:
+            kw = kw[0] if kw else {}
+            assert ran(op, direction, C, N, H, W, D, **kw) == want, (op, C, N, H, W, D, kw)
+
+
+def test_forward_launches_of_few_waves_keep_a_lane_per_channel():
+    """Double and idle lanes: below a wave per SIMD the chain of one wave is all there is, and a lane per
+    channel has the shorter one."""
+    f32, low = dict(dtype="f32"), dict(reduce="MIN")
+    sides("f",
+          [("v1", 32, 3, 38, 40, 6), ("v1", 32, 3, 38, 40, 24), ("v1", 32, 2, 38, 40, 12), ("v1", 32, 1, 20, 24, 12),
+           ("v1", 16, 3, 50, 56, 6), ("v2", 16, 3, 38, 40, 6), ("v2", 64, 6, 38, 40, 17), ("v2", 32, 3, 13, 15, 3),
+           ("v1", 24, 3, 38, 40, 24, f32), ("v1", 20, 3, 38, 40, 12, dict(dtype="bf16")), ("v2", 28, 2, 38, 40, 8, f32),
+           ("layer", 32, 4, 38, 40, 12), ("layer", 64, 3, 20, 24, 8), ("feat", 32, 4, 38, 40, 12),
+           ("v2", 8, 1, 200, 260, 48, low), ("v1", 8, 1, 200, 260, 86, low),
+           ("v1", 32, 5, 120, 160, 24, low), ("v1", 64, 6, 90, 110, 24, low)],
+          [("v1", 32, 3, 50, 56, 24), ("v1", 32, 6, 50, 56, 24), ("v1", 32, 2, 38, 40, 24), ("v1", 32, 1, 38, 40, 12),
+           ("v1", 16, 3, 60, 80, 8), ("v2", 16, 3, 50, 56, 12), ("v2", 64, 6, 60, 80, 8), ("v2", 32, 1, 13, 15, 3),
+           ("v1", 24, 3, 60, 80, 12, f32), ("v1", 8, 5, 38, 40, 6), ("v1", 32, 6, 128, 160, 64), ("v1", 64, 3, 200, 260, 6),
+           ("layer", 32, 4, 50, 56, 12), ("layer", 64, 3, 20, 24, 3), ("layer", 16, 4, 20, 24, 8), ("layer", 32, 1, 20, 24, 8),
+           ("feat", 32, 4, 50, 56, 12), ("v1", 32, 3, 13, 15, 3, dict(dtype="f32")),
+           ("v2", 8, 1, 200, 260, 24, low), ("v2", 8, 1, 200, 260, 48), ("v1", 8, 1, 100, 130, 86, dict(B=2, reduce="MIN")),
+           ("v1", 32, 5, 120, 160, 48, low), ("v1", 32, 5, 120, 160, 24), ("v1", 32, 5, 100, 130, 12, dict(B=2, reduce="MIN"))])
+
+
 def segments(*args, **kw):
     """Depth segments of the call; negative: all tiles' first segments before all second ones."""
     ran(*args, **kw)
