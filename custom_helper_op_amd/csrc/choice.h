@@ -59,6 +59,32 @@ bool lanes_are_faster_forward(const Args<S> &a) {
   return waves < line && (one_value ? 2 * a.D >= lpp : a.D >= 4 || a.N >= 3);
 }
 
+// Gradients in double of one view, or of two, in launches that leave most of the chip idle.  With so few
+// depths to a tile there is little to share in its window, and clearing it, collecting in it and writing it
+// back is a longer chain than the strips' atomic additions.  The line is a number of tiles times depths; it
+// lies higher for the gradients with one value per voxel (their strips read less) and for wide pixels (whose
+// tiles are small).  One view, 38 x 40 x 6, squared differences: 4 channels 9.7 : 14.4, 8 channels 10.1 :
+// 13.4, 32 channels 13.5 : 15.3, 64 channels 15.7 : 21.4; beyond the line 60 x 80 x 24, 8 channels 17.6 :
+// 17.6, 60 x 80 x 6, 32 channels 21.2 : 18.0, 60 x 80 x 12, 64 channels (1200 tiles) 45.6 : 34.9; with one
+// value per voxel 90 x 110 x 6, 8 channels 14.2 : 19.0, x 12 23.4 : 19.4.  Not group correlation of 32
+// channels (38 x 40 x 6 17.5 : 16.4) or its minimum of 64.  16 channels: tiles (38 x 40 x 12 15.0 : 11.4).
+// Two views, squared differences: 4 channels, 38 x 40 x 6 12.8 : 15.6, 60 x 80 x 12 22.1 : 17.6; 64 channels,
+// 20 x 24 x 12 17.6 : 22.3, 38 x 40 x 12 29.2 : 27.2.
+template <typename S>
+bool lanes_are_faster_few_tiles(const Args<S> &a) {
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64, steps = tiles * a.D;
+  if (a.corr == BEST_GROUP_PAIR || a.N > 2 || a.D < 3 || tiles >= 512) return false;
+  if (a.N == 2)
+    return lpp == 1    ? steps < 1024 && a.D < 16 && (a.D > 3 || tiles >= 128)
+           : lpp == 16 ? steps < 3072
+                       : false;
+  const bool correlation = a.corr == GROUP_CORRELATION;
+  return lpp <= 2    ? steps < (a.corr == SUM_SQUARED_DIFFERENCE ? 2048 : 1024)
+         : lpp == 8  ? steps < 2560 && !correlation
+         : lpp == 16 ? steps < 8192 && !(correlation && a.reduce != 0)
+                     : false;
+}
+
 template <typename S>
 bool lanes_are_faster(const Args<S> &a, bool backward) {
   if (!backward) return lanes_are_faster_forward(a);
@@ -79,11 +105,7 @@ bool lanes_are_faster(const Args<S> &a, bool backward) {
   if (a.corr == GROUP_CORRELATION &&
       ((4 * a.D < 3 * lpp && (lpp == 16 || !few_tiles)) || (lpp == 16 && a.reduce != 0)))
     return true;
-  // One view over a few depths, few tiles: narrow pixels have only the clearing and writing back to do
-  // (38 x 40 x 6, 8 channels: group correlation 10.6 : 13.6, squared differences 8.5 : 11.9; 16 channels
-  // 16.6 : 16.3).
-  return a.N == 1 && lpp <= 2 && a.D < 12 && few_tiles &&
-         (a.corr == GROUP_CORRELATION || a.corr == SQUARED_DIFFERENCE);
+  return lanes_are_faster_few_tiles(a);
 }
 
 }  // namespace chop

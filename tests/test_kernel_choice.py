@@ -108,6 +108,27 @@ def test_forward_launches_of_few_waves_keep_a_lane_per_channel():
            ("v1", 32, 5, 120, 160, 48, low), ("v1", 32, 5, 120, 160, 24), ("v1", 32, 5, 100, 130, 12, dict(B=2, reduce="MIN"))])
 
 
+@pytest.mark.parametrize("op", ["v1", "layer", "feat"])
+def test_gradients_of_one_and_two_views_in_small_launches(op):
+    """Double: little to share in a tile's window, and a longer chain than the strips' atomic additions."""
+    sides("b",
+          [(op, 4, 1, 60, 80, 8), (op, 8, 1, 38, 40, 6), (op, 32, 1, 38, 40, 12), (op, 24, 1, 20, 24, 12),
+           (op, 64, 1, 38, 40, 20), (op, 4, 2, 38, 40, 6), (op, 64, 2, 20, 24, 12)],
+          [(op, 4, 1, 120, 160, 12), (op, 8, 1, 60, 80, 24), (op, 32, 1, 60, 80, 6), (op, 32, 1, 38, 40, 24),
+           (op, 64, 1, 60, 80, 3), (op, 16, 1, 38, 40, 12), (op, 4, 2, 60, 80, 24), (op, 4, 2, 20, 24, 3),
+           (op, 64, 2, 38, 40, 12), (op, 8, 1, 38, 40, 6, dict(dtype="f32")), (op, 64, 1, 38, 40, 2)])
+
+
+def test_correlation_gradients_of_one_view():
+    sides("b",
+          [("v2", 8, 1, 38, 40, 6), ("v2", 64, 1, 38, 40, 12), ("v2", 8, 1, 38, 40, 6, dict(reduce="MIN"))],
+          [("v2", 32, 1, 38, 40, 6), ("v2", 8, 1, 60, 80, 24), ("v2", 16, 1, 38, 40, 6)])
+
+
+def test_gradients_of_one_view_and_one_value_per_voxel():
+    sides("b", [("layer", 8, 1, 90, 110, 6)], [("layer", 8, 1, 90, 110, 12), ("v1", 8, 1, 90, 110, 6)])
+
+
 def segments(*args, **kw):
     """Depth segments of the call; negative: all tiles' first segments before all second ones."""
     ran(*args, **kw)
