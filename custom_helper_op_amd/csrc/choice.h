@@ -85,27 +85,46 @@ bool lanes_are_faster_few_tiles(const Args<S> &a) {
                      : false;
 }
 
+// Gradients of group correlation in double over a few depths.  A workgroup clears its window and writes it
+// back once for two depths as for a whole chunk, and the minimum passes over every view's voxels to find its
+// own.  200 x 260 unless another size is given; the strips' time goes up with the depths, the tiles' hardly.
+//   Mean   64 channels, two views: 2 depths 261 : 343, 3 depths 370 : 423, 4 depths 487 : 461; four views:
+//          3 depths 736 : 853, 4 depths 955 : 910.  32 channels, four views: 2 depths 281 : 319, 3 depths 401
+//          : 371.  16 channels, four views: 3 depths 157 : 182, 4 depths 189 : 193, and with 1200 tiles (120
+//          x 160) 71 : 65.
+//   Minimum at 64 channels, two views and more: at any depth, as a wave holds four pixels.  Two views: 4
+//          depths 248 : 437, 12 depths 585 : 718; four views, 12 depths 1003 : 1464, 32 depths 1833 : 2454.
+//          One view has nothing to pass over: 4 depths 223 : 187.
+//   Minimum at 32 channels from four views on, eight rows to a window: 4 depths 246 : 346, 8 depths 415 :
+//          432, 12 depths 567 : 538; 60 x 80 x 6 41 : 51.  Three views: 4 depths 253 : 274, 6 depths 312 : 318,
+//          60 x 80 x 4 41 : 37.
+//   Minimum at 16 channels: two views 3 depths 96 : 104, 4 depths 112 : 110; four views 153 : 186, 179 : 192.
+//   Minimum at 8 channels, four views: 8 depths 132 : 139, 12 depths 191 : 177; 120 x 160 x 8 57 : 65; 60 x 80
+//          x 4 26 : 22.  Six views: 188 : 199, but 120 x 160 x 8 88 : 77.  Two views: 60 x 80 x 12 20.6 : 22.9,
+//          one depth 33.8 : 34.1.  One view: 120 x 160 x 8 21.4 : 24.8, 200 x 260 x 8 44.8 : 40.2.
+//   Minimum at 4 channels, three views: 8 depths 76 : 121, 12 depths 113 : 148, one depth 31.7 : 29.3; four
+//          views, 60 x 80 x 8 25.5 : 22.9, 120 x 160 x 8 44 : 51.
+template <typename S>
+bool lanes_are_faster_correlation(const Args<S> &a) {
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64;
+  if (a.reduce == 0)
+    return a.N > 1 && lpp >= 4 && a.D < (lpp == 8 ? 3 : 4) && tiles >= (lpp == 16 ? 1024 : 2048);
+  switch (lpp) {
+    case 16: return a.N > 1;
+    case 8: return a.N >= 4 ? a.D <= 8 : a.N > 1 && a.D <= 4 && tiles >= 2048;
+    case 4: return a.N > 1 && a.D <= 3 && tiles >= 2048;
+    case 2:
+      return a.D <= (a.N <= 2 && tiles < 256 ? 12 : 8) && (a.D > 1 || a.N > 2) &&
+             (a.N == 1 ? tiles < 1024 : tiles >= 256 * (a.N - 2));
+    default: return a.D > 1 && a.D <= 12 && tiles >= 64 * (a.N - 2);
+  }
+}
+
 template <typename S>
 bool lanes_are_faster(const Args<S> &a, bool backward) {
   if (!backward) return lanes_are_faster_forward(a);
   if (sizeof(S) != 8) return false;
-  const int64_t lpp = lanes_of_a_pixel(a);
-  const bool few_tiles = a.pixels() * lpp / 64 < 2048;
-  // Gradients of group correlation over a few depths: clearing and writing back a workgroup's window
-  // costs the same for two depths as for a whole chunk, and wide pixels share it between few pixels.
-  // The line: 3/4 depth per lane of a pixel.  64 channels, two views, 200 x 260: 4 depths 246 : 436, 8
-  // depths 415 : 595; three views, 90 x 100: 4 depths 100 : 146, 12 depths 166 : 161.  32 channels,
-  // three views, 138 x 151: 2 depths 140 : 175, 4 depths 190 : 200, 6 depths 227 : 219.  16 channels: 2
-  // depths 77 : 83, 4 depths 108 : 93.  Where the tiles do not fill the chip the launch is bound by
-  // latency and the tiles' shorter chains win up to 32 channels (five views, 60 x 80, 600 tiles: 32
-  // channels, 2 depths 45 : 38), but not at 64 (70 : 89).
-  // The minimum at 64 channels at any depth: each view's workgroups pass over the other views' voxels
-  // with four pixels to a wave.  200 x 260, four views: 12 depths 1001 : 1455, 32 depths 1833 : 2454,
-  // one hypothesis field 1421 : 1622; two views, 32 depths 1109 : 1224, one hypothesis field 886 : 842.
-  if (a.corr == GROUP_CORRELATION &&
-      ((4 * a.D < 3 * lpp && (lpp == 16 || !few_tiles)) || (lpp == 16 && a.reduce != 0)))
-    return true;
-  return lanes_are_faster_few_tiles(a);
+  return lanes_are_faster_few_tiles(a) || (a.corr == GROUP_CORRELATION && lanes_are_faster_correlation(a));
 }
 
 }  // namespace chop

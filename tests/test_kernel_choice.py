@@ -129,6 +129,25 @@ def test_gradients_of_one_view_and_one_value_per_voxel():
     sides("b", [("layer", 8, 1, 90, 110, 6)], [("layer", 8, 1, 90, 110, 12), ("v1", 8, 1, 90, 110, 6)])
 
 
+def test_correlation_gradients_of_few_depths():
+    """Double: a workgroup's window costs the same for two depths as for a chunk, and the minimum passes over
+    every view's voxels."""
+    low = dict(reduce="MIN")
+    sides("b",
+          [("v2", 64, 2, 200, 260, 3), ("v2", 64, 4, 60, 80, 2), ("v2", 32, 4, 200, 260, 2), ("v2", 16, 4, 200, 260, 3)],
+          [("v2", 64, 2, 200, 260, 4), ("v2", 64, 1, 200, 260, 3), ("v2", 32, 4, 200, 260, 3), ("v2", 16, 4, 120, 160, 3),
+           ("v2", 16, 4, 200, 260, 4), ("v2", 8, 4, 200, 260, 1), ("v2", 64, 3, 90, 100, 8)])
+    sides("b",
+          [(op, C, N, H, W, D, low) for op, C, N, H, W, D in
+           [("v2", 64, 2, 38, 40, 6), ("v2", 64, 6, 200, 260, 32), ("v2", 32, 4, 60, 80, 8), ("v2", 24, 6, 200, 260, 6),
+            ("v2", 32, 2, 200, 260, 4), ("v2", 16, 3, 200, 260, 3), ("v2", 8, 3, 120, 160, 8), ("v2", 8, 6, 200, 260, 8),
+            ("v2", 8, 2, 60, 80, 12), ("v2", 8, 1, 120, 160, 8), ("v2", 4, 3, 200, 260, 12), ("v2", 4, 1, 60, 80, 8)]],
+          [(op, C, N, H, W, D, low) for op, C, N, H, W, D in
+           [("v2", 64, 1, 200, 260, 4), ("v2", 32, 4, 200, 260, 9), ("v2", 32, 3, 60, 80, 4), ("v2", 32, 3, 200, 260, 5),
+            ("v2", 16, 3, 120, 160, 3), ("v2", 16, 3, 200, 260, 4), ("v2", 8, 6, 120, 160, 8), ("v2", 8, 2, 120, 160, 9),
+            ("v2", 8, 1, 200, 260, 8), ("v2", 4, 3, 200, 260, 1), ("v2", 4, 6, 60, 80, 8), ("v2", 4, 2, 200, 260, 13)]])
+
+
 def segments(*args, **kw):
     """Depth segments of the call; negative: all tiles' first segments before all second ones."""
     ran(*args, **kw)
