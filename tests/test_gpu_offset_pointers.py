@@ -191,3 +191,36 @@ def test_other_ops_shifted_inputs(oracle):
     assert lib.chop_last_kernel_family() != TILED
     for g, w in zip(got, want):
         assert_backward_close(host(g), w)
+
+
+@pytest.mark.parametrize("C", [8, 32])
+@pytest.mark.parametrize("which", ["all", "outputs"])
+def test_float64(oracle, C, which):
+    """Float64 at channel counts that run the tiled kernels when aligned: every pointer shifted by one
+    element, or only the outputs."""
+    lib = _lib.load()
+    N, H, W, D = 2, 40, 61, 25
+    t = reference_test_case(3, 1, N, H, W, C, D, np.float64, seed=31 + C)
+    args = tuple(t[k] for k in KEYS)
+    want_cost, want_mask = oracle.cost_volume_fwd(*args, "MEAN")
+    cg = np.random.default_rng(32).standard_normal(want_cost.shape)
+    want = oracle.cost_volume_bwd(*args, cg, want_mask, "MEAN")
+    stream = torch.cuda.current_stream().cuda_stream
+    dims = (1, H, W, C, D, N, H, W)
+    for put, out, shape in ((dev, lambda s: torch.empty(s, dtype=torch.float64, device="cuda"), TILED),
+                            (shifted if which == "all" else dev, lambda s: shifted_empty(s, torch.float64), 3)):
+        ins = [put(x) for x in args]
+        cost, mask = out(want_cost.shape), torch.empty((1, H, W, D, 1), dtype=torch.int32, device="cuda")
+        _lib.check(lib.chop_cost_volume_fwd_f64(stream, 0, 1, *dims, *[x.data_ptr() for x in ins],
+                                                cost.data_ptr(), mask.data_ptr()))
+        assert lib.chop_last_kernel_shape() == shape
+        assert np.array_equal(host(mask), want_mask) and np.array_equal(host(cost), want_cost)
+        d_cg = put(cg)
+        grads = [out((1, H, W, C)), out((1, N, H, W, C)), out((1, H, W, 1))]
+        for g in grads:
+            g.fill_(float("nan"))     # the library zeroes what it accumulates into
+        _lib.check(lib.chop_cost_volume_bwd_f64(stream, 0, 1, *dims, *[x.data_ptr() for x in ins],
+                                                d_cg.data_ptr(), mask.data_ptr(), *[g.data_ptr() for g in grads]))
+        assert lib.chop_last_kernel_shape() == shape
+        for g, w in zip(grads, want):
+            assert_backward_close(host(g), w, 1e-10)

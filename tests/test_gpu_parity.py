@@ -32,6 +32,12 @@ def _assert_family(family, expect_tiled=True):
     assert got == want, (got, want)
 
 
+def _assert_lanes():
+    """The last call ran a lane per channel (in float64 the family's code stands for the tiles as well)."""
+    _assert_family(2)
+    assert _lib.load().chop_last_kernel_shape() == 3
+
+
 def _v1_inputs(t, dtype=None):
     keys = ("ref", "src", "base_plane", "offsets", "Rs", "Ts")
     return [dev(t[k].astype(dtype) if dtype else t[k]) for k in keys]
@@ -774,15 +780,16 @@ def test_strip_float64_wide_pixels(oracle, C, N):
     depth_grid = t["base_plane"] + t["offsets"][:, None, None, :]
     a2 = (t["ref"], t["src"], depth_grid, t["Rs"], t["Ts"])
     in2 = [dev(x) for x in a2]
+    _lib.load().chop_set_kernel_family(2)    # (unasked, 20 and 32 channels run the tiled kernels)
     for reduce in ("MEAN", "MIN"):
         want_cost, want_mask = oracle.cost_volume_fwd(*args, reduce)
         cost, mask = chop.cost_volume_raw(*ins, reduce)
-        _assert_family(2)
+        _assert_lanes()
         assert np.array_equal(host(mask), want_mask) and np.array_equal(host(cost), want_cost)
         cg = rng.standard_normal(want_cost.shape)
         want = oracle.cost_volume_bwd(*args, cg, want_mask, reduce)
         got = chop.cost_volume_grad(*ins, dev(cg), mask, reduce)
-        _assert_family(2)
+        _assert_lanes()
         for g, w in zip(got, want):
             assert_backward_close(host(g), w)
 
@@ -792,7 +799,7 @@ def test_strip_float64_wide_pixels(oracle, C, N):
         cg = rng.standard_normal(want_cost.shape)
         want = oracle.cost_volume_v2_bwd(*a2, cg, want_mask, reduce, groups)
         got = chop.cost_volume_grad_v2(*in2, dev(cg), mask, reduce, groups)
-        _assert_family(2)
+        _assert_lanes()
         for g, w in zip(got, want):
             assert_backward_close(host(g), w)
 
@@ -802,7 +809,7 @@ def test_strip_float64_wide_pixels(oracle, C, N):
         cg = rng.standard_normal(want_cost.shape)
         want = oracle.cost_aggregate_bwd(*args, cg, want_mask, reduce)
         got = chop.cost_aggregate_grad(*ins, dev(cg), mask, reduce)
-        _assert_family(2)
+        _assert_lanes()
         for g, w in zip(got, want):
             assert_backward_close(host(g), w)
 
@@ -812,6 +819,7 @@ def test_strip_float64_wide_pixels(oracle, C, N):
         cg = rng.standard_normal(want_cost.shape)
         want = oracle.cost_volume_v3_bwd(*args, cg, want_mask, reduce, groups)
         got = chop.cost_volume_grad_v3(*ins, dev(cg), mask, reduce, groups)
+        _assert_lanes()
         for g, w in zip(got, want):
             assert_backward_close(host(g), w)
 
@@ -822,7 +830,7 @@ def test_strip_float64_wide_pixels(oracle, C, N):
     cg = rng.standard_normal(want_feat.shape)
     want = oracle.feature_aggregate_bwd(*fargs, cg, want_mask)
     got = chop.feature_aggregate_grad(*ins[1:], dev(cg), mask)
-    _assert_family(2)
+    _assert_lanes()
     for g, w in zip(got, want):
         assert_backward_close(host(g), w)
 

@@ -13,9 +13,8 @@ from gpu_util import assert_backward_close, dev, host
 pytestmark = pytest.mark.gpu
 
 
-def _tensors(seed, B, N, H, W, C, D, near, far, rot, shift):
+def _tensors(seed, B, N, H, W, C, D, near, far, rot, shift, f32=np.float32):
     rng = np.random.default_rng(seed)
-    f32 = np.float32
     ref = rng.standard_normal((B, H, W, C)).astype(f32)
     src = rng.standard_normal((B, N, H, W, C)).astype(f32)
     base = rng.uniform(0.0, 0.05, (B, H, W, 1)).astype(f32)
@@ -74,6 +73,62 @@ def test_spread_cells(oracle, C, sweep):
     got = chop.feature_aggregate_grad(*d_args[1:], dev(cg), dev(mask))
     for g, w in zip(got, oracle.feature_aggregate_bwd(*args[1:], cg, mask)):
         assert_backward_close(host(g), w)
+
+
+@pytest.fixture
+def tiles():
+    """The tiled kernels wherever they can serve the shape, also where a lane per channel is the faster one."""
+    lib = _lib.load()
+    lib.chop_set_kernel_family(3)
+    yield lib
+    lib.chop_set_kernel_family(0)
+
+
+@pytest.mark.parametrize("sweep", sorted(SWEEPS))
+@pytest.mark.parametrize("C", [4, 8, 16, 24, 32, 64])
+def test_spread_cells_float64(oracle, tiles, C, sweep):
+    """The same sweeps in float64, whose windows are smaller (six rows at 32 channels, four in
+    CostAggregate) and whose lanes own two pairs of channels apart: runs that end outside the window,
+    windows that move inside a chunk, cells on their way to memory.  Each sum has a few hundred terms: 1e-10
+    of the gradient's rms, as for the tiles on ordinary sweeps."""
+    near, far, rot, shift = SWEEPS[sweep]
+    N, D = (6, 19) if sweep == "mixed" else (2, 11)
+    rng, args = _tensors(C, 1, N, 31, 43, C, D, near, far, rot, shift, np.float64)
+    a2 = (args[0], args[1], args[2] + args[3][:, None, None, :], args[4], args[5])
+    calls = [("cost_volume", args, ("MEAN",)), ("cost_volume", args, ("MIN",)),
+             ("cost_aggregate", args, ("MEAN",)), ("cost_aggregate", args, ("MIN",)),
+             ("cost_volume_v2", a2, ("MEAN", C // 4)), ("cost_volume_v2", a2, ("MIN", C // 2)),
+             ("feature_aggregate", args[1:], ())]
+    if C in (8, 16, 32, 64):
+        calls += [("cost_volume_v3", args, ("MEAN", C // 4)), ("cost_volume_v3", args, ("MIN", C // 8))]
+    for name, a, extra in calls:
+        print("\n[case] C%d %s %s %s" % (C, sweep, name, extra), flush=True)
+        cost, mask = getattr(oracle, name + "_fwd")(*a, *extra)
+        cg = rng.standard_normal(cost.shape)
+        grad = getattr(chop, {"cost_volume_v2": "cost_volume_grad_v2", "cost_volume_v3": "cost_volume_grad_v3"}
+                       .get(name, name + "_grad"))
+        got = grad(*[dev(x) for x in a], dev(cg), dev(mask), *extra)
+        assert tiles.chop_last_kernel_shape() == 2
+        for g, w in zip(got, getattr(oracle, name + "_bwd")(*a, cg, mask, *extra)):
+            assert_backward_close(host(g), w, 1e-10)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("sweep", sorted(SWEEPS))
+@pytest.mark.parametrize("C,sub", [(8, 1), (16, 2), (32, 1), (32, 2), (64, 2)])
+def test_spread_cells_narrow_pairs(oracle, tiles, C, sub, sweep, dtype):
+    """CostVolumeV3 with groups of one and two channels."""
+    near, far, rot, shift = SWEEPS[sweep]
+    N, D = (4, 19) if sweep == "mixed" else (2, 11)
+    rng, args = _tensors(C + sub, 1, N, 27, 39, C, D, near, far, rot, shift, dtype)
+    for reduce in ("MEAN", "MIN"):
+        print("\n[case] C%d sub %d %s %s" % (C, sub, sweep, reduce), flush=True)
+        cost, mask = oracle.cost_volume_v3_fwd(*args, reduce, C // sub)
+        cg = rng.standard_normal(cost.shape).astype(dtype)
+        got = chop.cost_volume_grad_v3(*[dev(x) for x in args], dev(cg), dev(mask), reduce, C // sub)
+        assert tiles.chop_last_kernel_shape() == 2
+        for g, w in zip(got, oracle.cost_volume_v3_bwd(*args, cg, mask, reduce, C // sub)):
+            assert_backward_close(host(g), w, 1e-4 if dtype == np.float32 else 1e-10)
 
 
 def test_spread_cells_views_take_turns(oracle):

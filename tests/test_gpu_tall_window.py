@@ -1,6 +1,7 @@
 """The 32-channel gradients with the eight-row window in its tall form (8 x 6 texels over tiles of 4 x 2
 pixels): five and six views, sweeps of 32 depths and more on images that give 16384 workgroups, sizes
-that no tile divides, sweeps whose samples lie far apart.  Against the oracle at the float32 bar."""
+that no tile divides, sweeps whose samples lie far apart; and one a little too small for it, which runs the
+wide form.  Against the oracle at the float32 bar."""
 import numpy as np
 import pytest
 
@@ -13,8 +14,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("op", ["v1", "aggregate_mean", "aggregate_min", "feature"])
-@pytest.mark.parametrize("N,H,W,D,near", [(5, 123, 77, 33, 0.6), (6, 75, 77, 64, 3.0)])
-def test_tall_window(oracle, op, N, H, W, D, near):
+@pytest.mark.parametrize("N,H,W,D,near,tall", [(5, 131, 99, 33, 0.6, True), (6, 75, 77, 64, 3.0, True),
+                                               (5, 123, 77, 33, 0.6, False)])
+def test_tall_window(oracle, op, N, H, W, D, near, tall):
     print("\n[case] %s N%d %dx%dx%d near %g" % (op, N, H, W, D, near), flush=True)
     f32, C = np.float32, 32
     rng = np.random.default_rng(N + D)
@@ -38,5 +40,8 @@ def test_tall_window(oracle, op, N, H, W, D, near):
     cg = rng.standard_normal(shape).astype(f32)
     got = bwd(*ins, dev(cg), mask, *extra)
     assert _lib.load().chop_last_backward_window() == 8
+    # the number of workgroups as the tall form counts them: tiles of 4 x 2 pixels, views, segments
+    units = -(-H // 4) * -(-W // 2) * N * _lib.load().chop_last_segments()
+    assert (units >= 16384) == tall
     for g, w in zip(got, want_bwd(*args, cg, host(mask), *extra)):
         assert_backward_close(host(g), w)
