@@ -742,16 +742,30 @@ StripGeom strip_geometry(const Args<S> &a, bool backward) {
   // chunk then (3 channels, two views, 12 x 16 x 9, double, 12 tiles: forward 11.3 -> 5.8 us, gradient
   // 17.2 -> 9.5 us; bf16 group correlation, four views, 16 x 17 x 28: 50 -> 9 and 76 -> 16 us; forward at
   // one wave per SIMD instead: 24 channels, three views, 38 x 43 x 25 15 against 11 us).  Every segment of
-  // a gradient adds to its pixels' sums: two depths at least and 48 segments at most (two views, 15 x 21 x
-  // 94: 41 us in five segments, 17 in 47, 30 in 94; three views, 18 x 19 x 186: 40, 21 in 47, 36 in 93), and
-  // only below one wave per SIMD (bf16, 3 channels, five views, two images of 100 x 128 x 9, 1600 strips: 87
-  // us whole, 112 in two), half a wave where there is next to nothing to cut (double, group correlation of 32
-  // channels, five views, 38 x 40 x 5, 760 strips: 31 whole, 45 in two and three).  CostAggregate in
-  // double adds its rows up chunk by chunk: no less than one (64 channels, 26 x 34 x 3: 16.5 -> 20.3 us).
+  // a gradient adds to its pixels' sums: two depths at least and a 48th of the range (two views, 15 x 21 x
+  // 94: 41 us in five segments, 17 in 47, 30 in 94; three views, 18 x 19 x 186: 40, 21 in 47, 36 in 93).
+  // Beyond a chunk the length is rounded down to chunks, so ranges from 400 depths on go in 54 to 90 segments
+  // (C 5, 15 x 21 x 720: 42 us in 90, 34 in 48; 8 x 9 x 432 in double: 19 in 54, 25 in 48).
+  // The fewer depths, the less a gradient gains by being cut, and the more waves it has without, the less:
+  // measured on 6000 launches between half a wave and two waves per SIMD.  Up to five depths half a wave
+  // (double, group correlation of 32 channels, five views, 38 x 40 x 5, 760 strips: 31 whole, 45 in two and
+  // three), up to eight one wave (three quarters in double), up to twelve 1400 waves (0.81 of the time below
+  // them, 1.02 above; bf16, 3 channels, five views, two images of 100 x 128 x 9, 1600 strips: 87 us whole,
+  // 112 in two; double 1024: 0.95 and 1.03), up to 31 depths 1700 (0.76 and 1.02; double 1400: 0.84 and 1.09),
+  // from 32 on two (0.71, double 0.80; 12 channels, five views, 50 x 55 x 36 in double: 113 us in two, 59 in
+  // five).  CostAggregate in double adds its rows up chunk by chunk: no less than one beyond 32 channels (64
+  // channels, 26 x 34 x 3: 16.5 -> 20.3 us) or half a wave per SIMD (32 channels, 2 depths 1.11; below, 3
+  // channels, five views, 16 x 21 x 5 16.4 -> 10.8 us).
   // Segments as even as their number allows: the longest is what the launch lasts (double, 64 channels,
   // 38 x 40 x 6 in 5 + 1: gradient 15 -> 20 us).
-  const bool whole_chunks = !backward && a.corr == SUM_SQUARED_DIFFERENCE && sizeof(S) == 8 && a.D <= kDB;
-  const int64_t full = !backward ? 2048 : a.D <= 5 ? 512 : 1024;
+  const bool whole_chunks = !backward && a.corr == SUM_SQUARED_DIFFERENCE && sizeof(S) == 8 && a.D <= kDB &&
+                            (a.C > 32 || g.tiles >= 512);
+  constexpr bool kDouble = sizeof(S) == 8;
+  const int64_t full = !backward || a.D >= 32 ? 2048
+                       : a.D <= 5             ? 512
+                       : a.D <= 8             ? (kDouble ? 768 : 1024)
+                       : a.D <= 12            ? (kDouble ? 1024 : 1400)
+                                              : (kDouble ? 1400 : 1700);
   if (g.tiles * ((a.D + g.seg - 1) / g.seg) < full && !whole_chunks) {
     int64_t len = (g.tiles * a.D + 2047) / 2048;
     if (backward) {

@@ -169,6 +169,14 @@ def test_strips_are_cut_where_it_pays():
     assert segments("v1", "f", 64, 5, 26, 34, 3, family=2) == 2
     assert segments("v1", "f", 3, 2, 12, 16, 9, family=2) == 9              # twelve strips: depth by depth
     assert segments("v1", "b", 3, 2, 12, 16, 9, family=2) == 5
+    assert segments("v1", "b", 12, 5, 50, 55, 36, family=2) == 5            # 688 strips, two segments anyway
+    assert segments("v2", "b", 12, 2, 59, 77, 22, groups=3, family=2) == 3  # 1136 strips
+    assert segments("v1", "b", 12, 2, 72, 90, 22, dtype="f32") == 2         # 1620 strips
+    assert segments("v1", "b", 12, 2, 72, 90, 22) == 1
+    assert segments("v1", "b", 5, 3, 100, 100, 12, dtype="f32") == 2        # 1250 strips
+    assert segments("v1", "b", 5, 3, 100, 100, 12) == 1
+    assert segments("layer", "f", 3, 5, 16, 21, 5, family=2) == 5
+    assert segments("layer", "f", 32, 5, 30, 40, 5, family=2) == 1          # 600 strips
 
 
 def test_many_taps_stay_in_one_round():
