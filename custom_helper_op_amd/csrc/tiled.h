@@ -65,6 +65,7 @@ struct Geometry {
   int64_t grid;            // workgroups to launch
   int tiles_x;             // tiles per image row (a tile: tile_rows(PPW) rows of pixels)
   int sub;                 // channels per correlation group (1 for squared difference)
+  bool stream_halves;      // forward: rows that leave as half lines (half_lines) bypass the caches
   float src_h_max, src_w_max;  // (float)(srcH - 1), (float)(srcW - 1): acceptance bounds
 };
 
@@ -358,12 +359,38 @@ __device__ __forceinline__ void fold_groups(const R *ch, int sub, R *out) {
   }
 }
 
-template <typename S, int VEC, int LPP, bool PAD>
-__device__ __forceinline__ void store_groups(S *p, const typename Storage<S>::Real *v, int sub) {
+// In double the rows of 16 channels, and those of groups of one channel, leave in two stores that touch half
+// of every line each.  Streamed, the halves reach memory on their own as partial lines, which costs up to
+// twice the time where little else goes on -- one or two views, or a row for every view: these ask the
+// launcher (Geometry::stream_halves).  With more views the rows come seldom enough and streaming stays 5 to
+// 10 % ahead of the caches.
+constexpr bool half_lines(int lpp, int nv, int corr, int elem_bytes, bool pad) {
+  return elem_bytes == 8 && !pad && lpp >= 4 &&
+         ((corr == 1 && (nv == 1 || (nv == 2 && lpp >= 8))) || (lpp == 4 && (corr == 4 || (corr == 0 && nv == 1))));
+}
+template <typename S, int CNT, bool STREAM, bool ASK, int GAP = 2>
+__device__ __forceinline__ void store_row(S *p, const typename Storage<S>::Real *v, bool stream) {
+  if constexpr (ASK) {
+    // (uniform; the two empty statements keep the compiler from making one store of the two, which
+    // would be one that does not stream)
+    if (stream) {
+      asm volatile("");
+      store_vec<S, CNT, true, GAP>(p, v);
+      asm volatile("");
+    } else {
+      store_vec<S, CNT, false, GAP>(p, v);
+    }
+  } else {
+    store_vec<S, CNT, STREAM, GAP>(p, v);
+  }
+}
+
+template <typename S, int VEC, int LPP, bool PAD, bool ASK>
+__device__ __forceinline__ void store_groups(S *p, const typename Storage<S>::Real *v, int sub, bool stream) {
   // p already points at this lane's first group; a pixel's row holds VEC * LPP / sub values
   constexpr int C = VEC * LPP, B = (int)sizeof(S);
   if (sub == 1) {
-    store_vec<S, VEC, !PAD && whole_lines(C, B)>(p, v);
+    store_row<S, VEC, !PAD && whole_lines(C, B), ASK>(p, v, stream);
   } else if (sub == 2) {
     store_vec<S, VEC / 2, !PAD && whole_lines(C / 2, B)>(p, v);
   } else if (sub == 4) {
@@ -1018,6 +1045,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   // the cost rows of the per-channel ops (and the sample rows of the warp-only op) stream past
   // the caches where they cover whole lines
   constexpr bool kNtRows = !PAD && whole_lines(VEC * LPP, (int)sizeof(S));
+  constexpr bool kAsk = half_lines(LPP, NV, CORR, (int)sizeof(S), PAD);
+  const bool stream_halves = kAsk && g.stream_halves;
   // one value per voxel that is added up in channel order
   constexpr bool kRowSums = CORR == 2 && (REDUCE == 1 || LIT);
   const int d_lo = t.d_lo, d_hi = t.d_hi;
@@ -1196,7 +1225,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               smp[c] = wt.x * tap[0][0][c] + wt.y * tap[0][1][c] + wt.z * tap[0][2][c] + wt.w * tap[0][3][c];
           }
           if (t.pix_ok && ch_ok)
-            store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d0 + jj) * N + n) * C + ch0, smp);
+            store_row<S, VEC, kNtRows, kAsk, GAP>(a.cost + ((t.pix * D + d0 + jj) * N + n) * C + ch0, smp, stream_halves);
         }
       }
       if constexpr (LPP > 1) wave_sync();
@@ -1313,10 +1342,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               if (arg[jj][c] < 0) acc[jj][c] = dflt;
           }
           if (CORR == 0) {
-            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc[jj]);
+            store_row<S, VEC, kNtRows, kAsk, GAP>(out + ch0, acc[jj], stream_halves);
             store_winners<VEC, LPP, GAP, PAD>(mout + ch0, arg[jj]);
           } else {
-            store_groups<S, VEC, LPP, PAD>(out + goff, acc[jj], g.sub);
+            store_groups<S, VEC, LPP, PAD, kAsk>(out + goff, acc[jj], g.sub, stream_halves);
             if (g.sub == 1) store_ints<VEC, !PAD && whole_lines(VEC * LPP, 4)>(mout + goff, arg[jj]);
             else if (g.sub == 2) store_ints<VEC / 2, !PAD && whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg[jj]);
             else if (g.sub == 4 || (t.cl & 1)) store_ints<1, !PAD && whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg[jj]);
@@ -1328,7 +1357,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
               for (int c = 0; c < VEC; ++c) acc[jj][c] = dflt;
             }
-            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc[jj]);
+            store_row<S, VEC, kNtRows, kAsk, GAP>(out + ch0, acc[jj], stream_halves);
           } else {
             R grp[VEC];
             fold_or_keep<LIT>(acc[jj], g.sub, grp);
@@ -1336,7 +1365,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
               for (int c = 0; c < VEC; ++c) grp[c] = dflt;
             }
-            store_groups<S, VEC, LPP, PAD>(out + goff, grp, g.sub);
+            store_groups<S, VEC, LPP, PAD, kAsk>(out + goff, grp, g.sub, stream_halves);
           }
         }
       }
@@ -1431,7 +1460,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
                        wt.w * tap[n][3][c];
           }
           if (n < N && t.pix_ok && ch_ok)
-            store_vec<S, VEC, kNtRows, GAP>(a.cost + ((t.pix * D + d) * N + n) * C + ch0, smp);
+            store_row<S, VEC, kNtRows, kAsk, GAP>(a.cost + ((t.pix * D + d) * N + n) * C + ch0, smp, stream_halves);
           continue;
         }
         if (off >= 0) {
@@ -1516,10 +1545,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           S *out = out_pix + d * OC;  // d * OC is uniform: one add per lane
           int32_t *mout = mask_pix + d * OC;
           if (CORR == 0) {
-            store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc);
+            store_row<S, VEC, kNtRows, kAsk, GAP>(out + ch0, acc, stream_halves);
             store_winners<VEC, LPP, GAP, PAD>(mout + ch0, arg);
           } else {
-            store_groups<S, VEC, LPP, PAD>(out + goff, acc, g.sub);
+            store_groups<S, VEC, LPP, PAD, kAsk>(out + goff, acc, g.sub, stream_halves);
             if (g.sub == 1) store_ints<VEC, !PAD && whole_lines(VEC * LPP, 4)>(mout + goff, arg);
             else if (g.sub == 2) store_ints<VEC / 2, !PAD && whole_lines(VEC * LPP / 2, 4)>(mout + goff, arg);
             else if (g.sub == 4 || (t.cl & 1)) store_ints<1, !PAD && whole_lines(VEC * LPP / 4, 4)>(mout + goff, arg);
@@ -1548,7 +1577,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
             for (int c = 0; c < VEC; ++c) acc[c] = dflt;
           }
-          store_vec<S, VEC, kNtRows, GAP>(out + ch0, acc);
+          store_row<S, VEC, kNtRows, kAsk, GAP>(out + ch0, acc, stream_halves);
         } else {
           R grp[VEC];
           fold_or_keep<LIT>(acc, g.sub, grp);
@@ -1556,7 +1585,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
             for (int c = 0; c < VEC; ++c) grp[c] = dflt;
           }
-          store_groups<S, VEC, LPP, PAD>(out + goff, grp, g.sub);
+          store_groups<S, VEC, LPP, PAD, kAsk>(out + goff, grp, g.sub, stream_halves);
         }
       }
     }
@@ -2906,6 +2935,7 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
            : by_segment ? g.units_per_xcd * 8 * g.nseg
                         : g.units_per_xcd * 8;
   g.sub = sub;
+  g.stream_halves = false;
   g.src_h_max = g.src_w_max = 0.f;  // set by the launcher from the source image size
   return g;
 }

@@ -193,3 +193,24 @@ def test_difference_of_a_finished_sample(oracle, op, C, reduce):
         assert np.array_equal(got[0], want[0])
     else:
         np.testing.assert_allclose(got[0], want[0], rtol=3e-16)
+
+
+@pytest.mark.parametrize("op,C,N,sub", [("v1", 16, 1, 1), ("v2", 16, 1, 1), ("v2", 32, 2, 1), ("v2", 64, 1, 1),
+                                        ("feature", 16, 3, 1)])
+@pytest.mark.parametrize("H,W", [(32, 41), (256, 257)])
+def test_rows_of_half_lines(op, C, N, sub, H, W):
+    """Rows that leave in two stores of half a line each, through the caches (small launches) and past them
+    (65536 pixels and more): the bits of the lane-per-channel kernels."""
+    t = reference_test_case(3, 1, N, H, W, C, 3, np.float64, seed=C + N)
+    for reduce in ("MEAN",) if op == "feature" else ("MEAN", "MIN"):
+        if op == "v2":
+            grid = (t["base_plane"] + t["offsets"][:, None, None, :]).astype(np.float64)
+            ins = [dev(x) for x in (t["ref"], t["src"], grid, t["Rs"], t["Ts"])]
+            run = lambda: chop.cost_volume_v2_raw(*ins, reduce, C // sub)
+        else:
+            ins = [dev(t[k]) for k in ("ref", "src", "base_plane", "offsets", "Rs", "Ts")]
+            run = (lambda: chop.cost_volume_raw(*ins, reduce)) if op == "v1" else (
+                lambda: chop.feature_aggregate_raw(*ins[1:]))
+        tiles, lanes = _both(run)
+        for g, w in zip(tiles, lanes):
+            assert np.array_equal(g, w)
