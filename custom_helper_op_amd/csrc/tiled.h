@@ -2861,7 +2861,8 @@ inline int choose_segments(int64_t tiles, int64_t D, int lpp, int64_t target_uni
 
 template <int LPP>
 inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int sub, int ngroups = 1,
-                              int vper = 0, bool tall = false, bool row_sums = false, bool many_taps = false) {
+                              int vper = 0, bool tall = false, bool row_sums = false, bool many_taps = false,
+                              bool open_lines = false) {
   constexpr int PPW = 64 / LPP;
   Geometry g;
   g.hw = (int)(H * W);
@@ -2887,7 +2888,8 @@ inline Geometry make_geometry(int64_t B, int64_t H, int64_t W, int64_t D, int su
   // of more than 2048 waves goes in two rounds; one that has a wave for every SIMD is left as it is (minimum
   // of CostAggregate, 8 channels, six views, 135 x 181 x 24, 782 tiles: 2 segments 37 us, 3 segments 43;
   // samples of six views, 32 channels, 44 x 62 x 107, 352 tiles: 5 segments 52 us, 7 58).
-  if (vper == 0 && tiles * g.nseg < (many_taps ? 1024 : 2048)) {
+  // open_lines (see the launcher): not cut at all.
+  if (vper == 0 && !open_lines && tiles * g.nseg < (many_taps ? 1024 : 2048)) {
     const int64_t chunks = (D + LPP - 1) / LPP, want = many_taps ? 2048 / tiles : (2048 + tiles - 1) / tiles;
     g.nseg = (int)(want < chunks ? want : chunks);
   }

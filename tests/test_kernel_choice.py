@@ -191,6 +191,19 @@ def test_many_taps_stay_in_one_round():
     assert segments("feat", "f", 32, 6, 8, 12, 33, dtype="f32") == -5       # twelve tiles: single chunks
 
 
+def test_launches_of_narrow_pixels_are_not_cut_past_the_caches():
+    """Pieces of lines: more waves side by side keep more lines open than the caches hold."""
+    f32 = dict(dtype="f32")
+    assert segments("feat", "f", 4, 4, 314, 375, 19, **f32) == 1
+    assert segments("feat", "f", 4, 4, 314, 375, 3, **f32) == 2             # 23 MB
+    assert segments("feat", "f", 4, 1, 160, 208, 57, **f32) == 2
+    assert segments("feat", "f", 4, 1, 236, 263, 33, **f32) == 3            # a wave to every SIMD
+    assert segments("v1", "f", 4, 3, 120, 160, 100, **f32) == 4
+    assert segments("v1", "f", 4, 3, 120, 160, 57, **f32) == 7
+    assert segments("feat", "f", 8, 4, 236, 263, 19, **f32) == 1
+    assert segments("feat", "f", 8, 4, 160, 208, 19, **f32) == 2
+
+
 def test_uneven_segments_go_one_after_the_other():
     """Side by side a short last segment leaves every other compute unit idle; segments about as long as each
     other stay side by side, and so do narrow pixels with one value per voxel."""
