@@ -120,9 +120,58 @@ bool lanes_are_faster_correlation(const Args<S> &a) {
   }
 }
 
+// Gradients of CostVolumeV3's minimum.  One source group and one reference group of one view receive the
+// voxel's gradient, and the mask names them: nothing is searched for, and next to nothing is added up.  The
+// tiles' workgroup of each view still walks every voxel with all of a pixel's lanes and clears and writes
+// back its window; their work grows with the views times the channels, that of the others hardly.  Groups of
+// four and eight channels in float run the tiles at any size.
+//   More than 16 groups: a thread per voxel.  Its time is that of a few additions to memory, so the line is a
+//   number of depths per view.  Float, 200 x 260 unless another size is given: 32 channels in groups of one,
+//   two views, 8 depths 113 : 138, 12 depths 147 : 158, 32 depths 350 : 265; four views, 12 depths 144 : 215;
+//   one view 4 depths 46 : 48, 12 depths 116 : 79.  64 channels in groups of one, two views, 8 depths 119 :
+//   223, 32 depths 375 : 455; one view, 32 depths 316 : 287.  64 channels in groups of two, four views, 8
+//   depths 210 : 340; two views 211 : 224, one view, 4 depths 91 : 81.  Few tiles, 20 x 24: 32 channels, two
+//   views, 12 depths 8 : 18, 32 depths 13 : 18.  Double: the tiles take twice the time and more.  64
+//   channels in groups of one, four views, 8 depths 124 : 638; in groups of two 217 : 644; 32 channels, two
+//   views, 8 depths 103 : 208, 32 depths 330 : 484, 120 x 160 x 96 353 : 375.
+//   Up to 16 groups: a lane per channel.  It has no window to clear.  One view of 8 channels, 60 x 80 x 12 13 :
+//   15, x 32 24 : 16.  32 channels in groups of two, float: four views, 4 depths 70 : 95, 12 depths even; two
+//   views, 383 x 534 x 4 0.87 of the tiles' time; 20 x 24 x 12 10 : 14.  Double: four views, 8 depths 266 :
+//   326, two views, 8 depths 239 : 208 (four views' texel cache is the largest that the strips hold).  64
+//   channels in groups of four and eight, double: four views, 60 x 80 x 12 56 : 72, 200 x 260 x 4 296 : 515,
+//   60 x 80 x 96 293 : 239; six views, 4 depths 504 : 612, 120 x 160 x 12 353 : 319; one view 4 depths 1.26 of
+//   the tiles' time.  16 channels, float, four views, 383 x 534: 4 depths 0.76 of the tiles' time, 12 depths
+//   1.09; double: tiles.
+template <typename S>
+bool lanes_are_faster_best_pair(const Args<S> &a) {
+  const bool wide = sizeof(S) == 8;
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64, sub = a.C / a.groups;
+  if (a.reduce == 0 || (!wide && sub >= 4)) return false;
+  if (a.groups > 16) {
+    if ((tiles < 1024 && a.D <= 12) || (tiles < 256 && a.D <= (wide ? 160 : sub == 1 ? 64 : 32))) return true;
+    if (wide) return a.groups == 64 || a.D < (sub == 1 ? 64 * a.N - 32 : 32 * a.N - 12);
+    return sub == 1 ? a.D <= (lpp == 16 ? 16 : 6) * a.N : a.N > 1 && a.D <= 5 * a.N;
+  }
+  switch (lpp) {
+    case 2:
+      return (a.N == 1 && tiles < 256 && a.D <= 16) ||
+             (wide && a.N > 1 && a.N <= 4 && a.D <= (tiles >= 4096 ? 7 : 3) && tiles >= 1024);
+    case 4:
+      if (wide) return a.N > 1 && a.D == 1 && tiles >= 2048;
+      return (a.N == 1 && tiles < 64 && a.D <= 16) || (a.N > 1 && tiles >= 8192 && a.D <= 6);
+    case 8:
+      if (tiles < 128) return a.D >= 8 && a.D <= 16 && a.N <= 4;
+      if (!wide) return a.N > 1 && a.D <= 6 && tiles >= (a.N >= 4 ? 768 : 2048);
+      if (a.N == 2 || a.N == 3) return a.D <= 2 && tiles >= 4096;
+      return a.N >= 4 && ((a.D <= 4 && tiles >= 512) || (a.N == 4 && a.D <= 12 && tiles >= 1024));
+    default: return a.N > 4 ? a.D <= 6 && tiles >= 1024 : a.N > 2 ? a.D <= 32 : a.N > 1 && a.D <= 24;
+  }
+}
+
 template <typename S>
 bool lanes_are_faster(const Args<S> &a, bool backward) {
   if (!backward) return lanes_are_faster_forward(a);
+  if (a.corr == BEST_GROUP_PAIR) return lanes_are_faster_best_pair(a);
   if (sizeof(S) != 8) return false;
   return lanes_are_faster_few_tiles(a) || (a.corr == GROUP_CORRELATION && lanes_are_faster_correlation(a));
 }

@@ -148,6 +148,32 @@ def test_correlation_gradients_of_few_depths():
             ("v2", 8, 1, 200, 260, 8), ("v2", 4, 3, 200, 260, 1), ("v2", 4, 6, 60, 80, 8), ("v2", 4, 2, 200, 260, 13)]])
 
 
+def test_gradients_of_the_best_pair_by_winner():
+    """CostVolumeV3's minimum: one pair of groups of one view receives the voxel's gradient, while the tiles walk
+    every view with all of a pixel's lanes.  More than 16 groups: a thread per voxel, otherwise a lane per
+    channel."""
+    f32 = dict(dtype="f32")
+    for want, calls in (
+            (GENERAL, [(32, 1, 2, 200, 260, 12, f32), (32, 1, 2, 20, 24, 32, f32), (64, 1, 2, 383, 534, 27, f32),
+                       (64, 2, 4, 200, 260, 8, f32), (32, 1, 2, 200, 260, 32), (64, 1, 4, 200, 260, 8),
+                       (64, 1, 1, 60, 80, 96), (64, 2, 2, 60, 80, 32)]),
+            (LANES, [(8, 1, 1, 60, 80, 12, f32), (32, 2, 2, 20, 24, 12, f32), (32, 2, 4, 200, 260, 4, f32),
+                     (16, 2, 3, 383, 534, 4, f32), (32, 4, 4, 200, 260, 8), (64, 8, 4, 60, 80, 12),
+                     (64, 4, 2, 200, 260, 4), (64, 4, 6, 200, 260, 4)]),
+            (TILES, [(32, 1, 2, 200, 260, 32, f32), (32, 1, 1, 200, 260, 12, f32), (64, 1, 1, 200, 260, 32, f32),
+                     (64, 2, 1, 200, 260, 4, f32), (64, 2, 2, 200, 260, 32, f32), (64, 4, 4, 200, 260, 4, f32),
+                     (8, 1, 1, 60, 80, 32, f32), (8, 1, 2, 60, 80, 4, f32), (16, 2, 3, 200, 260, 12, f32),
+                     (32, 1, 2, 120, 160, 96), (16, 1, 4, 200, 260, 4), (32, 4, 2, 200, 260, 4),
+                     (64, 8, 1, 200, 260, 4), (64, 8, 6, 120, 160, 12), (64, 4, 2, 60, 80, 96)])):
+        for C, sub, N, H, W, D, *kw in calls:
+            kw = dict(reduce="MIN", groups=C // sub, **(kw[0] if kw else {}))
+            assert ran("v3", "b", C, N, H, W, D, **kw) == want, (C, sub, N, H, W, D, kw)
+            kw["reduce"] = "MEAN"
+            if D > 8 or "dtype" in kw:
+                assert ran("v3", "b", C, N, H, W, D, **kw) == TILES
+            assert ran("v3", "f", C, N, H, W, D, **dict(kw, reduce="MIN")) == TILES
+
+
 def segments(*args, **kw):
     """Depth segments of the call; negative: all tiles' first segments before all second ones."""
     ran(*args, **kw)
