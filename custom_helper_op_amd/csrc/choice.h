@@ -42,6 +42,9 @@ bool lanes_are_faster_forward(const Args<S> &a) {
            ((a.corr == GROUP_CORRELATION && waves >= 32768) ||
             (a.corr == SQUARED_DIFFERENCE && waves >= 65536));
   }
+  // (one view's minimum of 28 channels likewise, 160 x 200: 96 depths 0.83 of the tiles' time, 32 depths 1.06)
+  if (sizeof(S) == 8 && idle_lanes && a.corr == SQUARED_DIFFERENCE && a.reduce != 0 && a.N == 1 && waves >= 40960)
+    return true;
   // Two waves of the squared differences' minimum of many views fit a SIMD: a little over 2048 tiles leave a
   // second round nearly empty, until the depths can be cut to fill it (five views, 32 channels, 2400 tiles:
   // 12 depths 64.5 : 72.4, 24 depths 101 : 115, 48 depths 189 : 172; 3250 tiles, 12 depths 83.4 : 73.8).
@@ -56,7 +59,7 @@ bool lanes_are_faster_forward(const Args<S> &a) {
     line = a.N == 1 ? 0 : a.N == 2 ? 192 : 384;
   else
     line = a.N == 1 ? 192 : a.N == 2 || samples ? 384 : 768;
-  return waves < line && (one_value ? 2 * a.D >= lpp : a.D >= 4 || a.N >= 3);
+  return waves < line && (one_value ? 2 * a.D >= lpp : a.D >= 4 || (a.N >= 3 && a.D == 3 && !samples));
 }
 
 // Gradients in double of one view, or of two, in launches that leave most of the chip idle.  With so few
@@ -73,51 +76,105 @@ bool lanes_are_faster_forward(const Args<S> &a) {
 template <typename S>
 bool lanes_are_faster_few_tiles(const Args<S> &a) {
   const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64, steps = tiles * a.D;
-  if (a.corr == BEST_GROUP_PAIR || a.N > 2 || a.D < 3 || tiles >= 512) return false;
+  if (a.corr == BEST_GROUP_PAIR || a.N > 2 || tiles >= 512) return false;
+  if (a.D < 3) return a.corr == SUM_SQUARED_DIFFERENCE && a.N == 1 && lpp == 2;
+  const bool correlation = a.corr == GROUP_CORRELATION;
   if (a.N == 2)
-    return lpp == 1    ? steps < 1024 && a.D < 16 && (a.D > 3 || tiles >= 128)
+    return lpp == 1    ? steps < (correlation && a.reduce == 0 ? 256 : 1024) && a.D < 16 && (a.D > 3 || tiles >= 128)
            : lpp == 16 ? steps < 3072
                        : false;
-  const bool correlation = a.corr == GROUP_CORRELATION;
-  return lpp <= 2    ? steps < (a.corr == SUM_SQUARED_DIFFERENCE ? 2048 : 1024)
+  return lpp <= 2    ? steps < (a.corr == SUM_SQUARED_DIFFERENCE ? 2048 : correlation && a.reduce != 0 ? 2560 : 1024)
          : lpp == 8  ? steps < 2560 && !correlation
          : lpp == 16 ? steps < 8192 && !(correlation && a.reduce != 0)
                      : false;
 }
 
-// Gradients of group correlation in double over a few depths.  A workgroup clears its window and writes it
+// Gradients of group correlation in double.  Over a few depths: a workgroup clears its window and writes it
 // back once for two depths as for a whole chunk, and the minimum passes over every view's voxels to find its
-// own.  200 x 260 unless another size is given; the strips' time goes up with the depths, the tiles' hardly.
+// own, of which wider groups have fewer.  Groups of four channels, 200 x 260 and planes
+// from depth 2 on unless something else is given; the strips' time goes up with the depths and the number of groups, the tiles' hardly.
 //   Mean   64 channels, two views: 2 depths 261 : 343, 3 depths 370 : 423, 4 depths 487 : 461; four views:
-//          3 depths 736 : 853, 4 depths 955 : 910.  32 channels, four views: 2 depths 281 : 319, 3 depths 401
-//          : 371.  16 channels, four views: 3 depths 157 : 182, 4 depths 189 : 193, and with 1200 tiles (120
-//          x 160) 71 : 65.
+//          3 depths 736 : 853, 4 depths 955 : 910, 38 x 45 x 1 23 : 30.  32 channels, four views: 2 depths 281 :
+//          319, 3 depths 401 : 371.  16 channels, four views: 3 depths 157 : 182, 4 depths 189 : 193, and with
+//          1200 tiles (120 x 160) 71 : 65.
+//          4 channels, whose window is one texel column to a lane: long sweeps, from 0.7 of the tiles' time
+//          (planes from depth 5 on, 96 depths, four views) to 0.9 (planes from 0.7); 32 depths 0.85 and 1.56.
 //   Minimum at 64 channels, two views and more: at any depth, as a wave holds four pixels.  Two views: 4
 //          depths 248 : 437, 12 depths 585 : 718; four views, 12 depths 1003 : 1464, 32 depths 1833 : 2454.
 //          One view has nothing to pass over: 4 depths 223 : 187.
-//   Minimum at 32 channels from four views on, eight rows to a window: 4 depths 246 : 346, 8 depths 415 :
-//          432, 12 depths 567 : 538; 60 x 80 x 6 41 : 51.  Three views: 4 depths 253 : 274, 6 depths 312 : 318,
-//          60 x 80 x 4 41 : 37.
+//   Minimum at 32 channels, four views: groups of one and two, 2 depths 0.81 and 0.74 of the tiles' time, 4
+//          depths 1.21 and 1.02; of four, 4 depths 246 : 346, 8 depths 415 : 432; of eight, 6 depths 0.80, 8 depths
+//          0.92.  Six views: 2 depths 0.78, 60 x 80 x 4 1.06; groups of eight, 200 x 260 x 6 0.96.  Three views:
+//          4 depths 253 : 274, 6 depths 312 : 318, 60 x 80 x 4 41 : 37.
 //   Minimum at 16 channels: two views 3 depths 96 : 104, 4 depths 112 : 110; four views 153 : 186, 179 : 192.
-//   Minimum at 8 channels, four views: 8 depths 132 : 139, 12 depths 191 : 177; 120 x 160 x 8 57 : 65; 60 x 80
-//          x 4 26 : 22.  Six views: 188 : 199, but 120 x 160 x 8 88 : 77.  Two views: 60 x 80 x 12 20.6 : 22.9,
-//          one depth 33.8 : 34.1.  One view: 120 x 160 x 8 21.4 : 24.8, 200 x 260 x 8 44.8 : 40.2.
-//   Minimum at 4 channels, three views: 8 depths 76 : 121, 12 depths 113 : 148, one depth 31.7 : 29.3; four
-//          views, 60 x 80 x 8 25.5 : 22.9, 120 x 160 x 8 44 : 51.
+//   Minimum at 8 channels: groups of one and two, four views, 8 depths 1.2 and 1.0 of the tiles' time, planes
+//          from 5 on and 330 x 400 1.56 and 1.25; of four 132 : 139, 12 depths 191 : 177; 120 x 160 x 8 57 :
+//          65; 60 x 80 x 4 26 : 22; of eight, 8 depths 0.61 to 0.85, 16 depths 0.77 to 0.97.  Six views, groups
+//          of four: 188 : 199, but 120 x 160 x 8 88 : 77.  Two views, any groups: 60 x 80 x 12 20.6 : 22.9, x 16
+//          0.9, 120 x 160 x 8 0.9.  One view: 120 x 160 x 8 21.4 : 24.8, x 16 0.9, 200 x 260 x 8 44.8 : 40.2.
+//   Minimum at 4 channels: three views, 8 depths 76 : 121, 12 depths 113 : 148; 32 depths, two views, groups of
+//          one 0.75 to 1.15, of two 0.72 to 1.06, of four 0.70 to 0.91 of the tiles' time; 96 depths 0.6 to 0.75
+//          with any; 16 depths, groups of four, two views and more 0.76 to 0.99.  One view, 8 depths, 120 x
+//          160 0.76 and 0.94, 330 x 400 0.91 and 1.68.  Four views, 60 x 80 x 8 25.5 : 22.9, 120 x 160 x 8 44 : 51.
 template <typename S>
 bool lanes_are_faster_correlation(const Args<S> &a) {
-  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64;
-  if (a.reduce == 0)
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64, sub = a.C / a.groups;
+  if (a.reduce == 0) {
+    if (lpp == 1) return a.D >= 64 && tiles >= 256;
+    if (lpp == 16 && a.N > 1 && a.D <= 2) return tiles >= 256;
     return a.N > 1 && lpp >= 4 && a.D < (lpp == 8 ? 3 : 4) && tiles >= (lpp == 16 ? 1024 : 2048);
+  }
   switch (lpp) {
     case 16: return a.N > 1;
-    case 8: return a.N >= 4 ? a.D <= 8 : a.N > 1 && a.D <= 4 && tiles >= 2048;
+    case 8:
+      if (a.N >= 4 && a.D <= 2) return tiles >= 256;
+      if (a.N == 4) return a.D <= (sub == 1 ? 2 : sub == 2 ? 4 : 8) && tiles >= 256;
+      if (a.N > 4) return sub > 1 && a.D <= 2 + (sub < 8 ? sub : 6) && tiles >= 2048;
+      return a.N > 1 && a.D <= 4 && tiles >= 2048;
     case 4: return a.N > 1 && a.D <= 3 && tiles >= 2048;
     case 2:
-      return a.D <= (a.N <= 2 && tiles < 256 ? 12 : 8) && (a.D > 1 || a.N > 2) &&
-             (a.N == 1 ? tiles < 1024 : tiles >= 256 * (a.N - 2));
-    default: return a.D > 1 && a.D <= 12 && tiles >= 64 * (a.N - 2);
+      if (a.N <= 2 && tiles < 1024) return a.D <= (tiles < 256 ? 16 : 8) && a.D > (a.N == 1 || tiles >= 256 ? 1 : 3);
+      if (a.N == 1 || sub < 4) return false;
+      return a.D <= (sub == 8 && a.N <= 4 && tiles >= 1024 ? 16 : 8) && tiles >= 256 * (a.N - 2);
+    default:
+      if (a.D >= 64) return tiles >= 256;
+      if (a.D > 12) return tiles >= 256 && (a.D >= 24 ? sub > 1 || a.N == 1 : a.N > 1 && (sub == 4 || (sub == 2 && a.N >= 4)));
+      if (a.D <= 1 || tiles < 64 * (a.N - 2)) return false;
+      return a.N == 1 ? tiles < 512 : a.D > 2 && (sub == 4 || (sub == 2 && a.D <= 8));
   }
+}
+
+// Gradients in double over one to eight depths of the ops without groups, and of CostVolumeV3 (see above: the
+// window's cost is that of a chunk).  At 64 channels a workgroup has four pixels to share its window, with
+// idle lanes eight of fewer channels.  As a part of the tiles' time, 200 x 260 unless another size is given:
+//   Squared differences, 64 channels, two and four views: one depth 0.79 and 0.77, two depths 1.01 and 0.99;
+//   minimum 0.70 and 0.63, two depths 0.84 and 0.75, three 1.03.  24 channels, two views: 0.75, two depths
+//   0.84, three 0.99, but 60 x 80 x 2 1.09.  32 channels and fewer: even at one depth.
+//   CostAggregate's mean: the same.  Its minimum passes over every view's voxels: 64 channels, two views, two
+//   depths 0.79, four 1.00; three views, four 0.88, eight 1.15; four views, eight 0.91, 60 x 80 x 8 0.93,
+//   twelve 1.02; 24 channels, four views, four 0.77, eight 0.94; three views four 0.94 (120 x 160 1.05); 32
+//   channels, four views only, four 0.89; 8 channels, two to four views, two depths 0.79 to 0.87.
+//   CostVolumeV3's mean, up to 16 groups: 64 channels, groups of eight, two views, eight depths 0.79, three
+//   views 0.92, four views, four depths 0.93; of four, two views, four depths 0.82, three views 0.92, four
+//   views, two depths 0.92; 32 channels, two and four views, one depth 0.80 and 0.74, two 0.92 and 0.98; 16
+//   channels, one depth 0.82 and 0.71, two 0.98 and 0.93.
+template <typename S>
+bool lanes_are_faster_few_depths(const Args<S> &a) {
+  const int64_t lpp = lanes_of_a_pixel(a), tiles = a.pixels() * lpp / 64;
+  const bool idle_lanes = a.C > 16 && a.C < 32, low = a.reduce != 0, one_value = a.corr == SUM_SQUARED_DIFFERENCE;
+  if (a.N < 2 || a.D > 8 || tiles < 512) return false;
+  if (a.corr == BEST_GROUP_PAIR) {
+    if (a.groups > 16 || a.N > 4 || low) return false;
+    if (lpp == 16) return tiles >= 4096 && a.D * a.N <= (a.C == 8 * a.groups ? 16 : 8);
+    return (lpp == 8 && a.D <= 2 && tiles >= 4096) || (lpp == 4 && a.D == 1 && tiles >= 2048);
+  }
+  if (a.corr != SQUARED_DIFFERENCE && !one_value) return false;
+  if (one_value && low) {
+    if (lpp == 16) return a.D <= (a.N == 2 ? 2 : a.N == 3 ? 5 : 8);
+    if (idle_lanes) return a.D <= (a.N <= 3 ? 3 : 5) && tiles >= 2048;
+    return a.N <= 4 && ((lpp == 8 && a.N == 4 && a.D <= 4 && tiles >= 2048) || (lpp == 2 && a.D <= 2 && tiles >= 1024));
+  }
+  return lpp == 16 ? a.D <= (low ? 2 : 1) : idle_lanes && a.D <= 2 && tiles >= 2048;
 }
 
 // Gradients of CostVolumeV3's minimum.  One source group and one reference group of one view receive the
@@ -171,9 +228,10 @@ bool lanes_are_faster_best_pair(const Args<S> &a) {
 template <typename S>
 bool lanes_are_faster(const Args<S> &a, bool backward) {
   if (!backward) return lanes_are_faster_forward(a);
-  if (a.corr == BEST_GROUP_PAIR) return lanes_are_faster_best_pair(a);
+  if (a.corr == BEST_GROUP_PAIR && lanes_are_faster_best_pair(a)) return true;
   if (sizeof(S) != 8) return false;
-  return lanes_are_faster_few_tiles(a) || (a.corr == GROUP_CORRELATION && lanes_are_faster_correlation(a));
+  return lanes_are_faster_few_tiles(a) || lanes_are_faster_few_depths(a) ||
+         (a.corr == GROUP_CORRELATION && lanes_are_faster_correlation(a));
 }
 
 }  // namespace chop

@@ -145,7 +145,7 @@ def test_correlation_gradients_of_few_depths():
           [(op, C, N, H, W, D, low) for op, C, N, H, W, D in
            [("v2", 64, 1, 200, 260, 4), ("v2", 32, 4, 200, 260, 9), ("v2", 32, 3, 60, 80, 4), ("v2", 32, 3, 200, 260, 5),
             ("v2", 16, 3, 120, 160, 3), ("v2", 16, 3, 200, 260, 4), ("v2", 8, 6, 120, 160, 8), ("v2", 8, 2, 120, 160, 9),
-            ("v2", 8, 1, 200, 260, 8), ("v2", 4, 3, 200, 260, 1), ("v2", 4, 6, 60, 80, 8), ("v2", 4, 2, 200, 260, 13)]])
+            ("v2", 8, 1, 200, 260, 8), ("v2", 4, 3, 200, 260, 1), ("v2", 4, 6, 60, 80, 8), ("v2", 4, 1, 200, 260, 13)]])
 
 
 def test_gradients_of_the_best_pair_by_winner():
@@ -172,6 +172,38 @@ def test_gradients_of_the_best_pair_by_winner():
             if D > 8 or "dtype" in kw:
                 assert ran("v3", "b", C, N, H, W, D, **kw) == TILES
             assert ran("v3", "f", C, N, H, W, D, **dict(kw, reduce="MIN")) == TILES
+
+
+def test_gradients_of_few_depths():
+    """Double: a window costs the same for one depth as for a chunk, and the minimum of CostAggregate passes over
+    every view's voxels."""
+    low = dict(reduce="MIN")
+    sides("b",
+          [("v1", 64, 2, 200, 260, 1), ("v1", 64, 4, 60, 80, 2, low), ("v1", 28, 6, 200, 260, 2), ("layer", 64, 4, 200, 260, 1),
+           ("layer", 64, 6, 120, 160, 8, low), ("layer", 64, 3, 60, 80, 4, low), ("layer", 24, 4, 200, 260, 4, low),
+           ("layer", 20, 2, 200, 260, 2), ("layer", 32, 4, 200, 260, 4, low), ("layer", 8, 3, 200, 260, 2, low),
+           ("layer", 8, 1, 38, 40, 1), ("v3", 64, 2, 200, 260, 8, dict(groups=8)), ("v3", 64, 4, 200, 260, 2),
+           ("v3", 32, 2, 200, 260, 2), ("v3", 16, 4, 200, 260, 1), ("v3", 16, 4, 200, 260, 1, low)],
+          [("v1", 64, 2, 200, 260, 2), ("v1", 64, 4, 200, 260, 3, low), ("v1", 28, 6, 60, 80, 2), ("v1", 32, 4, 200, 260, 1),
+           ("v1", 64, 1, 200, 260, 1), ("layer", 64, 4, 200, 260, 9, low), ("layer", 64, 2, 200, 260, 4, low),
+           ("layer", 24, 4, 60, 80, 4, low), ("layer", 32, 3, 200, 260, 4, low), ("layer", 8, 4, 60, 80, 2, low),
+           ("feat", 64, 4, 200, 260, 1), ("v3", 64, 2, 200, 260, 9, dict(groups=8)), ("v3", 64, 2, 60, 80, 4),
+           ("v3", 32, 2, 200, 260, 3), ("v3", 64, 4, 200, 260, 2, dict(dtype="f32")),
+           ("layer", 64, 4, 200, 260, 4, dict(reduce="MIN", dtype="f32"))])
+
+
+def test_correlation_gradients_by_group_width():
+    """Double, minimum: the strips' time goes up with the number of groups.  Four channels: long sweeps too."""
+    call = lambda C, sub, N, H, W, D, **kw: ("v2", C, N, H, W, D, dict(dict(reduce="MIN"), groups=C // sub, **kw))
+    sides("b",
+          [call(32, 8, 4, 200, 260, 8), call(32, 1, 4, 200, 260, 2), call(32, 2, 6, 60, 80, 2), call(8, 8, 4, 200, 260, 16),
+           call(8, 4, 2, 330, 400, 8), call(8, 1, 2, 120, 160, 8), call(4, 4, 2, 120, 160, 16),
+           call(4, 1, 4, 120, 160, 96), call(4, 2, 4, 330, 400, 32), call(4, 4, 3, 200, 260, 8),
+           call(4, 1, 1, 60, 80, 16), call(4, 4, 2, 120, 160, 96, reduce="MEAN"), call(64, 4, 4, 38, 45, 1, reduce="MEAN")],
+          [call(32, 1, 4, 200, 260, 8), call(32, 2, 4, 120, 160, 6), call(32, 1, 6, 60, 80, 8), call(8, 1, 4, 200, 260, 8),
+           call(8, 2, 2, 330, 400, 8), call(8, 8, 1, 200, 260, 16), call(8, 4, 6, 120, 160, 8), call(4, 1, 2, 120, 160, 16),
+           call(4, 1, 4, 200, 260, 8), call(4, 1, 1, 330, 400, 8), call(4, 4, 4, 60, 80, 96), call(4, 1, 2, 60, 80, 8, reduce="MEAN"),
+           call(4, 4, 2, 120, 160, 32, reduce="MEAN")])
 
 
 def segments(*args, **kw):
