@@ -185,7 +185,8 @@ bool lanes_are_faster_few_depths(const Args<S> &a) {
 //   More than 16 groups: a thread per voxel.  Its time is that of a few additions to memory, so the line is a
 //   number of depths per view.  Float, 200 x 260 unless another size is given: 32 channels in groups of one,
 //   two views, 8 depths 113 : 138, 12 depths 147 : 158, 32 depths 350 : 265; four views, 12 depths 144 : 215;
-//   one view 4 depths 46 : 48, 12 depths 116 : 79.  64 channels in groups of one, two views, 8 depths 119 :
+//   one view 4 depths 46 : 48, 12 depths 116 : 79; 383 x 534 x 27, two views, planes from depth 0.7, 2 and 5 on
+//   1123 : 1492, 1138 : 1107 and 1126 : 851, and 300 x 400 x 27, four views, 683 : 1117, 693 : 921, 696 : 764.  64 channels in groups of one, two views, 8 depths 119 :
 //   223, 32 depths 375 : 455; one view, 32 depths 316 : 287.  64 channels in groups of two, four views, 8
 //   depths 210 : 340; two views 211 : 224, one view, 4 depths 91 : 81.  Few tiles, 20 x 24: 32 channels, two
 //   views, 12 depths 8 : 18, 32 depths 13 : 18.  Double: the tiles take twice the time and more.  64
@@ -207,7 +208,7 @@ bool lanes_are_faster_best_pair(const Args<S> &a) {
   if (a.groups > 16) {
     if ((tiles < 1024 && a.D <= 12) || (tiles < 256 && a.D <= (wide ? 160 : sub == 1 ? 64 : 32))) return true;
     if (wide) return a.groups == 64 || a.D < (sub == 1 ? 64 * a.N - 32 : 32 * a.N - 12);
-    return sub == 1 ? a.D <= (lpp == 16 ? 16 : 6) * a.N : a.N > 1 && a.D <= 5 * a.N;
+    return sub == 1 ? a.D <= (lpp == 16 ? 16 : a.N == 1 ? 6 : 9) * a.N : a.N > 1 && a.D <= 5 * a.N;
   }
   switch (lpp) {
     case 2:

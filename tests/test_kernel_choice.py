@@ -156,7 +156,8 @@ def test_gradients_of_the_best_pair_by_winner():
     for want, calls in (
             (GENERAL, [(32, 1, 2, 200, 260, 12, f32), (32, 1, 2, 20, 24, 32, f32), (64, 1, 2, 383, 534, 27, f32),
                        (64, 2, 4, 200, 260, 8, f32), (32, 1, 2, 200, 260, 32), (64, 1, 4, 200, 260, 8),
-                       (64, 1, 1, 60, 80, 96), (64, 2, 2, 60, 80, 32)]),
+                       (64, 1, 1, 60, 80, 96), (64, 2, 2, 60, 80, 32),
+                       (32, 1, 4, 300, 400, 27, f32)]),
             (LANES, [(8, 1, 1, 60, 80, 12, f32), (32, 2, 2, 20, 24, 12, f32), (32, 2, 4, 200, 260, 4, f32),
                      (16, 2, 3, 383, 534, 4, f32), (32, 4, 4, 200, 260, 8), (64, 8, 4, 60, 80, 12),
                      (64, 4, 2, 200, 260, 4), (64, 4, 6, 200, 260, 4)]),
