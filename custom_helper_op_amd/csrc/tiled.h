@@ -298,15 +298,15 @@ __device__ __forceinline__ void slot_write(R *p, const R (&v)[4]) {
   }
 }
 
-// Orders this wave's LDS traffic: the lanes of a wavefront execute in lockstep and the
-// LDS returns a wave's operations in issue order, so only the compiler has to be kept
-// from moving accesses across the phase boundary.
 // An LDS object at (lane-dependent byte offset) + (compile-time constant).
 template <typename T>
 __device__ __forceinline__ T &lds_at(unsigned char *base, unsigned lane_bytes, int const_bytes) {
   return *reinterpret_cast<T *>(base + lane_bytes + const_bytes);
 }
 
+// Orders this wave's LDS traffic: the lanes of a wavefront execute in lockstep and the
+// LDS returns a wave's operations in issue order, so only the compiler has to be kept
+// from moving accesses across the phase boundary.
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1700,12 +1700,13 @@ constexpr int kClaimLanes = 8;
 // LDS bytes of the backward kernel: the records of one chunk
 //   Four wts, dwt [NV*64] | int2 cell {slots, key|inside} [NV*64] | int off [NV*64] |
 //   R scale [64] | R dst [64] (per-voxel depth gradients and CostVolumeV3)
+// then the list of texels leaving a window, then the windows.  With one view per workgroup
+// the list shares the record space: a window that moves for a chunk as a whole does so before the
+// chunk's records are written.  One that follows the runs inside a chunk (end_spread_runs) has a list of
+// its own, backward_list_bytes.
 // The slim form (double, slim_double) keeps one Four {dh, dw, d sh / d depth, d sw / d depth} for both
 // sets of weights, which the lanes expand where a depth starts (eleven operations): 64 bytes less
 // per voxel.
-// then the list of texels leaving a window, then the windows.  With one view per workgroup
-// the list shares the record space: a window only moves before the chunk's records are
-// written.
 template <typename R, int VEC, int LPP, int NV, int FORM = kPlainWindow, bool SLIM = false, bool DST = true>
 constexpr int backward_record_bytes() {
   using WN = Window<VEC, LPP, FORM>;
