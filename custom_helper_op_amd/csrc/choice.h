@@ -26,7 +26,9 @@ int64_t lanes_of_a_pixel(const Args<S> &a) {
 //   CostAggregate and FeatureAggregate hold less per view (four views, 32 channels: with differences 180
 //   12.5 : 13.2, 380 14.7 : 16.0, 700 16.7 : 16.5; samples alone 380 12.2 : 16.4, 570 18.2 : 17.9).
 // Few depths shorten the tiles' chain, not the lanes' (one view, 38 x 40: 3 depths 5.4 : 4.5; CostAggregate,
-// four views, 64 channels, 20 x 24: 3 depths 13.4 : 9.7).
+// four views, 64 channels, 20 x 24: 3 depths 13.4 : 9.7; samples of 16 channels, six views, 19 x 20: one depth
+// 10.3 : 7.3; group correlation of 32 channels, six views, 58 x 61: 4 depths 19.3 : 15.2).  Not with the
+// squared differences of five and six views (64 channels, 19 x 21, one depth 6.2 : 9.1).
 template <typename S>
 bool lanes_are_faster_forward(const Args<S> &a) {
   const bool idle_lanes = a.C > 16 && a.C < 32;
@@ -58,8 +60,11 @@ bool lanes_are_faster_forward(const Args<S> &a) {
   else if (one_value)
     line = a.N == 1 ? 0 : a.N == 2 ? 192 : 384;
   else
-    line = a.N == 1 ? 192 : a.N == 2 || samples ? 384 : 768;
-  return waves < line && (one_value ? 2 * a.D >= lpp : a.D >= 4 || (a.N >= 3 && a.D == 3 && !samples));
+    line = a.N == 1 ? 192 : a.N == 2 || samples || (a.corr == GROUP_CORRELATION && a.D < 5) ? 384 : 768;
+  if (waves >= line) return false;
+  if (one_value) return 2 * a.D >= lpp;
+  return a.D >= 4 || (a.D == 3 && a.N >= 3 && !samples) ||
+         (a.corr == SQUARED_DIFFERENCE && a.N >= 5 && lpp >= 8);
 }
 
 // Gradients in double of one view, or of two, in launches that leave most of the chip idle.  With so few

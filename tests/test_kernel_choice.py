@@ -98,14 +98,16 @@ def test_forward_launches_of_few_waves_keep_a_lane_per_channel():
            ("v1", 24, 3, 38, 40, 24, f32), ("v1", 20, 3, 38, 40, 12, dict(dtype="bf16")), ("v2", 28, 2, 38, 40, 8, f32),
            ("layer", 32, 4, 38, 40, 12), ("layer", 64, 3, 20, 24, 8), ("feat", 32, 4, 38, 40, 12),
            ("v2", 8, 1, 200, 260, 48, low), ("v1", 8, 1, 200, 260, 86, low),
-           ("v1", 32, 5, 120, 160, 24, low), ("v1", 64, 6, 90, 110, 24, low)],
+           ("v1", 32, 5, 120, 160, 24, low), ("v1", 64, 6, 90, 110, 24, low), ("v1", 64, 5, 19, 21, 1),
+           ("v1", 28, 1, 160, 200, 96, low)],
           [("v1", 32, 3, 50, 56, 24), ("v1", 32, 6, 50, 56, 24), ("v1", 32, 2, 38, 40, 24), ("v1", 32, 1, 38, 40, 12),
            ("v1", 16, 3, 60, 80, 8), ("v2", 16, 3, 50, 56, 12), ("v2", 64, 6, 60, 80, 8), ("v2", 32, 1, 13, 15, 3),
            ("v1", 24, 3, 60, 80, 12, f32), ("v1", 8, 5, 38, 40, 6), ("v1", 32, 6, 128, 160, 64), ("v1", 64, 3, 200, 260, 6),
            ("layer", 32, 4, 50, 56, 12), ("layer", 64, 3, 20, 24, 3), ("layer", 16, 4, 20, 24, 8), ("layer", 32, 1, 20, 24, 8),
            ("feat", 32, 4, 50, 56, 12), ("v1", 32, 3, 13, 15, 3, dict(dtype="f32")),
            ("v2", 8, 1, 200, 260, 24, low), ("v2", 8, 1, 200, 260, 48), ("v1", 8, 1, 100, 130, 86, dict(B=2, reduce="MIN")),
-           ("v1", 32, 5, 120, 160, 48, low), ("v1", 32, 5, 120, 160, 24), ("v1", 32, 5, 100, 130, 12, dict(B=2, reduce="MIN"))])
+           ("v1", 32, 5, 120, 160, 48, low), ("v1", 32, 5, 120, 160, 24), ("v1", 32, 5, 100, 130, 12, dict(B=2, reduce="MIN")),
+           ("v1", 64, 4, 19, 21, 1), ("feat", 16, 6, 19, 20, 1), ("v2", 32, 6, 58, 61, 4), ("v1", 28, 1, 160, 200, 32, low)])
 
 
 @pytest.mark.parametrize("op", ["v1", "layer", "feat"])
