@@ -1884,6 +1884,13 @@ struct LooseSums {
   R v[4];
   __device__ __forceinline__ R &operator[](int k) { return v[k]; }
 };
+// The sum of tap `k` and channel `c` on top of `old`.  As many sums as channels: the channel's own.  Fewer
+// (group correlation): the sum of the channel's group, times the channel's reference value.
+template <int VEC, int NS, typename R, typename T>
+__device__ __forceinline__ R add_tap_sum(R old, T (&v)[NS], const R (&ref)[VEC], int c, int k) {
+  if constexpr (NS == VEC) return old + v[c][k];
+  else return mad(ref[c], v[c * NS / VEC][k], old);
+}
 
 // Adds the four tap images of a finished run into the window (a cell that sticks out of the
 // window never gets here: flush_cells_to_memory takes it).  Called from divergent code by all
@@ -1899,8 +1906,8 @@ struct LooseSums {
 // from 429 to 400 us; against LDS atomics it halved the time of the 8-channel workloads.
 // 16 lanes per pixel (four pixels per wave): the pixels that fire in the same instruction
 // take turns, one pixel per round with its four taps in flight together.
-template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP = 2, typename R, typename T>
-__device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC], R *data,
+template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP = 2, int NS, typename R, typename T>
+__device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[NS], const R (&ref)[VEC], R *data,
                                            int *tags, int lane, int cl) {
   using WN = Window<VEC, LPP, FORM>;
   if (key < 0) {
@@ -1929,7 +1936,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] += v[i][k];
+            for (int i = 0; i < VEC; ++i) old[k][i] = add_tap_sum(old[k][i], v, ref, i, k);
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
@@ -1948,7 +1955,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
             R old[VEC];
             slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] += v[i][k];
+            for (int i = 0; i < VEC; ++i) old[i] = add_tap_sum(old[i], v, ref, i, k);
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
           }
         } else {
@@ -1958,7 +1965,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] += v[i][k];
+            for (int i = 0; i < VEC; ++i) old[k][i] = add_tap_sum(old[k][i], v, ref, i, k);
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
           }
         }
@@ -1974,7 +1981,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
             R old[VEC];
             slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
 #pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] += v[i][k];
+            for (int i = 0; i < VEC; ++i) old[i] = add_tap_sum(old[i], v, ref, i, k);
             slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
             // (the next tap may be the texel another pixel has just updated: the LDS keeps a
             // wave's operations in order, the compiler is held to it here)
@@ -1989,7 +1996,7 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
   }
   // (a cell that sticks out of the window never gets here: flush_cells_to_memory took it)
 #pragma unroll
-  for (int i = 0; i < VEC; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
+  for (int i = 0; i < NS; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
 }
 
 // Cells that no window position covers (the tile's pixels of one depth further apart than the
@@ -1999,10 +2006,10 @@ __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[VEC],
 // and the whole wave adds each row as a dense run of 2*C consecutive floats.  Added lane by
 // lane from the registers, each 16-byte chunk of a texel would carry one float per
 // instruction, and the atomics cost per chunk, not per float.
-template <int VEC, int LPP, int GAP, typename R, typename T>
-__device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool mine, int key,
-                                                      T (&v)[VEC], R *stage, R *gview, int srcW, int lane, int cl,
-                                                      int cm) {
+template <int VEC, int LPP, int GAP, int NS, typename R, typename T>
+__device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool mine, int key, T (&v)[NS],
+                                                      const R (&ref)[VEC], R *stage, R *gview, int srcW, int lane,
+                                                      int cl, int cm) {
   constexpr int C = VEC * LPP;
   while (m) {
     const int lead = __ffsll((long long)m) - 1;
@@ -2013,7 +2020,9 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 #pragma unroll
       for (int k = 0; k < 4; ++k)
       {
-        const R w[VEC] = {v[0][k], v[1][k], v[2][k], v[3][k]};
+        R w[VEC];
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) w[i] = NS == VEC ? v[i * NS / VEC][k] : add_tap_sum(R(0), v, ref, i, k);
         slot_write<GAP>(stage + (k == 2 ? 3 : k == 3 ? 2 : k) * C + lane_first(cl, GAP), w);
       }
     }
@@ -2035,7 +2044,7 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
   }
   if (mine) {
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
+    for (int i = 0; i < NS; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
   }
 }
 
@@ -2061,6 +2070,8 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // with them the kernels spilled 44-68 bytes around the depth loop and four waves were slower
 // than three).  Up to 32 bytes of scratch remain in two of those instantiations, outside the
 // depth loop: bf16 group-correlation backward 479 -> 462 us cold, 447 -> 417 us warm.
+// Group correlation with the tap sums per group (run_sums): 112-128 registers lean; maxima of two
+// groups per lane keep three waves (28-44 bytes of scratch at four).
 // Sixteen lanes per pixel (64 channels): slimmed, all of them, to three waves (164-222 registers
 // left alone, 132-164 slimmed; LDS holds them to 13 workgroups per CU, see Window::ROWS).
 // Double: the slimmed code at two waves per SIMD (taps, tap sums and rows of four channels are 100
@@ -2072,17 +2083,22 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // channel: 940), minimum over three views x 64 751 against 372 (673).  CostAggregate has no rows and
 // does not spill: three views, 149 x 220 x 116, 524 against 584 us (1460); 64 channels, where LDS holds
 // either form to seven workgroups, 364 against 275 us (630); one lane per pixel has no records in LDS.
+// (tap sums per group instead of per channel, see backward_kernel's GV)
+constexpr bool run_sums(int lpp, int reduce, int gv) { return gv < 4 && (lpp != 2 || reduce != 0); }
 constexpr bool slim_double(int lpp, int corr) { return corr == 2 && lpp > 1 && lpp <= 8; }
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false,
-                             bool wide_real = false) {
+                             bool wide_real = false, int gv = 4) {
   return wide_real ? true : nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
                      (lpp == 4 && ((corr <= 1 && reduce == 0) || corr == 2 || corr == 4)) ||
-                     (lpp == 2 && corr <= 1 && reduce == 0));
+                     (lpp == 2 && corr <= 1 && reduce == 0) ||
+                     (corr == 1 && run_sums(lpp, reduce, gv) && lpp >= 4 && (reduce == 0 || gv == 1)));
 }
+// 32 channels: the gradients that have kernels for either window (six rows and eight).
+constexpr bool two_windows(int corr, int reduce) { return (corr == 0 && reduce == 0) || corr == 2 || corr == 4; }
 constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false,
-                             bool wide_real = false) {
+                             bool wide_real = false, int gv = 4) {
   return wide_real ? (slim_double(lpp, corr) ? 3 : 2) : lpp == 16 && nv == 1                             ? 3
-         : lean_backward(nv, lpp, corr, reduce, wide) ? 4
+         : lean_backward(nv, lpp, corr, reduce, wide, false, gv) ? 4
          : nv == 1 && lpp <= 8                       ? 3
          : nv <= 2                                   ? 2
                                                      : 1;
@@ -2111,15 +2127,30 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // lane-per-channel kernels have two pixels and none (training
 // passes of 24 channels: minimum over five views, 63 x 85 x 37, 219 -> 110 us; warped features, 212 x
 // 213 x 86, 627 -> 344 us).
+// GV (CORR 1): group values per lane -- four (groups of one channel), two, or one (of four; a group of eight
+// is one that two lanes share).  A compile-time flag: a run-time width in the depth loop cost the 8-channel
+// kernels 5 % (bf16, four views, 512 x 640 x 8, two images: 373 -> 353 us).
+// With fewer values than channels (kRunSums) everything a depth adds factors into its group value and the
+// channels, which stay what they are while a run lasts: the tap sums are kept per group, sum of cost_grad *
+// weight, and meet the reference channels when the run ends (in the window's addition), the taps there too
+// (ref_grad); the depth gradient takes the taps against the reference, formed once per run (`proj`).  Per
+// depth 10 operations per group where the channel loop takes 15 per channel, and 16 to 28 registers less,
+// which with 32 channels are a fourth wave per SIMD.  Gradient, two views unless said, 128 x 160: 32 channels in 8
+// groups x 48 104 -> 90 us (maximum, three views, 241 -> 179), in 4 groups, six views, x 64 378 -> 334; 64
+// channels in groups of four, maximum, 178 -> 154; 16 channels in 8 groups, maximum, four views, 150 x 200 x
+// 32, 241 -> 185; double 139 -> 130; 8 channels, maximum, bf16 as above, 609 -> 428.  The mean of 8 channels
+// keeps the channel loop: with 32 pixels in a wave a run ends at nearly every depth, and what a run costs
+// more is what its depths save (537 -> 545 us for the training pass with bf16 run sums).  Errors against
+// 64-bit sums are the channel loop's or below (1.03e-7 and 1.02e-7 of the norm; it: 1.04e-7, 1.05e-7).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool DG = true,
-          bool PV = (CORR == 1), bool VLOOP = false, int EIGHT = kNotEight, bool PAD = false>
-__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, sizeof(S) == 8)) void backward_kernel(
+          bool PV = (CORR == 1), bool VLOOP = false, int EIGHT = kNotEight, bool PAD = false, int GV = 4>
+__global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, sizeof(S) == 8, GV)) void backward_kernel(
     const Args<S> a, const Geometry g) {
   using R = typename Storage<S>::Real;
   using R4 = Four<R>;
   constexpr bool kDouble = sizeof(S) == 8;
   constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
-  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, kDouble);
+  constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, kDouble, GV);
   constexpr bool kSlim = kDouble && slim_double(LPP, CORR);
   constexpr int kForm = !(kLean && LPP == 8) ? kPlainWindow : kSlim ? kFourRows : EIGHT == kEightTall ? kSixColumns : kSixRows;
   using WN = Window<VEC, LPP, kForm>;
@@ -2185,6 +2216,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
     for (int c = 0; c < VEC; ++c) ref[c] = R(0);
   }
+  if constexpr (PAD && run_sums(LPP, REDUCE, GV)) {  // (idle lanes: their window slots stay zero)
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) ref[c] = ch_ok ? ref[c] : R(0);
+  }
   constexpr int kWideSub = CORR == 5 ? 2 : 8;  // CostVolumeV3: the wider of the kernel's two group widths
   Two<R> ends{};
   if constexpr (CORR == 5 && REDUCE == 0) ends = ref_ends<LPP>(ref);
@@ -2220,7 +2255,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   constexpr bool kEndLeft = kWinners && (CORR != 2 || LPP < 8);
   constexpr int kFewRuns = !kWinners ? 0 : best_pair_op(CORR) ? 4 : PPW / 8;
   const int OC = CORR == 1 ? a.groups : kVoxelGrad ? 1 : C;
-  const int gv = VEC / g.sub;  // group values per lane (a group of eight: one, shared by two lanes)
+  static_assert(VEC == 4 && (GV == 4 || (CORR == 1 && (GV == 2 || GV == 1))), "group values per lane");
+  constexpr bool kRunSums = run_sums(LPP, REDUCE, GV);
+  constexpr int NS = kRunSums ? GV : VEC;  // sums per tap
   const int goff = CORR == 1 ? group_offset<VEC>(clc, g.sub) : ch0;
   const int d_lo = t.d_lo, d_hi = t.d_hi;
   // upstream-gradient rows fetched ahead; the MIN reduce stages the mask rows beside them
@@ -2266,7 +2303,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     oy[n] = ox[n] = WN::kNone;
   }
   R tap[NV][4][VEC];
-  Sums sg[NV][VEC];
+  Sums sg[NV][NS];
+  R proj[NV][4][kRunSums && DG ? GV : 1];  // kRunSums: the taps of the open run against the reference, per group
   int cur[NV];     // tap offset of the open run, -1: none
   int2 cell[NV];   // its slots and key (bit 31: inside the window)
   unsigned ring_rows[NV];  // ring rows of the window this lane's accepted cells mapped to
@@ -2276,8 +2314,20 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     ring_rows[n] = 0u;
     cell[n] = make_int2(0, 0);
 #pragma unroll
-    for (int c = 0; c < VEC; ++c) sg[n][c] = Sums{R(0), R(0), R(0), R(0)};
+    for (int c = 0; c < NS; ++c) sg[n][c] = Sums{R(0), R(0), R(0), R(0)};
   }
+  // kRunSums: the reference gradient of a run that ends (its taps are still at hand)
+  auto take_run = [&](int n) __attribute__((always_inline)) {
+    if constexpr (kRunSums) {
+#pragma unroll
+      for (int c = 0; c < VEC; ++c) {
+        R run = tap[n][0][c] * sg[n][c * NS / VEC][0];  // (summed by itself: one rounding per run in racc)
+#pragma unroll
+        for (int k = 1; k < 4; ++k) run = mad(tap[n][k][c], sg[n][c * NS / VEC][k], run);
+        racc[c] += run;
+      }
+    }
+  };
   const S *cg_lane =
       CORR == 4 ? a.cost_grad + (t.pix * D * N + t.view0) * C + ch0
                 : a.cost_grad + t.pix * D * OC + (kVoxelGrad ? 0 : goff);
@@ -2323,7 +2373,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       const bool out = fire && !in;
       const unsigned long long m = __ballot(out);
       if (m != 0ull) {
-        flush_cells_to_memory<VEC, LPP, GAP>(m, out, key, sg[n], s_stage, gview[n], srcW, lane, cl, cm);
+        if (out) take_run(n);
+        flush_cells_to_memory<VEC, LPP, GAP>(m, out, key, sg[n], ref, s_stage, gview[n], srcW, lane, cl, cm);
         if (out) cur[n] = -1;
       }
     }
@@ -2367,24 +2418,16 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     // is fetched.  One cache state is slower this way (by 4 %): every line dirty with another
     // kernel's output, which a load that allocates has to push out first.
     // (whole rows are kept as loaded and widened to float where a depth uses them; group
-    // rows, whose width is a run-time value, are widened here and kept as float bits)
-    RawWord<S> cgw[kVoxelGrad ? 1 : PF][(CORR == 0 || CORR == 4) ? raw_words<S, VEC>() : VEC];
-    int mrow[kMaskRows ? PF : 1][VEC];
+    // rows are widened here and kept as float bits)
+    RawWord<S> cgw[kVoxelGrad ? 1 : PF][(CORR == 0 || CORR == 4) ? raw_words<S, VEC>() : GV];
+    int mrow[kMaskRows ? PF : 1][GV];
     auto load_rows = [&](int first) {
       if constexpr (CORR == 1) {
-        // the group width is a run-time value: one branch around all of the chunk's loads, so
-        // that they go out together (a branch per row makes each row wait for the one before)
-        auto group_rows = [&](auto cnt) {
-          constexpr int CNT = decltype(cnt)::value;
 #pragma unroll
-          for (int jj = 0; jj < PF; ++jj) {
-            const int d = min(first + jj, d_hi - 1);
-            load_vec<S, CNT, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<R *>(cgw[jj]));
-          }
-        };
-        if (g.sub == 1) group_rows(std::integral_constant<int, VEC>());
-        else if (g.sub == 2) group_rows(std::integral_constant<int, VEC / 2>());
-        else group_rows(std::integral_constant<int, 1>());
+        for (int jj = 0; jj < PF; ++jj) {
+          const int d = min(first + jj, d_hi - 1);
+          load_vec<S, GV, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<R *>(cgw[jj]));
+        }
       }
 #pragma unroll
       for (int jj = 0; jj < PF; ++jj) {
@@ -2398,19 +2441,16 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
           load_raw<S, VEC, whole_lines(VEC * LPP, (int)sizeof(S)), GAP>(src_cg, cgw[jj]);
         if constexpr (kMaskRows) {
           const int32_t *m = mask_lane + (int64_t)d * OC;
-          const int cntv = CORR == 0 ? VEC : gv;
-          if (GAP != 2) {
+          if constexpr (GAP != 2) {
             const int2 lo = *reinterpret_cast<const int2 *>(m), hi = *reinterpret_cast<const int2 *>(m + GAP);
             mrow[jj][0] = lo.x, mrow[jj][1] = lo.y, mrow[jj][2] = hi.x, mrow[jj][3] = hi.y;
-          } else if (cntv == 4) {
+          } else if constexpr (GV == 4) {
             typedef int i32x4 __attribute__((ext_vector_type(4)));
-            const i32x4 *q = reinterpret_cast<const i32x4 *>(m);
-            const i32x4 v = *q;
+            const i32x4 v = *reinterpret_cast<const i32x4 *>(m);
             mrow[jj][0] = v[0], mrow[jj][1] = v[1], mrow[jj][2] = v[2], mrow[jj][3] = v[3];
-          } else if (cntv == 2) {
+          } else if constexpr (GV == 2) {
             typedef int i32x2 __attribute__((ext_vector_type(2)));
-            const i32x2 *q = reinterpret_cast<const i32x2 *>(m);
-            const i32x2 v = *q;
+            const i32x2 v = *reinterpret_cast<const i32x2 *>(m);
             mrow[jj][0] = v[0], mrow[jj][1] = v[1];
           } else {
             mrow[jj][0] = *m;
@@ -2510,7 +2550,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               const bool left = !spread[n] && cur[n] >= 0 && !WN::inside(key, ny - sy / 2, nx - sx / 2);
               const unsigned long long m = __ballot(left);
               if (m != 0ull) {
-                flush_cells_to_memory<VEC, LPP, GAP>(m, left, key, sg[n], s_stage, gview[n], srcW, t.lane, t.cl, cm);
+                if (left) take_run(n);
+                flush_cells_to_memory<VEC, LPP, GAP>(m, left, key, sg[n], ref, s_stage, gview[n], srcW, t.lane, t.cl, cm);
                 if (left) cur[n] = -1;
               }
             }
@@ -2623,48 +2664,38 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       // (one view per workgroup: a tap offset implies a non-zero factor, phase 1 reprojects
       // only voxels that have one; one test instead of two per depth)
       if (NV == 1 ? rec_off[0] >= 0 : scl != R(0)) {
-        R cg[VEC];
+        R cg[GV];  // of this lane's channels (group correlation: groups)
         {
-          R raw[VEC];
+          R raw[GV];
           if constexpr (!kVoxelGrad) {
-            if (CORR == 0 || CORR == 4)
+            if constexpr (CORR == 0 || CORR == 4)
               widen_raw<S, VEC>(cgw[jj % PF], raw);
             else
 #pragma unroll
-              for (int c = 0; c < VEC; ++c) raw[c] = raw_to_real(cgw[jj % PF][c]);
+              for (int c = 0; c < GV; ++c) raw[c] = raw_to_real(cgw[jj % PF][c]);
           }
           if constexpr (kVoxelGrad) {
 #pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = scl;
+            for (int c = 0; c < GV; ++c) cg[c] = scl;
           } else if (CORR == 4) {
             // (each view of FeatureAggregate has rows of its own: no factor)
 #pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = raw[c];
-          } else if (CORR == 0 || g.sub == 1) {
-#pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = raw[c] * scl;
-          } else if (g.sub == 2) {
-#pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = raw[c / 2] * scl;
-          } else if (g.sub == 4) {
-#pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = raw[c / 4] * scl;
+            for (int c = 0; c < GV; ++c) cg[c] = raw[c];
           } else {
 #pragma unroll
-            for (int c = 0; c < VEC; ++c) cg[c] = raw[0] * scl;
+            for (int c = 0; c < GV; ++c) cg[c] = raw[c] * scl;
           }
           if constexpr (kMaskRows) {
             // only the channels (groups) this view won contribute
             static_assert(NV == 1, "the MIN gradient runs one view per workgroup");
             const int *mr = mrow[jj % PF];
 #pragma unroll
-            for (int c = 0; c < VEC; ++c) {
-              const int win = (CORR == 0 || g.sub == 1) ? mr[c]
-                              : g.sub == 2              ? mr[c / 2]
-                              : g.sub == 4              ? mr[c / 4]
-                                                        : mr[0];
-              if (win != t.view0) cg[c] = R(0);
-            }
+            for (int c = 0; c < GV; ++c)
+              if (mr[c] != t.view0) cg[c] = R(0);
+          }
+          if constexpr (PAD && kRunSums) {
+#pragma unroll
+            for (int c = 0; c < GV; ++c) cg[c] = ch_ok ? cg[c] : R(0);
           }
         }
 #pragma unroll
@@ -2686,6 +2717,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               // the run on the previous cell ends.  Start fetching the new cell's taps
               // first, then hand the old cell's image to the window while they arrive.
               // byte offsets in 32 bits: the loads take the view's base from scalar registers
+              if constexpr (kRunSums)
+                if (cur[n] >= 0) take_run(n);
               const unsigned e0 = ((unsigned)off + lane_ch) * (unsigned)sizeof(S);
               const unsigned e1 = e0 + (unsigned)row_step * (unsigned)sizeof(S);
               const char *vb = reinterpret_cast<const char *>(view[n]);
@@ -2695,14 +2728,42 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + (e1 + cb)), tap[n][2]);
               load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + e1), tap[n][3]);
               if (cur[n] >= 0)
-                window_add<VEC, LPP, kLean, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n],
+                window_add<VEC, LPP, kLean, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n], ref,
                                             s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
               cur[n] = off;
               if constexpr (LPP > 1)
                 cell[n] = lds_at<int2>(smem, p4 * 2u, kCell + ((n * LPP + jj) * PPW) * 8);
               else
                 cell[n] = r_cell[n];
+              if constexpr (kRunSums && DG) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                  for (int i = 0; i < GV; ++i) {
+                    constexpr int SUB = VEC / GV;
+                    R sum = ref[i * SUB] * tap[n][k][i * SUB];
+#pragma unroll
+                    for (int c = 1; c < SUB; ++c) sum = mad(ref[i * SUB + c], tap[n][k][i * SUB + c], sum);
+                    proj[n][k][i] = sum;
+                  }
+              }
             }
+            if constexpr (kRunSums) {
+#pragma unroll
+              for (int i = 0; i < GV; ++i) {
+                sg[n][i][0] = mad(cg[i], wt.x, sg[n][i][0]);
+                sg[n][i][1] = mad(cg[i], wt.y, sg[n][i][1]);
+                sg[n][i][2] = mad(cg[i], wt.z, sg[n][i][2]);
+                sg[n][i][3] = mad(cg[i], wt.w, sg[n][i][3]);
+                if constexpr (DG) {
+                  R ds = dwt.x * proj[n][0][i];
+                  ds = mad(dwt.y, proj[n][1][i], ds);
+                  ds = mad(dwt.z, proj[n][2][i], ds);
+                  ds = mad(dwt.w, proj[n][3][i], ds);
+                  dvox = mad(cg[i], ds, dvox);
+                }
+              }
+            } else {
             R gs3[VEC];
             if constexpr (best_pair_op(CORR)) {
               const int pair = REDUCE ? lds_at<int>(smem, p4, kDst + (jj * PPW) * 4) : 0;
@@ -2719,7 +2780,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               if constexpr (best_pair_op(CORR)) {
                 gsrc = gs3[c];
               } else if constexpr (CORR == 4) {
-                gsrc = cg[c];
+                gsrc = cg[c * GV / VEC];
               } else if (CORR != 1) {
                 // (double: the sample first, then the difference: sums of the sample's parts are the
                 // smaller numbers to round, and the lane-per-channel kernels have it so)
@@ -2728,15 +2789,15 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                 diff = mad(wt.z, tap[n][2][c], diff);
                 diff = mad(wt.w, tap[n][3][c], diff);
                 if constexpr (kDouble) diff -= ref[c];
-                gsrc = diff * cg[c];
+                gsrc = diff * cg[c * GV / VEC];
                 racc[c] -= gsrc;
               } else {
                 R smp = wt.x * tap[n][0][c];
                 smp = mad(wt.y, tap[n][1][c], smp);
                 smp = mad(wt.z, tap[n][2][c], smp);
                 smp = mad(wt.w, tap[n][3][c], smp);
-                racc[c] = mad(cg[c], smp, racc[c]);
-                gsrc = cg[c] * ref[c];
+                racc[c] = mad(cg[c * GV / VEC], smp, racc[c]);
+                gsrc = cg[c * GV / VEC] * ref[c];
               }
               if constexpr (PAD) gsrc = ch_ok ? gsrc : R(0);
               if constexpr (kMatrix) {
@@ -2754,6 +2815,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                 ds = mad(dwt.w, tap[n][3][c], ds);
                 dvox = mad(gsrc, ds, dvox);
               }
+            }
             }
           }
         }
@@ -2805,8 +2867,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
     if (__ballot(cur[n] >= 0 && cell[n].y >= 0) != 0ull) end_spread_runs(n, cur[n] >= 0);
+    if (cur[n] >= 0) take_run(n);
     if (cur[n] >= 0)
-      window_add<VEC, LPP, false, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n],
+      window_add<VEC, LPP, false, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n], ref,
                            s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
   }
   wave_sync();
