@@ -2059,8 +2059,13 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // no scratch.  Those three cost 5 % at three waves per SIMD; with the 10 KB of LDS of the
 // six-row window the fourth wave gains 11 % (MVSNet-stage backward 301 -> 277 us).
 // Likewise the gradients of CostAggregate (both reduces: 137 -> 117 registers) and of
-// FeatureAggregate (149 -> 119).  Not the MIN / MAX gradients of the per-channel ops (their mask
-// rows keep them above 140) and not CostVolumeV3 (its two extra LDS rows per pixel are 2 KB).
+// FeatureAggregate (149 -> 119).  The MIN / MAX gradients of the per-channel ops, whose mask rows kept them
+// at 141-166, keep the winners as lane masks in scalar registers instead (find_won: 120-128, no scratch in
+// float): 24 channels, six wide-baseline views, 200 x 260 x 64, 1075 -> 908 us; 32 channels, x 96, 1457 -> 1320, two
+// views, 128 x 160 x 96, 208 -> 206; 16 channels, three views, x 48, 282 -> 268, bf16, four, 221 -> 207.  The
+// wait for the winners costs up to 6 % where three waves per SIMD hold the whole launch: those keep the
+// other form (the launcher).  Not CostVolumeV3 (its two extra LDS rows per pixel are 2 KB), nor the
+// maximum of 8 channels whose views take turns (52-80 bytes of scratch).
 // Four lanes per pixel (16 channels), gradients of a mean: 130 registers left alone, 121 lean
 // (held to 128 without the slimming they spilled three to five); the window of the 4 x 4 pixel
 // tile is 4 KB.  CostAggregate and FeatureAggregate the same (134 -> 117-120; six views, 497 x 700 x 41:
@@ -2070,8 +2075,7 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // with them the kernels spilled 44-68 bytes around the depth loop and four waves were slower
 // than three).  Up to 32 bytes of scratch remain in two of those instantiations, outside the
 // depth loop: bf16 group-correlation backward 479 -> 462 us cold, 447 -> 417 us warm.
-// Group correlation with the tap sums per group (run_sums): 112-128 registers lean; maxima of two
-// groups per lane keep three waves (28-44 bytes of scratch at four).
+// Group correlation with the tap sums per group (run_sums): 112-128 registers lean, both reduces.
 // Sixteen lanes per pixel (64 channels): slimmed, all of them, to three waves (164-222 registers
 // left alone, 132-164 slimmed; LDS holds them to 13 workgroups per CU, see Window::ROWS).
 // Double: the slimmed code at two waves per SIMD (taps, tap sums and rows of four channels are 100
@@ -2088,10 +2092,11 @@ constexpr bool run_sums(int lpp, int reduce, int gv) { return gv < 4 && (lpp != 
 constexpr bool slim_double(int lpp, int corr) { return corr == 2 && lpp > 1 && lpp <= 8; }
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false,
                              bool wide_real = false, int gv = 4) {
-  return wide_real ? true : nv == 1 && !wide && (lpp == 16 || (lpp == 8 && ((corr == 0 && reduce == 0) || corr == 2 || corr == 4)) ||
-                     (lpp == 4 && ((corr <= 1 && reduce == 0) || corr == 2 || corr == 4)) ||
-                     (lpp == 2 && corr <= 1 && reduce == 0) ||
-                     (corr == 1 && run_sums(lpp, reduce, gv) && lpp >= 4 && (reduce == 0 || gv == 1)));
+  return wide_real ||
+         (nv == 1 && !wide &&
+          (lpp == 16 || (lpp == 8 && (corr == 0 || corr == 2 || corr == 4)) ||
+           (lpp == 4 && (corr <= 2 || corr == 4)) || (lpp == 2 && (corr == 0 || (corr == 1 && reduce == 0))) ||
+           (corr == 1 && run_sums(lpp, reduce, gv) && lpp >= 4)));
 }
 // 32 channels: the gradients that have kernels for either window (six rows and eight).
 constexpr bool two_windows(int corr, int reduce) { return (corr == 0 && reduce == 0) || corr == 2 || corr == 4; }
@@ -2118,7 +2123,8 @@ constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool
 // A compile-time flag: the loop around the kernel's body costs the wide instantiations
 // registers they do not have (the 32-channel kernel spills with it).
 // EIGHT: 32 channels with a window of eight rows, for many views.  kEightWide: 8 x 8 texels and the kernel
-// without the slimming of lean_backward, three waves per SIMD; kEightTall: 8 x 6 over tiles of 4 x 2
+// without the slimming of lean_backward, three waves per SIMD (also the small launches' form of the minimum,
+// any width); kEightTall: 8 x 6 over tiles of 4 x 2
 // pixels, the slimmed form turned by ninety degrees.  The launcher decides (tiled_launch.inc).
 // PAD: fewer channels than the pixel's lanes hold (20, 24, 28 on eight lanes).  The lanes past the
 // last channel compute what the last lane computes and contribute nothing: their gradients are
@@ -2264,6 +2270,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   constexpr int PFMAX = (REDUCE || kLean) ? 4 : 8;
   constexpr int PF = LPP < PFMAX ? LPP : PFMAX;
   constexpr bool kMaskRows = REDUCE == 1 && !kVoxelGrad;
+  static_assert(!kMaskRows || NV == 1, "the MIN gradient runs one view per workgroup");
+  constexpr bool kWonMasks = kMaskRows && kLean && !kDouble && LPP <= 8;  // (find_won)
   // mask entries per voxel: the MIN reduce of CostVolumeV3 records (view, reference group,
   // source group)
   const int mask_w = kMaskRows ? OC : (best_pair_op(CORR) && REDUCE == 1) ? 3 : 1;
@@ -2422,24 +2430,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     RawWord<S> cgw[kVoxelGrad ? 1 : PF][(CORR == 0 || CORR == 4) ? raw_words<S, VEC>() : GV];
     int mrow[kMaskRows ? PF : 1][GV];
     auto load_rows = [&](int first) {
-      if constexpr (CORR == 1) {
+      if constexpr (kMaskRows) {
 #pragma unroll
         for (int jj = 0; jj < PF; ++jj) {
           const int d = min(first + jj, d_hi - 1);
-          load_vec<S, GV, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<R *>(cgw[jj]));
-        }
-      }
-#pragma unroll
-      for (int jj = 0; jj < PF; ++jj) {
-        const int d = min(first + jj, d_hi - 1);
-        const S *src_cg = cg_lane + (int64_t)d * cg_step;
-        // (each view of FeatureAggregate has rows of its own: streamed where they cover whole
-        // lines)
-        if constexpr (CORR == 0)
-          load_raw<S, VEC, false, GAP>(src_cg, cgw[jj]);
-        if constexpr (CORR == 4)
-          load_raw<S, VEC, whole_lines(VEC * LPP, (int)sizeof(S)), GAP>(src_cg, cgw[jj]);
-        if constexpr (kMaskRows) {
           const int32_t *m = mask_lane + (int64_t)d * OC;
           if constexpr (GAP != 2) {
             const int2 lo = *reinterpret_cast<const int2 *>(m), hi = *reinterpret_cast<const int2 *>(m + GAP);
@@ -2457,8 +2451,57 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
           }
         }
       }
+      if constexpr (CORR == 1) {
+#pragma unroll
+        for (int jj = 0; jj < PF; ++jj) {
+          const int d = min(first + jj, d_hi - 1);
+          load_vec<S, GV, false>(cg_lane + (int64_t)d * cg_step, reinterpret_cast<R *>(cgw[jj]));
+        }
+      }
+#pragma unroll
+      for (int jj = 0; jj < PF; ++jj) {
+        const int d = min(first + jj, d_hi - 1);
+        const S *src_cg = cg_lane + (int64_t)d * cg_step;
+        // (each view of FeatureAggregate has rows of its own: streamed where they cover whole
+        // lines)
+        if constexpr (CORR == 0)
+          load_raw<S, VEC, false, GAP>(src_cg, cgw[jj]);
+        if constexpr (CORR == 4)
+          load_raw<S, VEC, whole_lines(VEC * LPP, (int)sizeof(S)), GAP>(src_cg, cgw[jj]);
+      }
+    };
+    // Only the channels (groups) this view won contribute: the rest of a staged row becomes zero.  The
+    // comparisons are made when the winners arrive, whose first entry the reprojection waits for anyway, and
+    // kept as lane masks in scalar registers, so that the winners hold no registers through the walk.
+    unsigned long long won[kWonMasks ? PF : 1][GV];
+    auto find_won = [&]() __attribute__((always_inline)) {
+      if constexpr (kWonMasks) {
+#pragma unroll
+        for (int jj = 0; jj < PF; ++jj)
+#pragma unroll
+          for (int i = 0; i < GV; ++i) won[jj][i] = __ballot(mrow[jj][i] == t.view0);
+      }
+    };
+    auto keep_won = [&]() __attribute__((always_inline)) {
+      if constexpr (kWonMasks) {
+        auto select = [](uint32_t w, unsigned long long m) __attribute__((always_inline)) {
+          return __builtin_amdgcn_inverse_ballot_w64(m) ? w : 0u;
+        };
+#pragma unroll
+        for (int jj = 0; jj < PF; ++jj) {
+          if constexpr (sizeof(S) == 2 && CORR == 0) {  // (two channels per word)
+#pragma unroll
+            for (int i = 0; i < GV / 2; ++i)
+              cgw[jj][i] &= select(0xffffu, won[jj][2 * i]) | select(0xffff0000u, won[jj][2 * i + 1]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < GV; ++i) cgw[jj][i] = select(cgw[jj][i], won[jj][i]);
+          }
+        }
+      }
     };
     if constexpr (!kVoxelGrad) load_rows(d0);
+    find_won();
     {
       const R depth = d0 + t.cl < d_hi ? (per_voxel_depth ? dv : base + dv) : R(1);
       // factor the reduce applies to the upstream gradient: squared difference 2/k,
@@ -2595,6 +2638,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       }
     }
     if constexpr (LPP > 1) wave_sync();
+    keep_won();
     int rb_off[2][NV];
     R4 rb_wt[2][NV], rb_dwt[2][NV];
     R rb_scl[2], own_w = R(0);
@@ -2624,7 +2668,11 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       // (no early exit past d_hi: the records of such depths carry a zero factor and no tap
       // offset, the row loads are clamped, and a loop without exits compiles to faster code)
       if constexpr (LPP > PF && !kVoxelGrad) {
-        if (jj > 0 && jj % PF == 0) load_rows(d0 + jj);  // next part of a deep chunk
+        if (jj > 0 && jj % PF == 0) {  // next part of a deep chunk
+          load_rows(d0 + jj);
+          find_won();
+          keep_won();
+        }
       }
       // The records of the NEXT depth are requested now, so that their LDS latency overlaps
       // this depth's arithmetic (jj is unrolled: the buffer index is a compile-time constant).
@@ -2685,13 +2733,11 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
             for (int c = 0; c < GV; ++c) cg[c] = raw[c] * scl;
           }
-          if constexpr (kMaskRows) {
+          if constexpr (kMaskRows && !kWonMasks) {
             // only the channels (groups) this view won contribute
-            static_assert(NV == 1, "the MIN gradient runs one view per workgroup");
-            const int *mr = mrow[jj % PF];
 #pragma unroll
             for (int c = 0; c < GV; ++c)
-              if (mr[c] != t.view0) cg[c] = R(0);
+              if (mrow[jj % PF][c] != t.view0) cg[c] = R(0);
           }
           if constexpr (PAD && kRunSums) {
 #pragma unroll
