@@ -318,7 +318,7 @@ __device__ __forceinline__ void wave_sync() {
 // row mirrors (a mirror pairs lane i with lane WIDTH-1-i; the quad steps finish the sum).
 template <int CTRL>
 __device__ __forceinline__ int dpp_move(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
+  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
@@ -514,42 +514,96 @@ __device__ __forceinline__ void load_cameras(const Args<S> &a, int b, int view0,
   }
 }
 
+// w / z and h / z, each correctly rounded, with one reciprocal between them.  The steps are those of a
+// correctly rounded division by Newton's iteration and residual corrections (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990), without the scaling that only divisors
+// and quotients at the ends of the exponent's range need: fourteen operations (double: twelve) where two
+// divisions are twenty-two.  Divisors outside 2^-60 .. 2^60 (double: 2^-500 .. 2^500) make the wave divide
+// the plain way, and `small`: quotients near zero matter too (without it one below a quarter, which no
+// caller accepts, may be off).
+__device__ __forceinline__ bool unusual_divisor(float z) { return __float_as_uint(z) - 0x21800000u > 0x3c000000u; }
+__device__ __forceinline__ bool unusual_divisor(double z) { return (unsigned)__double2hiint(z) - 0x20b00000u > 0x3e800000u; }
+__device__ __forceinline__ void quotients(float w, float h, float z, bool small, float &qw, float &qh) {
+  float r = __builtin_amdgcn_rcpf(z);
+  r = __builtin_fmaf(__builtin_fmaf(-z, r, 1.f), r, r);
+  qw = w * r, qh = h * r;
+  qw = __builtin_fmaf(__builtin_fmaf(-z, qw, w), r, qw);
+  qh = __builtin_fmaf(__builtin_fmaf(-z, qh, h), r, qh);
+  qw = __builtin_fmaf(__builtin_fmaf(-z, qw, w), r, qw);
+  qh = __builtin_fmaf(__builtin_fmaf(-z, qh, h), r, qh);
+  if (small || __ballot(unusual_divisor(z)) != 0ull) qw = w / z, qh = h / z;
+}
+__device__ __forceinline__ void quotients(double w, double h, double z, bool small, double &qw, double &qh) {
+  double r = __builtin_amdgcn_rcp(z);
+  r = __builtin_fma(__builtin_fma(-z, r, 1.0), r, r);
+  r = __builtin_fma(__builtin_fma(-z, r, 1.0), r, r);
+  qw = w * r, qh = h * r;
+  qw = __builtin_fma(__builtin_fma(-z, qw, w), r, qw);
+  qh = __builtin_fma(__builtin_fma(-z, qh, h), r, qh);
+  if (small || __ballot(unusual_divisor(z)) != 0ull) qw = w / z, qh = h / z;
+}
+__device__ __forceinline__ float fraction(float x) { return __builtin_amdgcn_fractf(x); }  // x - floor(x), exact for x >= 0
+__device__ __forceinline__ double fraction(double x) { return __builtin_amdgcn_fract(x); }
+
 // One reprojection with hoisted row products; bit-identical to warp.h's project().
 template <typename R>
 struct Hit {
-  int off;     // element offset of tap (fh,fw) inside the view's image, or -1
+  int cell;    // place of tap (fh,fw) in the view's image, or -1: not accepted, the rest means nothing
   int key;     // (fh << 16) | fw
   R k00, k01, k11, k10;
   R dh, dw;
   R z, w3d, h3d;
 };
 
+// Without branches: what a rejected sample leaves behind is never looked at.  `wanted`: this lane's voxel counts.
+// (image rows and columns fit 15 bits, see make_plan.)  With the shared reciprocal, 24-bit products, taps
+// addressed from a uniform base and the window's four slot numbers put together by byte permutes a view of a
+// chunk takes about 60 instructions less than it did (of 170 in the gradients, of 74 forward), and the forward
+// kernels up to nine registers: gradients -2 to -8 % (f16, 16 channels, four views, 256 x 320 x 32, 235 -> 219
+// us; 16-channel minimum, three views, 259 -> 244), forward 0 to -15 % (bf16 groups, four views, 512 x 640 x
+// 8, 137 -> 129 us; CostAggregate's minimum of 16 channels, four views, 69 -> 60).
 template <int NV, typename R>
-__device__ __forceinline__ void reproject(const Cameras<NV, R> &c, int n, R depth, R half,
-                                          R src_h_max, R src_w_max, int srcW, int C,
-                                          Hit<R> &r) {
-  r.off = -1;
-  r.key = 0;
-  r.k00 = r.k01 = r.k11 = r.k10 = R(0);
+__device__ __forceinline__ void reproject(const Cameras<NV, R> &c, int n, R depth, R half, R src_h_max, R src_w_max,
+                                          int srcW, bool wanted, Hit<R> &r) {
   r.z = c.zc[n] * depth + c.t2[n];
-  if (r.z <= R(0)) return;
   r.w3d = c.wc[n] * depth + c.t0[n];
-  R sw = r.w3d / r.z;
   r.h3d = c.hc[n] * depth + c.t1[n];
-  R sh = r.h3d / r.z;
+  R sw, sh;
+  quotients(r.w3d, r.h3d, r.z, half == R(0), sw, sh);
   sw = sw - half;
   sh = sh - half;
-  if (sh > R(0) && sw > R(0) && sh < src_h_max && sw < src_w_max) {
-    const int fh = static_cast<int>(sh), fw = static_cast<int>(sw);
-    r.dh = sh - static_cast<R>(fh);
-    r.dw = sw - static_cast<R>(fw);
-    r.k11 = r.dh * r.dw;
-    r.k10 = r.dh * (R(1) - r.dw);
-    r.k00 = (R(1) - r.dh) * (R(1) - r.dw);
-    r.k01 = (R(1) - r.dh) * r.dw;
-    r.off = (fh * srcW + fw) * C;
-    r.key = (fh << 16) | fw;
-  }
+  const bool ok = wanted && !(r.z <= R(0)) && sh > R(0) && sw > R(0) && sh < src_h_max && sw < src_w_max;
+  const int fh = static_cast<int>(sh), fw = static_cast<int>(sw);
+  r.dh = fraction(sh);
+  r.dw = fraction(sw);
+  const R eh = R(1) - r.dh, ew = R(1) - r.dw;
+  r.k11 = r.dh * r.dw;
+  r.k10 = r.dh * ew;
+  r.k00 = eh * ew;
+  r.k01 = eh * r.dw;
+  r.cell = ok ? (int)__umul24((unsigned)fh, (unsigned)srcW) + fw : -1;
+  r.key = (fh << 16) | (fw & 0xffff);
+}
+
+// The four taps (00, 01, 11, 10) of a cell, this lane's channels: the view's uniform base and 32 bits of
+// bytes (an image has less than 2^29 elements, make_plan).  `cell` counts units of UNIT elements: texels, or
+// elements where the channel count is a run-time value (its product is then formed once per voxel).
+constexpr int cell_unit(int channels, bool pad) { return pad ? 1 : channels; }
+template <typename S, int VEC, int GAP, int UNIT>
+__device__ __forceinline__ void load_cell(const S *view, int cell, int C, int row_step, unsigned lane_ch,
+                                          typename Storage<S>::Real (&tap)[4][VEC]) {
+  const unsigned e0 = ((unsigned)cell * (unsigned)UNIT + lane_ch) * (unsigned)sizeof(S);
+  const unsigned e1 = e0 + (unsigned)row_step * (unsigned)sizeof(S);
+  const char *base = reinterpret_cast<const char *>(view);
+  const unsigned step = (unsigned)C * (unsigned)sizeof(S);
+  // (the texel to the right at a distance known when compiling lands in the instruction's offset field)
+  const char *row0 = base + e0, *row1 = base + e1;
+  const char *right0 = UNIT > 1 ? row0 + UNIT * sizeof(S) : base + (e0 + step);
+  const char *right1 = UNIT > 1 ? row1 + UNIT * sizeof(S) : base + (e1 + step);
+  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(row0), tap[0]);
+  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(right0), tap[1]);
+  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(right1), tap[2]);
+  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(row1), tap[3]);
 }
 
 template <typename S>
@@ -987,7 +1041,9 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
     if constexpr (NV <= 2) keep_alive(touched);
     return;
   }
-  const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
+  const int C = PAD ? (int)a.C : VEC * LPP;
+  constexpr int kUnit = cell_unit(VEC * LPP, PAD);
+  const int D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
   const R half = a.half;
   const bool ch_ok = !PAD || t.cl * VEC < C;
   const int clc = PAD ? min(t.cl, C / VEC - 1) : t.cl;  // the lane whose channels this lane holds
@@ -1025,7 +1081,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
   const S *view[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n)
-    view[n] = a.src + ((int64_t)t.b * N + (n < N ? n : 0)) * srcH * srcW * C + ch0;
+    view[n] = a.src + ((int64_t)t.b * N + (n < N ? n : 0)) * srcH * srcW * C;  // (uniform)
   const int row_step = srcW * C;
 
   R tap[NT][4][VEC];
@@ -1070,23 +1126,21 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         Hit<R> hit;
-        hit.off = -1;
-        hit.k00 = hit.k01 = hit.k11 = hit.k10 = R(0);
         if constexpr (kOneSet) load_cameras<S, 1>(a, t.b, n, ref_w, ref_h, cam);
-        if (n < N && d_ok)
-          reproject<NT, R>(cam, kOneSet ? 0 : n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
-        cnt += hit.off >= 0;
-        if constexpr (kRowSums) vmask |= (hit.off >= 0 ? 1u : 0u) << n;
+        reproject<NT, R>(cam, kOneSet ? 0 : n, depth, half, g.src_h_max, g.src_w_max, srcW, n < N && d_ok, hit);
+        const int off = PAD && hit.cell >= 0 ? hit.cell * C : hit.cell;
+        cnt += off >= 0;
+        if constexpr (kRowSums) vmask |= (off >= 0 ? 1u : 0u) << n;
         if constexpr (CORR == 4) {
           if (n < N && d_ok && t.pix_ok)
-            a.mask[(t.pix * D + d) * N + n] = hit.off >= 0 ? 1 : 0;
+            a.mask[(t.pix * D + d) * N + n] = off >= 0 ? 1 : 0;
         }
         if constexpr (LPP > 1) {
-          lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = hit.off;
+          lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = off;
           lds_at<R4>(smem, q4 * kR4, kWts + (n * LPP * PPW) * (int)sizeof(R4)) =
               R4{hit.k00, hit.k01, hit.k11, hit.k10};
         } else {
-          r_off[n] = hit.off;
+          r_off[n] = off;
           r_wts[n] = R4{hit.k00, hit.k01, hit.k11, hit.k10};
         }
       }
@@ -1136,11 +1190,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           if (off >= 0) {
             if (off != cur1) {
               cur1 = off;
-              const S *q = view[n] + off;
-              load_vec<S, VEC, false, GAP>(q, tp[0]);
-              load_vec<S, VEC, false, GAP>(q + C, tp[1]);
-              load_vec<S, VEC, false, GAP>(q + row_step + C, tp[2]);
-              load_vec<S, VEC, false, GAP>(q + row_step, tp[3]);
+              load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tp);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
@@ -1214,11 +1264,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               wt = r_wts[n];
             if (off != cur1) {
               cur1 = off;
-              const S *q = view[n] + off;
-              load_vec<S, VEC, false, GAP>(q, tap[0][0]);
-              load_vec<S, VEC, false, GAP>(q + C, tap[0][1]);
-              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[0][2]);
-              load_vec<S, VEC, false, GAP>(q + row_step, tap[0][3]);
+              load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tap[0]);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
@@ -1278,11 +1324,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             wt = r_wts[n];
           if (off != cur1) {
             cur1 = off;
-            const S *q = view[n] + off;
-            load_vec<S, VEC, false, GAP>(q, tp[0]);
-            load_vec<S, VEC, false, GAP>(q + C, tp[1]);
-            load_vec<S, VEC, false, GAP>(q + row_step + C, tp[2]);
-            load_vec<S, VEC, false, GAP>(q + row_step, tp[3]);
+            load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tp);
           }
           ++kcnt[jj];
           if constexpr (REDUCE == 1 || LIT) {
@@ -1411,11 +1453,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           if (off >= 0) {
             if (off != cur[n]) {
               cur[n] = off;
-              const S *q = view[n] + off;
-              load_vec<S, VEC, false, GAP>(q, tap[n][0]);
-              load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
-              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
-              load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
+              load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tap[n]);
             }
             R smp[VEC];
 #pragma unroll
@@ -1448,11 +1486,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           if (off >= 0) {
             if (off != cur[n]) {
               cur[n] = off;
-              const S *q = view[n] + off;
-              load_vec<S, VEC, false, GAP>(q, tap[n][0]);
-              load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
-              load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
-              load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
+              load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tap[n]);
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
@@ -1466,11 +1500,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         if (off >= 0) {
           if (off != cur[n]) {
             cur[n] = off;
-            const S *q = view[n] + off;
-            load_vec<S, VEC, false, GAP>(q, tap[n][0]);
-            load_vec<S, VEC, false, GAP>(q + C, tap[n][1]);
-            load_vec<S, VEC, false, GAP>(q + row_step + C, tap[n][2]);
-            load_vec<S, VEC, false, GAP>(q + row_step, tap[n][3]);
+            load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tap[n]);
           }
           if constexpr (REDUCE == 1 || LIT) {
             R val[VEC];
@@ -1678,13 +1708,12 @@ struct Window {
   static constexpr bool kPacked = SLOTS <= 256;  // four slot numbers fit one word
   static constexpr int kInside = (int)0x80000000u;  // flag in the key word: cell lies in the window
 
-  // slots of the taps 00, 01, 11, 10 of cell `key`, one byte each
-  static __device__ __forceinline__ unsigned pack_slots(int key) {
-    const int fh = (key >> 16) & 0x7fff, fw = key & 0xffff;
-    const int r0 = ring_row((unsigned)fh), ry0 = r0 * COLS, ry1 = ring_next<ROWS>(r0) * COLS;
-    const int rx0 = ring_col((unsigned)fw), rx1 = ring_next<COLS>(rx0);
-    return (unsigned)(ry0 + rx0) | ((unsigned)(ry0 + rx1) << 8) | ((unsigned)(ry1 + rx1) << 16) |
-           ((unsigned)(ry1 + rx0) << 24);
+  // slots of the taps 00, 01, 11, 10 of the cell in row `fh` (ring row r0) and column `fw`, one byte each
+  static __device__ __forceinline__ unsigned pack_slots(int r0, int r1, unsigned fw) {
+    const unsigned rx0 = (unsigned)ring_col(fw), rx1 = (unsigned)ring_next<COLS>((int)rx0);
+    const unsigned ry0 = (unsigned)(r0 * COLS), ry1 = (unsigned)(r1 * COLS);
+    // bytes: rx0, rx1, rx1, rx0 plus ry0, ry0, ry1, ry1 (v_perm_b32: selectors 0-3 take the second operand's bytes)
+    return __builtin_amdgcn_perm(rx1, rx0, 0x00040400u) + __builtin_amdgcn_perm(ry1, ry0, 0x04040000u);
   }
   // whole cell inside the window at origin (oy, ox)?
   static __device__ __forceinline__ bool inside(int key, int oy, int ox) {
@@ -1696,6 +1725,10 @@ struct Window {
 // Pixels of up to this many lanes update the scatter window in claimed tap-by-tap rounds
 // (see window_add), which needs one claim word per window slot.
 constexpr int kClaimLanes = 8;
+// ... and from two lanes on the claim words also say which slots hold something: negative where nothing was
+// added since the window last let go of the slot (window_move, tagged_rows).  With one lane per pixel a
+// pixel would write all four by itself (minimum of CostAggregate, three views of 4 channels, 256 x 320 x 32: 123 -> 130 us).
+constexpr bool tagged_slots(int lpp) { return lpp >= 2 && lpp <= kClaimLanes; }
 
 // LDS bytes of the backward kernel: the records of one chunk
 //   Four wts, dwt [NV*64] | int2 cell {slots, key|inside} [NV*64] | int off [NV*64] |
@@ -1733,15 +1766,41 @@ constexpr int backward_lds_bytes() {
          (LPP <= kClaimLanes ? WN::SLOTS * 4 : 0) + backward_list_bytes<R, VEC, LPP, FORM>();
 }
 
-// Minimum over the 64 lanes, in registers: four DPP steps reduce each row of 16 lanes,
-// four lane reads combine the rows.
-__device__ __forceinline__ int wave_min(int v) {
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));   // quad_perm 2,3,0,1
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
-  v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));  // row_mirror
-  return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-             min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+// The box around the cells of the active lanes of a wave (at least one): `lo` and `hi` hold a lane's smallest
+// and largest row and column, packed like a key, kNoLow and kNoHigh for a lane without a cell.  Rows and columns
+// are reduced together, in 16-bit halves, by DPP moves within and then across the rows of 16 lanes: 26
+// instructions, where four 32-bit reductions took 88 -- a spread sweep makes a box at nearly every depth.
+constexpr int kNoLow = 0x7fff7fff, kNoHigh = 0;
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ int min_halves(int a, int b) {
+  return __builtin_bit_cast(int, __builtin_elementwise_min(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
+}
+__device__ __forceinline__ int max_halves(int a, int b) {
+  return __builtin_bit_cast(int, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void box_step(int &lo, int &hi) {
+  int l, h;
+  if constexpr (ROWS == 0xf) {  // (every lane reads one: what the register held before is of no interest)
+    l = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true), h = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
+  } else {
+    l = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+    h = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+  }
+  lo = min_halves(lo, l), hi = max_halves(hi, h);
+}
+struct Box {
+  int y0, x0, y1, x1;  // first row and column of the cells, last ones of their texels (uniform)
+};
+__device__ __forceinline__ Box wave_box(int lo, int hi) {
+  box_step<0xB1, 0xf>(lo, hi);   // quad_perm 1,0,3,2
+  box_step<0x4E, 0xf>(lo, hi);   // quad_perm 2,3,0,1
+  box_step<0x141, 0xf>(lo, hi);  // row_half_mirror
+  box_step<0x140, 0xf>(lo, hi);  // row_mirror
+  box_step<0x142, 0xa>(lo, hi);  // row_bcast15 into rows 1 and 3
+  box_step<0x143, 0xc>(lo, hi);  // row_bcast31 into rows 2 and 3: lane 63 has everything
+  const int l = __builtin_amdgcn_readlane(lo, 63), h = __builtin_amdgcn_readlane(hi, 63);
+  return Box{l >> 16, l & 0xffff, (h >> 16) + 1, (h & 0xffff) + 1};
 }
 
 // Adds to element `e` of a view's image, whose 2^29 elements at most (make_plan) are addressed as the
@@ -1751,13 +1810,15 @@ __device__ __forceinline__ void atomic_at(R *image, unsigned e, R v) {
   atomic_add(reinterpret_cast<R *>(reinterpret_cast<char *>(image) + e * (unsigned)sizeof(R)), v);
 }
 
-// Moves the window of one view to origin (ny, nx): every texel that falls outside the new
-// window is written out with dense global atomics (C consecutive floats per texel, 64/C
-// texels per instruction, UN instructions per round: their LDS reads go out together) and its
-// slot is cleared.  Uniform control flow.  `cm`: channels of a texel in memory (a slot may be
-// padded; padding stays zero and is never written out).
+// Moves the window of one view to origin (ny, nx): every texel that was added to and falls outside the new
+// window is written out with dense global atomics (C consecutive floats per texel, 64/C texels per
+// instruction, UN instructions per round: their LDS reads go out together) and its slot is cleared.
+// Uniform control flow.  `tags`: see tagged_slots.  A spread sweep leaves some fifteen of the 48 or 64 slots at a
+// time; with the empty ones left out, the list holding offsets instead of indices and the box of wave_box six
+// wide-baseline views, 288 x 384 x 128, take 10.5 ms instead of 11.6.  `cm`:
+// channels of a texel in memory (a slot may be padded; padding stays zero and is never written out).
 template <int VEC, int LPP, int FORM = kPlainWindow, int UN = 4, typename R>
-__device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R *data,
+__device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R *data, int *tags,
                                             int *list, R *gview, int srcW, int lane, int cm) {
   using WN = Window<VEC, LPP, FORM>;
   if (oy != WN::kNone) {
@@ -1767,14 +1828,16 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R 
       const int s = sb + lane;  // (a window of 48 slots: the last lanes have none)
       const int ry = s / WN::COLS, rx = s % WN::COLS;
       const int y = WN::image_row(ry, oy), x = WN::image_col(rx, ox);
-      const bool leaving = s < WN::SLOTS && !((unsigned)(y - ny) < (unsigned)WN::ROWS &&
-                                              (unsigned)(x - nx) < (unsigned)WN::COLS);
+      bool leaving = s < WN::SLOTS && !((unsigned)(y - ny) < (unsigned)WN::ROWS &&
+                                        (unsigned)(x - nx) < (unsigned)WN::COLS);
+      if constexpr (tagged_slots(LPP)) leaving = leaving && tags[s] >= 0;
       const unsigned long long m = __ballot(leaving);
       if (leaving) {
         const int rank = count + (int)__builtin_amdgcn_mbcnt_hi(
             (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));  // leaving lanes below me
-        list[2 * rank] = s;
-        list[2 * rank + 1] = y * srcW + x;
+        list[2 * rank] = s * WN::STRIDE;
+        list[2 * rank + 1] = (y * srcW + x) * cm;
+        if constexpr (tagged_slots(LPP)) tags[s] = -1;
       }
       count += __popcll(m);
     }
@@ -1787,18 +1850,14 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R 
         int2 le[UN];
         R v[UN];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
-          const int e = e0 + u * EPI + sub_e;
-          le[u] = pairs[e < count ? e : 0];
-          if (e >= count) le[u].x = -1;
-        }
+        for (int u = 0; u < UN; ++u) le[u] = pairs[min(e0 + u * EPI + sub_e, count - 1)];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) v[u] = le[u].x >= 0 ? data[le[u].x * WN::STRIDE + j] : R(0);
+        for (int u = 0; u < UN; ++u) v[u] = data[le[u].x + j];
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
-          if (v[u] != R(0)) {
-            data[le[u].x * WN::STRIDE + j] = R(0);
-            atomic_at(gview, (unsigned)le[u].y * (unsigned)cm + (unsigned)j, v[u]);
+          if (e0 + u * EPI + sub_e < count && v[u] != R(0)) {
+            data[le[u].x + j] = R(0);
+            atomic_at(gview, (unsigned)le[u].y + (unsigned)j, v[u]);
           }
         }
       }
@@ -1809,7 +1868,7 @@ __device__ __forceinline__ void window_move(int &oy, int &ox, int ny, int nx, R 
   ox = nx;
 }
 
-// Bitwise OR over the 64 lanes, in registers (as wave_min).
+// Bitwise OR over the 64 lanes, in registers.
 __device__ __forceinline__ unsigned wave_or(unsigned v) {
   v |= (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xf, 0xf, false);
   v |= (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xf, 0xf, false);
@@ -1819,9 +1878,30 @@ __device__ __forceinline__ unsigned wave_or(unsigned v) {
          (unsigned)__builtin_amdgcn_readlane((int)v, 32) | (unsigned)__builtin_amdgcn_readlane((int)v, 48);
 }
 
+// The ring rows of a window that hold something: those with a tag that is not negative (uniform).
+template <int VEC, int LPP, int FORM>
+__device__ __forceinline__ unsigned tagged_rows(const int *tags, int lane) {
+  using WN = Window<VEC, LPP, FORM>;
+  unsigned rows = 0u;
+#pragma unroll
+  for (int sb = 0; sb < WN::SLOTS; sb += 64) {
+    const int s = sb + lane;
+    const bool held = s < WN::SLOTS && tags[s] >= 0;
+    if constexpr (64 % WN::COLS == 0) {
+      const unsigned long long m = __ballot(held);
+#pragma unroll
+      for (int r = 0; r < 64 / WN::COLS; ++r)
+        rows |= (m >> (r * WN::COLS) & ((1ull << WN::COLS) - 1ull) ? 1u : 0u) << (sb / WN::COLS + r);
+    } else {
+      rows |= wave_or(held ? 1u << (s / WN::COLS) : 0u);
+    }
+  }
+  return rows;
+}
+
 // Writes out everything a window holds, when its view is done: row by row of the ring
-// buffer, and only the rows some accepted cell of this view ever mapped to (`rows`: bit r
-// set when a cell used ring row r; a short sweep over few hypotheses touches three or four
+// buffer, and only the rows that hold something, or that some accepted cell of this view ever
+// mapped to (`rows`: bit r set when a cell used ring row r; a short sweep over few hypotheses touches three or four
 // of the eight, and the untouched ones need neither their LDS reads nor their address
 // arithmetic).  All LDS reads of a row are issued together, then its atomics.
 template <int VEC, int LPP, int FORM = kPlainWindow, typename R>
@@ -1892,8 +1972,8 @@ __device__ __forceinline__ R add_tap_sum(R old, T (&v)[NS], const R (&ref)[VEC],
   else return mad(ref[c], v[c * NS / VEC][k], old);
 }
 
-// Adds the four tap images of a finished run into the window (a cell that sticks out of the
-// window never gets here: flush_cells_to_memory takes it).  Called from divergent code by all
+// Adds the four tap images of a finished run into the window (its cell lies inside: one that sticks out
+// never gets here, flush_cells_to_memory has taken it).  Called from divergent code by all
 // LPP lanes of every pixel whose run just ended.  Float LDS atomics cost about three cycles
 // per lane, so the window sums are updated with plain 16-byte read-add-write.  Cells of
 // different pixels overlap (a texel is tap 01 of one cell and tap 00 of its neighbour).
@@ -1910,91 +1990,80 @@ template <int VEC, int LPP, bool LEAN = false, int FORM = kPlainWindow, int GAP 
 __device__ __forceinline__ void window_add(unsigned slots, int key, T (&v)[NS], const R (&ref)[VEC], R *data,
                                            int *tags, int lane, int cl) {
   using WN = Window<VEC, LPP, FORM>;
-  if (key < 0) {
-    // the whole cell lies inside the window (the usual case)
-    if constexpr (!WN::kPacked) slots = 0;
-    int slot[4];
-    if constexpr (WN::kPacked) {
-      slot[0] = slots & 255u, slot[1] = (slots >> 8) & 255u, slot[2] = (slots >> 16) & 255u,
-      slot[3] = slots >> 24;
-    } else {
-      const int fh = (key >> 16) & 0x7fff, fw = key & 0xffff;
-      const int ry0 = WN::ring_row((unsigned)fh) * WN::COLS, ry1 = WN::ring_row((unsigned)fh + 1u) * WN::COLS;
-      const int rx0 = WN::ring_col((unsigned)fw), rx1 = WN::ring_col((unsigned)fw + 1u);
-      slot[0] = ry0 + rx0, slot[1] = ry0 + rx1, slot[2] = ry1 + rx1, slot[3] = ry1 + rx0;
+  int slot[4];
+  if constexpr (WN::kPacked) {
+    slot[0] = slots & 255u, slot[1] = (slots >> 8) & 255u, slot[2] = (slots >> 16) & 255u, slot[3] = slots >> 24;
+  } else {
+    const int fh = (key >> 16) & 0x7fff, fw = key & 0xffff;
+    const int ry0 = WN::ring_row((unsigned)fh) * WN::COLS, ry1 = WN::ring_row((unsigned)fh + 1u) * WN::COLS;
+    const int rx0 = WN::ring_col((unsigned)fw), rx1 = WN::ring_col((unsigned)fw + 1u);
+    slot[0] = ry0 + rx0, slot[1] = ry0 + rx1, slot[2] = ry1 + rx1, slot[3] = ry1 + rx0;
+  }
+  unsigned char *const base = reinterpret_cast<unsigned char *>(data + lane_first(cl, GAP));
+  R *texel[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) texel[k] = reinterpret_cast<R *>(base + slot[k] * (WN::STRIDE * (int)sizeof(R)));
+  auto all_at_once = [&]() __attribute__((always_inline)) {
+    R old[4][VEC];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) slot_read<GAP>(texel[k], old[k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) old[k][i] = add_tap_sum(old[k][i], v, ref, i, k);
+      slot_write<GAP>(texel[k], old[k]);
     }
-    R *base = data + lane_first(cl, GAP);
-    if constexpr (LPP > kClaimLanes) {
-      unsigned long long firing = __ballot(true);
-      while (firing) {
-        const int lead = __ffsll((long long)firing) - 1;
-        firing &= ~(((1ull << LPP) - 1ull) << lead);  // retire this pixel's lanes
-        if (lane - cl == lead) {
-          R old[4][VEC];
+  };
+  // (one tap after the other; `shared`: the next tap may be the texel another pixel has just updated -- the
+  // LDS keeps a wave's operations in order, the compiler is held to it here)
+  auto one_by_one = [&](bool shared) __attribute__((always_inline)) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) slot_read<GAP>(base + slot[k] * WN::STRIDE, old[k]);
+    for (int k = 0; k < 4; ++k) {
+      R old[VEC];
+      slot_read<GAP>(texel[k], old);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] = add_tap_sum(old[k][i], v, ref, i, k);
-            slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
-          }
-        }
-        if (firing) wave_sync();
-      }
+      for (int i = 0; i < VEC; ++i) old[i] = add_tap_sum(old[i], v, ref, i, k);
+      slot_write<GAP>(texel[k], old);
+      if (shared) wave_sync();
+    }
+  };
+  if constexpr (LPP > kClaimLanes) {
+    unsigned long long firing = __ballot(true);
+    while (firing) {
+      const int lead = __ffsll((long long)firing) - 1;
+      firing &= ~(((1ull << LPP) - 1ull) << lead);  // retire this pixel's lanes
+      if (lane - cl == lead) all_at_once();
+      if (firing) wave_sync();
+    }
+  } else {
+    const int me = lane - cl;  // the same in all lanes of a pixel
+    if (__popcll(__ballot(true)) == LPP) {
+      // one pixel alone (four of ten events on the headline workload): nothing to collide with, its four
+      // taps go in flight together -- or, in a kernel held to a register budget, one after the other
+      // (twelve registers less at the kernel's peak)
+      if constexpr (LEAN) one_by_one(false);
+      else all_at_once();
     } else {
-      const int me = lane - cl;  // the same in all lanes of a pixel
+      // (the wave leaves this loop together: a pixel that left it by itself would add after it, beside the others)
       bool pending = true;
-      if (__popcll(__ballot(true)) == LPP) {
-        // one pixel alone (four of ten events on the headline workload): nothing to
-        // collide with, its four taps go in flight together -- or, in a kernel held to a
-        // register budget, one after the other (twelve registers less at the kernel's peak)
-        if constexpr (LEAN) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            R old[VEC];
-            slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] = add_tap_sum(old[i], v, ref, i, k);
-            slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
-          }
-        } else {
-          R old[4][VEC];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) slot_read<GAP>(base + slot[k] * WN::STRIDE, old[k]);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) old[k][i] = add_tap_sum(old[k][i], v, ref, i, k);
-            slot_write<GAP>(base + slot[k] * WN::STRIDE, old[k]);
-          }
-        }
-        pending = false;
-      }
-      while (pending) {
+      do {
         if (pending) tags[slot[0]] = me;
         wave_sync();
         const bool go = pending && tags[slot[0]] == me;
-        if (go) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            R old[VEC];
-            slot_read<GAP>(base + slot[k] * WN::STRIDE, old);
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) old[i] = add_tap_sum(old[i], v, ref, i, k);
-            slot_write<GAP>(base + slot[k] * WN::STRIDE, old);
-            // (the next tap may be the texel another pixel has just updated: the LDS keeps a
-            // wave's operations in order, the compiler is held to it here)
-            wave_sync();
-          }
-        }
+        if (go) one_by_one(true);
         pending = pending && !go;
-        if (__ballot(pending) == 0ull) break;
-      }
-      wave_sync();
+      } while (__ballot(pending) != 0ull);
     }
+    if constexpr (tagged_slots(LPP)) {  // these four slots hold something now
+#pragma unroll
+      for (int i = 0; i < (LPP >= 4 ? 1 : 2); ++i) {
+        const unsigned k = (unsigned)(cl + i * LPP) & 3u;
+        static_assert(WN::kPacked, "slot numbers of a byte");
+        tags[(slots >> (k * 8u)) & 255u] = me;
+      }
+    }
+    wave_sync();
   }
-  // (a cell that sticks out of the window never gets here: flush_cells_to_memory took it)
 #pragma unroll
   for (int i = 0; i < NS; ++i) v[i] = T{R(0), R(0), R(0), R(0)};
 }
@@ -2165,7 +2234,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   extern __shared__ __align__(16) unsigned char smem[];
   Tile<LPP> t;
   if (!locate_tile<S, LPP, EIGHT == kEightTall>(a, g, t)) return;
-  const int C = (int)a.C, D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
+  const int C = PAD ? (int)a.C : VEC * LPP;
+  constexpr int kUnit = cell_unit(VEC * LPP, PAD);
+  const int D = (int)a.D, N = (int)a.N, srcH = (int)a.srcH, srcW = (int)a.srcW;
   const R half = a.half;
   constexpr bool per_voxel_depth = PV;
   constexpr bool kDstWords = !kSlim || PV;
@@ -2296,6 +2367,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   }
   for (int k = t.lane * 4; k < NV * WN::SLOTS * WN::STRIDE; k += 256)
     *reinterpret_cast<R4 *>(s_data + k) = R4{R(0), R(0), R(0), R(0)};
+  if constexpr (tagged_slots(LPP))
+    for (int k = t.lane; k < WN::SLOTS; k += 64) s_tags[k] = -1;
   Cameras<NV, R> cam;
   if constexpr (!kSlim)
     load_cameras<S, NV>(a, t.b, t.view0, static_cast<R>(t.w) + half, static_cast<R>(t.h) + half, cam);
@@ -2315,7 +2388,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   R proj[NV][4][kRunSums && DG ? GV : 1];  // kRunSums: the taps of the open run against the reference, per group
   int cur[NV];     // tap offset of the open run, -1: none
   int2 cell[NV];   // its slots and key (bit 31: inside the window)
-  unsigned ring_rows[NV];  // ring rows of the window this lane's accepted cells mapped to
+  unsigned ring_rows[NV];  // (without tags) ring rows of the window this lane's accepted cells mapped to
 #pragma unroll
   for (int n = 0; n < NV; ++n) {
     cur[n] = -1;
@@ -2370,12 +2443,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     const unsigned long long outside = __ballot(fire && !in);
     if (outside != 0ull) {
       if (kFewRuns == 0 || __popcll(outside) > kFewRuns * LPP) {
-        const int fh = key >> 16, fw = key & 0xffff;
-        const int ny = wave_min(fire ? fh : WN::kNone), nx = wave_min(fire ? fw : WN::kNone);
-        const int hy = -wave_min(fire ? -fh : WN::kNone) + 1, hx = -wave_min(fire ? -fw : WN::kNone) + 1;
-        const int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
-        window_move<VEC, LPP, kForm, 2>(oy[n], ox[n], ny - (sy > 0 ? sy / 2 : 0), nx - (sx > 0 ? sx / 2 : 0),
-                                    s_data + n * WN::SLOTS * WN::STRIDE, s_move_list, gview[n], srcW, lane, cm);
+        const Box b = wave_box(fire ? key : kNoLow, fire ? key : kNoHigh);
+        const int sy = WN::ROWS - (b.y1 - b.y0 + 1), sx = WN::COLS - (b.x1 - b.x0 + 1);
+        window_move<VEC, LPP, kForm, 2>(oy[n], ox[n], b.y0 - (sy > 0 ? sy / 2 : 0), b.x0 - (sx > 0 ? sx / 2 : 0),
+                                    s_data + n * WN::SLOTS * WN::STRIDE, s_tags, s_move_list, gview[n], srcW, lane, cm);
         in = WN::inside(key, oy[n], ox[n]);
       }
       const bool out = fire && !in;
@@ -2514,6 +2585,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
         asm volatile("" : "+v"(cam_w), "+v"(cam_h));
         load_cameras<S, NV>(a, t.b, t.view0, static_cast<R>(cam_w) + half, static_cast<R>(cam_h) + half, cam);
       }
+      static_assert(NV == 1, "one view at a time");
+      bool nothing = false;
       R scl = R(0);
       if constexpr (REDUCE == 0) {
         if (cnt > 0) {
@@ -2539,58 +2612,60 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
       }
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
+        // A chunk without a voxel that counts -- outside this view, or, where every voxel has one winner, won by
+        // the others -- leaves everything as it is.  (Not where every voxel's depth gradient is stored.)
+        if (!PV && kWinners && __ballot(scl != R(0)) == 0ull) {
+          nothing = true;
+          break;
+        }
         Hit<R> hit;
-        hit.off = -1;
-        hit.key = 0;
-        hit.k00 = hit.k01 = hit.k11 = hit.k10 = R(0);
-        hit.dh = hit.dw = R(0);
+        reproject<NV, R>(cam, n, depth, half, g.src_h_max, g.src_w_max, srcW, t.view0 + n < N && scl != R(0), hit);
+        if (!PV && __ballot(hit.cell >= 0) == 0ull) {
+          nothing = true;
+          break;
+        }
         R4 dw4 = R4{R(0), R(0), R(0), R(0)};
-        if (t.view0 + n < N && scl != R(0)) {
-          reproject<NV, R>(cam, n, depth, half, g.src_h_max, g.src_w_max, srcW, C, hit);
-          if (DG && hit.off >= 0) {
-            // d(sample)/d(depth) = sum over taps of dwt * tap, from
-            //   d/d(src_h) = t1*dw + (t10 - t00),  d/d(src_w) = t1*dh + (t01 - t00),
-            //   t1 = t11 - t10 - t01 + t00, chained through the perspective divide.
-            const R inv = quick_recip(hit.z * hit.z);
-            const R ah = (cam.hc[n] * hit.z - cam.zc[n] * hit.h3d) * inv;
-            const R aw = (cam.wc[n] * hit.z - cam.zc[n] * hit.w3d) * inv;
-            const R cp = ah * hit.dw + aw * hit.dh;
-            dw4 = R4{cp - ah - aw, aw - cp, cp, ah - cp};
-            if constexpr (kSlim) dw4 = R4{R(0), R(0), ah, aw};  // taps 00, 01, 11, 10
-          }
+        if constexpr (DG) {
+          // d(sample)/d(depth) = sum over taps of dwt * tap, from
+          //   d/d(src_h) = t1*dw + (t10 - t00),  d/d(src_w) = t1*dh + (t01 - t00),
+          //   t1 = t11 - t10 - t01 + t00, chained through the perspective divide.
+          const R inv = quick_recip(hit.z * hit.z);
+          const R ah = (cam.hc[n] * hit.z - cam.zc[n] * hit.h3d) * inv;
+          const R aw = (cam.wc[n] * hit.z - cam.zc[n] * hit.w3d) * inv;
+          const R cp = ah * hit.dw + aw * hit.dh;
+          dw4 = R4{cp - ah - aw, aw - cp, cp, ah - cp};
+          if constexpr (kSlim) dw4 = R4{R(0), R(0), ah, aw};  // taps 00, 01, 11, 10
         }
         // The scatter window has to cover this chunk's cells and the cell still open from
         // the last chunk.  Usually it already does (one vote); otherwise it is centred on
         // their bounding box.  A box larger than the window: the window follows the runs that
         // end, depth by depth (end_spread_runs).
-        const bool valid = hit.off >= 0;
-        if (valid) {
-          const int r0 = WN::ring_row((unsigned)hit.key >> 16);
-          ring_rows[n] |= (1u << r0) | (1u << WN::template ring_next<WN::ROWS>(r0));
+        const bool valid = hit.cell >= 0;
+        if constexpr (kMatrix) {  // (the matrix cores multiply the weights of lanes without a sample too, by zero)
+          if (!valid) hit.k00 = hit.k01 = hit.k11 = hit.k10 = R(0);
         }
+        const int r0 = WN::ring_row((unsigned)hit.key >> 16 & 0x7fffu), r1 = WN::template ring_next<WN::ROWS>(r0);
+        if constexpr (!tagged_slots(LPP))
+          if (valid) ring_rows[n] |= (1u << r0) | (1u << r1);
         bool in_new = !valid || WN::inside(hit.key, oy[n], ox[n]);
         spread[n] = false;
         if (__ballot(!(in_new && (cur[n] < 0 || cell[n].y < 0))) != 0ull) {
-          int my = WN::kNone, mx = WN::kNone, My = -WN::kNone, Mx = -WN::kNone;
-          if (valid) my = My = hit.key >> 16, mx = Mx = hit.key & 0xffff;
+          int lo = valid ? hit.key : kNoLow, hi = valid ? hit.key : kNoHigh;
           if (cur[n] >= 0) {
-            const int cy = (cell[n].y >> 16) & 0x7fff, cx = cell[n].y & 0xffff;
-            my = min(my, cy), mx = min(mx, cx), My = max(My, cy), Mx = max(Mx, cx);
+            const int open = cell[n].y & 0x7fffffff;
+            lo = min_halves(lo, open), hi = max_halves(hi, open);
           }
-          int ny = wave_min(my), nx = wave_min(mx);
-          int hy = -wave_min(-My) + 1, hx = -wave_min(-Mx) + 1;  // last row / column used
-          int sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);  // slack
+          Box b = wave_box(lo, hi);
+          int sy = WN::ROWS - (b.y1 - b.y0 + 1), sx = WN::COLS - (b.x1 - b.x0 + 1);  // slack
           spread[n] = sy < 0 || sx < 0;
           if constexpr (kEndLeft) {
             if (spread[n] && __ballot(valid) != 0ull) {
               // without the open runs: where the chunk's cells fit, the runs it leaves behind end
-              const int fh = hit.key >> 16, fw = hit.key & 0xffff;
-              ny = wave_min(valid ? fh : WN::kNone), nx = wave_min(valid ? fw : WN::kNone);
-              hy = -wave_min(valid ? -fh : WN::kNone) + 1, hx = -wave_min(valid ? -fw : WN::kNone) + 1;
-              sy = WN::ROWS - (hy - ny + 1), sx = WN::COLS - (hx - nx + 1);
+              b = wave_box(valid ? hit.key : kNoLow, valid ? hit.key : kNoHigh);
+              sy = WN::ROWS - (b.y1 - b.y0 + 1), sx = WN::COLS - (b.x1 - b.x0 + 1);
               spread[n] = sy < 0 || sx < 0;
               const int key = cell[n].y & 0x7fffffff;
-              const bool left = !spread[n] && cur[n] >= 0 && !WN::inside(key, ny - sy / 2, nx - sx / 2);
+              const bool left = !spread[n] && cur[n] >= 0 && !WN::inside(key, b.y0 - sy / 2, b.x0 - sx / 2);
               const unsigned long long m = __ballot(left);
               if (m != 0ull) {
                 if (left) take_run(n);
@@ -2603,16 +2678,16 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             in_new = false;  // decided when the run ends
             cell[n].y &= 0x7fffffff;
           } else {
-            window_move<VEC, LPP, kForm>(oy[n], ox[n], ny - sy / 2, nx - sx / 2,
-                                  s_data + n * WN::SLOTS * WN::STRIDE, s_list, gview[n], srcW, t.lane, cm);
+            window_move<VEC, LPP, kForm>(oy[n], ox[n], b.y0 - sy / 2, b.x0 - sx / 2,
+                                  s_data + n * WN::SLOTS * WN::STRIDE, s_tags, s_list, gview[n], srcW, t.lane, cm);
             in_new = true;
             cell[n].y |= WN::kInside;
           }
         }
-        const int2 rec = make_int2(WN::kPacked ? (int)WN::pack_slots(hit.key) : 0,
+        const int2 rec = make_int2(WN::kPacked ? (int)WN::pack_slots(r0, r1, (unsigned)hit.key & 0xffffu) : 0,
                                    (valid && in_new) ? (hit.key | WN::kInside) : hit.key);
         if constexpr (LPP > 1) {
-          lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = hit.off;
+          lds_at<int>(smem, q4, kOff + (n * LPP * PPW) * 4) = PAD && valid ? hit.cell * C : hit.cell;
           lds_at<int2>(smem, q4 * 2u, kCell + (n * LPP * PPW) * 8) = rec;
           if constexpr (kSlim) {
             lds_at<R4>(smem, qw, kWts + (n * LPP * PPW) * kB4) = R4{hit.dh, hit.dw, dw4.z, dw4.w};
@@ -2621,12 +2696,13 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             if constexpr (DG) lds_at<R4>(smem, qw, kDwt + (n * LPP * PPW) * kB4) = dw4;
           }
         } else {
-          r_off[n] = hit.off;
+          r_off[n] = hit.cell;
           r_cell[n] = rec;
           r_wts[n] = R4{hit.k00, hit.k01, hit.k11, hit.k10};
           r_dwt[n] = dw4;
         }
       }
+      if (nothing) continue;
       if constexpr (LPP > 1) {
         lds_at<R>(smem, q1, kScl) = scl;
         if constexpr (best_pair_op(CORR))
@@ -2762,17 +2838,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               // above, which left cur[n] = -1)
               // the run on the previous cell ends.  Start fetching the new cell's taps
               // first, then hand the old cell's image to the window while they arrive.
-              // byte offsets in 32 bits: the loads take the view's base from scalar registers
               if constexpr (kRunSums)
                 if (cur[n] >= 0) take_run(n);
-              const unsigned e0 = ((unsigned)off + lane_ch) * (unsigned)sizeof(S);
-              const unsigned e1 = e0 + (unsigned)row_step * (unsigned)sizeof(S);
-              const char *vb = reinterpret_cast<const char *>(view[n]);
-              const unsigned cb = (unsigned)C * (unsigned)sizeof(S);
-              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + e0), tap[n][0]);
-              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + (e0 + cb)), tap[n][1]);
-              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + (e1 + cb)), tap[n][2]);
-              load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(vb + e1), tap[n][3]);
+              load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, lane_ch, tap[n]);
               if (cur[n] >= 0)
                 window_add<VEC, LPP, kLean, kForm, GAP>((unsigned)cell[n].x, cell[n].y, sg[n], ref,
                                             s_data + n * WN::SLOTS * WN::STRIDE, s_tags, t.lane, t.cl);
@@ -2922,7 +2990,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
   for (int n = 0; n < NV; ++n)
     window_flush_all<VEC, LPP, kForm>(oy[n], ox[n], s_data + n * WN::SLOTS * WN::STRIDE, gview[n], srcW,
-                               t.lane, wave_or(ring_rows[n]), cm);
+                               t.lane, tagged_slots(LPP) ? tagged_rows<VEC, LPP, kForm>(s_tags, t.lane) : wave_or(ring_rows[n]),
+                               cm);
   wave_sync();  // the next view clears the window
   }  // views of the group
 
