@@ -1290,6 +1290,13 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
       // (double: blocks of four depths, whose accumulators take the registers of eight in float)
       constexpr int kMostDB = sizeof(R) == 8 ? 4 : 8;
       constexpr int DB = LPP < kMostDB ? LPP : kMostDB;
+      // Two views side by side where the registers hold two sets of taps: their gathers are in flight
+      // together, and what these kernels do most is wait for them (six wide-baseline views, VALU 45 %, waiting
+      // 75 % of the waves' time: 4.6 -> 4.3 ms; 200 x 260 x 96 477 -> 435 us, five views, 128 x 160 x 48, 85.7 ->
+      // 80.9; 16 channels, six views, 148 -> 128, four 108 -> 103; minima 2-4 %).  Not with 16-bit taps, which
+      // are widened, and so waited for, as soon as they are loaded (five views 94 -> 96), nor in double.
+      constexpr int VW = sizeof(S) == 4 && NV % 2 == 0 && LPP >= 4 ? 2 : 1;
+      static_assert(NV % VW == 0, "whole groups of views");
 #pragma unroll
       for (int j0 = 0; j0 < LPP; j0 += DB) {
       R acc[DB][VEC];
@@ -1305,33 +1312,41 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
         }
       }
 #pragma unroll
-      for (int n = 0; n < NV; ++n) {
-        int cur1 = -1;
-        R tp[4][VEC];
+      for (int n = 0; n < NV; n += VW) {
+        int cur1[VW];
+        R tp[VW][4][VEC];
+#pragma unroll
+        for (int v = 0; v < VW; ++v) cur1[v] = -1;
 #pragma unroll
         for (int jj = 0; jj < DB; ++jj) {
           if (d0 + j0 + jj >= d_hi) continue;
-          int off;  // -1 also for a view beyond N (phase 1 leaves those records empty)
-          if constexpr (LPP > 1)
-            off = lds_at<int>(smem, p4, kOff + ((n * LPP + j0 + jj) * PPW) * 4);
-          else
-            off = r_off[n];
-          if (off < 0) continue;
-          R4 wt;
-          if constexpr (LPP > 1)
-            wt = lds_at<R4>(smem, p4 * kR4, kWts + ((n * LPP + j0 + jj) * PPW) * (int)sizeof(R4));
-          else
-            wt = r_wts[n];
-          if (off != cur1) {
-            cur1 = off;
-            load_cell<S, VEC, GAP, kUnit>(view[n], off, C, row_step, (unsigned)ch0, tp);
+          int off[VW];  // -1 also for a view beyond N (phase 1 leaves those records empty)
+          R4 wt[VW];
+#pragma unroll
+          for (int v = 0; v < VW; ++v) {
+            if constexpr (LPP > 1)
+              off[v] = lds_at<int>(smem, p4, kOff + (((n + v) * LPP + j0 + jj) * PPW) * 4);
+            else
+              off[v] = r_off[n + v];
+            if (off[v] < 0) continue;
+            if constexpr (LPP > 1)
+              wt[v] = lds_at<R4>(smem, p4 * kR4, kWts + (((n + v) * LPP + j0 + jj) * PPW) * (int)sizeof(R4));
+            else
+              wt[v] = r_wts[n + v];
+            if (off[v] != cur1[v]) {
+              cur1[v] = off[v];
+              load_cell<S, VEC, GAP, kUnit>(view[n + v], off[v], C, row_step, (unsigned)ch0, tp[v]);
+            }
           }
+#pragma unroll
+          for (int v = 0; v < VW; ++v) {
+          if (off[v] < 0) continue;
           ++kcnt[jj];
           if constexpr (REDUCE == 1 || LIT) {
             R val[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const R smp = wt.x * tp[0][c] + wt.y * tp[1][c] + wt.z * tp[2][c] + wt.w * tp[3][c];
+              const R smp = wt[v].x * tp[v][0][c] + wt[v].y * tp[v][1][c] + wt[v].z * tp[v][2][c] + wt[v].w * tp[v][3][c];
               if (CORR == 0) {
                 const R diff = smp - ref[c];
                 val[c] = diff * diff;
@@ -1347,27 +1362,28 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             } else if (CORR == 0) {
 #pragma unroll
               for (int c = 0; c < VEC; ++c)
-                if (acc[jj][c] > val[c]) acc[jj][c] = val[c], arg[jj][c] = n;
+                if (acc[jj][c] > val[c]) acc[jj][c] = val[c], arg[jj][c] = n + v;
             } else {
-              keep_larger_groups(acc[jj], arg[jj], val, g.sub, t.cl, n);
+              keep_larger_groups(acc[jj], arg[jj], val, g.sub, t.cl, n + v);
             }
           } else {
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
               if (CORR != 1) {
-                R diff = mad(wt.x, tp[0][c], -ref[c]);
-                diff = mad(wt.y, tp[1][c], diff);
-                diff = mad(wt.z, tp[2][c], diff);
-                diff = mad(wt.w, tp[3][c], diff);
+                R diff = mad(wt[v].x, tp[v][0][c], -ref[c]);
+                diff = mad(wt[v].y, tp[v][1][c], diff);
+                diff = mad(wt[v].z, tp[v][2][c], diff);
+                diff = mad(wt[v].w, tp[v][3][c], diff);
                 acc[jj][c] = mad(diff, diff, acc[jj][c]);
               } else {
-                R smp = wt.x * tp[0][c];
-                smp = mad(wt.y, tp[1][c], smp);
-                smp = mad(wt.z, tp[2][c], smp);
-                smp = mad(wt.w, tp[3][c], smp);
+                R smp = wt[v].x * tp[v][0][c];
+                smp = mad(wt[v].y, tp[v][1][c], smp);
+                smp = mad(wt[v].z, tp[v][2][c], smp);
+                smp = mad(wt[v].w, tp[v][3][c], smp);
                 acc[jj][c] = mad(smp, ref[c], acc[jj][c]);
               }
             }
+          }
           }
         }
       }
