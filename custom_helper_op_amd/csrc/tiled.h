@@ -585,13 +585,38 @@ __device__ __forceinline__ void reproject(const Cameras<NV, R> &c, int n, R dept
   r.key = (fh << 16) | (fw & 0xffff);
 }
 
+// Four taps of a cell, this lane's channels, in the arithmetic type -- or (RAW, f16 under a mean) as loaded: a
+// multiply-add takes half-precision factors as they are (v_fma_mix_f32, the same single rounding), so the
+// sixteen conversions at every cell change, which wait for the loads, and half the registers are not needed.
+// (f16: cascade stage, four views of 16 channels, 256 x 320 x 32, gradient 219 -> 201 us, forward 85 -> 78; 32
+// channels, two views, 128 x 160 x 96, 172 -> 164 and 61 -> 57; 8 channels, four views, 512 x 640 x 8, 67 -> 60.)
+// Literal forms round the product by itself, which costs them a conversion per depth: they keep the widened taps.
+template <typename S, int VEC, bool RAW = false>
+struct Taps {
+  typename Storage<S>::Real v[4][VEC];
+  __device__ __forceinline__ typename Storage<S>::Real operator()(int k, int c) const { return v[k][c]; }
+  template <int GAP>
+  __device__ __forceinline__ void load(int k, const S *p) { load_vec<S, VEC, false, GAP>(p, v[k]); }
+};
+template <int VEC>
+struct Taps<__half, VEC, true> {
+  uint32_t w[4][VEC / 2];
+  __device__ __forceinline__ float operator()(int k, int c) const {
+    return __half2float(__ushort_as_half((unsigned short)(c & 1 ? w[k][c / 2] >> 16 : w[k][c / 2] & 0xffffu)));
+  }
+  template <int GAP>
+  __device__ __forceinline__ void load(int k, const __half *p) { load_raw<__half, VEC, false, GAP>(p, w[k]); }
+};
+template <typename S>
+constexpr bool is_half() { return std::is_same<S, __half>::value; }
+
 // The four taps (00, 01, 11, 10) of a cell, this lane's channels: the view's uniform base and 32 bits of
 // bytes (an image has less than 2^29 elements, make_plan).  `cell` counts units of UNIT elements: texels, or
 // elements where the channel count is a run-time value (its product is then formed once per voxel).
 constexpr int cell_unit(int channels, bool pad) { return pad ? 1 : channels; }
-template <typename S, int VEC, int GAP, int UNIT>
+template <typename S, int VEC, int GAP, int UNIT, bool RAW>
 __device__ __forceinline__ void load_cell(const S *view, int cell, int C, int row_step, unsigned lane_ch,
-                                          typename Storage<S>::Real (&tap)[4][VEC]) {
+                                          Taps<S, VEC, RAW> &tap) {
   const unsigned e0 = ((unsigned)cell * (unsigned)UNIT + lane_ch) * (unsigned)sizeof(S);
   const unsigned e1 = e0 + (unsigned)row_step * (unsigned)sizeof(S);
   const char *base = reinterpret_cast<const char *>(view);
@@ -600,10 +625,10 @@ __device__ __forceinline__ void load_cell(const S *view, int cell, int C, int ro
   const char *row0 = base + e0, *row1 = base + e1;
   const char *right0 = UNIT > 1 ? row0 + UNIT * sizeof(S) : base + (e0 + step);
   const char *right1 = UNIT > 1 ? row1 + UNIT * sizeof(S) : base + (e1 + step);
-  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(row0), tap[0]);
-  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(right0), tap[1]);
-  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(right1), tap[2]);
-  load_vec<S, VEC, false, GAP>(reinterpret_cast<const S *>(row1), tap[3]);
+  tap.template load<GAP>(0, reinterpret_cast<const S *>(row0));
+  tap.template load<GAP>(1, reinterpret_cast<const S *>(right0));
+  tap.template load<GAP>(2, reinterpret_cast<const S *>(right1));
+  tap.template load<GAP>(3, reinterpret_cast<const S *>(row1));
 }
 
 template <typename S>
@@ -1001,6 +1026,13 @@ constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce, bool wide
   return nv >= 5 ? 4 : (nv >= 3 && lpp == 4) ? 5 : 1;
 }
 
+// At most five waves per SIMD: with six (the two-view instantiation needs only 80 VGPRs)
+// the waves of a CU evict each other's taps from L1 and the kernel is 6 % slower.  The minimum of three and
+// four views of 16 channels likewise with five instead of four (f16, 200 x 260 x 32: 85.8 against 81.6 us).
+constexpr int forward_max_waves(int lpp, int nv, int corr, int reduce) {
+  return reduce != 0 && corr == 0 && lpp == 4 && nv >= 3 && nv <= 4 ? 4 : 5;
+}
+
 // LIT: the mean in the reference's operand order too, every operation rounded by itself, so that the
 // result is the plain evaluation's to the bit.  Double is always evaluated that way: the rows are
 // twice as long and the stores bound the launch as before (two views, 32 channels, 128 x 160 x 192:
@@ -1014,11 +1046,10 @@ constexpr int forward_min_waves(int lpp, int nv, int corr, int reduce, bool wide
 // over five views, 63 x 85 x 37, 47 -> 36 us).
 template <typename S, int VEC, int LPP, int NV, int CORR, int REDUCE = 0, bool PAD = false,
           bool LIT = (sizeof(S) == 8 || PAD)>
-// At most five waves per SIMD: with six (the two-view instantiation needs only 80 VGPRs)
-// the waves of a CU evict each other's taps from L1 and the kernel is 6 % slower.  The lower
-// bound: see forward_min_waves.
+// (waves per SIMD: see forward_min_waves and forward_max_waves)
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, sizeof(S) == 8), 5))) void forward_kernel(
+__attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, sizeof(S) == 8),
+                                   forward_max_waves(LPP, NV, CORR, REDUCE)))) void forward_kernel(
     const Args<S> a, const Geometry g) {
   using R = typename Storage<S>::Real;
   using R4 = Four<R>;
@@ -1084,7 +1115,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
     view[n] = a.src + ((int64_t)t.b * N + (n < N ? n : 0)) * srcH * srcW * C;  // (uniform)
   const int row_step = srcW * C;
 
-  R tap[NT][4][VEC];
+  constexpr bool kRaw = is_half<S>() && REDUCE == 0 && !LIT;
+  Taps<S, VEC, kRaw> tap[NT];
   int cur[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) cur[n] = -1;
@@ -1162,7 +1194,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         constexpr int kMany = kOneSet ? 0 : 1;
-        R(&tp)[4][VEC] = tap[n * kMany];
+        Taps<S, VEC, kRaw> &tp = tap[n * kMany];
         int &cur1 = cur[n * kMany];
         if constexpr (kOneSet) cur1 = -1;
         R own[VEC];  // LPP == 1: this lane holds the whole pixel
@@ -1194,7 +1226,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const R smp = wt.x * tp[0][c] + wt.y * tp[1][c] + wt.z * tp[2][c] + wt.w * tp[3][c];
+              const R smp = wt.x * tp(0, c) + wt.y * tp(1, c) + wt.z * tp(2, c) + wt.w * tp(3, c);
               const R diff = smp - ref[c];
               sq[c] = diff * diff;
             }
@@ -1268,7 +1300,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
-              smp[c] = wt.x * tap[0][0][c] + wt.y * tap[0][1][c] + wt.z * tap[0][2][c] + wt.w * tap[0][3][c];
+              smp[c] = wt.x * tap[0](0, c) + wt.y * tap[0](1, c) + wt.z * tap[0](2, c) + wt.w * tap[0](3, c);
           }
           if (t.pix_ok && ch_ok)
             store_row<S, VEC, kNtRows, kAsk, GAP>(a.cost + ((t.pix * D + d0 + jj) * N + n) * C + ch0, smp, stream_halves);
@@ -1293,9 +1325,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
       // Two views side by side where the registers hold two sets of taps: their gathers are in flight
       // together, and what these kernels do most is wait for them (six wide-baseline views, VALU 45 %, waiting
       // 75 % of the waves' time: 4.6 -> 4.3 ms; 200 x 260 x 96 477 -> 435 us, five views, 128 x 160 x 48, 85.7 ->
-      // 80.9; 16 channels, six views, 148 -> 128, four 108 -> 103; minima 2-4 %).  Not with 16-bit taps, which
-      // are widened, and so waited for, as soon as they are loaded (five views 94 -> 96), nor in double.
-      constexpr int VW = sizeof(S) == 4 && NV % 2 == 0 && LPP >= 4 ? 2 : 1;
+      // 80.9; 16 channels, six views, 148 -> 128, four 108 -> 103; minima 2-4 %; f16, five
+      // views, 94 -> 88).  Not with taps that are widened, and so waited for, as soon as they are loaded (five
+      // views 94 -> 96), nor in double.
+      constexpr int VW = (sizeof(S) == 4 || kRaw) && NV % 2 == 0 && LPP >= 4 ? 2 : 1;
       static_assert(NV % VW == 0, "whole groups of views");
 #pragma unroll
       for (int j0 = 0; j0 < LPP; j0 += DB) {
@@ -1314,7 +1347,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
       for (int n = 0; n < NV; n += VW) {
         int cur1[VW];
-        R tp[VW][4][VEC];
+        Taps<S, VEC, kRaw> tp[VW];
 #pragma unroll
         for (int v = 0; v < VW; ++v) cur1[v] = -1;
 #pragma unroll
@@ -1346,7 +1379,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             R val[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const R smp = wt[v].x * tp[v][0][c] + wt[v].y * tp[v][1][c] + wt[v].z * tp[v][2][c] + wt[v].w * tp[v][3][c];
+              const R smp = wt[v].x * tp[v](0, c) + wt[v].y * tp[v](1, c) + wt[v].z * tp[v](2, c) + wt[v].w * tp[v](3, c);
               if (CORR == 0) {
                 const R diff = smp - ref[c];
                 val[c] = diff * diff;
@@ -1370,16 +1403,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
               if (CORR != 1) {
-                R diff = mad(wt[v].x, tp[v][0][c], -ref[c]);
-                diff = mad(wt[v].y, tp[v][1][c], diff);
-                diff = mad(wt[v].z, tp[v][2][c], diff);
-                diff = mad(wt[v].w, tp[v][3][c], diff);
+                R diff = mad(wt[v].x, tp[v](0, c), -ref[c]);
+                diff = mad(wt[v].y, tp[v](1, c), diff);
+                diff = mad(wt[v].z, tp[v](2, c), diff);
+                diff = mad(wt[v].w, tp[v](3, c), diff);
                 acc[jj][c] = mad(diff, diff, acc[jj][c]);
               } else {
-                R smp = wt[v].x * tp[v][0][c];
-                smp = mad(wt[v].y, tp[v][1][c], smp);
-                smp = mad(wt[v].z, tp[v][2][c], smp);
-                smp = mad(wt[v].w, tp[v][3][c], smp);
+                R smp = kRaw ? mad(wt[v].x, tp[v](0, c), R(0)) : wt[v].x * tp[v](0, c);
+                smp = mad(wt[v].y, tp[v](1, c), smp);
+                smp = mad(wt[v].z, tp[v](2, c), smp);
+                smp = mad(wt[v].w, tp[v](3, c), smp);
                 acc[jj][c] = mad(smp, ref[c], acc[jj][c]);
               }
             }
@@ -1474,8 +1507,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             R smp[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
-              smp[c] = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
-                       wt.w * tap[n][3][c];
+              smp[c] = wt.x * tap[n](0, c) + wt.y * tap[n](1, c) + wt.z * tap[n](2, c) +
+                       wt.w * tap[n](3, c);
             const R *ref_row = reinterpret_cast<const R *>(smem + kRec) + t.p * (VEC * LPP);
             R best;
             int code;
@@ -1506,8 +1539,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             }
 #pragma unroll
             for (int c = 0; c < VEC; ++c)
-              smp[c] = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
-                       wt.w * tap[n][3][c];
+              smp[c] = wt.x * tap[n](0, c) + wt.y * tap[n](1, c) + wt.z * tap[n](2, c) +
+                       wt.w * tap[n](3, c);
           }
           if (n < N && t.pix_ok && ch_ok)
             store_row<S, VEC, kNtRows, kAsk, GAP>(a.cost + ((t.pix * D + d) * N + n) * C + ch0, smp, stream_halves);
@@ -1522,8 +1555,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
             R val[VEC];
 #pragma unroll
             for (int c = 0; c < VEC; ++c) {
-              const R smp = wt.x * tap[n][0][c] + wt.y * tap[n][1][c] + wt.z * tap[n][2][c] +
-                            wt.w * tap[n][3][c];
+              const R smp = wt.x * tap[n](0, c) + wt.y * tap[n](1, c) + wt.z * tap[n](2, c) +
+                            wt.w * tap[n](3, c);
               if (CORR != 1) {
                 const R diff = smp - ref[c];
                 val[c] = diff * diff;
@@ -1550,16 +1583,16 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           for (int c = 0; c < VEC; ++c) {
             if (CORR != 1) {
               // sample - ref as one chain of fused multiply-adds
-              R diff = mad(wt.x, tap[n][0][c], -ref[c]);
-              diff = mad(wt.y, tap[n][1][c], diff);
-              diff = mad(wt.z, tap[n][2][c], diff);
-              diff = mad(wt.w, tap[n][3][c], diff);
+              R diff = mad(wt.x, tap[n](0, c), -ref[c]);
+              diff = mad(wt.y, tap[n](1, c), diff);
+              diff = mad(wt.z, tap[n](2, c), diff);
+              diff = mad(wt.w, tap[n](3, c), diff);
               acc[c] = mad(diff, diff, acc[c]);
             } else {
-              R smp = wt.x * tap[n][0][c];
-              smp = mad(wt.y, tap[n][1][c], smp);
-              smp = mad(wt.z, tap[n][2][c], smp);
-              smp = mad(wt.w, tap[n][3][c], smp);
+              R smp = kRaw ? mad(wt.x, tap[n](0, c), R(0)) : wt.x * tap[n](0, c);
+              smp = mad(wt.y, tap[n](1, c), smp);
+              smp = mad(wt.z, tap[n](2, c), smp);
+              smp = mad(wt.w, tap[n](3, c), smp);
               acc[c] = mad(smp, ref[c], acc[c]);
             }
           }
@@ -2399,7 +2432,8 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     gview[n] = src_grad_img + vo;
     oy[n] = ox[n] = WN::kNone;
   }
-  R tap[NV][4][VEC];
+  constexpr bool kRaw = is_half<S>();
+  Taps<S, VEC, kRaw> tap[NV];
   Sums sg[NV][NS];
   R proj[NV][4][kRunSums && DG ? GV : 1];  // kRunSums: the taps of the open run against the reference, per group
   int cur[NV];     // tap offset of the open run, -1: none
@@ -2418,9 +2452,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
     if constexpr (kRunSums) {
 #pragma unroll
       for (int c = 0; c < VEC; ++c) {
-        R run = tap[n][0][c] * sg[n][c * NS / VEC][0];  // (summed by itself: one rounding per run in racc)
+        R run = kRaw ? mad(tap[n](0, c), sg[n][c * NS / VEC][0], R(0)) : tap[n](0, c) * sg[n][c * NS / VEC][0];  // (summed by itself: one rounding per run in racc)
 #pragma unroll
-        for (int k = 1; k < 4; ++k) run = mad(tap[n][k][c], sg[n][c * NS / VEC][k], run);
+        for (int k = 1; k < 4; ++k) run = mad(tap[n](k, c), sg[n][c * NS / VEC][k], run);
         racc[c] += run;
       }
     }
@@ -2823,7 +2857,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             for (int c = 0; c < GV; ++c) cg[c] = raw[c];
           } else {
 #pragma unroll
-            for (int c = 0; c < GV; ++c) cg[c] = raw[c] * scl;
+            for (int c = 0; c < GV; ++c) cg[c] = kRaw && CORR == 0 ? mad(raw[c], scl, R(0)) : raw[c] * scl;
           }
           if constexpr (kMaskRows && !kWonMasks) {
             // only the channels (groups) this view won contribute
@@ -2871,9 +2905,9 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
 #pragma unroll
                   for (int i = 0; i < GV; ++i) {
                     constexpr int SUB = VEC / GV;
-                    R sum = ref[i * SUB] * tap[n][k][i * SUB];
+                    R sum = kRaw ? mad(ref[i * SUB], tap[n](k, i * SUB), R(0)) : ref[i * SUB] * tap[n](k, i * SUB);
 #pragma unroll
-                    for (int c = 1; c < SUB; ++c) sum = mad(ref[i * SUB + c], tap[n][k][i * SUB + c], sum);
+                    for (int c = 1; c < SUB; ++c) sum = mad(ref[i * SUB + c], tap[n](k, i * SUB + c), sum);
                     proj[n][k][i] = sum;
                   }
               }
@@ -2898,10 +2932,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
             if constexpr (best_pair_op(CORR)) {
               const int pair = REDUCE ? lds_at<int>(smem, p4, kDst + (jj * PPW) * 4) : 0;
               if (g.sub == kWideSub)
-                v3_pair_gradients<R, VEC, LPP, kWideSub, REDUCE>(wt, tap[n], ends, scl, pair, s_v3, t.p,
+                v3_pair_gradients<R, VEC, LPP, kWideSub, REDUCE>(wt, tap[n].v, ends, scl, pair, s_v3, t.p,
                                                                  t.cl, racc, gs3);
               else
-                v3_pair_gradients<R, VEC, LPP, kWideSub / 2, REDUCE>(wt, tap[n], ends, scl, pair, s_v3, t.p,
+                v3_pair_gradients<R, VEC, LPP, kWideSub / 2, REDUCE>(wt, tap[n].v, ends, scl, pair, s_v3, t.p,
                                                                      t.cl, racc, gs3);
             }
 #pragma unroll
@@ -2914,18 +2948,18 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
               } else if (CORR != 1) {
                 // (double: the sample first, then the difference: sums of the sample's parts are the
                 // smaller numbers to round, and the lane-per-channel kernels have it so)
-                R diff = kDouble ? wt.x * tap[n][0][c] : mad(wt.x, tap[n][0][c], -ref[c]);
-                diff = mad(wt.y, tap[n][1][c], diff);
-                diff = mad(wt.z, tap[n][2][c], diff);
-                diff = mad(wt.w, tap[n][3][c], diff);
+                R diff = kDouble ? wt.x * tap[n](0, c) : mad(wt.x, tap[n](0, c), -ref[c]);
+                diff = mad(wt.y, tap[n](1, c), diff);
+                diff = mad(wt.z, tap[n](2, c), diff);
+                diff = mad(wt.w, tap[n](3, c), diff);
                 if constexpr (kDouble) diff -= ref[c];
                 gsrc = diff * cg[c * GV / VEC];
                 racc[c] -= gsrc;
               } else {
-                R smp = wt.x * tap[n][0][c];
-                smp = mad(wt.y, tap[n][1][c], smp);
-                smp = mad(wt.z, tap[n][2][c], smp);
-                smp = mad(wt.w, tap[n][3][c], smp);
+                R smp = kRaw ? mad(wt.x, tap[n](0, c), R(0)) : wt.x * tap[n](0, c);
+                smp = mad(wt.y, tap[n](1, c), smp);
+                smp = mad(wt.z, tap[n](2, c), smp);
+                smp = mad(wt.w, tap[n](3, c), smp);
                 racc[c] = mad(cg[c * GV / VEC], smp, racc[c]);
                 gsrc = cg[c * GV / VEC] * ref[c];
               }
@@ -2939,10 +2973,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
                 sg[n][c][3] = mad(gsrc, wt.w, sg[n][c][3]);
               }
               if constexpr (DG) {
-                R ds = dwt.x * tap[n][0][c];
-                ds = mad(dwt.y, tap[n][1][c], ds);
-                ds = mad(dwt.z, tap[n][2][c], ds);
-                ds = mad(dwt.w, tap[n][3][c], ds);
+                R ds = kRaw ? mad(dwt.x, tap[n](0, c), R(0)) : dwt.x * tap[n](0, c);
+                ds = mad(dwt.y, tap[n](1, c), ds);
+                ds = mad(dwt.z, tap[n](2, c), ds);
+                ds = mad(dwt.w, tap[n](3, c), ds);
                 dvox = mad(gsrc, ds, dvox);
               }
             }
