@@ -2182,8 +2182,12 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // float): 24 channels, six wide-baseline views, 200 x 260 x 64, 1075 -> 908 us; 32 channels, x 96, 1457 -> 1320, two
 // views, 128 x 160 x 96, 208 -> 206; 16 channels, three views, x 48, 282 -> 268, bf16, four, 221 -> 207.  The
 // wait for the winners costs up to 6 % where three waves per SIMD hold the whole launch: those keep the
-// other form (the launcher).  Not CostVolumeV3 (its two extra LDS rows per pixel are 2 KB), nor the
-// maximum of 8 channels whose views take turns (52-80 bytes of scratch).
+// other form (the launcher).  Not the maximum of 8 channels whose views take turns (52-80 bytes of scratch).
+// CostVolumeV3 with groups of four and eight likewise, and since its rows of reference and sample are 2 KB of
+// LDS more, with a window of four rows (four_row_pairs): 10.1 instead of 14.3 KB and four waves instead of
+// 2.75 per SIMD (32 channels in four groups, two views, 120 x 152 x 64, 188 -> 162 us; five views, x 48, 317
+// -> 238; in double, 100 x 130 x 32, 171 -> 141; 16 channels 109 -> 96).  Narrower groups need 143 registers:
+// slimmed at three waves with the six-row window (12.2 KB: 237 -> 197 us for groups of two).
 // Four lanes per pixel (16 channels), gradients of a mean: 130 registers left alone, 121 lean
 // (held to 128 without the slimming they spilled three to five); the window of the 4 x 4 pixel
 // tile is 4 KB.  CostAggregate and FeatureAggregate the same (134 -> 117-120; six views, 497 x 700 x 41:
@@ -2212,15 +2216,16 @@ constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = 
                              bool wide_real = false, int gv = 4) {
   return wide_real ||
          (nv == 1 && !wide &&
-          (lpp == 16 || (lpp == 8 && (corr == 0 || corr == 2 || corr == 4)) ||
-           (lpp == 4 && (corr <= 2 || corr == 4)) || (lpp == 2 && (corr == 0 || (corr == 1 && reduce == 0))) ||
+          (lpp == 16 || (lpp == 8 && corr != 1) ||
+           (lpp == 4 && corr <= 4) || (lpp == 2 && (corr == 0 || (corr == 1 && reduce == 0))) ||
            (corr == 1 && run_sums(lpp, reduce, gv) && lpp >= 4)));
 }
+constexpr bool four_row_pairs(int corr, bool wide_real) { return corr == 3 || (corr == 5 && wide_real); }
 // 32 channels: the gradients that have kernels for either window (six rows and eight).
 constexpr bool two_windows(int corr, int reduce) { return (corr == 0 && reduce == 0) || corr == 2 || corr == 4; }
 constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false,
                              bool wide_real = false, int gv = 4) {
-  return wide_real ? (slim_double(lpp, corr) ? 3 : 2) : lpp == 16 && nv == 1                             ? 3
+  return wide_real ? (slim_double(lpp, corr) ? 3 : 2) : (lpp == 16 || corr == 5) && nv == 1               ? 3
          : lean_backward(nv, lpp, corr, reduce, wide, false, gv) ? 4
          : nv == 1 && lpp <= 8                       ? 3
          : nv <= 2                                   ? 2
@@ -2276,7 +2281,10 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
   constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, kDouble, GV);
   constexpr bool kSlim = kDouble && slim_double(LPP, CORR);
-  constexpr int kForm = !(kLean && LPP == 8) ? kPlainWindow : kSlim ? kFourRows : EIGHT == kEightTall ? kSixColumns : kSixRows;
+  constexpr int kForm = !(kLean && LPP == 8)                       ? kPlainWindow
+                        : kSlim || four_row_pairs(CORR, kDouble) ? kFourRows
+                        : EIGHT == kEightTall                      ? kSixColumns
+                                                                   : kSixRows;
   using WN = Window<VEC, LPP, kForm>;
   constexpr int PPW = 64 / LPP;
   constexpr bool kWide = sizeof(S) == 2;  // gradients accumulate in fp32 images
