@@ -1330,6 +1330,10 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
       // views 94 -> 96), nor in double.
       constexpr int VW = (sizeof(S) == 4 || kRaw) && NV % 2 == 0 && LPP >= 4 ? 2 : 1;
       static_assert(NV % VW == 0, "whole groups of views");
+      // One view at a time: its arithmetic in the branch that fetched its taps, not in a second one (bf16 groups
+      // of four, 64 channels, six views, 63 x 82 x 10, four images: 76 -> 63 us; mean 126 -> 120).  Double is
+      // faster with two branches (32 channels, four views, 120 x 160 x 48: 125 against 128; samples 362, 368).
+      constexpr bool kOneBranch = VW == 1 && sizeof(R) == 4;
 #pragma unroll
       for (int j0 = 0; j0 < LPP; j0 += DB) {
       R acc[DB][VEC];
@@ -1355,13 +1359,7 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
           if (d0 + j0 + jj >= d_hi) continue;
           int off[VW];  // -1 also for a view beyond N (phase 1 leaves those records empty)
           R4 wt[VW];
-#pragma unroll
-          for (int v = 0; v < VW; ++v) {
-            if constexpr (LPP > 1)
-              off[v] = lds_at<int>(smem, p4, kOff + (((n + v) * LPP + j0 + jj) * PPW) * 4);
-            else
-              off[v] = r_off[n + v];
-            if (off[v] < 0) continue;
+          auto fetch = [&](int v) __attribute__((always_inline)) {
             if constexpr (LPP > 1)
               wt[v] = lds_at<R4>(smem, p4 * kR4, kWts + (((n + v) * LPP + j0 + jj) * PPW) * (int)sizeof(R4));
             else
@@ -1370,10 +1368,8 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               cur1[v] = off[v];
               load_cell<S, VEC, GAP, kUnit>(view[n + v], off[v], C, row_step, (unsigned)ch0, tp[v]);
             }
-          }
-#pragma unroll
-          for (int v = 0; v < VW; ++v) {
-          if (off[v] < 0) continue;
+          };
+          auto add = [&](int v) __attribute__((always_inline)) {
           ++kcnt[jj];
           if constexpr (REDUCE == 1 || LIT) {
             R val[VEC];
@@ -1417,6 +1413,21 @@ __attribute__((amdgpu_waves_per_eu(forward_min_waves(LPP, NV, CORR, REDUCE, size
               }
             }
           }
+          };
+#pragma unroll
+          for (int v = 0; v < VW; ++v) {
+            if constexpr (LPP > 1)
+              off[v] = lds_at<int>(smem, p4, kOff + (((n + v) * LPP + j0 + jj) * PPW) * 4);
+            else
+              off[v] = r_off[n + v];
+            if (off[v] < 0) continue;
+            fetch(v);
+            if constexpr (kOneBranch) add(v);
+          }
+          if constexpr (!kOneBranch) {
+#pragma unroll
+            for (int v = 0; v < VW; ++v)
+              if (off[v] >= 0) add(v);
           }
         }
       }
@@ -2211,7 +2222,9 @@ __device__ __forceinline__ void flush_cells_to_memory(unsigned long long m, bool
 // either form to seven workgroups, 364 against 275 us (630); one lane per pixel has no records in LDS.
 // (tap sums per group instead of per channel, see backward_kernel's GV)
 constexpr bool run_sums(int lpp, int reduce, int gv) { return gv < 4 && (lpp != 2 || reduce != 0); }
-constexpr bool slim_double(int lpp, int corr) { return corr == 2 && lpp > 1 && lpp <= 8; }
+// The minimum of 8 channels: the third wave spills 28 bytes, two do not (one view, 173 x 194 x 91, 97 -> 87 us; two
+// views, 40 x 60 x 30, four images, 29 -> 25.5); the mean is faster with it (two views, 136 against 148).
+constexpr bool slim_double(int lpp, int corr, int reduce) { return corr == 2 && lpp > (reduce == 0 ? 1 : 2) && lpp <= 8; }
 constexpr bool lean_backward(int nv, int lpp, int corr, int reduce, bool wide = false,
                              bool wide_real = false, int gv = 4) {
   return wide_real ||
@@ -2225,7 +2238,7 @@ constexpr bool four_row_pairs(int corr, bool wide_real) { return corr == 3 || (c
 constexpr bool two_windows(int corr, int reduce) { return (corr == 0 && reduce == 0) || corr == 2 || corr == 4; }
 constexpr int backward_waves(int nv, int lpp, int corr = 0, int reduce = 1, bool wide = false,
                              bool wide_real = false, int gv = 4) {
-  return wide_real ? (slim_double(lpp, corr) ? 3 : 2) : (lpp == 16 || corr == 5) && nv == 1               ? 3
+  return wide_real ? (slim_double(lpp, corr, reduce) ? 3 : 2) : (lpp == 16 || corr == 5) && nv == 1               ? 3
          : lean_backward(nv, lpp, corr, reduce, wide, false, gv) ? 4
          : nv == 1 && lpp <= 8                       ? 3
          : nv <= 2                                   ? 2
@@ -2280,7 +2293,7 @@ __global__ __launch_bounds__(64, backward_waves(NV, LPP, CORR, REDUCE, EIGHT == 
   constexpr bool kDouble = sizeof(S) == 8;
   constexpr int GAP = lane_gap(LPP, CORR, (int)sizeof(S), PAD);
   constexpr bool kLean = lean_backward(NV, LPP, CORR, REDUCE, EIGHT == kEightWide, kDouble, GV);
-  constexpr bool kSlim = kDouble && slim_double(LPP, CORR);
+  constexpr bool kSlim = kDouble && slim_double(LPP, CORR, REDUCE);
   constexpr int kForm = !(kLean && LPP == 8)                       ? kPlainWindow
                         : kSlim || four_row_pairs(CORR, kDouble) ? kFourRows
                         : EIGHT == kEightTall                      ? kSixColumns
